@@ -154,6 +154,7 @@ void kc_swiglu_pack(kc_stream_t s, const float* g, const float* u, uint16_t* y, 
 int kc_mv_pack(kc_stream_t s, int fmt, WSlice w, int K, int R, const float* x, int xs, float* y, int ys, int T, uint16_t* px);
 void kq4_route_bucket(kc_stream_t s, const Qwen4Cfg* c, const float* logits, int32_t* ind, float* wt, int T, int32_t* perm,
                       MmTile* tiles, int32_t* ntiles);
+/* (ours: shared, and sh of the next, may be NULL - no shared expert, zeros that are not read) */
 void kc_moe_combine(kc_stream_t s, const float* D, const float* w, const float* shared, float* x, int d, int k, int T);
 /* engine/kernels_qwen4.h:71, engine/kernels_qwen4.cu:514-516 */
 void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* wt, const float* sh, const float* sg,

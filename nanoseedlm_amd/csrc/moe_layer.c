@@ -399,8 +399,8 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
             kc_mm_grouped_dev(s, c->fmt, down, ff, d, m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
         }
     }
-    if (c->router == NSLM_ROUTE_SOFTMAX) kq4_moe_combine(s, d, k, m->D, m->wt, m->zero, m->zero, 0, io, T);
-    else kc_moe_combine(s, m->D, m->wt, m->zero, io, d, k, T);
+    if (c->router == NSLM_ROUTE_SOFTMAX) kq4_moe_combine(s, d, k, m->D, m->wt, NULL, m->zero, 0, io, T);
+    else kc_moe_combine(s, m->D, m->wt, NULL, io, d, k, T);
     return kc_last_error() ? -1 : 0;
 }
 

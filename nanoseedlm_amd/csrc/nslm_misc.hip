@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(256) k_router_logits(RouterArgs a, const uint1
     const uint16_t* wr = W + (size_t) e * a.d;
     const bool vec = a.d % 8 == 0 && (((uintptr_t) W | (uintptr_t) x) & 15u) == 0;
     const float be = bf(bias[e]);
-    for (int t0 = 0; t0 < T; t0 += RL_TOK) {
+    for (int t0 = RL_TOK * (int) blockIdx.y; t0 < T; t0 += RL_TOK * (int) gridDim.y) {
         const int nt = min(RL_TOK, T - t0);
         float lo[RL_TOK], hi[RL_TOK];
 #pragma unroll
@@ -69,6 +69,79 @@ __global__ void __launch_bounds__(256) k_router_logits(RouterArgs a, const uint1
                 score[(size_t) (t0 + u) * a.n + e] = sg;
                 selout[(size_t) (t0 + u) * a.n + e] = sg + be;
             }
+        }
+    }
+}
+
+// Many tokens: the same logits, bit for bit (the lane's chain of multiply-adds over its 8-value pieces, then the wave's xor tree),
+// with the activations of RM_TOK tokens staged in LDS once for RM_EXP experts, so that a weight piece a wave reads serves RM_TOK tokens and
+// a token's row is read once a workgroup.  (The kernel above walks all tokens with a wave an expert: 64 experts are 16 workgroups,
+// 1218 us at 512 tokens of 2048, where this launch has 256 workgroups.)  A wave takes two experts at a time and sums all its
+// 2 RM_TOK x 2 partial sums in one folding tree: at each level a lane hands half of its values to its partner and adds the other
+// half - the additions of the xor tree, without forming every sum in every lane (33 exchanges instead of 192).
+#define RM_TOK 8
+#define RM_EXP 16
+__global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const uint16_t* W, const uint16_t* bias, const float* x, int T,
+                                                            float* score, float* selout) {
+    extern __shared__ __attribute__((aligned(16))) float xs[];   // [RM_TOK][2][d / 8][4]: a piece's first and last four values apart
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, np = a.d / 8, t0 = (int) blockIdx.x * RM_TOK;
+    for (int i = tid; i < RM_TOK * np * 2; i += 256) {
+        const int t = i / (2 * np), q = i - t * 2 * np;   // 16-byte unit q of token t's row
+        const float4 v = *(const float4*) (x + (size_t) min(t0 + t, T - 1) * a.d + 4 * (size_t) q);
+        *(float4*) &xs[((size_t) (t * 2 + (q & 1)) * np + (q >> 1)) * 4] = v;
+    }
+    __syncthreads();
+    for (int e0 = (int) blockIdx.y * RM_EXP + 2 * wv; e0 < min(a.n, ((int) blockIdx.y + 1) * RM_EXP); e0 += 8) {
+        const int e1 = min(e0 + 1, a.n - 1);
+        float lo[2][RM_TOK], hi[2][RM_TOK];
+#pragma unroll
+        for (int u = 0; u < RM_TOK; ++u) lo[0][u] = lo[1][u] = hi[0][u] = hi[1][u] = 0.0f;
+        for (int c = lane; c < np; c += 64) {
+            const uint4 q[2] = {*(const uint4*) (W + (size_t) e0 * a.d + 8 * (size_t) c), *(const uint4*) (W + (size_t) e1 * a.d + 8 * (size_t) c)};
+            float w[2][8];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                w[h][0] = bf(q[h].x & 0xFFFFu); w[h][1] = bf(q[h].x >> 16); w[h][2] = bf(q[h].y & 0xFFFFu); w[h][3] = bf(q[h].y >> 16);
+                w[h][4] = bf(q[h].z & 0xFFFFu); w[h][5] = bf(q[h].z >> 16); w[h][6] = bf(q[h].w & 0xFFFFu); w[h][7] = bf(q[h].w >> 16);
+            }
+            const bool low = 8 * c < a.hw;   // (hw in whole pieces)
+#pragma unroll
+            for (int u = 0; u < RM_TOK; ++u) {
+                const float4 x0 = *(const float4*) &xs[((size_t) (u * 2) * np + c) * 4], x1 = *(const float4*) &xs[((size_t) (u * 2 + 1) * np + c) * 4];
+                const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    float s = low ? lo[h][u] : hi[h][u];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) s = fmaf(w[h][i], xv[i], s);
+                    lo[h][u] = low ? s : lo[h][u];
+                    hi[h][u] = low ? hi[h][u] : s;
+                }
+            }
+        }
+        // value index v = (token, expert half, partition); after the level with stride o a lane holds the half of the values that its bit o picks
+        float v[4 * RM_TOK];
+#pragma unroll
+        for (int u = 0; u < RM_TOK; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) { v[4 * u + 2 * h] = lo[h][u]; v[4 * u + 2 * h + 1] = hi[h][u]; }
+#pragma unroll
+        for (int lv = 0; lv < 5; ++lv) {
+            const int o = 32 >> lv, n = (4 * RM_TOK) >> (lv + 1);   // n values stay
+            const bool up = (lane & o) != 0;
+#pragma unroll
+            for (int i = 0; i < n; ++i) {
+                const float give = up ? v[i] : v[i + n], keep = up ? v[i + n] : v[i];
+                v[i] = keep + __shfl_xor(give, o);
+            }
+        }
+        const float sum = v[0] + __shfl_xor(v[0], 1);          // lane: value index = lane >> 1
+        const float other = __shfl_xor(sum, 2);                // the other partition's sum
+        const int u = lane >> 3, h = (lane >> 2) & 1, e = h ? e0 + 1 : e0;
+        if ((lane & 3) == 0 && t0 + u < T && e < a.n) {
+            const float sg = 1.0f / (1.0f + expf(-(bfr(sum) + bfr(other))));
+            score[(size_t) (t0 + u) * a.n + e] = sg;
+            selout[(size_t) (t0 + u) * a.n + e] = sg + bf(bias[e]);
         }
     }
 }
@@ -168,21 +241,50 @@ __global__ void k_swiglu_pack(const float* g, const float* u, uint16_t* y, size_
                                  pack_bf2(bfr(silu_bf(g1.z) * u1.z), bfr(silu_bf(g1.w) * u1.w)));
 }
 // x[t][c] = bf16(x + bf16(bf16(sum_j bf16(D[t,j][c] * bf16(w[t,j]))) + shared[t][c]))
-__global__ void k_moe_combine(const float* D, const float* w, const float* shared, float* x, int d, int k) {
-    const int c = (int) (blockIdx.x * blockDim.x + threadIdx.x), t = (int) blockIdx.y;
-    if (c >= d) return;
-    float s = 0.0f;
-    for (int j = 0; j < k; ++j) s += bfr(D[((size_t) t * k + j) * d + c] * bfr(w[t * k + j]));
-    const size_t i = (size_t) t * d + c;
-    x[i] = bfr(x[i] + bfr(bfr(s) + shared[i]));
-}
 // out[t][i] = sigmoid(sg[t * sgld]) * sh[t][i] + sum_j wt[t][j] D[t,j][i], all f32
-__global__ void k_q4_moe_combine(int d, int k, const float* D, const float* wt, const float* sh, const float* sg, int sgld, float* out) {
-    const int i = (int) (blockIdx.x * blockDim.x + threadIdx.x), t = (int) blockIdx.y;
-    if (i >= d) return;
-    float acc = (1.0f / (1.0f + expf(-sg[(size_t) t * sgld]))) * sh[(size_t) t * d + i];
-    for (int j = 0; j < k; ++j) acc = fmaf(wt[t * k + j], D[((size_t) t * k + j) * d + i], acc);
-    out[(size_t) t * d + i] = acc;
+// Bound by the reads of D (k rows of d a token).  V = 4: a thread takes four columns, all its rows' 16-byte loads requested before the
+// first is added (a column a thread, each load behind the last add: 45 us at 2048 tokens, top-8, d = 2048; now 30, where
+// 150 MB at a large copy's rate are 29).  Q4 = false: the first form, with sh = shared, io = x.  sh NULL: zeros, not read.
+template <int V, bool Q4>
+__global__ void __launch_bounds__(256) k_combine(const float* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k) {
+    const int c = V * (int) (blockIdx.x * blockDim.x + threadIdx.x), t = (int) blockIdx.y;
+    if (c >= d) return;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const size_t at = (size_t) t * d + c;
+    const float* Dt = D + (size_t) t * k * d + c;
+    vec s = {}, h = {}, x = {};
+    if (sh) h = *(const vec*) (sh + at);
+    if (!Q4) x = *(const vec*) (io + at);
+    if (Q4) {
+        const float gate = 1.0f / (1.0f + expf(-sg[(size_t) t * sgld]));
+#pragma unroll
+        for (int i = 0; i < V; ++i) s[i] = gate * h[i];
+    }
+    for (int j0 = 0; j0 < k; j0 += 8) {
+        vec v[8];
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {   // (clamped: the loads stay unconditional)
+            v[j] = *(const vec*) (Dt + (size_t) min(j0 + j, k - 1) * d);
+            w[j] = wt[t * k + min(j0 + j, k - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j0 + j >= k) break;
+#pragma unroll
+            for (int i = 0; i < V; ++i) s[i] = Q4 ? fmaf(w[j], v[j][i], s[i]) : s[i] + bfr(v[j][i] * bfr(w[j]));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) x[i] = Q4 ? s[i] : bfr(x[i] + bfr(bfr(s[i]) + h[i]));
+    *(vec*) (io + at) = x;
+}
+template <bool Q4>
+void combine(hipStream_t st, const float* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, int T) {
+    if (d % 4 == 0 && (((uintptr_t) D | (uintptr_t) sh | (uintptr_t) io) & 15u) == 0)
+        hipLaunchKernelGGL((k_combine<4, Q4>), dim3((unsigned) (d / 4 + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
+    else
+        hipLaunchKernelGGL((k_combine<1, Q4>), dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
 }
 __global__ void k_pack_input_bf16(const float* x, uint16_t* y, size_t n) {
     const size_t b = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -558,7 +660,17 @@ void kc_router_topk(kc_stream_t s, RouterArgs a, const float* score, const float
 void kc_router(kc_stream_t s, RouterArgs a, const uint16_t* W, const uint16_t* bias, const float* x, float* score,
                float* sel, int32_t* inds, float* wts, int T) {
     if (T < 1) return;
-    hipLaunchKernelGGL(k_router_logits, dim3((unsigned) (a.n + 3) / 4), dim3(256), 0, (hipStream_t) s, a, W, bias, x, T, score, sel);
+    // From 16 tokens on, the tokens' rows staged in LDS (below, a wave an expert and four tokens fills a decode step's launch better);
+    // rows in whole 16-byte pieces, both partitions too, and RM_TOK of them within a workgroup's LDS.
+    if (T >= 16 && a.d % 8 == 0 && a.hw % 8 == 0 && a.d <= 4096 && (((uintptr_t) W | (uintptr_t) x) & 15u) == 0) {
+        static const hipError_t once = hipFuncSetAttribute((const void*) k_router_logits_many, hipFuncAttributeMaxDynamicSharedMemorySize, RM_TOK * 4096 * 4);
+        (void) once;
+        hipLaunchKernelGGL(k_router_logits_many, dim3((unsigned) (T + RM_TOK - 1) / RM_TOK, (unsigned) (a.n + RM_EXP - 1) / RM_EXP), dim3(256),
+                           (size_t) RM_TOK * a.d * sizeof(float), (hipStream_t) s, a, W, bias, x, T, score, sel);
+    } else {
+        hipLaunchKernelGGL(k_router_logits, dim3((unsigned) (a.n + 3) / 4, (unsigned) (T + RL_TOK - 1) / RL_TOK), dim3(256), 0, (hipStream_t) s, a, W,
+                           bias, x, T, score, sel);
+    }
     kc_router_topk(s, a, score, sel, inds, wts, T);
 }
 void kq4_route_ld(kc_stream_t s, const Qwen4Cfg* c, const float* logits, int ld, int32_t* ind, float* wt, int T) {
@@ -580,12 +692,12 @@ void kc_swiglu_pack(kc_stream_t s, const float* g, const float* u, uint16_t* y, 
 }
 void kc_moe_combine(kc_stream_t s, const float* D, const float* w, const float* shared, float* x, int d, int k, int T) {
     if (T < 1) return;
-    hipLaunchKernelGGL(k_moe_combine, dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, (hipStream_t) s, D, w, shared, x, d, k);
+    combine<false>((hipStream_t) s, D, w, shared, nullptr, 0, x, d, k, T);
 }
 void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* wt, const float* sh, const float* sg,
                      int sgld, float* out, int T) {
     if (T < 1) return;
-    hipLaunchKernelGGL(k_q4_moe_combine, dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, (hipStream_t) s, d, k, D, wt, sh, sg, sgld, out);
+    combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T);
 }
 void kc_pack_input_bf16(kc_stream_t s, const float* x, uint16_t* y, size_t n) {
     if (n < 8) return;

@@ -839,3 +839,31 @@ def test_grouped_launches_over_matrices_that_share_an_input(T):
     assert np.array_equal(got16.to_array(np.uint16, (T, R)), want16.to_array(np.uint16, (T, R)))
     for b in bufs + alone + [tab, px, y3, perm, tiles, nt, want16, got16, perm1, tile1, nt1]:
         b.free()
+
+
+@pytest.mark.parametrize("T,n,d", [(16, 17, 512), (33, 64, 2048), (70, 6, 1040)])
+def test_router_of_many_tokens_equals_runs_of_few(be, T, n, d):
+    """kc_router from 16 tokens on (the tokens' rows staged in LDS for 16 experts) gives every token the selection and the weights
+    of a call of a few tokens, bit for bit: token counts, expert counts and row lengths that leave partial workgroups."""
+    rng = np.random.default_rng(T + n)
+    W = packs.f32_to_bf16_bits((rng.standard_normal((n, d)) * 0.05).astype(np.float32))
+    bias = packs.f32_to_bf16_bits((rng.standard_normal(n) * 0.01).astype(np.float32))
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    k = min(4, n)
+    ind, wt = be.kt_router(W, bias, x, k, d // 2, 1.0)
+    for t0 in range(0, T, 7):
+        i1, w1 = be.kt_router(W, bias, x[t0:t0 + 7], k, d // 2, 1.0)
+        assert np.array_equal(ind[t0:t0 + 7], i1) and np.array_equal(wt[t0:t0 + 7].view(np.uint32), w1.view(np.uint32)), t0
+
+
+@pytest.mark.parametrize("d", [6, 132, 2048])
+@pytest.mark.parametrize("k", [1, 8, 11])
+def test_combine_widths(be, oracle, d, k):
+    """Both combines with four columns a thread (d % 4 == 0) and one, and more rows than one batch of loads holds."""
+    rng = np.random.default_rng(d + k)
+    T = 3
+    D, x, sh = (packs.round_bf16(rng.standard_normal(s).astype(np.float32)) for s in ((T * k, d), (T, d), (T, d)))
+    w, sg = rng.random((T, k)).astype(np.float32), rng.standard_normal((T, 1)).astype(np.float32)
+    assert np.array_equal(be.kt_combine(D, w, sh, x).view(np.uint32), oracle.moe_combine(D, w, sh, x).view(np.uint32))
+    ref = sh.astype(np.float64) / (1 + np.exp(-sg.astype(np.float64))) + (w[:, :, None].astype(np.float64) * D.reshape(T, k, d)).sum(1)
+    assert np.allclose(be.kt_q4_combine(D, w, sh, sg), ref, rtol=1e-5, atol=1e-5)
