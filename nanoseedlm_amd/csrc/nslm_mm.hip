@@ -10,28 +10,13 @@
 // accumulator columns are consecutive output addresses).  f32 accumulation.  In exact mode (kc_seed_gemm_f32) a seed
 // weight is carried as three BF16 terms hi + mid + lo whose sum is the f32 value, three MFMAs per step, as the reference.
 // Other formats (BF16, Q8, Q4) dequantize to BF16 values exactly and take the same path.
-#include <stdlib.h>
-
-#include <type_traits>
-
-#include "nslm_mv_dev.h"
+#include "nslm_mm_dev.h"
 
 using namespace nslm;
 
 namespace {
 
 int g_seed_exact = 0;   // kc_seed_gemm_f32
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-struct MmArgs {
-    int K, R, T, xs, ys, xdiv, add, f32out;
-    const WSlice* ws2;   // grouped launches of two matrices over the same tiles (grid.z = 2): the second slice table ..
-    float* y2;           // .. and its output
-    uint16_t* a16;       // non-null: a workgroup's 64 weight rows are 32 gate rows (ws) and the same 32 up rows (ws2), and what it
-                         // stores is their SwiGLU as BF16 bits [pair][ys] (the two GEMMs and the SwiGLU + pack pass in one launch)
-};
 
 // A workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every outstanding global load of the
 // wave, which would serialise the producers' prefetches (issued steps ahead on purpose) with each step.
@@ -79,6 +64,7 @@ __global__ void __launch_bounds__(512) k_mm(int fmt, MmArgs a, WSlice wd, const 
     WSlice wt;
     if (grouped) {
         const MmTile tl = tiles[blockIdx.y];
+        if (tl.count <= a.least) return;   // another launch's
         wt = ws[tl.slice];
         start = tl.start;
         count = tl.count;
@@ -310,14 +296,6 @@ __global__ void __launch_bounds__(512) k_mm(int fmt, MmArgs a, WSlice wd, const 
             }
 }
 
-// a kernel that asks for more dynamic LDS than the default limit has the limit raised to what it needs, once (the kernel is a
-// template argument so that every kernel has its own "once": kernels of one signature share a pointer type)
-template <auto K>
-void allow_big_lds(size_t bytes) {
-    static const hipError_t once = bytes > 48 * 1024 ? hipFuncSetAttribute((const void*) K, hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes)
-                                                     : hipSuccess;
-    (void) once;
-}
 template <int MT, int NTERM>
 constexpr size_t mm_lds() { return (size_t) (2 * NTERM * BM * LDW + 2 * 128 * MT * LDW) * sizeof(uint16_t); }
 
@@ -357,13 +335,6 @@ void launch_mm(hipStream_t st, int fmt, const MmArgs& a, WSlice wd, const WSlice
 #define XCHUNK 2048      // BF16 elements of an activation chunk: 32 tokens x 64 K
 #define RECD 4           // weight steps between a record's request and its decode
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
-    const f32x2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
-__device__ __forceinline__ int x_swizzle(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
 template <int N>
 __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -383,15 +354,6 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     WTile* Wsm = (WTile*) (smem + NCW * XCH * XCHUNK);          // [2]
     __shared__ int srow[BN], drow[BN];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
-    // FSYNC (one consumer wave: the grouped launches of a batched step, whose time is the decoders'): the weight tiles change hands
-    // by counters in LDS instead of a workgroup barrier a step.  A decoder waits only for the consumer to have read the tile it
-    // is about to overwrite (two steps back - it has, when the decode is what takes the time), never for the other decoders: with
-    // the barrier every step cost each decoder wave the wait for the slowest of the four (C2 at 32 rows: 271.2 -> 263.5 us, C3 at 16:
-    // 627 -> 609; with no hand-over at all and garbage computed: 247 and 540).  The dense 512-token GEMM with its eight consumer
-    // waves is indifferent to the barrier and keeps it.
-    constexpr bool FSYNC = NCW == 1;
-    constexpr int NWT = FSYNC && XCH == 2 ? 3 : 2;   // weight tiles in LDS: a third one where the activation ring leaves room for it
-    __shared__ __attribute__((aligned(16))) uint32_t flg[8];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wv >= NCW;
     const bool grouped = tiles != nullptr;
@@ -409,19 +371,8 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
         // (gate / up tiles: the decoder waves of the tile's upper 32 rows read the up slice)
         wt = gu && tid >= 64 * NCW + 128 ? a.ws2[tl.slice] : ws[tl.slice];
         start = tl.start;
-        count = min(tl.count, BN);   // (a tile never holds more than the launch was told: see mm_grouped)
-        if (BN < MMT_BN && tl.count > BN) {
-            // a broken promise is made visible: the pairs this launch cannot reach are stored as NaN, not left stale
-            const int rows = gu ? BM / 2 : BM;
-            for (int i = BN * rows + tid; i < tl.count * rows; i += NTHR) {
-                const int orow = r0 + i % rows;
-                const size_t at = (size_t) perm[tl.start + i / rows] * a.ys + orow;
-                if (orow < a.R) {
-                    if (gu) a.a16[at] = 0x7FC0u;
-                    else Y[at] = __uint_as_float(0x7FC00000u);
-                }
-            }
-        }
+        count = tl.count;
+        if (count <= a.least) return;   // another launch's
     } else {
         wt = wd;
         start = (int) blockIdx.y * BN;
@@ -429,56 +380,6 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     }
     if (count < 1) return;
     if (seedf) load_tables(tab);
-    if (FSYNC && tid < 8) flg[tid] = 0u;
-    // flg[w], w < 4: weight steps decoder wave w has written; flg[4]: steps the consumer has read.  (One word a decoder, not a sum:
-    // with two tiles a decoder may be a step ahead of another, and three waves a step ahead would make up for one a step behind.)
-    // The polls and the posts are a few instructions of inline code with registers of their own: written in the language (volatile
-    // reads in a loop, s_setprio builtins around it) they cost 20 registers and with them the fifth wave a SIMD, i.e. a resident
-    // workgroup - a quarter more time instead of less.  A poll is bounded; a waiting wave drops to priority 0, so its polls take
-    // only the issue slots nobody else wants.
-    auto wait_written = [&](uint32_t need) {   // all four decoders have written `need` steps; back at priority 3
-        uint32_t g0, g1, g2, g3, spins = 1u << 24;
-        asm volatile("s_setprio 0\n\t"
-                     "1:\n\t"
-                     "ds_read_b32 %0, %5\n\t"
-                     "ds_read_b32 %1, %5 offset:4\n\t"
-                     "ds_read_b32 %2, %5 offset:8\n\t"
-                     "ds_read_b32 %3, %5 offset:12\n\t"
-                     "s_waitcnt lgkmcnt(0)\n\t"
-                     "v_min3_u32 %0, %0, %1, %2\n\t"
-                     "v_min_u32 %0, %0, %3\n\t"
-                     "v_cmp_ge_u32 vcc, %0, %6\n\t"
-                     "s_cbranch_vccnz 2f\n\t"
-                     "s_sub_u32 %4, %4, 1\n\t"
-                     "s_cmp_lg_u32 %4, 0\n\t"
-                     "s_cbranch_scc1 1b\n\t"
-                     "2:\n\t"
-                     "s_setprio 3"
-                     : "=&v"(g0), "=&v"(g1), "=&v"(g2), "=&v"(g3), "+s"(spins)
-                     : "v"((uint32_t) (uintptr_t) &flg[0]), "v"(need)
-                     : "vcc", "scc", "memory");
-    };
-    auto wait_read = [&](uint32_t need) {   // the consumer has read `need` steps; back at priority 2
-        uint32_t got, spins = 1u << 24;
-        asm volatile("s_setprio 0\n\t"
-                     "1:\n\t"
-                     "ds_read_b32 %0, %2\n\t"
-                     "s_waitcnt lgkmcnt(0)\n\t"
-                     "v_cmp_ge_u32 vcc, %0, %3\n\t"
-                     "s_cbranch_vccnz 2f\n\t"
-                     "s_sub_u32 %1, %1, 1\n\t"
-                     "s_cmp_lg_u32 %1, 0\n\t"
-                     "s_cbranch_scc1 1b\n\t"
-                     "2:\n\t"
-                     "s_setprio 2"
-                     : "=&v"(got), "+s"(spins)
-                     : "v"((uint32_t) (uintptr_t) &flg[4]), "v"(need)
-                     : "vcc", "scc", "memory");
-    };
-    // (every lane stores the same word; the wave's LDS accesses before it are complete)
-    auto post = [&](int which, uint32_t v) {
-        asm volatile("s_waitcnt lgkmcnt(0)\n\tds_write_b32 %0, %1" ::"v"((uint32_t) (uintptr_t) &flg[which]), "v"(v) : "memory");
-    };
     for (int i = tid; i < BN; i += NTHR) {
         const bool ok = i < count;
         const int j = start + (ok ? i : 0);   // padding rows load the tile's first row; their results are never stored
@@ -489,7 +390,6 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     const int nsteps = a.K / WK;
 
     if (producer) {
-        if (FSYNC) __builtin_amdgcn_s_setprio(2);
         // rows past R decode row R - 1 again (never stored)
         const int ptid = tid - 64 * NCW, rr = ptid >> 2, jb = ptid & 3, row = min(r0 + (gu ? rr & 31 : rr), a.R - 1), nbk = a.K / 8;
         // This thread's two blocks of step s.  Always the same loads - steps past the end request the last step again, and a
@@ -573,10 +473,9 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                     }
                 }
             }
-            if (FSYNC && s >= NWT) wait_read((uint32_t) (s - NWT + 1));
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                *(uint4*) &Wsm[NWT == 2 ? s & 1 : s % NWT][rr][16 * jb + 8 * h] = make_uint4(cvt_pk_bf16(f[h][0], f[h][1]), cvt_pk_bf16(f[h][2], f[h][3]),
+                *(uint4*) &Wsm[s & 1][rr][16 * jb + 8 * h] = make_uint4(cvt_pk_bf16(f[h][0], f[h][1]), cvt_pk_bf16(f[h][2], f[h][3]),
                                                                        cvt_pk_bf16(f[h][4], f[h][5]), cvt_pk_bf16(f[h][6], f[h][7]));
         };
         MmRec2 rec[RECD] = {};
@@ -589,8 +488,7 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
             lookup(rec[(u + 1) % RECD], look[(u + 1) & 1]);   // the next step's table reads travel under this step's decode
             produce(s, rec[u], look[u & 1]);
             load_rec(s + RECD, rec[u]);
-            if (FSYNC) post(wv - NCW, (uint32_t) s + 1u);
-            else lds_barrier();
+            lds_barrier();
         };
         // whole rounds of the record ring in a loop with one way out (a conditional exit per step costs the loop a
         // register move per record word and step), the steps left over after it
@@ -611,11 +509,10 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     // ---- consumer side ---------------------------------------------------------------------------------------------------
     const int wtok = wv * 32 * CT;          // this wave's first token of the tile
     if (wtok >= count) {                    // a wave whose tokens are all padding has nothing to multiply
-        if (FSYNC) post(4, 0x7FFFFFFFu);
-        else for (int s = 0; s < nsteps; ++s) lds_barrier();
+        for (int s = 0; s < nsteps; ++s) lds_barrier();
         return;
     }
-    __builtin_amdgcn_s_setprio(FSYNC ? 3 : 2);   // the matrix pipeline's instruction stream goes first when both roles are ready
+    __builtin_amdgcn_s_setprio(2);   // the matrix pipeline's instruction stream goes first when both roles are ready
     f32x16 acc[CT][2];
 #pragma unroll
     for (int m = 0; m < CT; ++m)
@@ -652,14 +549,12 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     // One weight step: chunk m multiplies out of fragment set (m even ? fa : fb) while the next chunk's fragments travel
     // into the other set; with MT odd the sets have swapped roles when the step ends.
     auto step = [&](int s, bf16x8 (&fa)[4], bf16x8 (&fb)[4]) {
-        if (FSYNC) wait_written((uint32_t) s + 1u);
-        else lds_barrier();   // weight step s is in tile s & 1
+        lds_barrier();   // weight step s is in tile s & 1
         bf16x8 bq[4][2];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-            for (int n = 0; n < 2; ++n) bq[kk][n] = *(const bf16x8*) &Wsm[NWT == 2 ? s & 1 : s % NWT][32 * n + frow][16 * kk + 8 * fhi];
-        if (FSYNC) post(4, (uint32_t) s + 1u);
+            for (int n = 0; n < 2; ++n) bq[kk][n] = *(const bf16x8*) &Wsm[s & 1][32 * n + frow][16 * kk + 8 * fhi];
 #pragma unroll
         for (int m = 0; m < CT; ++m) {
             const int c = s * CT + m;
@@ -721,7 +616,7 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
         }
 }
 template <int NCW, int XCH>
-constexpr size_t mm_stream_lds() { return (size_t) (NCW * XCH * XCHUNK + (NCW == 1 && XCH == 2 ? 3 : 2) * BM * LDW2) * sizeof(uint16_t); }
+constexpr size_t mm_stream_lds() { return (size_t) (NCW * XCH * XCHUNK + 2 * BM * LDW2) * sizeof(uint16_t); }
 // the streamed kernel takes BF16 activations in 16-byte aligned rows, one BF16 term per weight, K in whole weight steps
 // (xrows > 0: the row count, for the variants that address rows by 32-bit byte offsets)
 bool stream_ok(int fmt, int K, int xs, const void* x, long long xrows) {
@@ -748,11 +643,21 @@ void launch_mm_stream(hipStream_t st, int fmt, const MmArgs& a, WSlice wd, const
     }
 }
 
+// the kernel for few tokens takes activations in 16-byte aligned rows (BF16 or f32), one BF16 term per weight, K in whole chunks
+template <bool PACKED>
+bool rows_ok(int fmt, int K, int xs, const void* x) {
+    const bool exact = g_seed_exact && (fmt == MF_SEED4 || fmt == MF_SEED4P4);
+    return !exact && K % 64 == 0 && xs % (PACKED ? 8 : 4) == 0 && ((uintptr_t) x & 15u) == 0;
+}
 template <bool PACKED>
 void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, int xs, float* y, int ys, int T, int add) {
     if (T < 1 || R < 1) return;
-    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), nullptr, nullptr, nullptr};
+    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, nullptr, nullptr, nullptr};
     const unsigned gx = (unsigned) (R + BM - 1) / BM;
+    if (rows_ok<PACKED>(fmt, K, xs, x) && mm_rows_better(fmt, R, T)) {
+        mm_rows_dense(st, fmt, a, w, x, PACKED, y);
+        return;
+    }
     if (PACKED && stream_ok(fmt, K, xs, x, T)) {
         if (T > 256) launch_mm_stream<2, 8, 4>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, (unsigned) (T + 511) / 512));
         else if (T > 128) launch_mm_stream<2, 4, 8>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
@@ -763,31 +668,32 @@ void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, in
     else if (T > 128) launch_mm<2, PACKED>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
     else launch_mm<1, PACKED>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
 }
+// A grouped launch's tiles of up to ROWS_MOST pairs go to the kernel for few tokens, which decodes as fast as the chip can (E 128, top-8,
+// d 2048, ff 768, P = 4: 64 rows 304 -> 255 us a layer step, 32 rows 245 -> 223) but passes over a tile's weights once every 32 pairs;
+// fuller tiles go to the streamed kernel, one decode a tile of up to 128 (512 rows, 32 pairs a tile: 434 there, 384 here).  The rule looks
+// at a tile alone.  A caller that bounds its tiles by 64 is spared the second launch.
+#define ROWS_MOST 32
 template <bool PACKED>
 void mm_grouped(hipStream_t st, int fmt, const WSlice* ws, int K, int R, const void* x, int xs, float* y, int ys, int xdiv,
                 const int32_t* perm, const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows,
                 const WSlice* ws2 = nullptr, float* y2 = nullptr) {
     if (grid_tiles < 1 || R < 1) return;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), ws2, y2, nullptr};
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), 0, MMT_BN, ws2, y2, nullptr};
     WSlice none = {};
+    const dim3 grid((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles, ws2 ? 2u : 1u);
+    if (rows_ok<PACKED>(fmt, K, xs, x)) {
+        if (tile_rows > 64) a.least = a.most = ROWS_MOST;
+        mm_rows_grouped(st, fmt, a, ws, x, PACKED, y, perm, tiles, ntiles, grid_tiles, tile_rows);
+        if (tile_rows <= 64) return;
+    }
     if (PACKED && stream_ok(fmt, K, xs, x, 0)) {
-        // grouped tiles are mostly a few pairs of one expert: decode-bound, so a short ring buys two workgroups a CU - and
-        // where the caller knows that no tile holds more than 32 pairs, one multiplying wave instead of four buys four
-        const dim3 grid((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles, ws2 ? 2u : 1u);
-        // (one multiplying wave: four workgroups a CU fit either three weight tiles and a ring of two activation chunks or two and
-        // three.  C2 at 32 rows, P = 4: 260.3 against 263.5 us; C3 at 16 rows, P = 3, whose steps are shorter than an activation
-        // chunk's way from memory: 620 against 609; three and three, three workgroups a CU: 265.2 and 615.6)
-        if (tile_rows <= 32 && fmt == MF_SEED4P4) launch_mm_stream<1, 1, 2>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
-        else if (tile_rows <= 32) launch_mm_stream<1, 1, 3>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
-        else launch_mm_stream<1, 4, 3>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
+        launch_mm_stream<1, 4, 3>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
         return;
     }
-    launch_mm<1, PACKED>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, dim3((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles));
-    if (ws2) {   // (the first-generation kernel takes one matrix a launch)
-        a.ws2 = nullptr;
-        a.y2 = nullptr;
-        launch_mm<1, PACKED>(st, fmt, a, none, ws2, x, y2, perm, tiles, ntiles, dim3((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles));
-    }
+    a.ws2 = nullptr;   // (the first-generation kernel takes one matrix a launch)
+    a.y2 = nullptr;
+    launch_mm<1, PACKED>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, dim3(grid.x, grid.y));
+    if (ws2) launch_mm<1, PACKED>(st, fmt, a, none, ws2, x, y2, perm, tiles, ntiles, dim3(grid.x, grid.y));
 }
 
 }   // namespace
@@ -832,12 +738,13 @@ int kc_mm_grouped_swiglu(kc_stream_t s, int fmt, const WSlice* gate, const WSlic
                          int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows) {
     if (max_tiles < 1 || R < 1) return 0;
     if (!stream_ok(fmt, K, xs, x, 0) || host_store_f32()) return -1;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, up, nullptr, a16};
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, 0, MMT_BN, up, nullptr, a16};
+    if (tile_rows < 1) tile_rows = MMT_BN;
+    if (tile_rows > 64) a.least = a.most = ROWS_MOST;   // (as in mm_grouped)
+    mm_rows_grouped((hipStream_t) s, fmt, a, gate, x, true, nullptr, perm, tiles, nt, max_tiles, tile_rows);
     WSlice none = {};
     const dim3 grid((unsigned) (R + BM / 2 - 1) / (BM / 2), (unsigned) max_tiles);
-    if (tile_rows >= 1 && tile_rows <= 32 && fmt == MF_SEED4P4) launch_mm_stream<1, 1, 2>((hipStream_t) s, fmt, a, none, gate, x, nullptr, perm, tiles, nt, grid);   // (as in mm_grouped)
-    else if (tile_rows >= 1 && tile_rows <= 32) launch_mm_stream<1, 1, 3>((hipStream_t) s, fmt, a, none, gate, x, nullptr, perm, tiles, nt, grid);
-    else launch_mm_stream<1, 4, 3>((hipStream_t) s, fmt, a, none, gate, x, nullptr, perm, tiles, nt, grid);
+    if (tile_rows > 64) launch_mm_stream<1, 4, 3>((hipStream_t) s, fmt, a, none, gate, x, nullptr, perm, tiles, nt, grid);
     return 0;
 }
 void kc_mm_grouped_packed_pair(kc_stream_t s, int fmt, const WSlice* ws_a, const WSlice* ws_b, int K, int R, const uint16_t* x, int xs,

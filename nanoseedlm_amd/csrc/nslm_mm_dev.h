@@ -1,0 +1,47 @@
+// nslm_mm_dev.h - what the GEMM sources share: the launch arguments, BF16 packing, and the launcher of the kernel for few tokens.
+#pragma once
+#include <type_traits>
+
+#include "nslm_mv_dev.h"
+
+namespace nslm {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct MmArgs {
+    int K, R, T, xs, ys, xdiv, add, f32out;
+    int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's
+    const WSlice* ws2;   // grouped launches of two matrices over the same tiles (grid.z = 2): the second slice table ..
+    float* y2;           // .. and its output
+    uint16_t* a16;       // non-null: a workgroup's weight rows are gate rows (ws) and the same rows of up (ws2), half and half, and what
+                         // it stores is their SwiGLU as BF16 bits [pair][ys] (the two GEMMs and the SwiGLU + pack pass in one launch)
+};
+
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// a kernel that asks for more dynamic LDS than the default limit has the limit raised to what it needs, once (the kernel is a
+// template argument so that every kernel has its own "once": kernels of one signature share a pointer type)
+template <auto K>
+void allow_big_lds(size_t bytes) {
+    static const hipError_t once = bytes > 48 * 1024 ? hipFuncSetAttribute((const void*) K, hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes)
+                                                     : hipSuccess;
+    (void) once;
+}
+
+// 16-byte slot s of row r of a [rows][64] BF16 tile in LDS holds piece s ^ x_swizzle(r): the fragment reads of 16 or 32 rows spread over the banks
+__device__ __forceinline__ int x_swizzle(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
+
+// the kernel for few tokens a matrix (nslm_mm_rows.hip); packed: X holds BF16 bits, else f32
+bool mm_rows_better(int fmt, int R, int T);
+void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, const void* X, bool packed, float* Y);
+void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
+                     const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows);
+
+}   // namespace nslm

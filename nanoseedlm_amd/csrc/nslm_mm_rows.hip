@@ -1,0 +1,423 @@
+// nslm_mm_rows.hip - the GEMM for few tokens a matrix: Y[n][r] = sum_k W[r][k] X[n][k], dense or grouped by expert.
+//
+// With few tokens what a launch takes is the decode of the weights (about 100 vector instructions a seed block, four clocks each), and the
+// chip has to be filled from R / 16 row tiles.  The streamed kernel's workgroups take 64 rows and decode with one wave a SIMD: 64
+// workgroups for 4096 rows, each decoding alone.  Here
+//   * a lane's decoded 8-weight block never leaves its registers: eight BF16 weights of one row are exactly a lane's operand of
+//     v_mfma_f32_16x16x32_bf16 (lane l: row l % 16, K block l / 16), so nothing is handed over or waited for between the decode and the
+//     matrix core, and every wave decodes, independently of the others until their sums meet;
+//   * the waves of a workgroup share its rows and split K: 64-weight chunk c belongs to segment c % 8, and a segment's sum is one
+//     chain of MFMAs.  8 waves a workgroup: a segment each; 4 waves (grouped launches, whose many workgroups overlap): two each.
+//     Either way y = sum over w < 4 of (segment w + segment w + 4), so a token's bits depend on K alone, not on the launch's
+//     shape, the tile or the tile's other tokens.
+// Measured (us, streamed kernel -> this one): P = 4, 4096 x 4096: 9 tokens 40.1 -> 9.7, 48 tokens 42.8 -> 11.1, 200 tokens 51.8 -> 23.0;
+// 1024 x 4096, 100 tokens 44.7 -> 11.2; Q4 2880 x 2880, 301 tokens 43.0 -> 17.8; BF16 151936 x 2048, 16 tokens 155.7 -> 115.3 (5.5 TB/s).
+// What bounds it: vector issue of the decode for the seed formats, the activations' way from L2 for Q4 / Q8 / BF16 at many tokens,
+// HBM for BF16 at few.
+#include "nslm_mm_dev.h"
+
+using namespace nslm;
+
+namespace {
+
+// ---- a step: 64 K (one chunk) of a wave's 16 RT rows and 16 NT tokens, staged in the wave's own part of the LDS ------------------------
+// Loads in an MFMA operand's layout (consecutive lanes in different rows) cost the address unit a cycle a lane; staged by
+// global_load_lds, consecutive lanes take consecutive 16-byte pieces of a row.  The wave reads a step into registers at once and
+// requests the next one into the same place, so the LDS holds one step a wave and its decode covers the latency.
+//   activations  [16 NT][64] BF16, the 16-byte pieces of a row swizzled (x_swizzle) so that a fragment read spreads over the banks
+//   seeds        per row tile: 16 rows x 16 bytes of seeds, 16 x 16 of coefficient words; then 16 x 4 of codes
+//   Q4 / Q8      16 rows x 32 / 64 bytes a row tile (Q8: pieces swizzled); scales and biases stay in registers
+//   BF16         like the activations
+template <int FMT>
+constexpr bool seed_fmt() { return FMT == MF_SEED4P4 || FMT == MF_SEED4; }
+template <int FMT>
+constexpr int row_bytes() { return seed_fmt<FMT>() || FMT == MF_Q4 ? 32 : FMT == MF_Q8 ? 64 : 128; }   // of weights, a chunk
+template <int FMT, int RT, int NT, bool PACKED>
+constexpr int step_bytes() { return 16 * RT * (row_bytes<FMT>() + (FMT == MF_SEED4P4 ? 4 : 0)) + (PACKED ? NT * 2048 : 0); }
+
+__device__ __forceinline__ void to_lds16(const void* src, uint8_t* dst) {   // dst: the wave's base, lane l lands at dst + 16 l
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 16, 0, 0);
+}
+__device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
+}
+
+// The 16 RT rows from r0 (with a.a16: 8 RT gate rows and the same 8 RT up rows) x the 16 NT tokens n0 .. of a workgroup of NW waves.
+// lds: NW x max(step, RT NT KB).
+template <int FMT, int RT, int NT, int NW, bool PACKED, bool GROUPED>
+__device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, const WSlice& m1, const void* X, float* Y, const int32_t* perm, int start, int count,
+                                          int n0, int r0, const uint32_t* tab, uint8_t* lds) {
+    constexpr bool SEED = seed_fmt<FMT>();
+    constexpr int RB = row_bytes<FMT>();
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
+    const bool gu = GROUPED && a.a16 != nullptr;
+    const int nch = a.K / 64;
+    uint8_t* const ws = lds + w * step_bytes<FMT, RT, NT, PACKED>();
+    uint8_t* const wc = ws + 16 * RT * RB;                                     // codes
+    uint8_t* const wx = wc + (FMT == MF_SEED4P4 ? 64 * RT : 0);                // activations
+    // rows past R: the last one again, never stored
+    auto row_of = [&](int i) { return min(r0 + (gu ? i % (8 * RT) : i), a.R - 1); };   // i: row of the workgroup's 16 RT
+    auto second = [&](int rt) { return gu && rt >= RT / 2; };   // a row tile of the second matrix (up)
+    auto stream = [&](int rt, int s) { return (const uint8_t*) (second(rt) ? m1.p[s] : m0.p[s]); };
+    auto src_of = [&](int i) {   // token i of the tile's 16 NT (past the end: the last one again, never stored)
+        const int n = start + min(n0 + i, count - 1);
+        return (size_t) (GROUPED ? perm[n] / a.xdiv : n) * (size_t) a.xs;
+    };
+    // the lane's addresses in chunk 0
+    constexpr int NA = SEED || FMT == MF_Q4 ? (RT + 1) / 2 : FMT == MF_Q8 ? RT : 2 * RT;   // 16-byte weight loads a step
+    const uint8_t* pa[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        if constexpr (SEED) {   // groups of 16 lanes: seeds, words of row tile 2i, the same of 2i + 1
+            const int rt = min(2 * i + (g >> 1), RT - 1);
+            pa[i] = ((g & 1) ? stream(rt, 1) : stream(rt, 0)) + (size_t) row_of(16 * rt + t) * (size_t) (a.K / 4);
+        } else {
+            const int at = 1024 * i + 16 * lane, r = min(at / RB, 16 * RT - 1), piece = (at % RB) / 16;
+            const int sw = FMT == MF_BF16 ? piece ^ x_swizzle(r & 15) : FMT == MF_Q8 ? piece ^ ((r >> 2) & 3) : piece;
+            pa[i] = stream(r >> 4, 0) + (size_t) row_of(r) * (size_t) (a.K / 64 * RB) + 16 * sw;
+        }
+    }
+    const uint8_t* pcode = nullptr;
+    if constexpr (FMT == MF_SEED4P4) {
+        const int rt = min(g, RT - 1);
+        pcode = stream(rt, 3) + (size_t) row_of(16 * rt + t) * (size_t) (a.K / 16);
+    }
+    uint32_t px[PACKED ? 2 * NT : NT];   // in 16-byte pieces
+    if constexpr (PACKED) {
+#pragma unroll
+        for (int i = 0; i < 2 * NT; ++i) {
+            const int n = 8 * i + (lane >> 3);
+            px[i] = (uint32_t) (src_of(n) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle(n & 15));
+        }
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) px[nt] = (uint32_t) (src_of(16 * nt + t) >> 2) + 4u * (uint32_t) g;
+    }
+    uint32_t sc[RT], bi[RT];   // Q4 / Q8: scale and bias bits of the step that is staged
+    // streams may start at any 2-byte (codes: any) boundary; those that are not aligned go through registers
+    auto low = [&](const WSlice& m) { return (uintptr_t) m.p[0] | (SEED ? (uintptr_t) m.p[1] : 0) | (FMT == MF_SEED4P4 ? ((uintptr_t) m.p[3] & 3u) << 2 : 0); };
+    const bool aligned = ((low(m0) | (GROUPED ? low(m1) : 0)) & 15u) == 0;
+    auto request = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const uint8_t* src = pa[i] + (size_t) c * (SEED ? 16 : RB);
+            if (!((SEED || FMT == MF_Q4) && 2 * i + 1 == RT) || lane < 32) {   // (an odd row tile: half a load)
+                if (aligned) to_lds16(src, ws + 1024 * i);
+                else *(u32x4*) (ws + 1024 * i + 16 * lane) = *(const NSLM_GLOBAL u32x4_a2*) src;
+            }
+        }
+        if constexpr (FMT == MF_SEED4P4) {
+            if (RT >= 4 || lane < 16 * RT) {
+                if (aligned) to_lds4(pcode + 4 * (size_t) c, wc);
+                else *(uint32_t*) (wc + 4 * lane) = *(const NSLM_GLOBAL u32_a1*) (pcode + 4 * (size_t) c);
+            }
+        }
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int i = 0; i < 2 * NT; ++i) to_lds16((const uint8_t*) X + (size_t) (px[i] + 8u * (uint32_t) c) * 16, wx + 1024 * i);
+        }
+        if constexpr (FMT == MF_Q4 || FMT == MF_Q8) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const size_t gi = ((size_t) row_of(16 * rt + t) * a.K + (size_t) c * 64 + 16 * g) >> (second(rt) ? group_shift(m1) : group_shift(m0));
+                sc[rt] = gp<uint16_t>(stream(rt, 1))[gi];
+                bi[rt] = gp<uint16_t>(stream(rt, 2))[gi];
+            }
+        }
+    };
+    f32x4 acc[RT][NT], tot[RT][NT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = tot[rt][nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+    const int n = (nch - w + NW - 1) / NW;   // this wave's chunks: those of segment w, then (4 waves) of segment w + 4
+    int c = w;
+    auto next = [&](int at) { at += 8; if (NW == 4 && at >= nch) at = at % 8 >= 4 ? nch : w + 4; return at; };
+    if (n > 0) request(c);
+    for (int s = 0; s < n; ++s) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        bf16x8 xb[2][NT];
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) xb[h][nt] = *(const bf16x8*) (wx + nt * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const NSLM_GLOBAL uint8_t* xp = gp<uint8_t>(X) + (size_t) (px[nt] + 16u * (uint32_t) c + 2u * h) * 16;
+                    const uint4 va = ldg16(xp), vb = ldg16(xp + 16);
+#define F(w) __uint_as_float(w)
+                    xb[h][nt] = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(F(va.x), F(va.y)), cvt_pk_bf16(F(va.z), F(va.w)),
+                                                                      cvt_pk_bf16(F(vb.x), F(vb.y)), cvt_pk_bf16(F(vb.z), F(vb.w))));
+#undef F
+                }
+        }
+        uint32_t u[RT], v[RT], cd[RT];   // seeds: two seeds, two words, their codes.  Q4 / Q8: scale and bias
+        uint4 raw[RT][2];                // BF16: the two blocks; Q8: raw[0]; Q4: raw[0].xy
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            if constexpr (SEED) {
+                u[rt] = *(const uint32_t*) (ws + 512 * rt + 16 * t + 4 * g);
+                v[rt] = *(const uint32_t*) (ws + 512 * rt + 256 + 16 * t + 4 * g);
+                if (FMT == MF_SEED4P4) cd[rt] = wc[64 * rt + 4 * t + g];
+            } else if constexpr (FMT == MF_BF16) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+            } else {
+                u[rt] = sc[rt];
+                v[rt] = bi[rt];
+                if (FMT == MF_Q8) raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ ((t >> 2) & 3)));
+                else {
+                    const uint2 b = *(const uint2*) (ws + 512 * rt + 32 * t + 8 * g);
+                    raw[rt][0] = make_uint4(b.x, b.y, 0, 0);
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the step is in registers: its place is free
+        const int cn = next(c);
+        if (s + 1 < n) request(cn);
+        loads_issued();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 wb[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                if constexpr (FMT == MF_BF16) {
+                    wb[rt] = __builtin_bit_cast(bf16x8, raw[rt][h]);
+                    continue;
+                }
+                float f[8];
+                if constexpr (SEED) {
+                    const uint32_t seed = h ? u[rt] >> 16 : u[rt] & 0xFFFFu, word = h ? v[rt] >> 16 : v[rt] & 0xFFFFu, up = h ? u[rt] : u[rt] << 16;
+                    const uint32_t gs = stream_of(tab, seed);
+                    int is[8], code;
+                    if (FMT == MF_SEED4P4) {
+                        isum_p4(up, gs, tab[512 + (word & 0xFFu)], tab[512 + (word >> 8)], is);
+                        code = (int) ((cd[rt] >> (4 * h)) & 15u);
+                    } else {
+                        isum_p3(up, gs, tab[512 + ((word >> 4) & 0xFFu)], tab[512 + (word >> 12)], is);
+                        code = (int) (word & 15u);
+                    }
+                    const float e = pow2f((second(rt) ? m1.eb : m0.eb) + code) * NSLM_R32;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) f[i] = (float) is[i] * e;
+                } else {
+                    const float e = bf(u[rt]), b = bf(v[rt]);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const uint4& r = raw[rt][0];
+                        const uint32_t qv = FMT == MF_Q8 ? ((h ? (i < 4 ? r.z : r.w) : (i < 4 ? r.x : r.y)) >> (8 * (i & 3))) & 255u
+                                                         : ((h ? r.y : r.x) >> (4 * i)) & 15u;
+                        f[i] = e * (float) qv + b;
+                    }
+                }
+                wb[rt] = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], xb[h][nt], acc[rt][nt], 0, 0, 0);
+        }
+        if (NW == 4 && c < nch && c + 8 >= nch) {   // the segment is complete
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    tot[rt][nt] += acc[rt][nt];
+                    acc[rt][nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+                }
+        }
+        c = cn;
+    }
+    __syncthreads();
+    // accumulator element i of lane l: token l % 16, row 4 (l / 16) + i
+    f32x4* red = (f32x4*) lds;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) red[((w * RT + rt) * NT + nt) * 64 + lane] = NW == 4 ? tot[rt][nt] : acc[rt][nt];
+    __syncthreads();
+    auto sum = [&](int tile, int l) {
+        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 p = red[(i * RT * NT + tile) * 64 + l];
+            if (NW == 8) p = ((f32x4) {0.0f, 0.0f, 0.0f, 0.0f} + p) + red[((i + 4) * RT * NT + tile) * 64 + l];
+            s += p;
+        }
+        return s;
+    };
+    const int nout = (gu ? RT / 2 : RT) * NT * 64;
+    for (int i = tid; i < nout; i += 64 * NW) {
+        const int tile = i >> 6, l = i & 63, rt = tile / NT, nt = tile % NT, tok = n0 + 16 * nt + (l & 15), orow = r0 + 16 * rt + 4 * (l >> 4);
+        if (tok >= count || orow >= a.R) continue;
+        const int dst = GROUPED ? perm[start + tok] : start + tok;
+        const f32x4 s = sum(tile, l);
+        const bool vec = (a.ys & 3) == 0 && orow + 4 <= a.R;
+        if (gu) {   // the values the two GEMMs would have stored (rounded to BF16), then SwiGLU and its rounding, stored as BF16 bits
+            const f32x4 up = sum(tile + RT / 2 * NT, l);
+            uint32_t v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(bfr(silu_bf(bfr(s[j])) * bfr(up[j]))) >> 16;
+            uint16_t* ao = a.a16 + (size_t) dst * a.ys + orow;
+            if (vec && ((uintptr_t) ao & 7u) == 0) *(uint2*) ao = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+            else
+                for (int j = 0; j < 4 && orow + j < a.R; ++j) ao[j] = (uint16_t) v[j];
+            continue;
+        }
+        float* yo = Y + (size_t) dst * a.ys + orow;
+        if (vec && !a.add && !a.f32out && ((uintptr_t) yo & 15u) == 0) *(f32x4*) yo = (f32x4) {bfr(s[0]), bfr(s[1]), bfr(s[2]), bfr(s[3])};
+        else
+            for (int j = 0; j < 4 && orow + j < a.R; ++j) store_y(yo + j, s[j], a.add, a.f32out);
+    }
+}
+
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
+template <int FMT, int RT, int NT, int NW, bool PACKED>
+constexpr size_t rows_lds() { return (size_t) NW * max_of(step_bytes<FMT, RT, NT, PACKED>(), RT * NT * 1024); }
+constexpr size_t MOST_LDS = 156 * 1024;   // beside the decode tables
+
+template <int FMT, int RT, int NT, bool PACKED>
+__global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const void* X, float* Y) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    if (seed_fmt<FMT>()) {
+        load_tables(tab);
+        __syncthreads();
+    }
+    rows_tile<FMT, RT, NT, 8, PACKED, false>(a, w, w, X, Y, nullptr, 0, a.T, (int) blockIdx.y * 16 * NT, (int) blockIdx.x * 16 * RT, tab, lds);
+}
+
+#define GRT 2   // row tiles of the grouped kernel's workgroups
+template <int FMT, bool PACKED>
+__global__ void __launch_bounds__(256, 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles,
+                                                            const int32_t* ntiles, int limit) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    if (ntiles && (int) blockIdx.y >= *ntiles) return;
+    const bool gu = a.a16 != nullptr;
+    const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
+    const MmTile tl = tiles[blockIdx.y];
+    if (tl.count > a.most) return;   // another launch's
+    if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
+        ws = a.ws2;
+        Y = a.y2;
+    }
+    const WSlice m0 = ws[tl.slice], m1 = gu ? a.ws2[tl.slice] : m0;
+    if (tl.count > limit)   // a broken promise is made visible: pairs beyond the launch's bound are stored as NaN, not left stale
+        for (int i = limit * rows + (int) threadIdx.x; i < tl.count * rows; i += 256) {
+            const int orow = r0 + i % rows;
+            const size_t at = (size_t) perm[tl.start + i / rows] * a.ys + orow;
+            if (orow < a.R) {
+                if (gu) a.a16[at] = 0x7FC0u;
+                else Y[at] = __uint_as_float(0x7FC00000u);
+            }
+        }
+    const int count = min(tl.count, limit);
+    if (seed_fmt<FMT>()) {
+        load_tables(tab);
+        __syncthreads();
+    }
+    for (int n0 = 0; n0 < count; n0 += 32) {
+        if (n0) __syncthreads();   // the sums of the tokens before are read
+        if (count - n0 <= 16) rows_tile<FMT, GRT, 1, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds);
+        else rows_tile<FMT, GRT, 2, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds);
+    }
+}
+
+template <int FMT, int RT, int NT, bool PACKED>
+void launch(hipStream_t st, const MmArgs& a, const WSlice& w, const void* X, float* Y) {
+    constexpr size_t lds = rows_lds<FMT, RT, NT, 8, PACKED>();
+    static_assert(lds <= MOST_LDS, "a step of every wave fits the CU's LDS");
+    allow_big_lds<k_mm_rows<FMT, RT, NT, PACKED>>(lds);
+    const dim3 grid((unsigned) (a.R + 16 * RT - 1) / (16 * RT), (unsigned) (a.T + 16 * NT - 1) / (16 * NT));
+    hipLaunchKernelGGL((k_mm_rows<FMT, RT, NT, PACKED>), grid, dim3(512), lds, st, a, w, X, Y);
+    host_note_launch();
+}
+
+// The workgroup's shape: what a CU spends on a workgroup's step is RT decodes + NT token tiles' loads and MFMAs (beta: a token
+// tile's share against a row tile's decode, from the times of matrices of 300 .. 14336 rows at 9 .. 1024 tokens), and the launch
+// takes as many workgroups one after the other as the fullest of 256 CUs gets.
+struct Shape {
+    int rt, nt;
+    double cost;
+};
+double beta_of(int fmt) { return fmt == MF_BF16 ? 1.0 : fmt == MF_Q8 || fmt == MF_Q4 ? 0.3 : 0.13; }
+bool fits(int fmt, int rt, int nt) { return !(fmt == MF_BF16 && rt + nt > 9); }   // (BF16 weights: 2 KB of LDS a wave and tile)
+Shape shape_of(int fmt, int R, int T, bool packed) {
+    static const int rts[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 6}, {1, 8}, {2, 1}, {2, 2}, {2, 3}, {2, 4}, {2, 6}, {2, 8}, {4, 1}, {4, 2}, {4, 4}};
+    Shape best = {0, 0, 1e30};
+    for (const auto& s : rts) {
+        const int rt = s[0], nt = s[1];
+        if (!fits(fmt, rt, nt) || (!packed && !(rt == 1 && (nt == 1 || nt == 4)) && !(rt == 4 && nt == 4))) continue;
+        const long long wgs = (long long) ((R + 16 * rt - 1) / (16 * rt)) * ((T + 16 * nt - 1) / (16 * nt));
+        const double cost = (double) ((wgs + 255) / 256) * (rt + nt * beta_of(fmt));
+        if (cost < best.cost) best = {rt, nt, cost};
+    }
+    return best;
+}
+
+template <int FMT, bool PACKED>
+void dense(hipStream_t st, const MmArgs& a, const WSlice& w, const void* X, float* Y) {
+    const Shape s = shape_of(FMT, a.R, a.T, PACKED);
+#define C(RT, NT) case 10 * RT + NT: launch<FMT, RT, NT, PACKED>(st, a, w, X, Y); return;
+    if constexpr (PACKED) {
+        switch (10 * s.rt + s.nt) { C(1, 1) C(1, 2) C(1, 3) C(1, 4) C(1, 6) C(1, 8) C(2, 1) C(2, 2) C(2, 3) C(2, 4) C(2, 6) C(4, 1) C(4, 2) C(4, 4) }
+        if constexpr (FMT != MF_BF16) launch<FMT, 2, 8, PACKED>(st, a, w, X, Y);
+    } else {
+        switch (10 * s.rt + s.nt) { C(1, 1) C(1, 4) C(4, 4) }
+    }
+#undef C
+}
+template <int FMT, bool PACKED>
+void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles,
+             const int32_t* ntiles, int grid_tiles, int tile_rows) {
+    const int rows = a.a16 ? 8 * GRT : 16 * GRT;
+    const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
+    constexpr size_t lds = rows_lds<FMT, GRT, 2, 4, PACKED>();
+    allow_big_lds<k_mm_rows_grouped<FMT, PACKED>>(lds);
+    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y,
+                       perm, tiles, ntiles, tile_rows <= 32 ? 32 : MMT_BN);
+    host_note_launch();
+}
+
+}   // namespace
+
+namespace nslm {
+
+#define BY_FORMAT(CALL)                                        \
+    switch (fmt) {                                             \
+        case MF_SEED4P4: CALL(MF_SEED4P4); break;              \
+        case MF_SEED4: CALL(MF_SEED4); break;                  \
+        case MF_BF16: CALL(MF_BF16); break;                    \
+        case MF_Q8: CALL(MF_Q8); break;                        \
+        default: CALL(MF_Q4); break;                           \
+    }
+
+// Against the streamed kernel, whose workgroup takes 64 rows x up to 512 tokens and spends on a step, in row decodes, what `stream`
+// says (it was timed with 64 .. 224 workgroups, one a CU): that one wins where its workgroups fill the chip.
+bool mm_rows_better(int fmt, int R, int T) {
+    const int q = T <= 128 ? 0 : T <= 256 ? 1 : 2;
+    static const double seeds[] = {6.2, 7.5, 8.8}, ints[] = {8.4, 12.7, 14.5}, bfs[] = {13.7, 23.0, 34.0};
+    const double* stream = fmt == MF_BF16 ? bfs : fmt == MF_Q8 || fmt == MF_Q4 ? ints : seeds;
+    const long long wgs = (long long) ((R + 63) / 64) * ((T + 511) / 512);
+    return shape_of(fmt, R, T, true).cost < (double) ((wgs + 255) / 256) * stream[q];
+}
+void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, const void* X, bool packed, float* Y) {
+#define D(F) packed ? dense<F, true>(st, a, w, X, Y) : dense<F, false>(st, a, w, X, Y)
+    BY_FORMAT(D)
+#undef D
+}
+void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
+                     const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows) {
+#define G(F)                                                                                                 \
+    packed ? grouped<F, true>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)             \
+           : grouped<F, false>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)
+    BY_FORMAT(G)
+#undef G
+}
+
+}   // namespace nslm

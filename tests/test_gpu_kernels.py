@@ -294,6 +294,51 @@ def test_mm_token_tiles(be, oracle, T):
     assert np.max(np.abs(yf - ref)) / np.max(np.abs(ref)) < 1e-2   # the bar for the BF16 MFMA prefill
 
 
+# R 1 / 17 / 70: a row tile's edge inside; K 64: seven of a workgroup's eight waves without a chunk, 576: nine chunks, 1088: seventeen;
+# T: both sides of a token tile and of the workgroup shapes (one to eight token tiles, one to four row tiles)
+@pytest.mark.parametrize("R,K", [(1, 64), (17, 576), (70, 1088), (4100, 128)])
+@pytest.mark.parametrize("fmt", ALL_FMT)
+def test_mm_few_tokens(be, oracle, fmt, R, K):
+    rng = np.random.default_rng(R + 10 * K + fmt)
+    p = make_pack(rng, fmt, 1, R, K)
+    x = packs.round_bf16(rng.standard_normal((129, K)).astype(np.float32))
+    ref, mag = ref_mm(oracle, p, 0, x, 0)
+    y9 = None
+    for T in (1, 9, 16, 17, 33, 64, 65, 129):
+        y = be.kt_mm_plain(p, x[:T], packed=1)
+        assert close_bf(y, packs.round_bf16(ref[:T].astype(np.float32)).astype(np.float64), F32B * mag[:T]).all(), (NAMES[fmt], R, K, T)
+        assert np.array_equal(y.view(np.uint32), be.kt_mm_plain(p, x[:T], packed=0).view(np.uint32)), (NAMES[fmt], R, K, T)
+        y9 = y if T == 9 else y9
+        if y9 is not None and R < 4100:   # every shape of workgroup adds up a token's products in the same order
+            assert np.array_equal(y[:9].view(np.uint32), y9.view(np.uint32)), (NAMES[fmt], R, K, T)
+
+
+@pytest.mark.parametrize("off", [0, 2, 6])
+def test_mm_few_tokens_streams_at_any_boundary(be, oracle, off):
+    """Seed, coefficient and code streams that start 2 or 6 (codes: 1 or 3) bytes off a 16-byte boundary give the aligned streams' bits."""
+    from nanoseedlm_amd import backend, moe
+    L = backend.hip()
+    rng = np.random.default_rng(off)
+    R, K, T = 40, 192, 20
+    p = packs.seed4p4(rng, 1, R, K, eb=-20)
+    x = moe.DevBuf.from_array(packs.f32_to_bf16_bits(rng.standard_normal((T, K)).astype(np.float32)))
+    ys = []
+    for o in (0, off):
+        bufs = [moe.DevBuf.from_array(np.concatenate([np.zeros(n, np.uint8), np.ascontiguousarray(a[0]).view(np.uint8).ravel()]))
+                for a, n in ((p["seeds"], o), (p["coefs"], o), (p["codes"], o // 2))]
+        w = backend.WSlice()
+        w.p[0], w.p[1], w.p[3], w.eb = bufs[0].ptr.value + o, bufs[1].ptr.value + o, bufs[2].ptr.value + o // 2, int(p["eb"][0])
+        y = moe.DevBuf(4 * T * R)
+        L.kc_mm_packed(None, packs.MF_SEED4P4, w, K, R, x.ptr, K, y.ptr, R, T, 0, None)
+        moe.device_sync()
+        ys.append(y.to_array(np.uint32, (T, R)))
+        for b in bufs + [y]:
+            b.free()
+    x.free()
+    assert L.kc_last_error() == 0 and np.abs(ys[0].view(np.float32)).max() > 0
+    assert np.array_equal(ys[0], ys[1])
+
+
 # ---- grouping, routers, elementwise, slot table -------------------------------------------------------------------------------
 
 def test_bucket(be, oracle):
