@@ -266,6 +266,158 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
     }
 }
 
+// ---- several tokens: the products on the matrix cores, with the one-token pass's bits --------------------------------------------
+// A block's products with 4 tokens are 4 x 8 (P = 4: 4 x 12) multiply-adds beside its 70 to 90 instructions of decode, and they are what
+// grows with the tokens.  v_mfma_f32_4x4x1_16b_f32 is sixteen 4 x 4 outer products, one fused multiply-add an element: with a wave's four
+// adjacent lanes on the same chunk of four rows, A = a lane's own weight (column sum) and B = its token's activation, element (i, j)
+// runs through chunk_dot's chain of multiply-adds for row i and token j, in its order - the same bits as a one-token call - at one
+// instruction a weight for 4 tokens, on a pipe of its own.  Lane j of the quad ends up with token j's sums of the four rows, and
+// takes each row's block scale from the lane that decoded it (a quad permutation inside the multiply-add).
+// Chunk sums meet in LDS and are added in the order of the one-token kernels.  Against the staged pass (four tokens' multiply-adds on the
+// vector ALUs, a decode for every four tokens), us: 2880 x 2880, P = 3, 6 tokens 20.4 -> 11.0; 4096 x 4096, P = 4, 8 tokens 50.5 -> 24.8, 2
+// tokens 20.3 -> 13.2; 1000 x 8192 (which went a token a launch), P = 3, 8 tokens 87.2 -> 15.9.  Bound by the decode's vector issue and,
+// in small matrices, the staging of the activations.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int I>
+__device__ __forceinline__ float quad_lane(float v) {   // lane I of the lane's quad
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x55 * I, 0xF, 0xF, true));
+}
+template <int P, int NQ>
+__global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, int rb, int tstride, bool shfl) {
+    constexpr int XW = xw<P>(), XP = xpad<P>();
+    extern __shared__ float xl[];   // [tr tokens][chunk][XP], tstride floats a token; then the chunk sums [row][token][L | 1]
+    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    const int tid = threadIdx.x, nthr = blockDim.x, L = a.L, LS = L | 1;
+    float* const part = xl + tr * tstride;
+    const int quad = tid >> 2, ti = tid & 3, nquad = nthr >> 2;
+    const int t0 = (int) blockIdx.y * tr, nt = min(tr, a.ttot - t0);
+    const float* const xb = a.x + (size_t) t0 * a.xs;
+    float* const yb = a.y + (size_t) t0 * a.ys;
+    const int q0 = (int) blockIdx.x * rq_wg, q1 = min(q0 + rq_wg, (a.R + 3) / 4);   // the workgroup's row quads, rb a round
+    auto fetch = [&](int base, int item) {   // (past a round's end: its last item again)
+        const int it = min(item, (min(base + rb, q1) - base) * L - 1), rq = it / L, row = min(4 * (base + rq) + ti, a.R - 1);
+        return load_chunk<P>(a.wd, (uint32_t) row * (uint32_t) L + (uint32_t) (it - rq * L));
+    };
+    // requested in this order (see k_mv_seed): the tables, the first blocks of the activations, the records
+    uint32_t tw[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int i = min(tid + nthr * j, NSLM_TAB_WORDS - 1);
+        tw[j] = i < 512 ? kBasis.v[i] : kPairs.v[i - 512];
+    }
+    const int nb = a.K / 8, tot = nt * nb;
+    Chunk cur;
+    for (int base = tid; base == tid || base < tot; base += nthr * 4) {   // four blocks a thread and round, their loads in flight together
+        float4 q[4][2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int idx = min(base + nthr * j, tot - 1), t = idx / nb, i = idx - t * nb;
+            q[j][0] = ((const float4*) (xb + (size_t) t * a.xs))[2 * i];
+            q[j][1] = ((const float4*) (xb + (size_t) t * a.xs))[2 * i + 1];
+        }
+        loads_issued();
+        if (base == tid) {
+            cur = fetch(q0, quad);
+            loads_issued();
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (tid + nthr * j < NSLM_TAB_WORDS) tab[tid + nthr * j] = tw[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int idx = base + nthr * j;
+            if (idx >= tot) break;
+            const int t = idx / nb, i = idx - t * nb;
+            const float x8[8] = {q[j][0].x, q[j][0].y, q[j][0].z, q[j][0].w, q[j][1].x, q[j][1].y, q[j][1].z, q[j][1].w};
+            store_block<P>(xl + t * tstride, i, x8);
+        }
+    }
+    __syncthreads();
+    const uint32_t ebase = (uint32_t) (a.wd.eb + 127) << 23;
+    for (int base = q0; base < q1; base += rb) {
+        const int nrq = min(rb, q1 - base), items = nrq * L;
+        for (int item = quad; item - quad < items; item += nquad) {
+            const bool more = item - quad + nquad < items;
+            const Chunk nxt = more ? fetch(base, item + nquad) : fetch(base + rb < q1 ? base + rb : base, quad);
+            const int it = min(item, items - 1), rq = it / L, ch = it - rq * L;
+            const float* xr[NQ];   // (tokens past the run's end: its last one again, never stored)
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) xr[n] = xl + min(4 * n + ti, nt - 1) * tstride + ch * XP;
+            f32x4 acc[NQ];
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) acc[n] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const uint32_t ss = word_of(cur.sd, b >> 1), cc = word_of(cur.cw, b >> 1);
+                const uint32_t g = stream_of(tab, (b & 1) ? ss >> 16 : ss & 0xFFFFu), up = (b & 1) ? ss : ss << 16;
+                float z[XW], e2;
+                if constexpr (P == 4) {
+                    const uint32_t be = coef_bytes(cc, b & 1), bo = be << 4;
+                    uint32_t G[6];
+                    col_bytes_p4(up, g, G);
+#pragma unroll
+                    for (int m = 0; m < 12; ++m) z[m] = (float) (m == 11 ? dot8ones(be) : dot8z(G[m >> 1], (m & 1) ? bo : be));
+                    e2 = __uint_as_float((((cur.codes >> (4 * b)) & 15u) << 23) + ebase);
+                } else {
+                    const uint32_t word = (b & 1) ? cc >> 16 : cc & 0xFFFFu;
+                    int is[8];
+                    isum_p3(up, g, tab[512 + ((word >> 4) & 0xFFu)], tab[512 + (word >> 12)], is);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) z[c] = (float) is[c];
+                    e2 = __uint_as_float(((word & 15u) << 23) + ebase);
+                }
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) {
+                    const float* xt = xr[n] + XW * b;
+                    f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int m = 0; m < XW; m += 4) {
+                        const float4 v = *(const float4*) (xt + m);
+                        d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m], v.x, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m + 1], v.y, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m + 2], v.z, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m + 3], v.w, d, 0, 0, 0);
+                    }
+                    acc[n][0] = fmaf(quad_lane<0>(e2), d[0], acc[n][0]);
+                    acc[n][1] = fmaf(quad_lane<1>(e2), d[1], acc[n][1]);
+                    acc[n][2] = fmaf(quad_lane<2>(e2), d[2], acc[n][2]);
+                    acc[n][3] = fmaf(quad_lane<3>(e2), d[3], acc[n][3]);
+                }
+            }
+            if (item < items) {
+#pragma unroll
+                for (int n = 0; n < NQ; ++n)
+                    if (4 * n + ti < nt) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) part[((4 * rq + i) * tr + 4 * n + ti) * LS + ch] = acc[n][i];
+                    }
+            }
+            cur = nxt;
+        }
+        __syncthreads();
+        const int sums = 4 * nrq * nt;   // (row, token), rows side by side so that a token's results leave together
+        if (shfl) {
+            const int l = tid & (L - 1);
+            for (int w = tid / L; w < (sums + nthr / L - 1) / (nthr / L) * (nthr / L); w += nthr / L) {
+                const int wc = min(w, sums - 1), t = wc / (4 * nrq), r = wc - t * 4 * nrq, row = 4 * base + r;
+                float s = part[(r * tr + t) * LS + l];
+                for (int o = L >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
+                if (l == 0 && w < sums && row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_R32, a.add, a.f32out);
+            }
+        } else {
+            for (int w = tid; w < sums; w += nthr) {
+                const int t = w / (4 * nrq), r = w - t * 4 * nrq, row = 4 * base + r;
+                const float* p = part + (r * tr + t) * LS;
+                float s = 0.0f;
+#pragma unroll 4
+                for (int j = 0; j < L; ++j) s += p[j];
+                if (row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_R32, a.add, a.f32out);
+            }
+        }
+        if (base + rb < q1) __syncthreads();
+    }
+}
+
 // ---- generic path: every format, one wave per row --------------------------------------------------------------------
 template <int MODE>
 __global__ void __launch_bounds__(256) k_mv_any(int fmt, MvArgs a) {
@@ -704,10 +856,13 @@ int pick_threads(int V, int L, bool shfl) {
 #define MV_LDS_MAX (128 * 1024)
 // (the kernel is a template argument so that every kernel has its own "once": kernels of one signature share a pointer type)
 template <auto K>
-void allow_big_lds() {
-    static const hipError_t once = hipFuncSetAttribute((const void*) K, hipFuncAttributeMaxDynamicSharedMemorySize, MV_LDS_MAX);
+void allow_lds(int bytes) {
+    static const hipError_t once = hipFuncSetAttribute((const void*) K, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void) once;
 }
+template <auto K>
+void allow_big_lds() { allow_lds<K>(MV_LDS_MAX); }
+#define MV_TOK_LDS (152 * 1024)   // k_mv_tok's, beside its tables
 template <int P, int MODE, int NT, bool COLS>
 void launch_seed256(hipStream_t st, const MvArgs& a, bool shfl, dim3 grid, size_t lds) {
     if (shfl) {
@@ -792,6 +947,53 @@ int wide_run(int fmt, int K, int R, int T) {
     return run;
 }
 
+// A launch of 2 .. 8 tokens by k_mv_tok; false: another kernel's.  The tokens go in runs that fit the LDS beside the chunk sums of enough row
+// quads to keep 1024 threads busy, dealt to grid.y; a matrix whose chunks fill little more than a third of the chip's threads gives it two runs
+// instead of one (2048 x 2048, P = 3, 8 tokens: 9.5 us in two runs of four, 12.2 in one: what it takes is the staging).  A workgroup's share
+// of the row quads is a CU's, or half or a quarter of it where there is work for so many workgroups and their tokens fit the LDS: one
+// stages while another decodes.  A round is as many row quads as two passes of the threads and the LDS hold.
+// Rows of up to 32 chunks whose sums go by shuffles stay with the staged pass of k_mv_seed where that was as fast or faster: two tokens
+// (8192 x 2048: 11.6 us there, 12.0 here), and 5 to 8 of a matrix near 2048 x 2048 (8.0 and 9.0).
+template <int P>
+bool launch_tok(hipStream_t st, MvArgs a, int T, bool shfl) {
+    const int L = a.L, rq = (a.R + 3) / 4, LS = L | 1;
+    const long quads = (long) rq * L;
+    if (shfl && L <= 32 && (T == 2 || (T > 4 && quads >= 32L * cu_count() && quads <= 96L * cu_count()))) return false;
+    // token stride: 16 banks apart, so that the 16-byte reads of a quad's four tokens do not meet
+    const int tstride = ((L * xpad<P>() + 63) / 64) * 64 + 16;
+    const size_t tok = (size_t) tstride * sizeof(float), tok_sums = (size_t) 4 * LS * sizeof(float);   // a token's, of a row quad
+    auto held = [&](int tr, size_t lds) { return tr * tok >= lds ? 0 : (int) ((lds - tr * tok) / (tr * tok_sums)); };   // row quads' sums beside a run's tokens
+    const int all = (rq + cu_count() - 1) / cu_count();   // row quads a CU
+    auto want = [&](int per_cu) { const int n = 256 / per_cu / L < 1 ? 1 : 256 / per_cu / L; return all < n ? all : n; };
+    int runs = (T + MV_MAXT - 1) / MV_MAXT;
+    while (runs <= T && held((T + runs - 1) / runs, MV_TOK_LDS) < (runs < T ? want(1) : 1)) ++runs;
+    if (runs > T) return false;
+    if (runs == 1 && T > 4 && quads <= 96L * cu_count()) runs = 2;
+    const int tr = (T + runs - 1) / runs;
+    runs = (T + tr - 1) / tr;
+    int per_cu = (int) (quads * runs / (64L * cu_count()));
+    per_cu = per_cu >= 4 ? 4 : per_cu >= 2 ? 2 : 1;
+    while (per_cu > 1 && held(tr, MV_TOK_LDS / per_cu) < want(per_cu)) per_cu /= 2;
+    const int share = (int) (((long) rq * runs + per_cu * cu_count() - 1) / (per_cu * cu_count()));
+    int most = 512 / per_cu / L < 1 ? 1 : 512 / per_cu / L;
+    if (most > held(tr, MV_TOK_LDS / per_cu)) most = held(tr, MV_TOK_LDS / per_cu);
+    const int rounds = (share + most - 1) / most, rb = (share + rounds - 1) / rounds;
+    const int at_once = 256 / per_cu, passes = (rb * L + at_once - 1) / at_once;
+    int nthr = (4 * ((rb * L + passes - 1) / passes) + 63) / 64 * 64;
+    if (nthr < 256) nthr = 256;
+    a.ttot = T;
+    const size_t lds = tr * (tok + rb * tok_sums);
+    const dim3 grid((unsigned) (rq + share - 1) / share, (unsigned) runs);
+    if (tr > 4) {
+        allow_lds<k_mv_tok<P, 2>>(MV_TOK_LDS);
+        hipLaunchKernelGGL((k_mv_tok<P, 2>), grid, dim3(nthr), lds, st, a, tr, share, rb, tstride, shfl);
+    } else {
+        allow_lds<k_mv_tok<P, 1>>(MV_TOK_LDS);
+        hipLaunchKernelGGL((k_mv_tok<P, 1>), grid, dim3(nthr), lds, st, a, tr, share, rb, tstride, shfl);
+    }
+    return true;
+}
+
 #define MV_TG 4   // tokens a workgroup of the multi-token fast path stages in LDS
 #define MV_MULTI_MAXT 64
 
@@ -837,6 +1039,10 @@ void kc_mv(kc_stream_t s, int fmt, WSlice w, int K, int R, const float* x, int x
         // (a token's arithmetic does not depend on the run it is in).  One workgroup for all of 16 tokens needed 139 KB of
         // LDS, i.e. one workgroup a CU: 2048 x 2048 at 16 tokens 21.5 us, in runs of four 14.1 us (8 tokens: 12.6 -> 9.9).
         // Rows too long for the staging take one launch per token with the activations in registers.
+        if (T > 1 && T <= MV_MAXT && (fmt == MF_SEED4P4 ? launch_tok<4>(st, a, T, shfl) : launch_tok<3>(st, a, T, shfl))) {
+            note_launch();
+            return;
+        }
         const bool cols = cols_for(T);
         if (T > 1 && (size_t) MV_TG * L * xpad_of(fmt, cols) * sizeof(float) <= MV_LDS_MAX) {
             a.ttot = T;

@@ -228,6 +228,19 @@ def test_mv_more_rows_than_a_pass_on_the_general_path(be, oracle, fmt, K):
     assert np.array_equal(y[9].view(np.uint32), y1[0].view(np.uint32))
 
 
+# R 70 / 1101 / 4099: a last row quad of 2, 1 and 3 rows, one and several rounds a workgroup; K 8192: the tokens in runs (P = 4: of two)
+@pytest.mark.parametrize("fmt,K,R", [(packs.MF_SEED4P4, 2880, 1101), (packs.MF_SEED4, 2880, 70), (packs.MF_SEED4, 4096, 4099), (packs.MF_SEED4P4, 8192, 70),
+                                     (packs.MF_SEED4P4, 1024, 1101), (packs.MF_SEED4P4, 64, 5)])
+def test_mv_two_to_eight_tokens_equal_one(be, fmt, K, R):
+    rng = np.random.default_rng(K + R)
+    p = make_pack(rng, fmt, 1, R, K)
+    x = packs.round_bf16(rng.standard_normal((8, K)).astype(np.float32))
+    one = np.concatenate([be.kt_mv(p, x[t:t + 1]) for t in range(8)])
+    assert np.abs(one).max() > 0
+    for T in (2, 3, 4, 5, 7, 8):
+        assert np.array_equal(be.kt_mv(p, x[:T]).view(np.uint32), one[:T].view(np.uint32)), T
+
+
 # ---- GEMM -----------------------------------------------------------------------------------------------------------------------
 
 def ref_mm(orc, p, s, x, exact):
