@@ -173,10 +173,11 @@ void kc_heads_deq(kc_stream_t s, int fmt, WSlice W, const uint32_t* G, int H, in
 /* Rows [0,R) of one slice of any format decoded to BF16 bits [R][K] (seeds with the slice's own eb; SEED4 too):
  * the bit-exact weight regeneration check. */
 void kc_slice_deq(kc_stream_t s, int fmt, WSlice w, int K, int R, uint16_t* out);
-/* kc_mm_grouped_packed for a caller that knows an upper bound of MmTile.count: a decode step of T rows chooses no expert
- * more than T times, so no tile holds more than tile_rows = T pairs.  Up to 32 the launch uses workgroups with one
- * multiplying wave (four a CU instead of two; the tiles are decode-bound).  The bound is a promise: pairs of a tile beyond
- * it are not computed, and their results are stored as NaN so that a broken promise shows.  tile_rows < 1 or > 32: as kc_mm_grouped_packed. */
+/* kc_mm_grouped_packed for a caller that knows its tiles.  tile_rows up to 32: an upper bound of MmTile.count (a decode step of T rows
+ * chooses no expert more than T times); the bound is a promise: pairs of a tile beyond it are not computed, and their results are
+ * stored as NaN so that a broken promise shows.  33 .. 48, 49 .. 64, 65 .. 96: tiles hold few pairs, mostly up to 32, 64, 96 - fuller ones
+ * are computed too, in several passes.  Above MMT_BN: the tiles are mostly full, and an expert's adjoin.  Anything else: as
+ * kc_mm_grouped_packed. */
 void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, float* y,
                                int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles,
                                int tile_rows);
@@ -186,10 +187,10 @@ void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, 
 void kc_mm_grouped_packed_pair(kc_stream_t s, int fmt, const WSlice* ws_a, const WSlice* ws_b, int K, int R, const uint16_t* x, int xs,
                                float* ya, float* yb, int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt,
                                int max_tiles, int tile_rows);
-/* The gate GEMM, the up GEMM and kc_swiglu_pack in one launch: a workgroup's 64 weight rows are 32 gate rows and the same 32 up
- * rows of the tile's expert, so a lane holds both sums of a (pair, row) and stores a16[pair][row] = the BF16 bits kc_swiglu_pack
+/* The gate GEMM, the up GEMM and kc_swiglu_pack in one launch: a workgroup's weight rows are gate rows and the same up rows of the
+ * tile's expert, half and half, so it holds both sums of a (pair, row) and stores a16[pair][row] = the BF16 bits kc_swiglu_pack
  * would have stored from the two GEMMs' outputs (bit for bit).  R = the expert width, ys = a16's row stride.  -1 (nothing
- * launched) where kc_mm_grouped_packed would not take its streamed kernel (K % 64, alignment) or kc_store_f32(1) is set.
+ * launched) where K % 64, x or xs is not aligned, the weights are in exact mode or kc_store_f32(1) is set.
  * No counterpart in the reference (three launches, engine/mova_cuda.c:1308-1312). */
 int kc_mm_grouped_swiglu(kc_stream_t s, int fmt, const WSlice* gate, const WSlice* up, int K, int R, const uint16_t* x, int xs, uint16_t* a16,
                          int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows);

@@ -384,14 +384,16 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
         if (!routed_and_grouped) kc_bucket(s, m->ind, P, E, m->perm, m->tiles, m->ntiles);
         if (packed) {
             if (c->router != NSLM_ROUTE_SOFTMAX) kc_pack_input_bf16(s, xn, m->px, (size_t) T * d);   /* else: made for the router */
-            /* a step of T rows chooses no expert more than T times: no tile holds more than T pairs */
+            /* a step of T rows chooses no expert more than T times: no tile holds more than T pairs.  More rows than a pass of the
+               grouped kernels takes: the pairs an expert gets on average say which passes pay (kernels_hip.h) */
+            const int mean = P / E, pairs = T <= 32 ? T : mean <= 12 ? 48 : mean <= 52 ? 64 : mean <= 88 && E * ((ff + 63) / 64) < 512 ? 96 : MMT_BN + 1;
             /* gate, up and SwiGLU in one launch (else: the two GEMMs in one launch, then SwiGLU) */
-            if (kc_mm_grouped_swiglu(s, c->fmt, gate, up, d, ff, m->px, d, (uint16_t*) m->A, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, T)) {
-                kc_mm_grouped_packed_pair(s, c->fmt, gate, up, d, ff, m->px, d, m->G, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, T);
+            if (kc_mm_grouped_swiglu(s, c->fmt, gate, up, d, ff, m->px, d, (uint16_t*) m->A, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, pairs)) {
+                kc_mm_grouped_packed_pair(s, c->fmt, gate, up, d, ff, m->px, d, m->G, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, pairs);
                 kc_swiglu_pack(s, m->G, m->U, (uint16_t*) m->A, (size_t) P * ff);
             }
             kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles,
-                                      m->max_tiles, T);
+                                      m->max_tiles, pairs);
         } else {
             kc_mm_grouped_dev(s, c->fmt, gate, d, ff, xn, d, m->G, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
             kc_mm_grouped_dev(s, c->fmt, up, d, ff, xn, d, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);

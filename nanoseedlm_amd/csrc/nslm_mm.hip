@@ -343,9 +343,36 @@ struct MmRec2 {
     uint32_t u, v, c;  // seeds: two seeds, two coefficient words, the codes byte; Q8 / Q4: the group's scale and bias bits
 };
 
+// Two blocks' sums (isum_p4's / isum_p3's) in phase order, every operand a dozen instructions old, as a decoder wave that has a SIMD's vector
+// issue to itself needs them.  By multiply-adds on the windows' halves where they are (mad16): as many instructions as pairing the halves for
+// dot products, but a dot product runs on the matrix pipe and waits there for the consumers' MFMAs (C1: 80.0 -> MAD us).
+template <int P>
+__device__ __forceinline__ void isum2_mad(const uint32_t (&up)[2], const uint32_t (&g)[2], const uint32_t (&qa)[2], const uint32_t (&qb)[2], int (&is)[2][8]) {
+    uint32_t A[2][17];
+#pragma unroll
+    for (int k = 1; k <= 15; ++k)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) A[h][k] = __builtin_amdgcn_alignbit(g[h], up[h], 16 + k);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 1; k <= 16; ++k)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) A[h][k] = (k < 16 ? A[h][k] : g[h]) ^ 0x80008000u;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k = P * c + 1 + p;
+                is[h][c] = mad16(A[h][k <= 16 ? k : k - 16], k > 16, p < 2 ? qa[h] : qb[h], p & 1, p ? is[h][c] : 0, p == 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
 template <int CT, int NCW, int XCH, int FMT>
-__global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice wd, const WSlice* ws, const uint16_t* X, float* Y,
-                                                   const int32_t* perm, const MmTile* tiles, const int32_t* ntiles) {
+__global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice wt, const uint16_t* X, float* Y) {
     constexpr int BN = 32 * CT * NCW, NTHR = 64 * (NCW + 4);   // XCH: chunks in a consumer wave's ring
     constexpr bool seedf = FMT == MF_SEED4P4 || FMT == MF_SEED4;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
@@ -356,54 +383,34 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wv >= NCW;
-    const bool grouped = tiles != nullptr;
-    if (grouped && ntiles && (int) blockIdx.y >= *ntiles) return;
-    const bool gu = a.a16 != nullptr;   // (grouped launches only)
-    const int r0 = (int) blockIdx.x * (gu ? BM / 2 : BM);
-    int start, count;
-    WSlice wt;
-    if (grouped) {
-        const MmTile tl = tiles[blockIdx.y];
-        if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
-            ws = a.ws2;
-            Y = a.y2;
-        }
-        // (gate / up tiles: the decoder waves of the tile's upper 32 rows read the up slice)
-        wt = gu && tid >= 64 * NCW + 128 ? a.ws2[tl.slice] : ws[tl.slice];
-        start = tl.start;
-        count = tl.count;
-        if (count <= a.least) return;   // another launch's
-    } else {
-        wt = wd;
-        start = (int) blockIdx.y * BN;
-        count = min(BN, a.T - start);
-    }
+    const int r0 = (int) blockIdx.x * BM, start = (int) blockIdx.y * BN, count = min(BN, a.T - start);
     if (count < 1) return;
     if (seedf) load_tables(tab);
     for (int i = tid; i < BN; i += NTHR) {
         const bool ok = i < count;
-        const int j = start + (ok ? i : 0);   // padding rows load the tile's first row; their results are never stored
-        srow[i] = grouped ? perm[j] / a.xdiv : j;
-        drow[i] = !ok ? -1 : grouped ? perm[j] : j;
+        srow[i] = start + (ok ? i : 0);   // padding rows load the tile's first row; their results are never stored
+        drow[i] = ok ? start + i : -1;
     }
     __syncthreads();
     const int nsteps = a.K / WK;
 
     if (producer) {
         // rows past R decode row R - 1 again (never stored)
-        const int ptid = tid - 64 * NCW, rr = ptid >> 2, jb = ptid & 3, row = min(r0 + (gu ? rr & 31 : rr), a.R - 1), nbk = a.K / 8;
+        const int ptid = tid - 64 * NCW, rr = ptid >> 2, jb = ptid & 3, row = min(r0 + rr, a.R - 1), nbk = a.K / 8;
         // This thread's two blocks of step s.  Always the same loads - steps past the end request the last step again, and a
         // stream at any 2-byte boundary is read by the same instruction (the load is typed with that alignment) - so that the
         // compiler knows how many loads are in flight at every use: with the loads inside conditions it had waited, after
         // every third and fourth step, for the records it had requested a moment before.
         typedef uint32_t u32_a2 __attribute__((aligned(2)));
+        const size_t g0 = (size_t) row * nbk + 2 * jb;
+        const NSLM_GLOBAL uint8_t *pu = gp<uint8_t>(wt.p[0]) + 2 * g0, *pv = gp<uint8_t>(wt.p[1]) + 2 * g0, *pcd = gp<uint8_t>(wt.p[3]) + (g0 >> 1);
         auto load_rec = [&](int s_, MmRec2& r) {
             const int s = min(s_, nsteps - 1);
             if (seedf) {
-                const size_t g = (size_t) row * nbk + (size_t) s * (WK / 8) + 2 * jb;   // even: the pair shares a dword and a codes byte
-                r.u = *(const NSLM_GLOBAL u32_a2*) (gp<uint16_t>(wt.p[0]) + g);
-                r.v = *(const NSLM_GLOBAL u32_a2*) (gp<uint16_t>(wt.p[1]) + g);
-                if (FMT == MF_SEED4P4) r.c = gp<uint8_t>(wt.p[3])[g >> 1];
+                // (the pair shares a dword and a codes byte)
+                r.u = *(const NSLM_GLOBAL u32_a2*) (pu + (size_t) s * (WK / 4));
+                r.v = *(const NSLM_GLOBAL u32_a2*) (pv + (size_t) s * (WK / 4));
+                if (FMT == MF_SEED4P4) r.c = *(pcd + (size_t) s * (WK / 16));
                 return;
             }
             const size_t e0 = (size_t) row * a.K + (size_t) s * WK + 16 * jb;   // first of 16 elements
@@ -436,8 +443,7 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                 if (seedf) {
                     const uint32_t up[2] = {r.u << 16, r.u}, word[2] = {r.v & 0xFFFFu, r.v >> 16};
                     int is[2][8];
-                    if (FMT == MF_SEED4P4) isum2_p4(up, k.g, k.qa, k.qb, is);
-                    else isum2_p3(up, k.g, k.qa, k.qb, is);
+                    isum2_mad<FMT == MF_SEED4P4 ? 4 : 3>(up, k.g, k.qa, k.qb, is);
                     float sc[2];
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
@@ -522,14 +528,13 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
             for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.0f;
     // Chunk c = s MT + m is the 32 tokens of m-tile m x the 64 K of weight step s: 4 KB, four instructions, instruction i
     // landing rows 8 i + lane / 8, slot lane % 8 (whole 128-byte lines per row).  The wave's ring holds XCH chunks.
-    // Offsets from X are 32-bit where the host has checked that they fit (MT > 1), so the loads take the scalar base +
+    // Offsets from X are 32-bit (the host has checked that they fit), so the loads take the scalar base +
     // vector offset form and cost no address arithmetic.
-    typedef typename std::conditional<CT == 1, size_t, uint32_t>::type xoff_t;
-    xoff_t xoff[4 * CT];
+    uint32_t xoff[4 * CT];
 #pragma unroll
     for (int i = 0; i < 4 * CT; ++i) {
         const int row = 8 * (i & 3) + (lane >> 3), n = wtok + 32 * (i >> 2) + row, piece = (lane & 7) ^ x_swizzle(row);
-        xoff[i] = (xoff_t) (((size_t) srow[n] * (size_t) a.xs + 8u * (size_t) piece) * 2u);
+        xoff[i] = (uint32_t) (((size_t) srow[n] * (size_t) a.xs + 8u * (size_t) piece) * 2u);
     }
     uint16_t* ring = Xs + wv * (XCH * XCHUNK);
     auto fetch = [&](int sf, int mf, int slot) {   // chunk (sf, mf) -> ring slot (past the end: a harmless reload of the last step)
@@ -584,20 +589,6 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     wait_vm<0>();
     // accumulator element v of lane l: token row 8 * (v / 4) + 4 * (l / 32) + v % 4, weight column l % 32
     const bool plain = !a.add && !a.f32out;
-    if (gu) {   // n = 0: the gate rows, n = 1: the same rows of up, in the same lane: the values the two GEMMs would have stored
-                // (rounded to BF16), then SwiGLU and its rounding, stored as BF16 bits
-#pragma unroll
-        for (int m = 0; m < CT; ++m)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int tok = wtok + 32 * m + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                const int dst = drow[tok], orow = r0 + (lane & 31);
-                if (dst < 0 || orow >= a.R) continue;
-                const float av = bfr(silu_bf(bfr(acc[m][0][v])) * bfr(acc[m][1][v]));
-                a.a16[(size_t) dst * a.ys + orow] = (uint16_t) (__float_as_uint(av) >> 16);
-            }
-        return;
-    }
 #pragma unroll
     for (int m = 0; m < CT; ++m)
 #pragma unroll
@@ -618,28 +609,26 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
 template <int NCW, int XCH>
 constexpr size_t mm_stream_lds() { return (size_t) (NCW * XCH * XCHUNK + 2 * BM * LDW2) * sizeof(uint16_t); }
 // the streamed kernel takes BF16 activations in 16-byte aligned rows, one BF16 term per weight, K in whole weight steps
-// (xrows > 0: the row count, for the variants that address rows by 32-bit byte offsets)
+// (xrows: the row count - rows are addressed by 32-bit byte offsets)
 bool stream_ok(int fmt, int K, int xs, const void* x, long long xrows) {
     const bool exact = g_seed_exact && (fmt == MF_SEED4 || fmt == MF_SEED4P4);
     return !exact && K % WK == 0 && xs % 8 == 0 && ((uintptr_t) x & 15u) == 0 && (xrows * xs + K) * 2 < (1ll << 32);
 }
 template <int CT, int NCW, int XCH, int FMT>
-void launch_mm_stream_f(hipStream_t st, const MmArgs& a, WSlice wd, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
-                        const MmTile* tiles, const int32_t* ntiles, dim3 grid) {
+void launch_mm_stream_f(hipStream_t st, const MmArgs& a, WSlice w, const void* X, float* Y, dim3 grid) {
     const size_t lds = mm_stream_lds<NCW, XCH>();
     allow_big_lds<k_mm_stream<CT, NCW, XCH, FMT>>(lds);
-    hipLaunchKernelGGL((k_mm_stream<CT, NCW, XCH, FMT>), grid, dim3(64 * (NCW + 4)), lds, st, a, wd, ws, (const uint16_t*) X, Y, perm, tiles, ntiles);
+    hipLaunchKernelGGL((k_mm_stream<CT, NCW, XCH, FMT>), grid, dim3(64 * (NCW + 4)), lds, st, a, w, (const uint16_t*) X, Y);
     host_note_launch();
 }
 template <int CT, int NCW, int XCH>
-void launch_mm_stream(hipStream_t st, int fmt, const MmArgs& a, WSlice wd, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
-                      const MmTile* tiles, const int32_t* ntiles, dim3 grid) {
+void launch_mm_stream(hipStream_t st, int fmt, const MmArgs& a, WSlice w, const void* X, float* Y, dim3 grid) {
     switch (fmt) {
-        case MF_SEED4P4: launch_mm_stream_f<CT, NCW, XCH, MF_SEED4P4>(st, a, wd, ws, X, Y, perm, tiles, ntiles, grid); break;
-        case MF_SEED4: launch_mm_stream_f<CT, NCW, XCH, MF_SEED4>(st, a, wd, ws, X, Y, perm, tiles, ntiles, grid); break;
-        case MF_BF16: launch_mm_stream_f<CT, NCW, XCH, MF_BF16>(st, a, wd, ws, X, Y, perm, tiles, ntiles, grid); break;
-        case MF_Q8: launch_mm_stream_f<CT, NCW, XCH, MF_Q8>(st, a, wd, ws, X, Y, perm, tiles, ntiles, grid); break;
-        default: launch_mm_stream_f<CT, NCW, XCH, MF_Q4>(st, a, wd, ws, X, Y, perm, tiles, ntiles, grid); break;
+        case MF_SEED4P4: launch_mm_stream_f<CT, NCW, XCH, MF_SEED4P4>(st, a, w, X, Y, grid); break;
+        case MF_SEED4: launch_mm_stream_f<CT, NCW, XCH, MF_SEED4>(st, a, w, X, Y, grid); break;
+        case MF_BF16: launch_mm_stream_f<CT, NCW, XCH, MF_BF16>(st, a, w, X, Y, grid); break;
+        case MF_Q8: launch_mm_stream_f<CT, NCW, XCH, MF_Q8>(st, a, w, X, Y, grid); break;
+        default: launch_mm_stream_f<CT, NCW, XCH, MF_Q4>(st, a, w, X, Y, grid); break;
     }
 }
 
@@ -652,48 +641,65 @@ bool rows_ok(int fmt, int K, int xs, const void* x) {
 template <bool PACKED>
 void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, int xs, float* y, int ys, int T, int add) {
     if (T < 1 || R < 1) return;
-    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, nullptr, nullptr, nullptr};
+    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, 0, nullptr, nullptr, nullptr};
     const unsigned gx = (unsigned) (R + BM - 1) / BM;
     if (rows_ok<PACKED>(fmt, K, xs, x) && mm_rows_better(fmt, R, T)) {
         mm_rows_dense(st, fmt, a, w, x, PACKED, y);
         return;
     }
     if (PACKED && stream_ok(fmt, K, xs, x, T)) {
-        if (T > 256) launch_mm_stream<2, 8, 4>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, (unsigned) (T + 511) / 512));
-        else if (T > 128) launch_mm_stream<2, 4, 8>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
-        else launch_mm_stream<1, 4, 8>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
+        if (T > 256) launch_mm_stream<2, 8, 4>(st, fmt, a, w, x, y, dim3(gx, (unsigned) (T + 511) / 512));
+        else if (T > 128) launch_mm_stream<2, 4, 8>(st, fmt, a, w, x, y, dim3(gx, 1));
+        else launch_mm_stream<1, 4, 8>(st, fmt, a, w, x, y, dim3(gx, 1));
         return;
     }
     if (T > 256) launch_mm<4, PACKED>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, (unsigned) (T + 511) / 512));
     else if (T > 128) launch_mm<2, PACKED>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
     else launch_mm<1, PACKED>(st, fmt, a, w, nullptr, x, y, nullptr, nullptr, nullptr, dim3(gx, 1));
 }
-// A grouped launch's tiles of up to ROWS_MOST pairs go to the kernel for few tokens, which decodes as fast as the chip can (E 128, top-8,
-// d 2048, ff 768, P = 4: 64 rows 304 -> 255 us a layer step, 32 rows 245 -> 223) but passes over a tile's weights once every 32 pairs;
-// fuller tiles go to the streamed kernel, one decode a tile of up to 128 (512 rows, 32 pairs a tile: 434 there, 384 here).  The rule looks
-// at a tile alone.  A caller that bounds its tiles by 64 is spared the second launch.
+// Grouped launches, by what the caller says of its tiles (tile_rows, kernels_hip.h):
+//   up to 96 pairs: the kernel for few tokens, which decodes as fast as the chip can but passes over a tile's weights once every 32, 64 or 96
+//   pairs (E 128, top-8, d 2048, ff 768, P = 4, us a layer step against the streamed kernel's workgroups of 128 pairs: 64 rows 304 -> 237,
+//   512 rows - 32 pairs a tile - 387 -> 306);
+//   more than a tile holds: the tiles are mostly full - k_mm_wide, one decode for up to 256 pairs (2048 rows: 640 -> 507);
+//   nothing: both, tiles of up to ROWS_MOST pairs to the first, fuller ones to the other.
+// f32 activations have no k_mm_wide: there tiles of more than ROWS_MOST pairs take the first-generation kernel.
 #define ROWS_MOST 32
+#define ROWS_TILE 96
+template <class Rows, class Wide>
+void by_tiles(MmArgs& a, int tile_rows, Rows rows, Wide wide) {
+    if (tile_rows < 1) tile_rows = MMT_BN;
+    if (tile_rows > MMT_BN) wide(a);
+    else if (tile_rows <= ROWS_TILE) rows(a, tile_rows);
+    else {
+        a.least = a.most = ROWS_MOST;
+        a.paired = 1;
+        rows(a, tile_rows);
+        wide(a);
+    }
+}
 template <bool PACKED>
 void mm_grouped(hipStream_t st, int fmt, const WSlice* ws, int K, int R, const void* x, int xs, float* y, int ys, int xdiv,
                 const int32_t* perm, const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows,
                 const WSlice* ws2 = nullptr, float* y2 = nullptr) {
     if (grid_tiles < 1 || R < 1) return;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), 0, MMT_BN, ws2, y2, nullptr};
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), 0, MMT_BN, 0, ws2, y2, nullptr};
     WSlice none = {};
-    const dim3 grid((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles, ws2 ? 2u : 1u);
+    const dim3 grid((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles);
     if (rows_ok<PACKED>(fmt, K, xs, x)) {
-        if (tile_rows > 64) a.least = a.most = ROWS_MOST;
-        mm_rows_grouped(st, fmt, a, ws, x, PACKED, y, perm, tiles, ntiles, grid_tiles, tile_rows);
-        if (tile_rows <= 64) return;
-    }
-    if (PACKED && stream_ok(fmt, K, xs, x, 0)) {
-        launch_mm_stream<1, 4, 3>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
-        return;
+        if (PACKED) {
+            by_tiles(a, tile_rows, [&](const MmArgs& ar, int n) { mm_rows_grouped(st, fmt, ar, ws, x, true, y, perm, tiles, ntiles, grid_tiles, n); },
+                     [&](const MmArgs& aw) { mm_wide_grouped(st, fmt, aw, ws, (const uint16_t*) x, y, perm, tiles, ntiles, grid_tiles); });
+            return;
+        }
+        if (tile_rows > ROWS_TILE) a.least = a.most = ROWS_MOST;
+        mm_rows_grouped(st, fmt, a, ws, x, false, y, perm, tiles, ntiles, grid_tiles, tile_rows);
+        if (tile_rows <= ROWS_TILE) return;
     }
     a.ws2 = nullptr;   // (the first-generation kernel takes one matrix a launch)
     a.y2 = nullptr;
-    launch_mm<1, PACKED>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, dim3(grid.x, grid.y));
-    if (ws2) launch_mm<1, PACKED>(st, fmt, a, none, ws2, x, y2, perm, tiles, ntiles, dim3(grid.x, grid.y));
+    launch_mm<1, PACKED>(st, fmt, a, none, ws, x, y, perm, tiles, ntiles, grid);
+    if (ws2) launch_mm<1, PACKED>(st, fmt, a, none, ws2, x, y2, perm, tiles, ntiles, grid);
 }
 
 }   // namespace
@@ -737,14 +743,10 @@ void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, 
 int kc_mm_grouped_swiglu(kc_stream_t s, int fmt, const WSlice* gate, const WSlice* up, int K, int R, const uint16_t* x, int xs, uint16_t* a16,
                          int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows) {
     if (max_tiles < 1 || R < 1) return 0;
-    if (!stream_ok(fmt, K, xs, x, 0) || host_store_f32()) return -1;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, 0, MMT_BN, up, nullptr, a16};
-    if (tile_rows < 1) tile_rows = MMT_BN;
-    if (tile_rows > 64) a.least = a.most = ROWS_MOST;   // (as in mm_grouped)
-    mm_rows_grouped((hipStream_t) s, fmt, a, gate, x, true, nullptr, perm, tiles, nt, max_tiles, tile_rows);
-    WSlice none = {};
-    const dim3 grid((unsigned) (R + BM / 2 - 1) / (BM / 2), (unsigned) max_tiles);
-    if (tile_rows > 64) launch_mm_stream<1, 4, 3>((hipStream_t) s, fmt, a, none, gate, x, nullptr, perm, tiles, nt, grid);
+    if (!rows_ok<true>(fmt, K, xs, x) || host_store_f32()) return -1;
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, 0, MMT_BN, 0, up, nullptr, a16};
+    by_tiles(a, tile_rows, [&](const MmArgs& ar, int n) { mm_rows_grouped((hipStream_t) s, fmt, ar, gate, x, true, nullptr, perm, tiles, nt, max_tiles, n); },
+             [&](const MmArgs& aw) { mm_wide_grouped((hipStream_t) s, fmt, aw, gate, x, nullptr, perm, tiles, nt, max_tiles); });
     return 0;
 }
 void kc_mm_grouped_packed_pair(kc_stream_t s, int fmt, const WSlice* ws_a, const WSlice* ws_b, int K, int R, const uint16_t* x, int xs,

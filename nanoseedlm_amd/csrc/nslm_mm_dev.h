@@ -14,7 +14,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct MmArgs {
     int K, R, T, xs, ys, xdiv, add, f32out;
-    int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's
+    int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's;
+    int paired;          // so is, where adjoining tiles of a slice go in pairs, the second of a pair
     const WSlice* ws2;   // grouped launches of two matrices over the same tiles (grid.z = 2): the second slice table ..
     float* y2;           // .. and its output
     uint16_t* a16;       // non-null: a workgroup's weight rows are gate rows (ws) and the same rows of up (ws2), half and half, and what
@@ -24,6 +25,19 @@ struct MmArgs {
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
     const f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// half ha of a x half hb of b, int16, + c (ha, hb: constants once unrolled; the first product of a sum takes its zero inline)
+#define NSLM_MAD16(HA, HB)                                                                                                                             \
+    if (first) asm("v_mad_i32_i16 %0, %1, %2, 0 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b));                                              \
+    else asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b), "v"(c))
+__device__ __forceinline__ int mad16(uint32_t a, int ha, uint32_t b, int hb, int c, bool first) {
+    int d;
+    if (ha && hb) { NSLM_MAD16(1, 1); }
+    else if (ha) { NSLM_MAD16(1, 0); }
+    else if (hb) { NSLM_MAD16(0, 1); }
+    else { NSLM_MAD16(0, 0); }
+    return d;
 }
 
 // a kernel that asks for more dynamic LDS than the default limit has the limit raised to what it needs, once (the kernel is a
@@ -43,5 +57,8 @@ bool mm_rows_better(int fmt, int R, int T);
 void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, const void* X, bool packed, float* Y);
 void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
                      const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows);
+
+void mm_wide_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
+                     const int32_t* ntiles, int grid_tiles);
 
 }   // namespace nslm

@@ -42,46 +42,195 @@ __device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
 }
 
+// A seed block as BF16 weights; up: any word whose upper 16 bits are the seed.  hook(0 .. 7) is called between the phases: a caller with
+// matrix instructions to issue puts them there, where the vector ALU has work beside them.
+// isum_p4's / isum_p3's sums by multiply-adds on the halves where they are: as many instructions as pairing halves for dot products, but a
+// dot product runs on the matrix pipe and waits there for, and holds up, every wave's MFMAs.
+template <int FMT, class Hook>
+__device__ __forceinline__ bf16x8 seed_weights(uint32_t up, uint32_t seed, uint32_t word, uint32_t code, int eb, const uint32_t* tab, Hook hook) {
+    constexpr int P = FMT == MF_SEED4P4 ? 4 : 3;
+    const uint32_t gs = stream_of(tab, seed), qa = P == 4 ? tab[512 + (word & 0xFFu)] : tab[512 + ((word >> 4) & 0xFFu)],
+                   qb = P == 4 ? tab[512 + (word >> 8)] : tab[512 + (word >> 12)];
+    const float e = pow2f(eb + (int) code) * NSLM_R32;
+    hook(0);
+    uint32_t A[17];
+#pragma unroll
+    for (int k = 1; k <= 15; ++k) A[k] = __builtin_amdgcn_alignbit(gs, up, 16 + k);
+    A[16] = gs;
+    hook(1);
+#pragma unroll
+    for (int k = 1; k <= 16; ++k) A[k] ^= 0x80008000u;
+    int is[8];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        hook(2 + p);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int k = P * c + 1 + p;   // state k: A[k]'s low half, or A[k - 16]'s high half
+            is[c] = mad16(A[k <= 16 ? k : k - 16], k > 16, p < 2 ? qa : qb, p & 1, p ? is[c] : 0, p == 0);
+        }
+    }
+    if (P == 3) hook(5);
+    hook(6);
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = (float) is[i];
+    hook(7);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] *= e;
+    return __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
+}
+// eight Q4 (q.x) or Q8 weights
+template <int FMT>
+__device__ __forceinline__ bf16x8 affine_weights(uint2 q, float scale, float bias) {
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t v = FMT == MF_Q8 ? ((i < 4 ? q.x : q.y) >> (8 * (i & 3))) & 255u : (q.x >> (4 * i)) & 15u;
+        f[i] = scale * (float) v + bias;
+    }
+    return __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
+}
+
+// A wave's weights: 16 RT rows from r0 (with gu: 8 RT gate rows of m0 and the same 8 RT rows of up, m1), a chunk a step, staged in the wave's
+// own part of the LDS.
+template <int FMT, int RT>
+struct Weights {
+    static constexpr bool SEED = seed_fmt<FMT>();
+    static constexpr int RB = row_bytes<FMT>(), CODES = 16 * RT * RB;
+    static constexpr int NA = SEED || FMT == MF_Q4 ? (RT + 1) / 2 : FMT == MF_Q8 ? RT : 2 * RT;   // 16-byte loads a step
+    const WSlice &m0, &m1;
+    const bool gu;
+    const int K, R, r0, lane, t, g;
+    const uint8_t *pa[NA], *pcode;   // the lane's addresses in chunk 0
+    uint32_t sc[RT], bi[RT];         // Q4 / Q8: scale and bias bits of the step that is staged
+    bool aligned;
+    // what a step's decode reads.  u, v, cd: two seeds, two words, their codes; Q4 / Q8: scale and bias.  raw: BF16: the two blocks; Q8: [0]; Q4: [0].xy
+    struct Step {
+        uint32_t u[RT], v[RT], cd[RT];
+        uint4 raw[RT][2];
+    };
+
+    __device__ __forceinline__ int row_of(int i) const { return min(r0 + (gu ? i % (8 * RT) : i), R - 1); }   // rows past R: the last one again, never stored
+    __device__ __forceinline__ bool second(int rt) const { return gu && rt >= RT / 2; }
+    __device__ __forceinline__ const uint8_t* stream(int rt, int s) const { return (const uint8_t*) (second(rt) ? m1.p[s] : m0.p[s]); }
+
+    __device__ __forceinline__ Weights(const WSlice& a_, const WSlice& b_, bool gu_, int K_, int R_, int r0_, int lane_)
+        : m0(a_), m1(b_), gu(gu_), K(K_), R(R_), r0(r0_), lane(lane_), t(lane_ & 15), g(lane_ >> 4) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            if constexpr (SEED) {   // groups of 16 lanes: seeds, words of row tile 2i, the same of 2i + 1
+                const int rt = min(2 * i + (g >> 1), RT - 1);
+                pa[i] = ((g & 1) ? stream(rt, 1) : stream(rt, 0)) + (size_t) row_of(16 * rt + t) * (size_t) (K / 4);
+            } else {
+                const int at = 1024 * i + 16 * lane, r = min(at / RB, 16 * RT - 1), piece = (at % RB) / 16;
+                const int sw = FMT == MF_BF16 ? piece ^ x_swizzle(r & 15) : FMT == MF_Q8 ? piece ^ ((r >> 2) & 3) : piece;
+                pa[i] = stream(r >> 4, 0) + (size_t) row_of(r) * (size_t) (K / 64 * RB) + 16 * sw;
+            }
+        }
+        if constexpr (FMT == MF_SEED4P4) {
+            const int rt = min(g, RT - 1);
+            pcode = stream(rt, 3) + (size_t) row_of(16 * rt + t) * (size_t) (K / 16);
+        }
+        // streams may start at any 2-byte (codes: any) boundary; those that are not aligned go through registers
+        auto low = [&](const WSlice& m) { return (uintptr_t) m.p[0] | (SEED ? (uintptr_t) m.p[1] : 0) | (FMT == MF_SEED4P4 ? ((uintptr_t) m.p[3] & 3u) << 2 : 0); };
+        aligned = ((low(m0) | (gu ? low(m1) : 0)) & 15u) == 0;
+    }
+    __device__ __forceinline__ void request(int c, uint8_t* ws) {   // chunk c -> the LDS at ws
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const uint8_t* src = pa[i] + (size_t) c * (SEED ? 16 : RB);
+            if (!((SEED || FMT == MF_Q4) && 2 * i + 1 == RT) || lane < 32) {   // (an odd row tile: half a load)
+                if (aligned) to_lds16(src, ws + 1024 * i);
+                else *(u32x4*) (ws + 1024 * i + 16 * lane) = *(const NSLM_GLOBAL u32x4_a2*) src;
+            }
+        }
+        if constexpr (FMT == MF_SEED4P4) {
+            if (RT >= 4 || lane < 16 * RT) {
+                if (aligned) to_lds4(pcode + 4 * (size_t) c, ws + CODES);
+                else *(uint32_t*) (ws + CODES + 4 * lane) = *(const NSLM_GLOBAL u32_a1*) (pcode + 4 * (size_t) c);
+            }
+        }
+        if constexpr (FMT == MF_Q4 || FMT == MF_Q8) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const size_t gi = ((size_t) row_of(16 * rt + t) * K + (size_t) c * 64 + 16 * g) >> (second(rt) ? group_shift(m1) : group_shift(m0));
+                sc[rt] = gp<uint16_t>(stream(rt, 1))[gi];
+                bi[rt] = gp<uint16_t>(stream(rt, 2))[gi];
+            }
+        }
+    }
+    __device__ __forceinline__ void read(const uint8_t* ws, Step& s) const {   // a step that has landed, into registers
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            if constexpr (SEED) {
+                s.u[rt] = *(const uint32_t*) (ws + 512 * rt + 16 * t + 4 * g);
+                s.v[rt] = *(const uint32_t*) (ws + 512 * rt + 256 + 16 * t + 4 * g);
+                if (FMT == MF_SEED4P4) s.cd[rt] = ws[CODES + 64 * rt + 4 * t + g];
+            } else if constexpr (FMT == MF_BF16) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) s.raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+            } else {
+                s.u[rt] = sc[rt];
+                s.v[rt] = bi[rt];
+                if (FMT == MF_Q8) s.raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ ((t >> 2) & 3)));
+                else {
+                    const uint2 b = *(const uint2*) (ws + 512 * rt + 32 * t + 8 * g);
+                    s.raw[rt][0] = make_uint4(b.x, b.y, 0, 0);
+                }
+            }
+        }
+    }
+    template <class Hook>
+    __device__ __forceinline__ bf16x8 block(const Step& s, int rt, int h, const uint32_t* tab, Hook hook) const {   // the lane's block 2 g + h of the chunk's eight
+        if constexpr (SEED) {
+            const uint32_t word = h ? s.v[rt] >> 16 : s.v[rt] & 0xFFFFu;
+            return seed_weights<FMT>(h ? s.u[rt] : s.u[rt] << 16, h ? s.u[rt] >> 16 : s.u[rt] & 0xFFFFu, word,
+                                     FMT == MF_SEED4P4 ? (s.cd[rt] >> (4 * h)) & 15u : word & 15u, second(rt) ? m1.eb : m0.eb, tab, hook);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) hook(i);
+            const uint4& r = s.raw[rt][0];
+            if constexpr (FMT == MF_BF16) return __builtin_bit_cast(bf16x8, s.raw[rt][h]);
+            else return affine_weights<FMT>(FMT == MF_Q8 ? (h ? make_uint2(r.z, r.w) : make_uint2(r.x, r.y)) : make_uint2(h ? r.y : r.x, 0), bf(s.u[rt]), bf(s.v[rt]));
+        }
+    }
+    __device__ __forceinline__ bf16x8 block(const Step& s, int rt, int h, const uint32_t* tab) const { return block(s, rt, h, tab, [](int) {}); }
+};
+
+// four sums of pair / token dst, rows orow .. orow + 3 (those below R)
+__device__ __forceinline__ void store_rows(const MmArgs& a, float* Y, int dst, int orow, const f32x4& s) {
+    float* yo = Y + (size_t) dst * a.ys + orow;
+    if ((a.ys & 3) == 0 && orow + 4 <= a.R && !a.add && !a.f32out && ((uintptr_t) yo & 15u) == 0) *(f32x4*) yo = (f32x4) {bfr(s[0]), bfr(s[1]), bfr(s[2]), bfr(s[3])};
+    else
+        for (int j = 0; j < 4 && orow + j < a.R; ++j) store_y(yo + j, s[j], a.add, a.f32out);
+}
+// the values the two GEMMs would have stored (rounded to BF16), then SwiGLU and its rounding, stored as BF16 bits
+__device__ __forceinline__ void store_swiglu(const MmArgs& a, int dst, int orow, const f32x4& gate, const f32x4& up) {
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(bfr(silu_bf(bfr(gate[j])) * bfr(up[j]))) >> 16;
+    uint16_t* ao = a.a16 + (size_t) dst * a.ys + orow;
+    if ((a.ys & 3) == 0 && orow + 4 <= a.R && ((uintptr_t) ao & 7u) == 0) *(uint2*) ao = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+    else
+        for (int j = 0; j < 4 && orow + j < a.R; ++j) ao[j] = (uint16_t) v[j];
+}
+
 // The 16 RT rows from r0 (with a.a16: 8 RT gate rows and the same 8 RT up rows) x the 16 NT tokens n0 .. of a workgroup of NW waves.
 // lds: NW x max(step, RT NT KB).
 template <int FMT, int RT, int NT, int NW, bool PACKED, bool GROUPED>
 __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, const WSlice& m1, const void* X, float* Y, const int32_t* perm, int start, int count,
                                           int n0, int r0, const uint32_t* tab, uint8_t* lds) {
-    constexpr bool SEED = seed_fmt<FMT>();
-    constexpr int RB = row_bytes<FMT>();
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x & (64 * NW - 1), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
     const bool gu = GROUPED && a.a16 != nullptr;
     const int nch = a.K / 64;
+    Weights<FMT, RT> W(m0, m1, gu, a.K, a.R, r0, lane);
     uint8_t* const ws = lds + w * step_bytes<FMT, RT, NT, PACKED>();
-    uint8_t* const wc = ws + 16 * RT * RB;                                     // codes
-    uint8_t* const wx = wc + (FMT == MF_SEED4P4 ? 64 * RT : 0);                // activations
-    // rows past R: the last one again, never stored
-    auto row_of = [&](int i) { return min(r0 + (gu ? i % (8 * RT) : i), a.R - 1); };   // i: row of the workgroup's 16 RT
-    auto second = [&](int rt) { return gu && rt >= RT / 2; };   // a row tile of the second matrix (up)
-    auto stream = [&](int rt, int s) { return (const uint8_t*) (second(rt) ? m1.p[s] : m0.p[s]); };
+    uint8_t* const wx = ws + step_bytes<FMT, RT, NT, false>();   // activations
     auto src_of = [&](int i) {   // token i of the tile's 16 NT (past the end: the last one again, never stored)
         const int n = start + min(n0 + i, count - 1);
         return (size_t) (GROUPED ? perm[n] / a.xdiv : n) * (size_t) a.xs;
     };
-    // the lane's addresses in chunk 0
-    constexpr int NA = SEED || FMT == MF_Q4 ? (RT + 1) / 2 : FMT == MF_Q8 ? RT : 2 * RT;   // 16-byte weight loads a step
-    const uint8_t* pa[NA];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        if constexpr (SEED) {   // groups of 16 lanes: seeds, words of row tile 2i, the same of 2i + 1
-            const int rt = min(2 * i + (g >> 1), RT - 1);
-            pa[i] = ((g & 1) ? stream(rt, 1) : stream(rt, 0)) + (size_t) row_of(16 * rt + t) * (size_t) (a.K / 4);
-        } else {
-            const int at = 1024 * i + 16 * lane, r = min(at / RB, 16 * RT - 1), piece = (at % RB) / 16;
-            const int sw = FMT == MF_BF16 ? piece ^ x_swizzle(r & 15) : FMT == MF_Q8 ? piece ^ ((r >> 2) & 3) : piece;
-            pa[i] = stream(r >> 4, 0) + (size_t) row_of(r) * (size_t) (a.K / 64 * RB) + 16 * sw;
-        }
-    }
-    const uint8_t* pcode = nullptr;
-    if constexpr (FMT == MF_SEED4P4) {
-        const int rt = min(g, RT - 1);
-        pcode = stream(rt, 3) + (size_t) row_of(16 * rt + t) * (size_t) (a.K / 16);
-    }
     uint32_t px[PACKED ? 2 * NT : NT];   // in 16-byte pieces
     if constexpr (PACKED) {
 #pragma unroll
@@ -93,135 +242,71 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) px[nt] = (uint32_t) (src_of(16 * nt + t) >> 2) + 4u * (uint32_t) g;
     }
-    uint32_t sc[RT], bi[RT];   // Q4 / Q8: scale and bias bits of the step that is staged
-    // streams may start at any 2-byte (codes: any) boundary; those that are not aligned go through registers
-    auto low = [&](const WSlice& m) { return (uintptr_t) m.p[0] | (SEED ? (uintptr_t) m.p[1] : 0) | (FMT == MF_SEED4P4 ? ((uintptr_t) m.p[3] & 3u) << 2 : 0); };
-    const bool aligned = ((low(m0) | (GROUPED ? low(m1) : 0)) & 15u) == 0;
     auto request = [&](int c) {
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            const uint8_t* src = pa[i] + (size_t) c * (SEED ? 16 : RB);
-            if (!((SEED || FMT == MF_Q4) && 2 * i + 1 == RT) || lane < 32) {   // (an odd row tile: half a load)
-                if (aligned) to_lds16(src, ws + 1024 * i);
-                else *(u32x4*) (ws + 1024 * i + 16 * lane) = *(const NSLM_GLOBAL u32x4_a2*) src;
-            }
-        }
-        if constexpr (FMT == MF_SEED4P4) {
-            if (RT >= 4 || lane < 16 * RT) {
-                if (aligned) to_lds4(pcode + 4 * (size_t) c, wc);
-                else *(uint32_t*) (wc + 4 * lane) = *(const NSLM_GLOBAL u32_a1*) (pcode + 4 * (size_t) c);
-            }
-        }
+        W.request(c, ws);
         if constexpr (PACKED) {
 #pragma unroll
             for (int i = 0; i < 2 * NT; ++i) to_lds16((const uint8_t*) X + (size_t) (px[i] + 8u * (uint32_t) c) * 16, wx + 1024 * i);
         }
-        if constexpr (FMT == MF_Q4 || FMT == MF_Q8) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const size_t gi = ((size_t) row_of(16 * rt + t) * a.K + (size_t) c * 64 + 16 * g) >> (second(rt) ? group_shift(m1) : group_shift(m0));
-                sc[rt] = gp<uint16_t>(stream(rt, 1))[gi];
-                bi[rt] = gp<uint16_t>(stream(rt, 2))[gi];
-            }
-        }
     };
-    f32x4 acc[RT][NT], tot[RT][NT];
+    constexpr bool SEGS = NW == 4 && NT < 4;   // (four token tiles: one chain a wave, and half a step's activations at a time - the registers)
+    f32x4 acc[RT][NT], tot[SEGS ? RT : 1][SEGS ? NT : 1];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = tot[rt][nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int nt = 0; nt < NT; ++nt) {
+            acc[rt][nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+            if (SEGS) tot[rt][nt] = acc[rt][nt];
+        }
     const int n = (nch - w + NW - 1) / NW;   // this wave's chunks: those of segment w, then (4 waves) of segment w + 4
     int c = w;
     auto next = [&](int at) { at += 8; if (NW == 4 && at >= nch) at = at % 8 >= 4 ? nch : w + 4; return at; };
     if (n > 0) request(c);
     for (int s = 0; s < n; ++s) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        bf16x8 xb[2][NT];
-        if constexpr (PACKED) {
+        constexpr bool HALVES = NW == 4 && NT >= 4;
+        bf16x8 xb[HALVES ? 1 : 2][NT];
+        auto read_x = [&](int h) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) xb[h][nt] = *(const bf16x8*) (wx + nt * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
+            for (int nt = 0; nt < NT; ++nt) {
+                if constexpr (PACKED) {
+                    xb[HALVES ? 0 : h][nt] = *(const bf16x8*) (wx + nt * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+                } else {
                     const NSLM_GLOBAL uint8_t* xp = gp<uint8_t>(X) + (size_t) (px[nt] + 16u * (uint32_t) c + 2u * h) * 16;
                     const uint4 va = ldg16(xp), vb = ldg16(xp + 16);
 #define F(w) __uint_as_float(w)
-                    xb[h][nt] = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(F(va.x), F(va.y)), cvt_pk_bf16(F(va.z), F(va.w)),
-                                                                      cvt_pk_bf16(F(vb.x), F(vb.y)), cvt_pk_bf16(F(vb.z), F(vb.w))));
+                    xb[HALVES ? 0 : h][nt] = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(F(va.x), F(va.y)), cvt_pk_bf16(F(va.z), F(va.w)),
+                                                                                   cvt_pk_bf16(F(vb.x), F(vb.y)), cvt_pk_bf16(F(vb.z), F(vb.w))));
 #undef F
                 }
-        }
-        uint32_t u[RT], v[RT], cd[RT];   // seeds: two seeds, two words, their codes.  Q4 / Q8: scale and bias
-        uint4 raw[RT][2];                // BF16: the two blocks; Q8: raw[0]; Q4: raw[0].xy
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            if constexpr (SEED) {
-                u[rt] = *(const uint32_t*) (ws + 512 * rt + 16 * t + 4 * g);
-                v[rt] = *(const uint32_t*) (ws + 512 * rt + 256 + 16 * t + 4 * g);
-                if (FMT == MF_SEED4P4) cd[rt] = wc[64 * rt + 4 * t + g];
-            } else if constexpr (FMT == MF_BF16) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
-            } else {
-                u[rt] = sc[rt];
-                v[rt] = bi[rt];
-                if (FMT == MF_Q8) raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ ((t >> 2) & 3)));
-                else {
-                    const uint2 b = *(const uint2*) (ws + 512 * rt + 32 * t + 8 * g);
-                    raw[rt][0] = make_uint4(b.x, b.y, 0, 0);
-                }
             }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the step is in registers: its place is free
+        };
+        read_x(0);
+        if (!HALVES) read_x(1);
+        typename Weights<FMT, RT>::Step st;
+        W.read(ws, st);
         const int cn = next(c);
-        if (s + 1 < n) request(cn);
-        loads_issued();
+        auto go_on = [&]() {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the step is in registers: its place is free
+            if (s + 1 < n) request(cn);
+            loads_issued();
+        };
+        if (!HALVES) go_on();
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+            if (HALVES && h) {
+                read_x(1);
+                go_on();
+            }
             bf16x8 wb[RT];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                if constexpr (FMT == MF_BF16) {
-                    wb[rt] = __builtin_bit_cast(bf16x8, raw[rt][h]);
-                    continue;
-                }
-                float f[8];
-                if constexpr (SEED) {
-                    const uint32_t seed = h ? u[rt] >> 16 : u[rt] & 0xFFFFu, word = h ? v[rt] >> 16 : v[rt] & 0xFFFFu, up = h ? u[rt] : u[rt] << 16;
-                    const uint32_t gs = stream_of(tab, seed);
-                    int is[8], code;
-                    if (FMT == MF_SEED4P4) {
-                        isum_p4(up, gs, tab[512 + (word & 0xFFu)], tab[512 + (word >> 8)], is);
-                        code = (int) ((cd[rt] >> (4 * h)) & 15u);
-                    } else {
-                        isum_p3(up, gs, tab[512 + ((word >> 4) & 0xFFu)], tab[512 + (word >> 12)], is);
-                        code = (int) (word & 15u);
-                    }
-                    const float e = pow2f((second(rt) ? m1.eb : m0.eb) + code) * NSLM_R32;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) f[i] = (float) is[i] * e;
-                } else {
-                    const float e = bf(u[rt]), b = bf(v[rt]);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const uint4& r = raw[rt][0];
-                        const uint32_t qv = FMT == MF_Q8 ? ((h ? (i < 4 ? r.z : r.w) : (i < 4 ? r.x : r.y)) >> (8 * (i & 3))) & 255u
-                                                         : ((h ? r.y : r.x) >> (4 * i)) & 15u;
-                        f[i] = e * (float) qv + b;
-                    }
-                }
-                wb[rt] = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
-            }
+            for (int rt = 0; rt < RT; ++rt) wb[rt] = W.block(st, rt, h, tab);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], xb[h][nt], acc[rt][nt], 0, 0, 0);
+                for (int rt = 0; rt < RT; ++rt) acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], xb[HALVES ? 0 : h][nt], acc[rt][nt], 0, 0, 0);
         }
-        if (NW == 4 && c < nch && c + 8 >= nch) {   // the segment is complete
+        if (SEGS && c < nch && c + 8 >= nch) {   // the segment is complete
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -238,7 +323,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) red[((w * RT + rt) * NT + nt) * 64 + lane] = NW == 4 ? tot[rt][nt] : acc[rt][nt];
+        for (int nt = 0; nt < NT; ++nt) red[((w * RT + rt) * NT + nt) * 64 + lane] = SEGS ? tot[rt][nt] : acc[rt][nt];
     __syncthreads();
     auto sum = [&](int tile, int l) {
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -255,24 +340,106 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
         const int tile = i >> 6, l = i & 63, rt = tile / NT, nt = tile % NT, tok = n0 + 16 * nt + (l & 15), orow = r0 + 16 * rt + 4 * (l >> 4);
         if (tok >= count || orow >= a.R) continue;
         const int dst = GROUPED ? perm[start + tok] : start + tok;
-        const f32x4 s = sum(tile, l);
-        const bool vec = (a.ys & 3) == 0 && orow + 4 <= a.R;
-        if (gu) {   // the values the two GEMMs would have stored (rounded to BF16), then SwiGLU and its rounding, stored as BF16 bits
-            const f32x4 up = sum(tile + RT / 2 * NT, l);
-            uint32_t v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(bfr(silu_bf(bfr(s[j])) * bfr(up[j]))) >> 16;
-            uint16_t* ao = a.a16 + (size_t) dst * a.ys + orow;
-            if (vec && ((uintptr_t) ao & 7u) == 0) *(uint2*) ao = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
-            else
-                for (int j = 0; j < 4 && orow + j < a.R; ++j) ao[j] = (uint16_t) v[j];
-            continue;
-        }
-        float* yo = Y + (size_t) dst * a.ys + orow;
-        if (vec && !a.add && !a.f32out && ((uintptr_t) yo & 15u) == 0) *(f32x4*) yo = (f32x4) {bfr(s[0]), bfr(s[1]), bfr(s[2]), bfr(s[3])};
-        else
-            for (int j = 0; j < 4 && orow + j < a.R; ++j) store_y(yo + j, s[j], a.add, a.f32out);
+        if (gu) store_swiglu(a, dst, orow, sum(tile, l), sum(tile + RT / 2 * NT, l));
+        else store_rows(a, Y, dst, orow, sum(tile, l));
     }
+}
+
+// ---- fuller tiles of a grouped launch -----------------------------------------------------------------------------------------------
+// Up to 256 pairs of an expert - two table tiles - against 128 weight rows (64 gate and 64 up) a workgroup, so that an expert's weights are
+// decoded once.  Each of the 8 waves decodes its own 16 rows into operands and multiplies them with every pair; the pairs' activations of a step
+// sit once a workgroup in one of two LDS buffers, and the waves meet at one barrier a step, where the buffer before the last is free.
+// Two workgroups a CU, four waves a SIMD: 16 rows a wave leave the registers for that (64 of accumulators at 256 pairs), and the decode
+// needs them - with 32 rows and two waves a SIMD a block took 650 clocks instead of 430.
+template <int FMT, int NT>
+constexpr int wide_lds() { return 2 * (NT * 2048 + 8 * step_bytes<FMT, 1, NT, false>()); }
+template <int FMT, int NT>
+__device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, const uint16_t* X, float* Y, const int32_t* perm, int start, int count,
+                                          int r0, const uint32_t* tab, uint8_t* lds) {
+    constexpr int SB = step_bytes<FMT, 1, NT, false>();
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
+    const bool gu = a.a16 != nullptr;   // waves 0 - 3: gate rows, 4 - 7: the same rows of up
+    const int nch = a.K / 64, rw = r0 + 16 * (gu ? w & 3 : w);
+    Weights<FMT, 1> W(m, m, false, a.K, a.R, rw, lane);
+    uint8_t* const ws = lds + 2 * NT * 2048 + w * 2 * SB;
+    uint32_t px[NT / 4];   // in 16-byte pieces: the wave stages eight pairs' rows of every 64
+#pragma unroll
+    for (int i = 0; i < NT / 4; ++i) {
+        const int n = 64 * i + 8 * w + (lane >> 3);
+        px[i] = (uint32_t) (((size_t) (perm[start + min(n, count - 1)] / a.xdiv) * (size_t) a.xs) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle(n & 15));
+    }
+    auto request_x = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NT / 4; ++i) to_lds16((const uint8_t*) X + (size_t) (px[i] + 8u * (uint32_t) c) * 16, lds + (c & 1) * NT * 2048 + 1024 * (8 * i + w));
+    };
+    f32x4 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
+    // The matrix instructions of half a chunk are issued among the vector instructions that decode the next half.  A wave's records run a chunk
+    // ahead of its activations.
+    constexpr int NG = (NT + 7) / 8;   // token tiles a hook
+    constexpr int XD = 2;               // hooks a fragment is read ahead of its use
+    typename Weights<FMT, 1>::Step st;
+    bf16x8 wb, xq[XD][NG];
+    auto half = [&](int c, int h) {   // multiplies (c, h) while the next half's weights are formed
+        const uint8_t* const xt = lds + (c & 1) * NT * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t));
+        auto fetch = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < NG; ++j)
+                if (i < 8 && NG * i + j < NT) xq[i % XD][j] = *(const bf16x8*) (xt + (NG * i + j) * 2048);
+        };
+#pragma unroll
+        for (int i = 0; i < XD; ++i) fetch(i);
+        wb = W.block(st, 0, h ^ 1, tab, [&](int i) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NG; ++j)
+                if (NG * i + j < NT) acc[NG * i + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, xq[i % XD][j], acc[NG * i + j], 0, 0, 0);
+            fetch(i + XD);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    W.request(0, ws);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    W.read(ws, st);
+    wb = W.block(st, 0, 0, tab, [](int) {});
+    request_x(0);
+    if (nch > 1) W.request(1, ws + SB);
+    for (int c = 0; c < nch; ++c) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the activations of chunk c have landed, those of c - 1 are read
+        if (c + 1 < nch) request_x(c + 1);
+        half(c, 0);
+        if (c + 1 < nch) W.read(ws + ((c + 1) & 1) * SB, st);
+        if (c + 2 < nch) W.request(c + 2, ws + (c & 1) * SB);
+        loads_issued();
+        half(c, 1);   // (past the end: some block again)
+    }
+    const int orow = rw + 4 * g;
+    if (gu) {   // the up sums meet the gate sums in LDS
+        f32x4* const red = (f32x4*) lds;
+        __syncthreads();
+        if (w >= 4) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) red[((w - 4) * NT + nt) * 64 + lane] = acc[nt];
+        }
+        __syncthreads();
+        if (w >= 4) return;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            if (16 * nt + t < count && orow < a.R) store_swiglu(a, perm[start + 16 * nt + t], orow, acc[nt], red[(w * NT + nt) * 64 + lane]);
+        return;
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+        if (16 * nt + t < count && orow < a.R) store_rows(a, Y, perm[start + 16 * nt + t], orow, acc[nt]);
+}
+
+// An expert's tiles go in pairs where another launch takes them so: the tile's place (0, 1, 2, ..) in its run of adjoining tiles
+__device__ __forceinline__ bool follows(const MmTile& b, const MmTile& a) { return b.slice == a.slice && b.start == a.start + a.count; }
+__device__ __forceinline__ int place_of(const MmTile* tiles, int y) {
+    int n = 0;
+    for (; y > 0 && follows(tiles[y], tiles[y - 1]); --y) ++n;
+    return n;
 }
 
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
@@ -292,16 +459,17 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
 }
 
 #define GRT 2   // row tiles of the grouped kernel's workgroups
-template <int FMT, bool PACKED>
-__global__ void __launch_bounds__(256, 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles,
-                                                            const int32_t* ntiles, int limit) {
+// MOST: token tiles a pass.  Two (or four): four waves a SIMD.  Six: three, what their LDS leaves.
+template <int FMT, int MOST, bool PACKED>
+__global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
+                                                                           const MmTile* tiles, const int32_t* ntiles, int limit) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     if (ntiles && (int) blockIdx.y >= *ntiles) return;
     const bool gu = a.a16 != nullptr;
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
     const MmTile tl = tiles[blockIdx.y];
-    if (tl.count > a.most) return;   // another launch's
+    if (tl.count > a.most || (a.paired && (place_of(tiles, (int) blockIdx.y) & 1))) return;   // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -321,11 +489,50 @@ __global__ void __launch_bounds__(256, 4) k_mm_rows_grouped(MmArgs a, const WSli
         load_tables(tab);
         __syncthreads();
     }
-    for (int n0 = 0; n0 < count; n0 += 32) {
+    for (int n0 = 0; n0 < count; n0 += 16 * MOST) {
         if (n0) __syncthreads();   // the sums of the tokens before are read
-        if (count - n0 <= 16) rows_tile<FMT, GRT, 1, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds);
-        else rows_tile<FMT, GRT, 2, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds);
+        const int left = count - n0;
+#define T(NT) rows_tile<FMT, GRT, NT, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds)
+        if (left <= 16) T(1);
+        else if (MOST == 2 || left <= 32) T(2);
+        else if constexpr (MOST == 4) T(4);
+        else if constexpr (MOST == 6) {
+            if (left <= 64) T(4);
+            else T(6);
+        }
+#undef T
     }
+}
+
+// A grouped launch's tiles of more than a.least pairs, each with the tile that follows it
+template <int FMT>
+__global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
+                                                    const int32_t* ntiles, int grid_tiles) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
+    if (y >= nt) return;
+    const MmTile tl = tiles[y];
+    if (tl.count <= a.least || (place_of(tiles, y) & 1)) return;
+    if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
+        ws = a.ws2;
+        Y = a.y2;
+    }
+    const bool gu = a.a16 != nullptr;
+    const WSlice m = gu && threadIdx.x >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
+    int count = tl.count;
+    if (y + 1 < nt && follows(tiles[y + 1], tl)) count += tiles[y + 1].count;
+    if (seed_fmt<FMT>()) {
+        load_tables(tab);
+        __syncthreads();
+    }
+    const int r0 = (int) blockIdx.x * (gu ? 64 : 128);
+#define W(NT) wide_tile<FMT, NT>(a, m, X, Y, perm, tl.start, count, r0, tab, lds)
+    if (count <= 64) W(4);
+    else if (count <= 128) W(8);
+    else if (count <= 192) W(12);
+    else W(16);
+#undef W
 }
 
 template <int FMT, int RT, int NT, bool PACKED>
@@ -372,15 +579,35 @@ void dense(hipStream_t st, const MmArgs& a, const WSlice& w, const void* X, floa
     }
 #undef C
 }
-template <int FMT, bool PACKED>
-void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles,
-             const int32_t* ntiles, int grid_tiles, int tile_rows) {
+template <int FMT, int MOST, bool PACKED>
+void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
+             int grid_tiles, int limit) {
     const int rows = a.a16 ? 8 * GRT : 16 * GRT;
     const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
-    constexpr size_t lds = rows_lds<FMT, GRT, 2, 4, PACKED>();
-    allow_big_lds<k_mm_rows_grouped<FMT, PACKED>>(lds);
-    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y,
-                       perm, tiles, ntiles, tile_rows <= 32 ? 32 : MMT_BN);
+    constexpr size_t lds = rows_lds<FMT, GRT, MOST, 4, PACKED>();
+    allow_big_lds<k_mm_rows_grouped<FMT, MOST, PACKED>>(lds);
+    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit);
+    host_note_launch();
+}
+// tile_rows: what the caller says of its tiles' pairs.  The fewer token tiles a pass, the more the kernel's registers leave the decode
+template <int FMT, bool PACKED>
+void grouped_any(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
+                 int grid_tiles, int tile_rows) {
+    const int limit = tile_rows <= 32 ? 32 : MMT_BN;
+    if constexpr (PACKED) {
+        if (a.most > 64 && tile_rows > 64) { grouped<FMT, 6, true>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, limit); return; }
+        if (a.most > 32 && tile_rows > 48) { grouped<FMT, 4, true>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, limit); return; }
+    }
+    grouped<FMT, 2, PACKED>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, limit);
+}
+template <int FMT>
+void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
+          int grid_tiles) {
+    const int rows = a.a16 ? 64 : 128;
+    const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
+    constexpr size_t lds = wide_lds<FMT, 16>();
+    allow_big_lds<k_mm_wide<FMT>>(lds);
+    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles);
     host_note_launch();
 }
 
@@ -414,8 +641,15 @@ void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, co
 void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
                      const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows) {
 #define G(F)                                                                                                 \
-    packed ? grouped<F, true>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)             \
-           : grouped<F, false>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)
+    packed ? grouped_any<F, true>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)             \
+           : grouped_any<F, false>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, tile_rows)
+    BY_FORMAT(G)
+#undef G
+}
+
+void mm_wide_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
+                     const int32_t* ntiles, int grid_tiles) {
+#define G(F) wide<F>(st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles)
     BY_FORMAT(G)
 #undef G
 }

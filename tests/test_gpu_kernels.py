@@ -720,6 +720,61 @@ def test_route_bucket_equals_route_then_bucket(E, k, T):
         b.free()
 
 
+@pytest.mark.parametrize("fmt", ALL_FMT)
+@pytest.mark.parametrize("tile_rows", [0, 48, 64, 96, 129])
+def test_mm_grouped_tile_sizes(be, oracle, fmt, tile_rows):
+    """kc_mm_grouped_packed_rows and kc_mm_grouped_swiglu under every word on the tiles, over tables with 1 to 300 pairs an expert (an
+    expert of more than 128: adjoining tiles; 300: three), 150 weight rows, K of 5 chunks, against the oracle's products."""
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    L = backend.hip()
+    rng = np.random.default_rng(31 * fmt + tile_rows)
+    counts = [1, 17, 64, 65, 0, 128, 129, 200, 300]
+    E, R, K, P = len(counts), 150, 320, sum(counts)
+    keep, tabs, pk = [], [], []
+    for _ in range(2):
+        p = make_pack(rng, fmt, E, R, K)
+        arr = (backend.WSlice * E)()
+        names = {packs.MF_SEED4P4: [("seeds", 0), ("coefs", 1), ("codes", 3)], packs.MF_SEED4: [("seeds", 0), ("nibs", 1)],
+                 packs.MF_BF16: [("w", 0)]}.get(fmt, [("words", 0), ("scales", 1), ("biases", 2)])
+        for name, i in names:
+            buf = moe.DevBuf.from_array(np.ascontiguousarray(p[name]))
+            keep.append(buf)
+            for e in range(E):
+                arr[e].p[i] = buf.ptr.value + e * (buf.nbytes // E)
+        for e in range(E):
+            arr[e].eb, arr[e].gs = (int(p["eb"][e]), 0) if "eb" in p else (0, 6)
+        tab = moe.DevBuf(C.sizeof(arr))
+        backend.check(L.nh_memcpy_h2d(tab.ptr, arr, C.c_size_t(C.sizeof(arr))), "nh_memcpy_h2d")
+        tabs.append(tab); pk.append(p)
+    slc = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)
+    perm, tiles = oracle.bucket(slc, E, 128)
+    x = packs.round_bf16(rng.standard_normal((P, K)).astype(np.float32))
+    dx = moe.DevBuf.from_array(packs.f32_to_bf16_bits(x))
+    dperm, dtiles, dn = (moe.DevBuf.from_array(np.ascontiguousarray(v, dtype=np.int32)) for v in (perm, tiles, [len(tiles)]))
+    y, a16 = [moe.DevBuf(4 * P * R) for _ in range(2)], moe.DevBuf(2 * P * R)
+    mt = len(tiles) + 3
+    for j in range(2):
+        L.kc_mm_grouped_packed_rows(None, fmt, tabs[j].ptr, K, R, dx.ptr, K, y[j].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
+    assert L.kc_mm_grouped_swiglu(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, a16.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows) == 0
+    moe.device_sync()
+    assert L.kc_last_error() == 0
+    got = [v.to_array(np.float32, (P, R)) for v in y]
+    for j in range(2):
+        for e in range(E):
+            rows = np.flatnonzero(slc == e)
+            if len(rows):
+                r, m = ref_mm(oracle, pk[j], e, x[rows], 0)
+                assert close_bf(got[j][rows], packs.round_bf16(r.astype(np.float32)).astype(np.float64), F32B * m).all(), (NAMES[fmt], j, e)
+    sa = moe.DevBuf(2 * P * R)
+    L.kc_swiglu_pack(None, y[0].ptr, y[1].ptr, sa.ptr, C.c_size_t(P * R // 8 * 8))
+    moe.device_sync()
+    n = P * R // 8 * 8
+    assert np.array_equal(sa.to_array(np.uint16, (P * R,))[:n], a16.to_array(np.uint16, (P * R,))[:n])
+    for b in keep + tabs + y + [dx, dperm, dtiles, dn, a16, sa]:
+        b.free()
+
+
 def _grouped_rows_case(fmt, T, ind, rng):
     """kc_bucket on ind [T][4] of 9 experts, then kc_mm_grouped_packed and kc_mm_grouped_packed_rows(tile_rows = T) on the same
     tiles (R 72: not a multiple of a tile): both results as uint32 [P][R], and the permutation."""
