@@ -15,7 +15,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 struct MmArgs {
     int K, R, T, xs, ys, xdiv, add, f32out;
     int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's;
-    int paired;          // so is, where adjoining tiles of a slice go in pairs, the second of a pair
+    int paired;          // so is, beside k_mm_wide, the second tile of a pair that it takes together (second_of_pair)
     const WSlice* ws2;   // grouped launches of two matrices over the same tiles (grid.z = 2): the second slice table ..
     float* y2;           // .. and its output
     uint16_t* a16;       // non-null: a workgroup's weight rows are gate rows (ws) and the same rows of up (ws2), half and half, and what

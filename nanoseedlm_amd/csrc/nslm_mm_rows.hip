@@ -434,12 +434,19 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
         if (16 * nt + t < count && orow < a.R) store_rows(a, Y, perm[start + 16 * nt + t], orow, acc[nt]);
 }
 
-// An expert's tiles go in pairs where another launch takes them so: the tile's place (0, 1, 2, ..) in its run of adjoining tiles
+// Who computes a tile of a grouped launch, whatever table the host made: k_mm_wide takes every tile of more than `least` pairs, alone or together
+// with the tile that follows it in the same slice (of any count, none too), and k_mm_rows_grouped beside it takes what is left: the tiles
+// of up to `least` pairs that are not such a second.  A tile is a second when the tile before it is one that k_mm_wide takes, follows()
+// holds, and that one is no second itself; so a tile's part in it is the parity of the run of such tiles before it, up to the last one that
+// is not.  A wave looks at 64 tiles at once (a token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile
+// is a chain of as many loads).
 __device__ __forceinline__ bool follows(const MmTile& b, const MmTile& a) { return b.slice == a.slice && b.start == a.start + a.count; }
-__device__ __forceinline__ int place_of(const MmTile* tiles, int y) {
-    int n = 0;
-    for (; y > 0 && follows(tiles[y], tiles[y - 1]); --y) ++n;
-    return n;
+__device__ __forceinline__ bool second_of_pair(const MmTile* tiles, int y, int least) {   // all 64 lanes, the same arguments
+    for (int n = 0;; n += 64) {
+        const int i = y - n - (int) (threadIdx.x & 63);
+        const unsigned long long stop = ~__ballot(i > 0 && tiles[max(i - 1, 0)].count > least && follows(tiles[max(i, 0)], tiles[max(i - 1, 0)]));
+        if (stop) return (__ffsll(stop) - 1) & 1;   // (i <= 0 stops)
+    }
 }
 
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
@@ -469,7 +476,7 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     const bool gu = a.a16 != nullptr;
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
     const MmTile tl = tiles[blockIdx.y];
-    if (tl.count > a.most || (a.paired && (place_of(tiles, (int) blockIdx.y) & 1))) return;   // another launch's
+    if (tl.count > a.most || (a.paired && second_of_pair(tiles, (int) blockIdx.y, a.least))) return;   // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -504,7 +511,7 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     }
 }
 
-// A grouped launch's tiles of more than a.least pairs, each with the tile that follows it
+// A grouped launch's tiles of more than a.least pairs, each with the tile that follows it (second_of_pair)
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles) {
@@ -513,7 +520,7 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
-    if (tl.count <= a.least || (place_of(tiles, y) & 1)) return;
+    if (tl.count <= a.least || second_of_pair(tiles, y, a.least)) return;
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;

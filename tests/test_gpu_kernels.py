@@ -775,6 +775,98 @@ def test_mm_grouped_tile_sizes(be, oracle, fmt, tile_rows):
         b.free()
 
 
+# (slice, pairs) in table order: runs of a slice's adjoining tiles that kc_bucket, which fills a tile before it begins the next, never makes
+HAND_TILES = {
+    "small_first": [(0, 20), (0, 20), (1, 20), (1, 100), (2, 32), (2, 32), (2, 32), (2, 64), (3, 1), (3, 33), (3, 33)],
+    "empty_between": [(0, 64), (0, 0), (0, 64), (1, 0), (1, 100), (2, 0), (2, 0), (2, 20), (2, 0), (2, 128), (3, 40), (3, 0)],
+    "mixed": [(0, 128), (0, 128), (0, 40), (0, 128), (1, 33), (1, 32), (1, 33), (1, 33), (1, 7), (2, 128), (2, 20), (2, 128), (2, 128)],
+    "long": [(0, 40)] * 131 + [(0, 5)] + [(0, 40)] * 66 + [(1, 33)] * 3,   # runs of more tiles than a wave has lanes
+}
+
+
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_Q4])
+@pytest.mark.parametrize("table", list(HAND_TILES))
+def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
+    """Every pair of every tile of a hand-made table is computed, whatever a tile's count and its neighbours, by every grouped launch and
+    under every word on the tiles: the outputs hold NaN before, and what stays NaN was skipped."""
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    L = backend.hip()
+    rng = np.random.default_rng(7 * fmt + len(table))
+    tl = HAND_TILES[table]
+    E, R, K, P = 4, (40 if table == "long" else 150), (64 if table == "long" else 320), sum(n for _, n in tl)
+    pk = [make_pack(rng, fmt, E, R, K) for _ in range(2)]
+    keep, tabs = [], []
+    for p in pk:
+        arr = (backend.WSlice * E)()
+        names = [("seeds", 0), ("coefs", 1), ("codes", 3)] if fmt == packs.MF_SEED4P4 else [("words", 0), ("scales", 1), ("biases", 2)]
+        for name, i in names:
+            buf = moe.DevBuf.from_array(np.ascontiguousarray(p[name]))
+            keep.append(buf)
+            for e in range(E):
+                arr[e].p[i] = buf.ptr.value + e * (buf.nbytes // E)
+        for e in range(E):
+            arr[e].eb, arr[e].gs = (int(p["eb"][e]), 0) if "eb" in p else (0, 6)
+        tab = moe.DevBuf(C.sizeof(arr))
+        backend.check(L.nh_memcpy_h2d(tab.ptr, arr, C.c_size_t(C.sizeof(arr))), "nh_memcpy_h2d")
+        tabs.append(tab)
+    start = np.concatenate([[0], np.cumsum([n for _, n in tl])])
+    tiles = np.array([[s, start[i], n, 0] for i, (s, n) in enumerate(tl)], dtype=np.int32)
+    perm = rng.permutation(P).astype(np.int32)
+    slc = np.empty(P, dtype=np.int32)
+    slc[perm] = np.repeat([s for s, _ in tl], [n for _, n in tl])
+    x = packs.round_bf16(rng.standard_normal((P, K)).astype(np.float32))
+    ref, mag = [np.zeros((P, R)) for _ in range(2)], [np.zeros((P, R)) for _ in range(2)]
+    for j in range(2):
+        for e in np.unique(slc):
+            r, m = ref_mm(oracle, pk[j], e, x[slc == e], 0)
+            ref[j][slc == e], mag[j][slc == e] = packs.round_bf16(r.astype(np.float32)), m
+    dx, dxf = moe.DevBuf.from_array(packs.f32_to_bf16_bits(x)), moe.DevBuf.from_array(x)
+    dperm, dtiles, dn = (moe.DevBuf.from_array(np.ascontiguousarray(v, dtype=np.int32)) for v in (perm, tiles, [len(tiles)]))
+    mt = len(tl) + 2
+    nan = np.full((P, R), np.nan, dtype=np.float32)
+
+    def check(j, y, what):
+        got = y.to_array(np.float32, (P, R))
+        left = np.flatnonzero(np.isnan(got).any(axis=1))
+        assert left.size == 0, (what, "pairs not computed", left.size, "of", P)
+        assert close_bf(got, ref[j], F32B * mag[j]).all(), what
+
+    # the same launches with the tile count on the device and without it
+    y = moe.DevBuf.from_array(nan)
+    L.kc_mm_grouped_packed(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, y.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, None)
+    moe.device_sync()
+    check(0, y, "packed")
+    y.free()
+    y = moe.DevBuf.from_array(nan)
+    L.kc_mm_grouped(None, fmt, tabs[0].ptr, K, R, dxf.ptr, K, y.ptr, R, 1, dperm.ptr, dtiles.ptr, len(tl), None)
+    moe.device_sync()
+    check(0, y, "f32")
+    y.free()
+    for tile_rows in (0, 40, 64, 96, 100, 128, 129, 2048):
+        ys = [moe.DevBuf.from_array(nan) for _ in range(2)]
+        a16 = moe.DevBuf.from_array(np.full((P, R), 0x7FC0, dtype=np.uint16))
+        L.kc_mm_grouped_packed_rows(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, ys[0].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
+        moe.device_sync()
+        check(0, ys[0], ("rows", tile_rows))
+        ys[0].free()
+        ys[0] = moe.DevBuf.from_array(nan)
+        L.kc_mm_grouped_packed_pair(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, ys[0].ptr, ys[1].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
+        assert L.kc_mm_grouped_swiglu(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, a16.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows) == 0
+        want = moe.DevBuf(2 * P * R)
+        n = P * R // 8 * 8
+        L.kc_swiglu_pack(None, ys[0].ptr, ys[1].ptr, want.ptr, C.c_size_t(n))
+        moe.device_sync()
+        for j in range(2):
+            check(j, ys[j], ("pair", tile_rows, j))
+        assert np.array_equal(want.to_array(np.uint16, (P * R,))[:n], a16.to_array(np.uint16, (P * R,))[:n]), ("swiglu", tile_rows)
+        for b in ys + [a16, want]:
+            b.free()
+    assert L.kc_last_error() == 0
+    for b in keep + tabs + [dx, dxf, dperm, dtiles, dn]:
+        b.free()
+
+
 def _grouped_rows_case(fmt, T, ind, rng):
     """kc_bucket on ind [T][4] of 9 experts, then kc_mm_grouped_packed and kc_mm_grouped_packed_rows(tile_rows = T) on the same
     tiles (R 72: not a multiple of a tile): both results as uint32 [P][R], and the permutation."""
