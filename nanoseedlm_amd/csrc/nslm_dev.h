@@ -330,6 +330,7 @@ __device__ __forceinline__ int group_shift(const WSlice& w) { return w.gs ? w.gs
 
 // process-wide switches and launch-error bookkeeping (defined in nslm_mv.hip)
 int host_store_f32();
+int host_cu_count();
 void host_note_launch();
 void host_note_unsupported();   // a launcher refused its arguments: kc_last_error() reports an invalid value
 

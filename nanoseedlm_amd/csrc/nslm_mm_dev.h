@@ -15,11 +15,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 struct MmArgs {
     int K, R, T, xs, ys, xdiv, add, f32out;
     int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's;
-    int paired;          // so is, beside k_mm_wide, the second tile of a pair that it takes together (second_of_pair)
+    int paired;          // so is, beside k_mm_wide, a tile that joins one of k_mm_wide's (Join)
     const WSlice* ws2;   // grouped launches of two matrices over the same tiles (grid.z = 2): the second slice table ..
     float* y2;           // .. and its output
     uint16_t* a16;       // non-null: a workgroup's weight rows are gate rows (ws) and the same rows of up (ws2), half and half, and what
                          // it stores is their SwiGLU as BF16 bits [pair][ys] (the two GEMMs and the SwiGLU + pack pass in one launch)
+    int pairs[3];        // grouped: mm_wide_pairs
 };
 
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
@@ -58,6 +59,7 @@ void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, co
 void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
                      const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows);
 
+void mm_wide_pairs(MmArgs& a);
 void mm_wide_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                      const int32_t* ntiles, int grid_tiles);
 

@@ -435,19 +435,33 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 }
 
 // Who computes a tile of a grouped launch, whatever table the host made: k_mm_wide takes every tile of more than `least` pairs, alone or together
-// with the tile that follows it in the same slice (of any count, none too), and k_mm_rows_grouped beside it takes what is left: the tiles
-// of up to `least` pairs that are not such a second.  A tile is a second when the tile before it is one that k_mm_wide takes, follows()
-// holds, and that one is no second itself; so a tile's part in it is the parity of the run of such tiles before it, up to the last one that
-// is not.  A wave looks at 64 tiles at once (a token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile
-// is a chain of as many loads).
-__device__ __forceinline__ bool follows(const MmTile& b, const MmTile& a) { return b.slice == a.slice && b.start == a.start + a.count; }
-__device__ __forceinline__ bool second_of_pair(const MmTile* tiles, int y, int least) {   // all 64 lanes, the same arguments
-    for (int n = 0;; n += 64) {
-        const int i = y - n - (int) (threadIdx.x & 63);
-        const unsigned long long stop = ~__ballot(i > 0 && tiles[max(i - 1, 0)].count > least && follows(tiles[max(i, 0)], tiles[max(i - 1, 0)]));
-        if (stop) return (__ffsll(stop) - 1) & 1;   // (i <= 0 stops)
+// with one that joins it, and k_mm_rows_grouped beside it takes what is left: the tiles of up to `least` pairs that join none.  A tile can join
+// the one before it where that one is k_mm_wide's and both are a slice's adjoining pairs (an empty tile, too), and does if that one did not
+// join another itself: the parity of the run of tiles that can, up to the last one that cannot.  A wave looks at 64 tiles at once (a
+// token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile is a chain of as many loads).
+// A pair saves a decode and leaves half the workgroups.  Two a CU run at once (512).  Up to so many, and in a second round that they fill, full
+// tiles are faster alone; us a layer step, P = 4, full tiles alone and in pairs, with the workgroups of tiles alone: E 16, top-2, d 2048,
+// ff 1024, 2048 rows on the same two experts (512) 171 and 222; E 32, top-4, d 512, ff 256, 2048 rows (312) 95 and 120; E 64, top-8, d 640,
+// ff 384, 1531 rows (768 and 640) 131 and 144; just past a round: E 16, top-2, d 4096, ff 2048, 512 rows (576) 299 and 269; E 128, top-8,
+// d 2048, ff 768, 2048 rows (2292 and 3056) 580 and 543.  A tile of up to FEW pairs joins at any number: with a full one it fits the 192 pairs of
+// a smaller pass (E 16, top-8, d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138; E 16, top-2, d 2048, ff
+// 1024, 2048 rows, one expert in all: 215, 179, 179; 138 cases of 60 to 600 pairs an expert, geometric mean against no rule: 0.944, 0.943, 0.941).
+#define FEW 64
+struct Join {
+    int least, few;   // k_mm_wide's tiles; the pairs of a tile that can join one
+    __device__ __forceinline__ Join(const MmArgs& a, int nt) : least(a.least), few(nt >= a.pairs[2] || (nt > a.pairs[0] && nt < a.pairs[1]) ? MMT_BN : FEW) {}
+    __device__ __forceinline__ bool can(const MmTile& t, const MmTile& before) const {
+        return before.count > least && t.count <= few && t.slice == before.slice && t.start == before.start + before.count;
     }
-}
+    __device__ __forceinline__ bool joins(const MmTile* tiles, int y) const {   // all 64 lanes, the same y: tile y goes with tile y - 1
+        if (y < 1 || !can(tiles[y], tiles[y - 1])) return false;   // (most: by scalar loads)
+        for (int n = 0;; n += 64) {
+            const int i = y - n - (int) (threadIdx.x & 63);
+            const unsigned long long stop = ~__ballot(i > 0 && can(tiles[max(i, 0)], tiles[max(i - 1, 0)]));
+            if (stop) return (__ffsll(stop) - 1) & 1;   // (i <= 0 stops)
+        }
+    }
+};
 
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
 template <int FMT, int RT, int NT, int NW, bool PACKED>
@@ -472,11 +486,12 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
                                                                            const MmTile* tiles, const int32_t* ntiles, int limit) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
-    if (ntiles && (int) blockIdx.y >= *ntiles) return;
+    const int nt = ntiles ? *ntiles : (int) gridDim.y, y = (int) blockIdx.y;
+    if (y >= nt) return;
     const bool gu = a.a16 != nullptr;
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
-    const MmTile tl = tiles[blockIdx.y];
-    if (tl.count > a.most || (a.paired && second_of_pair(tiles, (int) blockIdx.y, a.least))) return;   // another launch's
+    const MmTile tl = tiles[y];
+    if (tl.count > a.most || (a.paired && Join(a, nt).joins(tiles, y))) return;   // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -511,7 +526,7 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     }
 }
 
-// A grouped launch's tiles of more than a.least pairs, each with the tile that follows it (second_of_pair)
+// A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join)
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles) {
@@ -520,15 +535,16 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
-    if (tl.count <= a.least || second_of_pair(tiles, y, a.least)) return;
+    const Join join(a, nt);
+    if (tl.count <= a.least || join.joins(tiles, y)) return;
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
     }
     const bool gu = a.a16 != nullptr;
-    const WSlice m = gu && threadIdx.x >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
+    const WSlice m = gu && __builtin_amdgcn_readfirstlane((int) threadIdx.x) >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
     int count = tl.count;
-    if (y + 1 < nt && follows(tiles[y + 1], tl)) count += tiles[y + 1].count;
+    if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
     if (seed_fmt<FMT>()) {
         load_tables(tab);
         __syncthreads();
@@ -621,6 +637,14 @@ void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, 
 }   // namespace
 
 namespace nslm {
+
+// the tile counts from which k_mm_wide takes full tiles in pairs (Join): past one round of its workgroups, until a quarter into a second, from two rounds on
+void mm_wide_pairs(MmArgs& a) {
+    const int blocks = a.a16 ? (a.R + 63) / 64 : (a.R + 127) / 128 * (a.ws2 ? 2 : 1), round = 2 * host_cu_count();   // a tile's; at once
+    a.pairs[0] = round / blocks;
+    a.pairs[1] = (5 * round / 4 + blocks - 1) / blocks;
+    a.pairs[2] = (2 * round + blocks - 1) / blocks;
+}
 
 #define BY_FORMAT(CALL)                                        \
     switch (fmt) {                                             \

@@ -1001,6 +1001,7 @@ bool launch_tok(hipStream_t st, MvArgs a, int T, bool shfl) {
 
 namespace nslm {
 int host_store_f32() { return g_store_f32; }
+int host_cu_count() { return cu_count(); }
 void host_note_unsupported() { g_last_error = (int) hipErrorInvalidValue; }
 void host_note_launch() {
     const hipError_t e = hipGetLastError();

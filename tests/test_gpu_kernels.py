@@ -780,7 +780,8 @@ HAND_TILES = {
     "small_first": [(0, 20), (0, 20), (1, 20), (1, 100), (2, 32), (2, 32), (2, 32), (2, 64), (3, 1), (3, 33), (3, 33)],
     "empty_between": [(0, 64), (0, 0), (0, 64), (1, 0), (1, 100), (2, 0), (2, 0), (2, 20), (2, 0), (2, 128), (3, 40), (3, 0)],
     "mixed": [(0, 128), (0, 128), (0, 40), (0, 128), (1, 33), (1, 32), (1, 33), (1, 33), (1, 7), (2, 128), (2, 20), (2, 128), (2, 128)],
-    "long": [(0, 40)] * 131 + [(0, 5)] + [(0, 40)] * 66 + [(1, 33)] * 3,   # runs of more tiles than a wave has lanes
+    "long": [(0, 40)] * 131 + [(0, 5)] + [(0, 40)] * 66 + [(1, 33)] * 3,   # runs of more tiles than a wave has lanes; passes all by the tiles' own rows
+    "round": [(0, 66)] * 261 + [(1, 66)] * 4,                                # workgroups enough that tiles of more than 64 pairs go in pairs
 }
 
 
@@ -794,7 +795,7 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
     L = backend.hip()
     rng = np.random.default_rng(7 * fmt + len(table))
     tl = HAND_TILES[table]
-    E, R, K, P = 4, (40 if table == "long" else 150), (64 if table == "long" else 320), sum(n for _, n in tl)
+    E, R, K, P = 4, (200 if len(tl) > 100 else 150), (64 if len(tl) > 100 else 320), sum(n for _, n in tl)
     pk = [make_pack(rng, fmt, E, R, K) for _ in range(2)]
     keep, tabs = [], []
     for p in pk:
@@ -843,7 +844,8 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
     moe.device_sync()
     check(0, y, "f32")
     y.free()
-    for tile_rows in (0, 40, 64, 96, 100, 128, 129, 2048):
+    # (a table's unused rows take later passes over its tiles: two of them, and more than there are passes)
+    for tile_rows, mt in [(t, len(tl) + 2) for t in (0, 40, 64, 96, 100, 128, 129, 2048)] + [(t, 5 * len(tl)) for t in (0, 40, 64, 96)]:
         ys = [moe.DevBuf.from_array(nan) for _ in range(2)]
         a16 = moe.DevBuf.from_array(np.full((P, R), 0x7FC0, dtype=np.uint16))
         L.kc_mm_grouped_packed_rows(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, ys[0].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
