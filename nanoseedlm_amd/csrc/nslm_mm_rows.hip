@@ -483,15 +483,31 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
 // MOST: token tiles a pass.  Two (or four): four waves a SIMD.  Six: three, what their LDS leaves.
 template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
-                                                                           const MmTile* tiles, const int32_t* ntiles, int limit) {
+                                                                           const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
-    const int nt = ntiles ? *ntiles : (int) gridDim.y, y = (int) blockIdx.y;
-    if (y >= nt) return;
+    // The grid has a workgroup row for as many tiles as the host's table holds.  Of fewer than `few` tiles, whose own workgroups do not fill the
+    // chip, those past *ntiles take the later passes over 16 MOST pairs: pass 1 of every tile, then pass 2, .. (row nt + e: pass 1 + e / nt of
+    // tile e % nt); the passes that they do not reach are the tile's own workgroups', after pass 0.  Tokens that agree on a few experts make
+    // few and full tiles (E 128, top-2, d 2048, ff 768, 100 rows on the same two experts: 66 -> 47 us a layer step).
+    constexpr int PASS = 16 * MOST;
+    const int nt = ntiles ? *ntiles : (int) gridDim.y, extra = (int) blockIdx.y - nt;
+    int y = (int) blockIdx.y, first = 0, next = PASS;   // the first pair, and that of the pass after it
+    if (nt >= few) {
+        if (extra >= 0) return;
+    } else if (extra < 0) {
+        next = PASS * (1 + (max((int) gridDim.y - nt - y, 0) + nt - 1) / nt);
+    } else {
+        if (nt < 1) return;
+        y = extra % nt;
+        first = PASS * (1 + extra / nt);
+        next = 2 * MMT_BN;   // (none)
+    }
     const bool gu = a.a16 != nullptr;
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
     const MmTile tl = tiles[y];
-    if (tl.count > a.most || (a.paired && Join(a, nt).joins(tiles, y))) return;   // another launch's
+    if (tl.count > a.most || tl.count <= first) return;                             // another launch's, or no such pass
+    if (a.paired && Join(a, nt).joins(tiles, y)) return;                            // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -511,8 +527,8 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
         load_tables(tab);
         __syncthreads();
     }
-    for (int n0 = 0; n0 < count; n0 += 16 * MOST) {
-        if (n0) __syncthreads();   // the sums of the tokens before are read
+    for (int n0 = first; n0 < count; n0 = next, next += PASS) {
+        if (n0 != first) __syncthreads();   // the sums of the tokens before are read
         const int left = count - n0;
 #define T(NT) rows_tile<FMT, GRT, NT, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds)
         if (left <= 16) T(1);
@@ -609,7 +625,10 @@ void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, f
     const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
     constexpr size_t lds = rows_lds<FMT, GRT, MOST, 4, PACKED>();
     allow_big_lds<k_mm_rows_grouped<FMT, MOST, PACKED>>(lds);
-    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit);
+    // Four workgroups a CU run at once.  (Passes of 32: half of that; most tiles there have one pass, and the rows that find none cost small matrices
+    // more than they give: E 128, top-2, d 512, ff 256, 96 rows 28 -> 32 us.  Passes of 64, E 16, top-2, d 2688, ff 384, 1010 rows: 135 and 121.)
+    const int few = (limit < a.most ? limit : a.most) > 16 * MOST ? (MOST > 2 ? 4 : 2) * host_cu_count() / (int) (grid.x * grid.z) + 1 : 0;
+    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few);
     host_note_launch();
 }
 // tile_rows: what the caller says of its tiles' pairs.  The fewer token tiles a pass, the more the kernel's registers leave the decode
