@@ -296,6 +296,27 @@ int nslm_moe_step_layer(NslmMoe* m, kc_stream_t s, int layer, const float* xn, i
     return kc_last_error() ? -1 : 0;
 }
 
+/* What a batched step says of its tiles to the grouped GEMMs (tile_rows, kernels_hip.h).  A step of T rows chooses no expert more than T times;
+ * past a pass's pairs, it is the pairs an expert gets on average, and the workgroups that k_mm_wide (the kernel of mostly full tiles) would have
+ * at a tile an expert, that say which passes pay: 64 and 96 up to where the fuller half of the tiles still fits (the mean and twice its root).
+ * us a layer step by the word 48 / 64 / 96 / 129, P = 4 where not said, [the word taken]:
+ *   a mean of up to 12   E 128, top-8, d 2048, ff 768: 3: [234] 236 292 289, 12: [248] 256 319 302; E 64, top-4, d 1024, ff 512: 12: [69] 70 83 75
+ *   up to 52             E 128, top-8: 25: 312 [291] 349 314, 50: 536 [357] 419 344; E 16, top-2, d 2048, ff 1024: 50: 115 [86] 88 97
+ *   up to 76 (88), few   E 16, top-2: 65: 135 107 [99] 102; E 16, top-8, d 3072, ff 512: 75: 121 98 [86] 114
+ *             many       E 64, top-4, d 1024, ff 448: 65: 145 118 121 [102]; E 128, top-4, d 512, ff 192, P = 3: 64: 114 101 112 [93]
+ *   up to a tile, few    E 16, top-8, d 3072, ff 512: 87: 129 [100] 98 115, 115: 148 [106] 127 118
+ *   else                 E 128, top-8: 128: 1146 786 970 [543]; E 16, top-4, d 1024, ff 2048, P = 3: 87: 148 112 113 [105]
+ * Skewed routing is the kernels' to see to, by the tiles' own counts: with a tenth of the experts taking half of the pairs, E 128, top-8, T = 128 /
+ * 512 / 2048: 266 / 350 / 621 (by the kernel of one 128-pair pass a tile that came before these: 323 / 412 / 656). */
+static int tile_word(int T, int P, int E, int d, int ff) {
+    const int mean = P / E, gu = E * ((ff + 63) / 64), dn = E * ((d + 127) / 128);
+    if (T <= 32) return T;
+    if (mean <= 12) return 48;
+    if (mean <= 52) return 64;
+    if (gu + dn < 768 && mean <= (gu <= 128 ? 88 : 76)) return 96;
+    return mean <= MMT_BN && gu <= 128 ? 64 : MMT_BN + 1;
+}
+
 int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, float* io) {
     const NslmMoeCfg* c = &m->c;
     if (!m->final || T < 1 || T > c->max_rows || layer < 0 || layer >= c->n_layer) return -1;
@@ -384,16 +405,14 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
         if (!routed_and_grouped) kc_bucket(s, m->ind, P, E, m->perm, m->tiles, m->ntiles);
         if (packed) {
             if (c->router != NSLM_ROUTE_SOFTMAX) kc_pack_input_bf16(s, xn, m->px, (size_t) T * d);   /* else: made for the router */
-            /* a step of T rows chooses no expert more than T times: no tile holds more than T pairs.  More rows than a pass of the
-               grouped kernels takes: the pairs an expert gets on average say which passes pay (kernels_hip.h) */
-            const int mean = P / E, pairs = T <= 32 ? T : mean <= 12 ? 48 : mean <= 52 ? 64 : mean <= 88 && E * ((ff + 63) / 64) < 512 ? 96 : MMT_BN + 1;
+            const int word = tile_word(T, P, E, d, ff);
             /* gate, up and SwiGLU in one launch (else: the two GEMMs in one launch, then SwiGLU) */
-            if (kc_mm_grouped_swiglu(s, c->fmt, gate, up, d, ff, m->px, d, (uint16_t*) m->A, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, pairs)) {
-                kc_mm_grouped_packed_pair(s, c->fmt, gate, up, d, ff, m->px, d, m->G, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, pairs);
+            if (kc_mm_grouped_swiglu(s, c->fmt, gate, up, d, ff, m->px, d, (uint16_t*) m->A, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, word)) {
+                kc_mm_grouped_packed_pair(s, c->fmt, gate, up, d, ff, m->px, d, m->G, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, word);
                 kc_swiglu_pack(s, m->G, m->U, (uint16_t*) m->A, (size_t) P * ff);
             }
             kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles,
-                                      m->max_tiles, pairs);
+                                      m->max_tiles, word);
         } else {
             kc_mm_grouped_dev(s, c->fmt, gate, d, ff, xn, d, m->G, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
             kc_mm_grouped_dev(s, c->fmt, up, d, ff, xn, d, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
