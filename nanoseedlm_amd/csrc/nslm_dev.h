@@ -243,47 +243,8 @@ __device__ __forceinline__ void col_bytes_p4(uint32_t up, uint32_t g, uint32_t (
 
 // Two blocks at once, written in phases (all windows, then all sign flips, all pairings, all products) with the
 // scheduler held to that order: a VALU result is not available to the next instruction slots, and a wave that has a SIMD's
-// vector issue to itself (the GEMM's decoder waves) loses those slots unless dependent instructions sit far apart.  In
-// phase order every operand is at least a dozen instructions old.
-__device__ __forceinline__ void isum2_p4(const uint32_t (&up)[2], const uint32_t (&g)[2], const uint32_t (&q01)[2],
-                                         const uint32_t (&q23)[2], int (&is)[2][8]) {
-    uint32_t A[2][17], lo[2][8], hi[2][8];
-#pragma unroll
-    for (int k = 1; k <= 15; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = __builtin_amdgcn_alignbit(g[h], up[h], 16 + k);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 1; k <= 16; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = (k < 16 ? A[h][k] : g[h]) ^ 0x80008000u;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j)   // pair j = states 2j+1, 2j+2 (low halves) and 2j+17, 2j+18 (high halves)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            lo[h][j] = halves(A[h][2 * j + 1], 0, A[h][2 * j + 2], 0);
-            hi[h][j] = halves(A[h][2 * j + 1], 1, A[h][2 * j + 2], 1);
-        }
-    __builtin_amdgcn_sched_barrier(0);
-    int t[2][8];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            t[h][c] = dot2z(lo[h][2 * c + 1], q23[h]);
-            t[h][c + 4] = dot2z(hi[h][2 * c + 1], q23[h]);
-        }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            is[h][c] = dot2(lo[h][2 * c], q01[h], t[h][c]);
-            is[h][c + 4] = dot2(hi[h][2 * c], q01[h], t[h][c + 4]);
-        }
-    __builtin_amdgcn_sched_barrier(0);
-}
+// vector issue to itself loses those slots unless dependent instructions sit far apart.  In phase order every operand is at
+// least a dozen instructions old.
 __device__ __forceinline__ void isum2_p3(const uint32_t (&up)[2], const uint32_t (&g)[2], const uint32_t (&q01)[2],
                                          const uint32_t (&q2)[2], int (&is)[2][8]) {
     uint32_t A[2][17], pr[2][8];

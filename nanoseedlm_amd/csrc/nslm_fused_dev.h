@@ -150,10 +150,6 @@ __device__ __forceinline__ void router_fetch_input(RouterRegs& r, const float* x
         }
     }
 }
-__device__ __forceinline__ void router_fetch(RouterRegs& r, const uint16_t* wr, const float* xr, int nb, const float* nw, int j0) {
-    router_fetch_row(r, wr, nb, j0);
-    router_fetch_input(r, xr, nb, nw, j0);
-}
 __device__ __forceinline__ float router_add(const RouterRegs& r, int nb, bool normed, float rn, int j0, float acc) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {

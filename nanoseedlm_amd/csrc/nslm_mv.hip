@@ -947,7 +947,8 @@ int wide_run(int fmt, int K, int R, int T) {
     return run;
 }
 
-// A launch of 2 .. 8 tokens by k_mv_tok; false: another kernel's.  The tokens go in runs that fit the LDS beside the chunk sums of enough row
+// A launch of 2 .. 8 tokens by k_mv_tok; false: another kernel's.  The tokens go in runs (of two at least: rows hold up to 128
+// chunks, and two of the longest fit) that fit the LDS beside the chunk sums of enough row
 // quads to keep 1024 threads busy, dealt to grid.y; a matrix whose chunks fill little more than a third of the chip's threads gives it two runs
 // instead of one (2048 x 2048, P = 3, 8 tokens: 9.5 us in two runs of four, 12.2 in one: what it takes is the staging).  A workgroup's share
 // of the row quads is a CU's, or half or a quarter of it where there is work for so many workgroups and their tokens fit the LDS: one

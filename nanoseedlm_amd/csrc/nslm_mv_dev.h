@@ -183,7 +183,7 @@ __device__ __forceinline__ void cols_post(const uint32_t (&zp)[8][6], uint32_t c
         acc = fmaf(d, e2, acc);
     }
 }
-// PAIRED (P = 3 only): two blocks at a time in phase order (isum2_p3), as the GEMM's decoder waves decode: measured 1 % faster
+// PAIRED (P = 3 only): two blocks at a time in phase order (isum2_p3): measured 1 % faster
 // in the persistent MoE kernel (three waves a SIMD), 6 % slower in the stand-alone matvec, which keeps the compiler's own order.
 template <int P, int NT, bool PAIRED = false, bool COLS = (P == 4)>
 __device__ __forceinline__ void chunk_dot(const Chunk& ck, int eb, const uint32_t* tab, const float* xr, int xstride, int nt,
