@@ -642,7 +642,7 @@ bool rows_ok(int fmt, int K, int xs, const void* x) {
 template <bool PACKED>
 void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, int xs, float* y, int ys, int T, int add) {
     if (T < 1 || R < 1) return;
-    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, 0, nullptr, nullptr, nullptr, {}};
+    MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, 0, nullptr, nullptr, nullptr};
     const unsigned gx = (unsigned) (R + BM - 1) / BM;
     if (rows_ok<PACKED>(fmt, K, xs, x) && mm_rows_better(fmt, R, T)) {
         mm_rows_dense(st, fmt, a, w, x, PACKED, y);
@@ -669,7 +669,6 @@ void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, in
 #define ROWS_TILE 96
 template <class Rows, class Wide>
 void by_tiles(MmArgs& a, int tile_rows, Rows rows, Wide wide) {
-    mm_wide_pairs(a);
     if (tile_rows < 1) tile_rows = MMT_BN;
     if (tile_rows > MMT_BN) wide(a);
     else if (tile_rows <= ROWS_TILE) rows(a, tile_rows);
@@ -685,7 +684,7 @@ void mm_grouped(hipStream_t st, int fmt, const WSlice* ws, int K, int R, const v
                 const int32_t* perm, const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows,
                 const WSlice* ws2 = nullptr, float* y2 = nullptr) {
     if (grid_tiles < 1 || R < 1) return;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), 0, MMT_BN, 0, ws2, y2, nullptr, {}};
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, host_store_f32(), 0, MMT_BN, 0, ws2, y2, nullptr};
     WSlice none = {};
     const dim3 grid((unsigned) (R + BM - 1) / BM, (unsigned) grid_tiles);
     if (rows_ok<PACKED>(fmt, K, xs, x)) {
@@ -746,7 +745,7 @@ int kc_mm_grouped_swiglu(kc_stream_t s, int fmt, const WSlice* gate, const WSlic
                          int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows) {
     if (max_tiles < 1 || R < 1) return 0;
     if (!rows_ok<true>(fmt, K, xs, x) || host_store_f32()) return -1;
-    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, 0, MMT_BN, 0, up, nullptr, a16, {}};
+    MmArgs a = {K, R, 0, xs, ys, xdiv, 0, 0, 0, MMT_BN, 0, up, nullptr, a16};
     by_tiles(a, tile_rows, [&](const MmArgs& ar, int n) { mm_rows_grouped((hipStream_t) s, fmt, ar, gate, x, true, nullptr, perm, tiles, nt, max_tiles, n); },
              [&](const MmArgs& aw) { mm_wide_grouped((hipStream_t) s, fmt, aw, gate, x, nullptr, perm, tiles, nt, max_tiles); });
     return 0;

@@ -20,7 +20,6 @@ struct MmArgs {
     float* y2;           // .. and its output
     uint16_t* a16;       // non-null: a workgroup's weight rows are gate rows (ws) and the same rows of up (ws2), half and half, and what
                          // it stores is their SwiGLU as BF16 bits [pair][ys] (the two GEMMs and the SwiGLU + pack pass in one launch)
-    int pairs[3];        // grouped: mm_wide_pairs
 };
 
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
@@ -59,7 +58,6 @@ void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, co
 void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
                      const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows);
 
-void mm_wide_pairs(MmArgs& a);
 void mm_wide_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                      const int32_t* ntiles, int grid_tiles);
 

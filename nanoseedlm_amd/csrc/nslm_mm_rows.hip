@@ -447,9 +447,18 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 // a smaller pass (E 16, top-8, d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138; E 16, top-2, d 2048, ff
 // 1024, 2048 rows, one expert in all: 215, 179, 179; 138 cases of 60 to 600 pairs an expert, geometric mean against no rule: 0.944, 0.943, 0.941).
 #define FEW 64
+struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and between [0] and [1].  (An argument of its own: in MmArgs it moved the dense kernel's: 17.74 -> 17.94 us)
+    int n[3];
+    explicit JoinAt(const MmArgs& a) {
+        const int blocks = a.a16 ? (a.R + 63) / 64 : (a.R + 127) / 128 * (a.ws2 ? 2 : 1), round = 2 * host_cu_count();   // a tile's workgroups; at once
+        n[0] = round / blocks;
+        n[1] = (5 * round / 4 + blocks - 1) / blocks;
+        n[2] = (2 * round + blocks - 1) / blocks;
+    }
+};
 struct Join {
     int least, few;   // k_mm_wide's tiles; the pairs of a tile that can join one
-    __device__ __forceinline__ Join(const MmArgs& a, int nt) : least(a.least), few(nt >= a.pairs[2] || (nt > a.pairs[0] && nt < a.pairs[1]) ? MMT_BN : FEW) {}
+    __device__ __forceinline__ Join(const MmArgs& a, const JoinAt& at, int nt) : least(a.least), few(nt >= at.n[2] || (nt > at.n[0] && nt < at.n[1]) ? MMT_BN : FEW) {}
     __device__ __forceinline__ bool can(const MmTile& t, const MmTile& before) const {
         return before.count > least && t.count <= few && t.slice == before.slice && t.start == before.start + before.count;
     }
@@ -483,7 +492,7 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
 // MOST: token tiles a pass.  Two (or four): four waves a SIMD.  Six: three, what their LDS leaves.
 template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
-                                                                           const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
+                                                                           const MmTile* tiles, const int32_t* ntiles, int limit, int few, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     // The grid has a workgroup row for as many tiles as the host's table holds.  Of fewer than `few` tiles, whose own workgroups do not fill the
@@ -507,7 +516,7 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
     const MmTile tl = tiles[y];
     if (tl.count > a.most || tl.count <= first) return;                             // another launch's, or no such pass
-    if (a.paired && Join(a, nt).joins(tiles, y)) return;                            // another launch's
+    if (a.paired && Join(a, at, nt).joins(tiles, y)) return;                            // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -545,13 +554,13 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
 // A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join)
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
-                                                    const int32_t* ntiles, int grid_tiles) {
+                                                    const int32_t* ntiles, int grid_tiles, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
-    const Join join(a, nt);
+    const Join join(a, at, nt);
     if (tl.count <= a.least || join.joins(tiles, y)) return;
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
@@ -628,7 +637,7 @@ void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, f
     // Four workgroups a CU run at once.  (Passes of 32: half of that; most tiles there have one pass, and the rows that find none cost small matrices
     // more than they give: E 128, top-2, d 512, ff 256, 96 rows 28 -> 32 us.  Passes of 64, E 16, top-2, d 2688, ff 384, 1010 rows: 135 and 121.)
     const int few = (limit < a.most ? limit : a.most) > 16 * MOST ? (MOST > 2 ? 4 : 2) * host_cu_count() / (int) (grid.x * grid.z) + 1 : 0;
-    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few);
+    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few, JoinAt(a));
     host_note_launch();
 }
 // tile_rows: what the caller says of its tiles' pairs.  The fewer token tiles a pass, the more the kernel's registers leave the decode
@@ -649,21 +658,13 @@ void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, 
     const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
     constexpr size_t lds = wide_lds<FMT, 16>();
     allow_big_lds<k_mm_wide<FMT>>(lds);
-    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles);
+    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(a));
     host_note_launch();
 }
 
 }   // namespace
 
 namespace nslm {
-
-// the tile counts from which k_mm_wide takes full tiles in pairs (Join): past one round of its workgroups, until a quarter into a second, from two rounds on
-void mm_wide_pairs(MmArgs& a) {
-    const int blocks = a.a16 ? (a.R + 63) / 64 : (a.R + 127) / 128 * (a.ws2 ? 2 : 1), round = 2 * host_cu_count();   // a tile's; at once
-    a.pairs[0] = round / blocks;
-    a.pairs[1] = (5 * round / 4 + blocks - 1) / blocks;
-    a.pairs[2] = (2 * round + blocks - 1) / blocks;
-}
 
 #define BY_FORMAT(CALL)                                        \
     switch (fmt) {                                             \
