@@ -644,7 +644,7 @@ void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, in
     if (T < 1 || R < 1) return;
     MmArgs a = {K, R, T, xs, ys, 1, add, host_store_f32(), 0, MMT_BN, 0, nullptr, nullptr, nullptr};
     const unsigned gx = (unsigned) (R + BM - 1) / BM;
-    if (rows_ok<PACKED>(fmt, K, xs, x) && mm_rows_better(fmt, R, T)) {
+    if (rows_ok<PACKED>(fmt, K, xs, x) && mm_rows_better(fmt, R, T, PACKED)) {
         mm_rows_dense(st, fmt, a, w, x, PACKED, y);
         return;
     }

@@ -53,7 +53,7 @@ void allow_big_lds(size_t bytes) {
 __device__ __forceinline__ int x_swizzle(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
 
 // the kernel for few tokens a matrix (nslm_mm_rows.hip); packed: X holds BF16 bits, else f32
-bool mm_rows_better(int fmt, int R, int T);
+bool mm_rows_better(int fmt, int R, int T, bool packed);
 void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, const void* X, bool packed, float* Y);
 void mm_rows_grouped(hipStream_t st, int fmt, const MmArgs& a, const WSlice* ws, const void* X, bool packed, float* Y, const int32_t* perm,
                      const MmTile* tiles, const int32_t* ntiles, int grid_tiles, int tile_rows);

@@ -595,7 +595,7 @@ void launch(hipStream_t st, const MmArgs& a, const WSlice& w, const void* X, flo
 
 // The workgroup's shape: what a CU spends on a workgroup's step is RT decodes + NT token tiles' loads and MFMAs (beta: a token
 // tile's share against a row tile's decode, from the times of matrices of 300 .. 14336 rows at 9 .. 1024 tokens), and the launch
-// takes as many workgroups one after the other as the fullest of 256 CUs gets.
+// takes as many workgroups one after the other as the fullest CU gets.
 struct Shape {
     int rt, nt;
     double cost;
@@ -604,12 +604,13 @@ double beta_of(int fmt) { return fmt == MF_BF16 ? 1.0 : fmt == MF_Q8 || fmt == M
 bool fits(int fmt, int rt, int nt) { return !(fmt == MF_BF16 && rt + nt > 9); }   // (BF16 weights: 2 KB of LDS a wave and tile)
 Shape shape_of(int fmt, int R, int T, bool packed) {
     static const int rts[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 6}, {1, 8}, {2, 1}, {2, 2}, {2, 3}, {2, 4}, {2, 6}, {2, 8}, {4, 1}, {4, 2}, {4, 4}};
+    const int cus = host_cu_count();
     Shape best = {0, 0, 1e30};
     for (const auto& s : rts) {
         const int rt = s[0], nt = s[1];
         if (!fits(fmt, rt, nt) || (!packed && !(rt == 1 && (nt == 1 || nt == 4)) && !(rt == 4 && nt == 4))) continue;
         const long long wgs = (long long) ((R + 16 * rt - 1) / (16 * rt)) * ((T + 16 * nt - 1) / (16 * nt));
-        const double cost = (double) ((wgs + 255) / 256) * (rt + nt * beta_of(fmt));
+        const double cost = (double) ((wgs + cus - 1) / cus) * (rt + nt * beta_of(fmt));
         if (cost < best.cost) best = {rt, nt, cost};
     }
     return best;
@@ -675,14 +676,17 @@ namespace nslm {
         default: CALL(MF_Q4); break;                           \
     }
 
-// Against the streamed kernel, whose workgroup takes 64 rows x up to 512 tokens and spends on a step, in row decodes, what `stream`
-// says (it was timed with 64 .. 224 workgroups, one a CU): that one wins where its workgroups fill the chip.
-bool mm_rows_better(int fmt, int R, int T) {
-    const int q = T <= 128 ? 0 : T <= 256 ? 1 : 2;
-    static const double seeds[] = {6.2, 7.5, 8.8}, ints[] = {8.4, 12.7, 14.5}, bfs[] = {13.7, 23.0, 34.0};
-    const double* stream = fmt == MF_BF16 ? bfs : fmt == MF_Q8 || fmt == MF_Q4 ? ints : seeds;
+// Against the kernel of 64 rows x up to 512 tokens a workgroup - for packed activations the streamed one, for f32 the first-generation one -, which
+// spends on a step, in row decodes, what `step` says: that one wins where its workgroups fill the chip.  The streamed kernel was timed with 64 ..
+// 224 workgroups, one a CU.  f32: 290 matrices of 300 .. 32000 rows at 9 .. 2048 tokens on both kernels; the lines lie where the faster one
+// changes (up to 128 tokens, and for Q4, Q8 and BF16 up to 256, it never does), and the kernel taken is 0.1 % off the faster one on average,
+// 16 % at worst (4096 x 4096, 1000 tokens, P = 4: first generation 236 us, this 165; 14336 x 4096, 400 tokens: 216 and 270).
+bool mm_rows_better(int fmt, int R, int T, bool packed) {
+    static const double step[2][3][3] = {{{6.2, 7.5, 8.8}, {8.4, 12.7, 14.5}, {13.7, 23.0, 34.0}},
+                                         {{16.0, 16.0, 24.0}, {24.0, 24.0, 31.6}, {32.0, 40.0, 60.0}}};
+    const int q = T <= 128 ? 0 : T <= 256 ? 1 : 2, f = fmt == MF_BF16 ? 2 : fmt == MF_Q8 || fmt == MF_Q4 ? 1 : 0, cus = host_cu_count();
     const long long wgs = (long long) ((R + 63) / 64) * ((T + 511) / 512);
-    return shape_of(fmt, R, T, true).cost < (double) ((wgs + 255) / 256) * stream[q];
+    return shape_of(fmt, R, T, packed).cost < (double) ((wgs + cus - 1) / cus) * step[packed ? 0 : 1][f][q];
 }
 void mm_rows_dense(hipStream_t st, int fmt, const MmArgs& a, const WSlice& w, const void* X, bool packed, float* Y) {
 #define D(F) packed ? dense<F, true>(st, a, w, X, Y) : dense<F, false>(st, a, w, X, Y)

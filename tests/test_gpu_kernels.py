@@ -326,6 +326,19 @@ def test_mm_few_tokens(be, oracle, fmt, R, K):
             assert np.array_equal(y[:9].view(np.uint32), y9.view(np.uint32)), (NAMES[fmt], R, K, T)
 
 
+# f32 activations at token counts that the first-generation kernel had (seeds: from 200 tokens; BF16: at 130): the last token tile partial, one row past a tile
+@pytest.mark.parametrize("T,R", [(130, 16385), (1000, 2881)])
+@pytest.mark.parametrize("fmt", ALL_FMT)
+def test_mm_f32_many_tokens(be, oracle, fmt, T, R):
+    K = 64
+    rng = np.random.default_rng(T + fmt)
+    p = make_pack(rng, fmt, 1, R, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)   # rounded to BF16 on the way in
+    ref, mag = ref_mm(oracle, p, 0, packs.round_bf16(x), 0)
+    y = be.kt_mm_plain(p, x, packed=0)
+    assert close_bf(y, packs.round_bf16(ref.astype(np.float32)).astype(np.float64), F32B * mag).all(), (NAMES[fmt], T)
+
+
 @pytest.mark.parametrize("off", [0, 2, 6])
 def test_mm_few_tokens_streams_at_any_boundary(be, oracle, off):
     """Seed, coefficient and code streams that start 2 or 6 (codes: 1 or 3) bytes off a 16-byte boundary give the aligned streams' bits."""
