@@ -439,15 +439,17 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 // the one before it where that one is k_mm_wide's and both are a slice's adjoining pairs (an empty tile, too), and does if that one did not
 // join another itself: the parity of the run of tiles that can, up to the last one that cannot.  A wave looks at 64 tiles at once (a
 // token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile is a chain of as many loads).
-// A pair saves a decode and leaves half the workgroups.  Two a CU run at once (512).  Up to so many, and in a second round that they fill, full
-// tiles are faster alone; us a layer step, P = 4, full tiles alone and in pairs, with the workgroups of tiles alone: E 16, top-2, d 2048,
-// ff 1024, 2048 rows on the same two experts (512) 171 and 222; E 32, top-4, d 512, ff 256, 2048 rows (312) 95 and 120; E 64, top-8, d 640,
-// ff 384, 1531 rows (768 and 640) 131 and 144; just past a round: E 16, top-2, d 4096, ff 2048, 512 rows (576) 299 and 269; E 128, top-8,
-// d 2048, ff 768, 2048 rows (2292 and 3056) 580 and 543.  A tile of up to FEW pairs joins at any number: with a full one it fits the 192 pairs of
-// a smaller pass (E 16, top-8, d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138; E 16, top-2, d 2048, ff
-// 1024, 2048 rows, one expert in all: 215, 179, 179; 138 cases of 60 to 600 pairs an expert, geometric mean against no rule: 0.944, 0.943, 0.941).
+// Beside k_mm_rows_grouped every tile can join: which kernel computes a tile, and with it its sums' order, is then a matter of the table alone,
+// not of the matrices in the launch.  Alone k_mm_wide pairs full tiles only where the pairs fill the chip: a pair saves a decode and leaves half
+// the workgroups.  Two a CU run at once (512).  Up to so many, and in a second round that they fill, full tiles are faster alone; us a layer
+// step, P = 4, full tiles alone and in pairs, with the workgroups of tiles alone: E 16, top-2, d 2048, ff 1024, 2048 rows on the same two
+// experts (512) 171 and 222; E 32, top-4, d 512, ff 256, 2048 rows (312) 95 and 120; E 64, top-8, d 640, ff 384, 1531 rows (768 and 640) 131
+// and 144; just past a round: E 16, top-2, d 4096, ff 2048, 512 rows (576) 299 and 269; E 128, top-8, d 2048, ff 768, 2048 rows (2292 and
+// 3056) 580 and 543.  A tile of up to FEW pairs joins at any number: with a full one it fits the 192 pairs of a smaller pass (E 16, top-8,
+// d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138; E 16, top-2, d 2048, ff 1024, 2048 rows, one expert
+// in all: 215, 179, 179; 138 cases of 60 to 600 pairs an expert, geometric mean against no rule: 0.944, 0.943, 0.941).
 #define FEW 64
-struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and between [0] and [1].  (An argument of its own: in MmArgs it moved the dense kernel's: 17.74 -> 17.94 us)
+struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and between [0] and [1]
     int n[3];
     explicit JoinAt(const MmArgs& a) {
         const int blocks = a.a16 ? (a.R + 63) / 64 : (a.R + 127) / 128 * (a.ws2 ? 2 : 1), round = 2 * host_cu_count();   // a tile's workgroups; at once
@@ -455,10 +457,10 @@ struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and betwee
         n[1] = (5 * round / 4 + blocks - 1) / blocks;
         n[2] = (2 * round + blocks - 1) / blocks;
     }
+    __device__ __forceinline__ bool pairs(int nt) const { return nt >= n[2] || (nt > n[0] && nt < n[1]); }
 };
 struct Join {
     int least, few;   // k_mm_wide's tiles; the pairs of a tile that can join one
-    __device__ __forceinline__ Join(const MmArgs& a, const JoinAt& at, int nt) : least(a.least), few(nt >= at.n[2] || (nt > at.n[0] && nt < at.n[1]) ? MMT_BN : FEW) {}
     __device__ __forceinline__ bool can(const MmTile& t, const MmTile& before) const {
         return before.count > least && t.count <= few && t.slice == before.slice && t.start == before.start + before.count;
     }
@@ -492,7 +494,7 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
 // MOST: token tiles a pass.  Two (or four): four waves a SIMD.  Six: three, what their LDS leaves.
 template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
-                                                                           const MmTile* tiles, const int32_t* ntiles, int limit, int few, JoinAt at) {
+                                                                           const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     // The grid has a workgroup row for as many tiles as the host's table holds.  Of fewer than `few` tiles, whose own workgroups do not fill the
@@ -515,8 +517,8 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     const bool gu = a.a16 != nullptr;
     const int rows = gu ? 8 * GRT : 16 * GRT, r0 = (int) blockIdx.x * rows;
     const MmTile tl = tiles[y];
-    if (tl.count > a.most || tl.count <= first) return;                             // another launch's, or no such pass
-    if (a.paired && Join(a, at, nt).joins(tiles, y)) return;                            // another launch's
+    if (tl.count > a.most || tl.count <= first) return;                  // another launch's, or no such pass
+    if (a.paired && Join {a.least, MMT_BN}.joins(tiles, y)) return;   // another launch's
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
         Y = a.y2;
@@ -560,7 +562,7 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
-    const Join join(a, at, nt);
+    const Join join = {a.least, a.least > 0 || at.pairs(nt) ? MMT_BN : FEW};
     if (tl.count <= a.least || join.joins(tiles, y)) return;
     if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
         ws = a.ws2;
@@ -638,7 +640,7 @@ void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, f
     // Four workgroups a CU run at once.  (Passes of 32: half of that; most tiles there have one pass, and the rows that find none cost small matrices
     // more than they give: E 128, top-2, d 512, ff 256, 96 rows 28 -> 32 us.  Passes of 64, E 16, top-2, d 2688, ff 384, 1010 rows: 135 and 121.)
     const int few = (limit < a.most ? limit : a.most) > 16 * MOST ? (MOST > 2 ? 4 : 2) * host_cu_count() / (int) (grid.x * grid.z) + 1 : 0;
-    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few, JoinAt(a));
+    hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few);
     host_note_launch();
 }
 // tile_rows: what the caller says of its tiles' pairs.  The fewer token tiles a pass, the more the kernel's registers leave the decode

@@ -795,6 +795,7 @@ HAND_TILES = {
     "mixed": [(0, 128), (0, 128), (0, 40), (0, 128), (1, 33), (1, 32), (1, 33), (1, 33), (1, 7), (2, 128), (2, 20), (2, 128), (2, 128)],
     "long": [(0, 40)] * 131 + [(0, 5)] + [(0, 40)] * 66 + [(1, 33)] * 3,   # runs of more tiles than a wave has lanes; passes all by the tiles' own rows
     "round": [(0, 66)] * 261 + [(1, 66)] * 4,                                # workgroups enough that tiles of more than 64 pairs go in pairs
+    "triples": [(0, 70), (0, 70), (0, 30)] * 100,                             # for one matrix not enough for that, for two at once enough
 }
 
 
@@ -802,13 +803,14 @@ HAND_TILES = {
 @pytest.mark.parametrize("table", list(HAND_TILES))
 def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
     """Every pair of every tile of a hand-made table is computed, whatever a tile's count and its neighbours, by every grouped launch and
-    under every word on the tiles: the outputs hold NaN before, and what stays NaN was skipped."""
+    under every word on the tiles: the outputs hold NaN before, and what stays NaN was skipped.  Under one word a matrix's results are the same
+    bits from a launch of its own, of two matrices, and of gate + up + SwiGLU."""
     import ctypes as C
     from nanoseedlm_amd import backend, moe
     L = backend.hip()
     rng = np.random.default_rng(7 * fmt + len(table))
     tl = HAND_TILES[table]
-    E, R, K, P = 4, (200 if len(tl) > 100 else 150), (64 if len(tl) > 100 else 320), sum(n for _, n in tl)
+    E, R, K, P = 4, {"long": 200, "round": 200, "triples": 128}.get(table, 150), (64 if table in ("long", "round") else 320), sum(n for _, n in tl)
     pk = [make_pack(rng, fmt, E, R, K) for _ in range(2)]
     keep, tabs = [], []
     for p in pk:
@@ -864,6 +866,7 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
         L.kc_mm_grouped_packed_rows(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, ys[0].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
         moe.device_sync()
         check(0, ys[0], ("rows", tile_rows))
+        alone = ys[0].to_array(np.uint32, (P, R))
         ys[0].free()
         ys[0] = moe.DevBuf.from_array(nan)
         L.kc_mm_grouped_packed_pair(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, ys[0].ptr, ys[1].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
@@ -874,6 +877,7 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
         moe.device_sync()
         for j in range(2):
             check(j, ys[j], ("pair", tile_rows, j))
+        assert np.array_equal(ys[0].to_array(np.uint32, (P, R)), alone), ("pair and rows", tile_rows)
         assert np.array_equal(want.to_array(np.uint16, (P * R,))[:n], a16.to_array(np.uint16, (P * R,))[:n]), ("swiglu", tile_rows)
         for b in ys + [a16, want]:
             b.free()
