@@ -107,6 +107,9 @@ void kc_mm_grouped_dev(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, c
                        const uint32_t* G);
 /* engine/kernels_cuda.h:110-114, engine/kernels_moe.cu:2384-2395 */
 void kc_pack_input_bf16(kc_stream_t s, const float* x, uint16_t* y, size_t n);
+/* kc_mm and kc_mm_packed take one of several kernels by fmt, R and T; a token's last bits (the order of its f32 sums) depend on K and on which one
+ * it is, not on the other tokens.  For up to 128 tokens and R up to 8192 that is one kernel, the same for both entry points (K % 64 == 0, rows
+ * 16-byte aligned, no exact mode). */
 void kc_mm_packed(kc_stream_t s, int fmt, WSlice w, int K, int R, const uint16_t* x, int xs, float* y, int ys, int T,
                   int add, const uint32_t* G);
 void kc_mm_grouped_packed(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, float* y,
@@ -177,7 +180,10 @@ void kc_slice_deq(kc_stream_t s, int fmt, WSlice w, int K, int R, uint16_t* out)
  * chooses no expert more than T times); the bound is a promise: pairs of a tile beyond it are not computed, and their results are
  * stored as NaN so that a broken promise shows.  33 .. 48, 49 .. 64, 65 .. 96: tiles hold few pairs, mostly up to 32, 64, 96 - fuller ones
  * are computed too, in several passes.  Above MMT_BN: the tiles are mostly full, and an expert's adjoin.  Anything else: as
- * kc_mm_grouped_packed. */
+ * kc_mm_grouped_packed.  Every tile of up to MMT_BN pairs of any table is computed under every word (but for a broken promise).
+ * A result's last bits: f32 sums of the same products in an order that depends on K alone up to 48 (the order of kc_mm_packed's launches of
+ * few tokens), above 128 on K alone again (one chain over K), and otherwise on the tile's count and the counts of the tiles that adjoin it
+ * in its slice too.  A host that wants a pair's bits whatever else is in the batch says 48 or less. */
 void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, float* y,
                                int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles,
                                int tile_rows);

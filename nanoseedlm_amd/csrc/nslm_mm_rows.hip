@@ -7,9 +7,10 @@
 //     v_mfma_f32_16x16x32_bf16 (lane l: row l % 16, K block l / 16), so nothing is handed over or waited for between the decode and the
 //     matrix core, and every wave decodes, independently of the others until their sums meet;
 //   * the waves of a workgroup share its rows and split K: 64-weight chunk c belongs to segment c % 8, and a segment's sum is one
-//     chain of MFMAs.  8 waves a workgroup: a segment each; 4 waves (grouped launches, whose many workgroups overlap): two each.
-//     Either way y = sum over w < 4 of (segment w + segment w + 4), so a token's bits depend on K alone, not on the launch's
-//     shape, the tile or the tile's other tokens.
+//     chain of MFMAs.  8 waves a workgroup: a segment each; 4 waves (grouped launches, whose many workgroups overlap): two each,
+//     y = sum over w < 4 of (segment w + segment w + 4).  So a token's bits depend on K alone, not on the launch's shape, the tile or its
+//     other tokens, in every dense launch of this file and in grouped passes of up to 32 pairs.  Passes of more have no registers for two
+//     sums a pair: a wave's two segments are one chain there, and k_mm_wide's sum is one chain over all of K.
 // Measured (us, streamed kernel -> this one): P = 4, 4096 x 4096: 9 tokens 40.1 -> 9.7, 48 tokens 42.8 -> 11.1, 200 tokens 51.8 -> 23.0;
 // 1024 x 4096, 100 tokens 44.7 -> 11.2; Q4 2880 x 2880, 301 tokens 43.0 -> 17.8; BF16 151936 x 2048, 16 tokens 155.7 -> 115.3 (5.5 TB/s).
 // What bounds it: vector issue of the decode for the seed formats, the activations' way from L2 for Q4 / Q8 / BF16 at many tokens,

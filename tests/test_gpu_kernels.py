@@ -804,7 +804,7 @@ HAND_TILES = {
 def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
     """Every pair of every tile of a hand-made table is computed, whatever a tile's count and its neighbours, by every grouped launch and
     under every word on the tiles: the outputs hold NaN before, and what stays NaN was skipped.  Under one word a matrix's results are the same
-    bits from a launch of its own, of two matrices, and of gate + up + SwiGLU."""
+    bits from a launch of its own, of two matrices, and of gate + up + SwiGLU; under a word of up to 48 they are kc_mm_packed's bits of few tokens."""
     import ctypes as C
     from nanoseedlm_amd import backend, moe
     L = backend.hip()
@@ -812,9 +812,10 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
     tl = HAND_TILES[table]
     E, R, K, P = 4, {"long": 200, "round": 200, "triples": 128}.get(table, 150), (64 if table in ("long", "round") else 320), sum(n for _, n in tl)
     pk = [make_pack(rng, fmt, E, R, K) for _ in range(2)]
-    keep, tabs = [], []
+    keep, tabs, slices = [], [], []
     for p in pk:
         arr = (backend.WSlice * E)()
+        slices.append(arr)
         names = [("seeds", 0), ("coefs", 1), ("codes", 3)] if fmt == packs.MF_SEED4P4 else [("words", 0), ("scales", 1), ("biases", 2)]
         for name, i in names:
             buf = moe.DevBuf.from_array(np.ascontiguousarray(p[name]))
@@ -867,6 +868,14 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
         moe.device_sync()
         check(0, ys[0], ("rows", tile_rows))
         alone = ys[0].to_array(np.uint32, (P, R))
+        if tile_rows == 40:   # passes of up to 32 pairs: the dense kernel's bits, whatever tile a pair is in
+            for e in np.unique(slc):
+                rows = moe.DevBuf.from_array(packs.f32_to_bf16_bits(x[slc == e][:64]))
+                n = rows.nbytes // (2 * K)
+                L.kc_mm_packed(None, fmt, slices[0][e], K, R, rows.ptr, K, ys[1].ptr, R, n, 0, None)
+                moe.device_sync()
+                assert np.array_equal(ys[1].to_array(np.uint32, (n, R)), alone[slc == e][:64]), ("dense and rows", e)
+                rows.free()
         ys[0].free()
         ys[0] = moe.DevBuf.from_array(nan)
         L.kc_mm_grouped_packed_pair(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, ys[0].ptr, ys[1].ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
