@@ -285,7 +285,7 @@ def moe_workload(name, steps, warmup, n_layers, no_graph, q4_gemm_from=9):
         res["roofline"] = dict(bound="hbm", achieved=bytes_step / ms / 1e6, peak=HBM_PEAK_GBS, unit="GB/s",
                                frac=bytes_step / ms / 1e6 / HBM_PEAK_GBS,
                                kernel=("k_moe_decode_grouped (one launch per step)" if T <= 24 and name[:2] == "c2" else
-                                       "k_mm_stream<1, %d, %d> grouped (two launches of the step: gate + up + SwiGLU, down; with its glue kernels)" % (1 if T <= 32 else 4, 2 if T <= 32 and name[:2] == "c2" else 3)),
+                                       "grouped GEMM (k_mm_rows_grouped, k_mm_wide for mostly full tiles; two launches of the step: gate + up + SwiGLU, down; with its glue kernels)"),
                                launch_us=ms * 1e3, algorithmic_bytes=bytes_step, **counters_of(name))
     desc = {"c2": "C2 MoE decode layer step: 128 experts seeded P=4, top-8 softmax, hidden 2048, intermediate 768",
             "c3": "C3 mixed-format layer step: 64 experts seeded P=3, top-4, hidden 2880, intermediate 2880, plus seven 2880 x 2880 Q4-g64 projections (q, k, v, o, shared gate / up / down)"}[name[:2]]
@@ -358,7 +358,7 @@ def model_workload(name, steps, warmup, no_graph, branches=False, splits=32):
     res = dict(ms_per_step=ms, wall_ms_per_step=wall_ms / steps, bytes_per_step=bytes_step, tokens=T, flops_per_step=flops)
     res["roofline"] = dict(bound="hbm", achieved=bytes_step / ms / 1e6, peak=HBM_PEAK_GBS, unit="GB/s", frac=bytes_step / ms / 1e6 / HBM_PEAK_GBS,
                            traffic=None, traffic_source=None, kernel="whole decode step (%s x 24 is the largest share)" % ("k_moe_decode_cu" if T == 1 else "k_moe_decode" if T <= 8 else "k_moe_decode_grouped")
-                           if T <= 24 else "whole decode step (grouped k_mm_stream launches are the largest share)",
+                           if T <= 24 else "whole decode step (the grouped GEMM launches are the largest share)",
                            launch_us=ms * 1e3, algorithmic_bytes=bytes_step)
     res["config"] = {"workload": f"C4 full synthetic model greedy decode: 24 layers, hidden 2048, MLA 16 heads (latent 512 + rope 64, FP8 cache), "
                                  f"128 seeded P=4 experts top-8 (intermediate 768) + shared expert, vocab 151936 BF16 LM head, batch {T}, "
