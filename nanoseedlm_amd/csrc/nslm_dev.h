@@ -241,6 +241,150 @@ __device__ __forceinline__ void col_bytes_p4(uint32_t up, uint32_t g, uint32_t (
     G[5] = __builtin_amdgcn_perm(h23, h01, 0x07060302u) ^ 0x88888888u;
 }
 
+#define NSLM_R32 (1.0f / 32767.0f)
+
+// ---- the eight sums by one multiply-add each (the GEMMs' form) -----------------------------------------------------------------
+// The P states of a weight are one window of the stream, shifted: all but the few bits at its two ends are the same bits.  So one state times
+// one multiplier, and two small corrections that depend on the end bits alone, give the whole sum:
+//   P = 4, weight c, T = state_(4c+4), l = the three stream bits below it, h = the three above it:  state_(4c+1+p) = 2^(3-p) T + (l >> p) - 65536 (h >> p), so
+//     isum_c = M (T - 32768) + H(l) - 65536 H(h) + 32768 L,   M = 8 q0 + 4 q1 + 2 q2 + q3,   H(b) = q0 b + q1 (b >> 1) + q2 (b >> 2),   L = H(7);
+//   P = 3, T = state_(3c+1), l = its two lowest bits, h = the two stream bits above it:  state_(3c+1+p) = (T - T mod 2^p + 65536 (h mod 2^p)) / 2^p, so
+//     4 isum_c = M (T - 32768) - H(l) + 65536 H(h) - 32768 L,  M = 4 q0 + 2 q1 + q2,   H(b) = 2 q1 (b & 1) + q2 b,   L = H(3).
+// H has 8 (4) entries of a byte: two registers, looked up by v_perm.  P = 4: l and h are bits 4i + 1 .. 4i + 3 of the stream, i = c and c + 4, so
+// one v_perm looks up four of them, and one more a weight joins the two corrections.  H is antisymmetric, H(7 - b) = L - H(b), so a
+// flipped index changes the sign; -M comes from one dot product over the nibbles (8 is no int4, -8 is), and everything is formed negated.
+// The bytes are offset to be positive, so what a multiply-add leaves is an integer 0 < y < 2^24, y = k - isum (P = 3: k + 4 isum):
+//   P = 4: k = 32769 L + 88 * 65537, 1.8e6 <= y <= 9.4e6;   P = 3: k = 32768 L + 40 + 80 * 65536, 0.8e6 <= y <= 9.6e6.
+// Such an integer is a float's bits: y * 2^-149, subnormal or of the first binade, so no convert is needed and k goes by an exact subtraction.
+// A block is about 70 vector instructions as BF16 weights, records and all (four multiply-adds a weight, a convert and a multiply: about 95).
+struct SumTab4 {
+    uint32_t v[256];
+};
+struct SumTab3 {
+    uint32_t v[512];
+};
+constexpr int sext4(uint32_t n) { return (int) (n & 15u) - (int) ((n & 8u) << 1); }
+constexpr SumTab4 make_sumtab4() {   // entry { q0, q1 }: H(0..3) + 88
+    SumTab4 t{};
+    for (uint32_t b = 0; b < 256; ++b) {
+        const int q0 = sext4(b), q1 = sext4(b >> 4);
+        t.v[b] = 88u | (uint32_t) (88 + q0) << 8 | (uint32_t) (88 + 2 * q0 + q1) << 16 | (uint32_t) (88 + 3 * q0 + q1) << 24;
+    }
+    return t;
+}
+constexpr SumTab3 make_sumtab3() {   // entry { q1, q2 }: 40 - H(0..3), 80 + H(0..3)
+    SumTab3 t{};
+    for (uint32_t b = 0; b < 256; ++b) {
+        const int q1 = sext4(b), q2 = sext4(b >> 4), H[4] = {0, 2 * q1 + q2, 2 * q2, 2 * q1 + 3 * q2};
+        for (int i = 0; i < 4; ++i) {
+            t.v[2 * b] |= (uint32_t) (40 - H[i]) << (8 * i);
+            t.v[2 * b + 1] |= (uint32_t) (80 + H[i]) << (8 * i);
+        }
+    }
+    return t;
+}
+__device__ const SumTab4 kSumTab4 = make_sumtab4();
+__device__ const SumTab3 kSumTab3 = make_sumtab3();
+template <int P>
+constexpr int sum_tab_words() { return P == 4 ? 768 : 1024; }   // LDS: [0, 512) the stream basis, then the table above
+template <int P>
+__device__ __forceinline__ void load_sum_tables(uint32_t* tab) {
+    for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = kBasis.v[i];
+    for (int i = threadIdx.x; i < sum_tab_words<P>() - 512; i += blockDim.x) tab[512 + i] = P == 4 ? kSumTab4.v[i] : kSumTab3.v[i];
+}
+// half ha of a x half hb of b, int16, + c (ha, hb: constants once unrolled)
+#define NSLM_MAD16(HA, HB) asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b), "v"(c))
+__device__ __forceinline__ int mad16(uint32_t a, int ha, uint32_t b, int hb, int c) {
+    int d;
+    if (ha && hb) { NSLM_MAD16(1, 1); }
+    else if (ha) { NSLM_MAD16(1, 0); }
+    else if (hb) { NSLM_MAD16(0, 1); }
+    else { NSLM_MAD16(0, 0); }
+    return d;
+}
+// the nibbles of w x the int4 constants of C, + 0
+template <uint32_t C>
+__device__ __forceinline__ int dot8c(uint32_t w) {
+    int d;
+    asm("v_dot8_i32_i4 %0, %1, %2, 0" : "=v"(d) : "v"(w), "s"(C));
+    return d;
+}
+struct SumCoefs {
+    uint32_t lo, hi;   // the tables
+    uint32_t m;        // the multiplier, int16
+    uint32_t k;
+};
+// cc: a packed pair of coefficient (nibble) words, of which block `odd` (0 / 1) is taken; t: its entry of the LDS table (sum_tab_at)
+template <int P>
+__device__ __forceinline__ uint32_t sum_tab_at(uint32_t cc, int odd) {
+    return P == 4 ? (odd ? (cc >> 16) & 0xFFu : cc & 0xFFu) : 2u * (odd ? cc >> 24 : (cc >> 8) & 0xFFu);
+}
+template <int P>
+__device__ __forceinline__ SumCoefs sum_coefs(uint32_t cc, int odd, const uint32_t* t) {
+    SumCoefs s;
+    s.lo = t[0];
+    if constexpr (P == 4) {
+        const int h = odd ? dot8c<0x01240000u>(cc) : dot8c<0x0124u>(cc), l = odd ? dot8c<0x01370000u>(cc) : dot8c<0x0137u>(cc);
+        uint32_t t3;   // H(b + 4) = H(b) + h, h = 4 q0 + 2 q1 + q2 (three bytes, then the fourth: left to itself the compiler takes a 64-bit multiply)
+        asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(t3) : "v"(h), "s"(0x010101), "v"(s.lo));
+        s.hi = t3 + ((uint32_t) h << 24);
+        s.m = (uint32_t) (odd ? dot8c<0xFEC80000u>(cc) : dot8c<0xFEC8u>(cc));
+        s.k = (uint32_t) (__mul24(l, 32769) + 88 * 65537);
+    } else {
+        s.hi = t[1];
+        s.m = (uint32_t) (odd ? dot8c<0x12400000u>(cc) : dot8c<0x1240u>(cc));
+        s.k = ((uint32_t) (odd ? dot8c<0x32000000u>(cc) : dot8c<0x3200u>(cc)) << 15) + (uint32_t) (40 + 80 * 65536);
+    }
+    return s;
+}
+// A block's eight y.  up: any word whose upper 16 bits are the seed; g: the 32 stream bits that follow.  hook(0 .. 3) is called between the phases:
+// a caller with matrix instructions to issue puts them there, where the vector ALU has work beside them.
+template <int P, class Hook>
+__device__ __forceinline__ void sums_of(uint32_t up, uint32_t g, const SumCoefs& s, uint32_t (&y)[8], Hook hook) {
+    if constexpr (P == 4) {
+        const uint32_t le = __builtin_amdgcn_alignbit(g, up, 17), lo = __builtin_amdgcn_alignbit(g, up, 21);   // bits 1 .., 5 ..: fields 0, 2, 4, 6; 1, 3, 5, 7
+        const uint32_t he = g >> 1, ho = g >> 5;                                                             // bits 17 .., 21 ..: fields 4, 6, 8, 10; 5, 7, 9, 11
+        const uint32_t xl[2] = {__builtin_amdgcn_perm(s.hi, s.lo, ~le & 0x07070707u), __builtin_amdgcn_perm(s.hi, s.lo, ~lo & 0x07070707u)};
+        const uint32_t xh[2] = {__builtin_amdgcn_perm(s.hi, s.lo, he & 0x07070707u), __builtin_amdgcn_perm(s.hi, s.lo, ho & 0x07070707u)};
+        hook(0);
+        uint32_t A[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) A[c] = (c < 3 ? __builtin_amdgcn_alignbit(g, up, 20 + 4 * c) : g) ^ 0x80008000u;   // states 4c + 4, 4c + 20
+        hook(1);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = __builtin_amdgcn_perm(xh[c & 1], xl[c & 1], 0x0C040C00u + 0x00010001u * (uint32_t) (c >> 1));
+        hook(2);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = (uint32_t) mad16(A[c & 3], c >> 2, s.m, 0, (int) y[c]);
+        hook(3);
+    } else {
+        uint32_t W[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) W[c] = c < 5 ? __builtin_amdgcn_alignbit(g, up, 17 + 3 * c) : g >> (3 * c - 15);   // state 3c + 1 and the bits above it
+        hook(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = __builtin_amdgcn_perm(s.hi, s.lo, (W[c] & 0x00030003u) | 0x0C040C00u);
+        hook(1);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) W[c] ^= 0x8000u;
+        hook(2);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = (uint32_t) mad16(W[c], 0, s.m, 0, (int) y[c]);
+        hook(3);
+    }
+}
+// The weights times 2^(-eb - 22): y as a float's bits, k off (exact), times the block's scale (one rounding).  The products' sums are these of
+// the weights themselves to the last bit once sums_scale has put the power of two back.
+template <int P>
+__device__ __forceinline__ void sums_scaled(const uint32_t (&y)[8], uint32_t k, uint32_t code, float (&f)[8]) {
+    const float s = __uint_as_float((code << 23) + ((P == 4 ? 239u : 237u) << 23 | 0x100u));   // R32 = 2^-15 (1 + 2^-15); 2^(149 + 15 - 15 - 37 + code)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] = P == 4 ? __uint_as_float(k) - __uint_as_float(y[c]) : __uint_as_float(y[c]) - __uint_as_float(k);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] *= s;
+}
+__device__ __forceinline__ float sums_scale(float v, int eb) { return ldexpf(v, eb + 22); }
+
 // Two blocks at once, written in phases (all windows, then all sign flips, all pairings, all products) with the
 // scheduler held to that order: a VALU result is not available to the next instruction slots, and a wave that has a SIMD's
 // vector issue to itself loses those slots unless dependent instructions sit far apart.  In phase order every operand is at
@@ -285,7 +429,6 @@ __device__ __forceinline__ void block_isum(const uint32_t* tab, uint32_t seed16,
 }
 // 2^e as f32 bits; e in the normal range
 __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t) (e + 127) << 23); }
-#define NSLM_R32 (1.0f / 32767.0f)
 
 __device__ __forceinline__ int group_shift(const WSlice& w) { return w.gs ? w.gs : 6; }
 

@@ -343,35 +343,6 @@ struct MmRec2 {
     uint32_t u, v, c;  // seeds: two seeds, two coefficient words, the codes byte; Q8 / Q4: the group's scale and bias bits
 };
 
-// Two blocks' sums (isum_p4's / isum_p3's) in phase order, every operand a dozen instructions old, as a decoder wave that has a SIMD's vector
-// issue to itself needs them.  By multiply-adds on the windows' halves where they are (mad16): as many instructions as pairing the halves for
-// dot products, but a dot product runs on the matrix pipe and waits there for the consumers' MFMAs (14336 x 4096, by dot products and so: 512 tokens
-// P = 4 87.9 -> 85.1 us, P = 3 77.9 -> 76.7; 2048 tokens 328.7 -> 321.5, 315.4 -> 308.9; 16384 x 4096, 256 tokens 57.5 -> 57.5, 56.4 -> 55.0).
-template <int P>
-__device__ __forceinline__ void isum2_mad(const uint32_t (&up)[2], const uint32_t (&g)[2], const uint32_t (&qa)[2], const uint32_t (&qb)[2], int (&is)[2][8]) {
-    uint32_t A[2][17];
-#pragma unroll
-    for (int k = 1; k <= 15; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = __builtin_amdgcn_alignbit(g[h], up[h], 16 + k);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 1; k <= 16; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = (k < 16 ? A[h][k] : g[h]) ^ 0x80008000u;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k = P * c + 1 + p;
-                is[h][c] = mad16(A[h][k <= 16 ? k : k - 16], k > 16, p < 2 ? qa[h] : qb[h], p & 1, p ? is[h][c] : 0, p == 0);
-            }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
 template <int CT, int NCW, int XCH, int FMT>
 __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice wt, const uint16_t* X, float* Y) {
     constexpr int BN = 32 * CT * NCW, NTHR = 64 * (NCW + 4);   // XCH: chunks in a consumer wave's ring
@@ -381,12 +352,12 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     typedef uint16_t WTile[BM][LDW2];
     WTile* Wsm = (WTile*) (smem + NCW * XCH * XCHUNK);          // [2]
     __shared__ int srow[BN], drow[BN];
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wv >= NCW;
     const int r0 = (int) blockIdx.x * BM, start = (int) blockIdx.y * BN, count = min(BN, a.T - start);
     if (count < 1) return;
-    if (seedf) load_tables(tab);
+    if constexpr (seedf) load_sum_tables<seed_p<FMT>()>(tab);
     for (int i = tid; i < BN; i += NTHR) {
         const bool ok = i < count;
         srow[i] = start + (ok ? i : 0);   // padding rows load the tile's first row; their results are never stored
@@ -427,40 +398,28 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
             }
         };
         // seeds: the table reads of a step's two blocks are issued one step early (its records are in registers by then)
-        struct Look { uint32_t g[2], qa[2], qb[2]; };
+        struct Look { uint32_t g[2], t[2][2]; };
         auto lookup = [&](const MmRec2& r, Look& k) {
             if (!seedf) return;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const uint32_t seed = h ? r.u >> 16 : r.u & 0xFFFFu, word = h ? r.v >> 16 : r.v & 0xFFFFu;
-                k.g[h] = stream_of(tab, seed);
-                k.qa[h] = FMT == MF_SEED4P4 ? tab[512 + (word & 0xFFu)] : tab[512 + ((word >> 4) & 0xFFu)];
-                k.qb[h] = FMT == MF_SEED4P4 ? tab[512 + (word >> 8)] : tab[512 + (word >> 12)];
+                const uint32_t* e = tab + 512 + sum_tab_at<seed_p<FMT>()>(r.v, h);
+                k.g[h] = stream_of(tab, h ? r.u >> 16 : r.u & 0xFFFFu);
+                k.t[h][0] = e[0];
+                if (FMT == MF_SEED4) k.t[h][1] = e[1];
             }
         };
         auto produce = [&](int s, const MmRec2& r, const Look& k) {
             float f[2][8];
             {
-                if (seedf) {
-                    const uint32_t up[2] = {r.u << 16, r.u}, word[2] = {r.v & 0xFFFFu, r.v >> 16};
-                    int is[2][8];
-                    isum2_mad<FMT == MF_SEED4P4 ? 4 : 3>(up, k.g, k.qa, k.qb, is);
-                    float sc[2];
+                if constexpr (seedf) {   // (both blocks phase by phase: a decoder wave has a SIMD's vector issue to itself and waits for every result)
+                    constexpr int P = seed_p<FMT>();
+                    const SumCoefs sc[2] = {sum_coefs<P>(r.v, 0, k.t[0]), sum_coefs<P>(r.v, 1, k.t[1])};
+                    uint32_t y[2][8];
+                    sums_of<P>(r.u << 16, k.g[0], sc[0], y[0], [](int) {});
+                    sums_of<P>(r.u, k.g[1], sc[1], y[1], [](int) {});
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int code = FMT == MF_SEED4P4 ? (int) ((r.c >> (4 * h)) & 15u) : (int) (word[h] & 15u);
-                        sc[h] = pow2f(wt.eb + code) * NSLM_R32;
-                    }
-#pragma unroll
-                    for (int c = 0; c < 8; ++c)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) f[h][c] = (float) is[h][c];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int c = 0; c < 8; ++c)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) f[h][c] *= sc[h];
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int h = 0; h < 2; ++h) sums_scaled<P>(y[h], sc[h].k, FMT == MF_SEED4P4 ? (r.c >> (4 * h)) & 15u : (r.v >> (16 * h)) & 15u, f[h]);
                 } else if (FMT == MF_BF16) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
@@ -581,29 +540,29 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     bf16x8 f0[4], f1[4];
     wait_vm<4 * (XCH - 2)>();   // chunk 0 has landed
     load_a(0, f0);
-    for (int s = 0; s < nsteps; s += 2) {
-        step(s, f0, f1);
-        if (s + 1 >= nsteps) break;
-        if (CT & 1) step(s + 1, f1, f0);
-        else step(s + 1, f0, f1);
+    int s0 = 0;
+    for (; s0 + 1 < nsteps; s0 += 2) {
+        step(s0, f0, f1);
+        if (CT & 1) step(s0 + 1, f1, f0);
+        else step(s0 + 1, f0, f1);
     }
+    if (s0 < nsteps) step(s0, f0, f1);
     wait_vm<0>();
     // accumulator element v of lane l: token row 8 * (v / 4) + 4 * (l / 32) + v % 4, weight column l % 32
     const bool plain = !a.add && !a.f32out;
 #pragma unroll
     for (int m = 0; m < CT; ++m)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int tok = wtok + 32 * m + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-            const int dst = drow[tok];
-            if (dst < 0) continue;
+        for (int n = 0; n < 2; ++n) {
+            const int orow = r0 + 32 * n + (lane & 31);
+            if (orow >= a.R) continue;
 #pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                const int orow = r0 + 32 * n + (lane & 31);
-                if (orow >= a.R) continue;
+            for (int v = 0; v < 16; ++v) {
+                const int dst = drow[wtok + 32 * m + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
+                if (dst < 0) continue;
                 float* yo = Y + (size_t) dst * a.ys + orow;
-                if (plain) __builtin_nontemporal_store(bfr(acc[m][n][v]), yo);
-                else store_y(yo, acc[m][n][v], a.add, a.f32out);
+                if (plain) __builtin_nontemporal_store(bfr(mm_scale<FMT>(acc[m][n][v], wt.eb)), yo);
+                else store_y(yo, mm_scale<FMT>(acc[m][n][v], wt.eb), a.add, a.f32out);
             }
         }
 }

@@ -27,18 +27,15 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {   // v_cvt
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// half ha of a x half hb of b, int16, + c (ha, hb: constants once unrolled; the first product of a sum takes its zero inline)
-#define NSLM_MAD16(HA, HB)                                                                                                                             \
-    if (first) asm("v_mad_i32_i16 %0, %1, %2, 0 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b));                                              \
-    else asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b), "v"(c))
-__device__ __forceinline__ int mad16(uint32_t a, int ha, uint32_t b, int hb, int c, bool first) {
-    int d;
-    if (ha && hb) { NSLM_MAD16(1, 1); }
-    else if (ha) { NSLM_MAD16(1, 0); }
-    else if (hb) { NSLM_MAD16(0, 1); }
-    else { NSLM_MAD16(0, 0); }
-    return d;
-}
+template <int FMT>
+constexpr bool seed_fmt() { return FMT == MF_SEED4P4 || FMT == MF_SEED4; }
+template <int FMT>
+constexpr int seed_p() { return FMT == MF_SEED4 ? 3 : 4; }
+template <int FMT>
+constexpr int mm_tab_words() { return seed_fmt<FMT>() ? sum_tab_words<seed_p<FMT>()>() : 1; }
+// a sum of products with the weights, scaled as the format has them
+template <int FMT>
+__device__ __forceinline__ float mm_scale(float v, int eb) { return seed_fmt<FMT>() ? sums_scale(v, eb) : v; }
 
 // a kernel that asks for more dynamic LDS than the default limit has the limit raised to what it needs, once (the kernel is a
 // template argument so that every kernel has its own "once": kernels of one signature share a pointer type)

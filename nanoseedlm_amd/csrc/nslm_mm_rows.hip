@@ -1,6 +1,6 @@
 // nslm_mm_rows.hip - the GEMM for few tokens a matrix: Y[n][r] = sum_k W[r][k] X[n][k], dense or grouped by expert.
 //
-// With few tokens what a launch takes is the decode of the weights (about 100 vector instructions a seed block, four clocks each), and the
+// With few tokens what a launch takes is the decode of the weights (about 70 vector instructions a seed block, four clocks each), and the
 // chip has to be filled from R / 16 row tiles.  The streamed kernel's workgroups take 64 rows and decode with one wave a SIMD: 64
 // workgroups for 4096 rows, each decoding alone.  Here
 //   * a lane's decoded 8-weight block never leaves its registers: eight BF16 weights of one row are exactly a lane's operand of
@@ -30,8 +30,6 @@ namespace {
 //   Q4 / Q8      16 rows x 32 / 64 bytes a row tile (Q8: pieces swizzled); scales and biases stay in registers
 //   BF16         like the activations
 template <int FMT>
-constexpr bool seed_fmt() { return FMT == MF_SEED4P4 || FMT == MF_SEED4; }
-template <int FMT>
 constexpr int row_bytes() { return seed_fmt<FMT>() || FMT == MF_Q4 ? 32 : FMT == MF_Q8 ? 64 : 128; }   // of weights, a chunk
 template <int FMT, int RT, int NT, bool PACKED>
 constexpr int step_bytes() { return 16 * RT * (row_bytes<FMT>() + (FMT == MF_SEED4P4 ? 4 : 0)) + (PACKED ? NT * 2048 : 0); }
@@ -43,43 +41,22 @@ __device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
 }
 
-// A seed block as BF16 weights; up: any word whose upper 16 bits are the seed.  hook(0 .. 7) is called between the phases: a caller with
-// matrix instructions to issue puts them there, where the vector ALU has work beside them.
-// isum_p4's / isum_p3's sums by multiply-adds on the halves where they are: as many instructions as pairing halves for dot products, but a
-// dot product runs on the matrix pipe and waits there for, and holds up, every wave's MFMAs.
+// Block `odd` of the pair of seeds u and words v as BF16 weights.  hook(0 .. 7) is called between the phases (sums_of).
 template <int FMT, class Hook>
-__device__ __forceinline__ bf16x8 seed_weights(uint32_t up, uint32_t seed, uint32_t word, uint32_t code, int eb, const uint32_t* tab, Hook hook) {
-    constexpr int P = FMT == MF_SEED4P4 ? 4 : 3;
-    const uint32_t gs = stream_of(tab, seed), qa = P == 4 ? tab[512 + (word & 0xFFu)] : tab[512 + ((word >> 4) & 0xFFu)],
-                   qb = P == 4 ? tab[512 + (word >> 8)] : tab[512 + (word >> 12)];
-    const float e = pow2f(eb + (int) code) * NSLM_R32;
+__device__ __forceinline__ bf16x8 seed_weights(uint32_t u, uint32_t v, int odd, uint32_t codes, const uint32_t* tab, Hook hook) {
+    constexpr int P = seed_p<FMT>();
+    const uint32_t g = stream_of(tab, odd ? u >> 16 : u & 0xFFFFu);
+    const SumCoefs sc = sum_coefs<P>(v, odd, tab + 512 + sum_tab_at<P>(v, odd));
     hook(0);
-    uint32_t A[17];
-#pragma unroll
-    for (int k = 1; k <= 15; ++k) A[k] = __builtin_amdgcn_alignbit(gs, up, 16 + k);
-    A[16] = gs;
-    hook(1);
-#pragma unroll
-    for (int k = 1; k <= 16; ++k) A[k] ^= 0x80008000u;
-    int is[8];
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        hook(2 + p);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const int k = P * c + 1 + p;   // state k: A[k]'s low half, or A[k - 16]'s high half
-            is[c] = mad16(A[k <= 16 ? k : k - 16], k > 16, p < 2 ? qa : qb, p & 1, p ? is[c] : 0, p == 0);
-        }
-    }
-    if (P == 3) hook(5);
-    hook(6);
+    uint32_t y[8];
+    sums_of<P>(odd ? u : u << 16, g, sc, y, [&](int i) { hook(1 + i); });
     float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = (float) is[i];
+    sums_scaled<P>(y, sc.k, P == 4 ? (codes >> (4 * odd)) & 15u : (v >> (16 * odd)) & 15u, f);
+    hook(5);
+    bf16x8 w = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
+    hook(6);
     hook(7);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] *= e;
-    return __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
+    return w;
 }
 // eight Q4 (q.x) or Q8 weights
 template <int FMT>
@@ -185,9 +162,7 @@ struct Weights {
     template <class Hook>
     __device__ __forceinline__ bf16x8 block(const Step& s, int rt, int h, const uint32_t* tab, Hook hook) const {   // the lane's block 2 g + h of the chunk's eight
         if constexpr (SEED) {
-            const uint32_t word = h ? s.v[rt] >> 16 : s.v[rt] & 0xFFFFu;
-            return seed_weights<FMT>(h ? s.u[rt] : s.u[rt] << 16, h ? s.u[rt] >> 16 : s.u[rt] & 0xFFFFu, word,
-                                     FMT == MF_SEED4P4 ? (s.cd[rt] >> (4 * h)) & 15u : word & 15u, second(rt) ? m1.eb : m0.eb, tab, hook);
+            return seed_weights<FMT>(s.u[rt], s.v[rt], h, FMT == MF_SEED4P4 ? s.cd[rt] : 0u, tab, hook);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) hook(i);
@@ -199,6 +174,10 @@ struct Weights {
     __device__ __forceinline__ bf16x8 block(const Step& s, int rt, int h, const uint32_t* tab) const { return block(s, rt, h, tab, [](int) {}); }
 };
 
+template <int FMT>
+__device__ __forceinline__ f32x4 scaled(const f32x4& s, int eb) {
+    return (f32x4) {mm_scale<FMT>(s[0], eb), mm_scale<FMT>(s[1], eb), mm_scale<FMT>(s[2], eb), mm_scale<FMT>(s[3], eb)};
+}
 // four sums of pair / token dst, rows orow .. orow + 3 (those below R)
 __device__ __forceinline__ void store_rows(const MmArgs& a, float* Y, int dst, int orow, const f32x4& s) {
     float* yo = Y + (size_t) dst * a.ys + orow;
@@ -326,7 +305,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) red[((w * RT + rt) * NT + nt) * 64 + lane] = SEGS ? tot[rt][nt] : acc[rt][nt];
     __syncthreads();
-    auto sum = [&](int tile, int l) {
+    auto sum = [&](int tile, int l, int eb) {
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -334,15 +313,15 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
             if (NW == 8) p = ((f32x4) {0.0f, 0.0f, 0.0f, 0.0f} + p) + red[((i + 4) * RT * NT + tile) * 64 + l];
             s += p;
         }
-        return s;
+        return scaled<FMT>(s, eb);
     };
     const int nout = (gu ? RT / 2 : RT) * NT * 64;
     for (int i = tid; i < nout; i += 64 * NW) {
         const int tile = i >> 6, l = i & 63, rt = tile / NT, nt = tile % NT, tok = n0 + 16 * nt + (l & 15), orow = r0 + 16 * rt + 4 * (l >> 4);
         if (tok >= count || orow >= a.R) continue;
         const int dst = GROUPED ? perm[start + tok] : start + tok;
-        if (gu) store_swiglu(a, dst, orow, sum(tile, l), sum(tile + RT / 2 * NT, l));
-        else store_rows(a, Y, dst, orow, sum(tile, l));
+        if (gu) store_swiglu(a, dst, orow, sum(tile, l, m0.eb), sum(tile + RT / 2 * NT, l, m1.eb));
+        else store_rows(a, Y, dst, orow, sum(tile, l, m0.eb));
     }
 }
 
@@ -416,6 +395,8 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
         half(c, 1);   // (past the end: some block again)
     }
     const int orow = rw + 4 * g;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = scaled<FMT>(acc[nt], m.eb);
     if (gu) {   // the up sums meet the gate sums in LDS
         f32x4* const red = (f32x4*) lds;
         __syncthreads();
@@ -483,9 +464,9 @@ constexpr size_t MOST_LDS = 156 * 1024;   // beside the decode tables
 template <int FMT, int RT, int NT, bool PACKED>
 __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const void* X, float* Y) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
-    if (seed_fmt<FMT>()) {
-        load_tables(tab);
+    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
+    if constexpr (seed_fmt<FMT>()) {
+        load_sum_tables<seed_p<FMT>()>(tab);
         __syncthreads();
     }
     rows_tile<FMT, RT, NT, 8, PACKED, false>(a, w, w, X, Y, nullptr, 0, a.T, (int) blockIdx.y * 16 * NT, (int) blockIdx.x * 16 * RT, tab, lds);
@@ -497,7 +478,7 @@ template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
                                                                            const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
     // The grid has a workgroup row for as many tiles as the host's table holds.  Of fewer than `few` tiles, whose own workgroups do not fill the
     // chip, those past *ntiles take the later passes over 16 MOST pairs: pass 1 of every tile, then pass 2, .. (row nt + e: pass 1 + e / nt of
     // tile e % nt); the passes that they do not reach are the tile's own workgroups', after pass 0.  Tokens that agree on a few experts make
@@ -535,8 +516,8 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
             }
         }
     const int count = min(tl.count, limit);
-    if (seed_fmt<FMT>()) {
-        load_tables(tab);
+    if constexpr (seed_fmt<FMT>()) {
+        load_sum_tables<seed_p<FMT>()>(tab);
         __syncthreads();
     }
     for (int n0 = first; n0 < count; n0 = next, next += PASS) {
@@ -559,7 +540,7 @@ template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
@@ -573,8 +554,8 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     const WSlice m = gu && __builtin_amdgcn_readfirstlane((int) threadIdx.x) >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
     int count = tl.count;
     if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
-    if (seed_fmt<FMT>()) {
-        load_tables(tab);
+    if constexpr (seed_fmt<FMT>()) {
+        load_sum_tables<seed_p<FMT>()>(tab);
         __syncthreads();
     }
     const int r0 = (int) blockIdx.x * (gu ? 64 : 128);
