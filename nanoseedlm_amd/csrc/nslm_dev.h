@@ -103,31 +103,6 @@ __device__ __forceinline__ void load_tables(uint32_t* tab) {
     for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = kBasis.v[i];
     for (int i = threadIdx.x; i < 256; i += blockDim.x) tab[512 + i] = kPairs.v[i];
 }
-// The same for a workgroup of exactly NTHR threads (256, 512 or 1024), in two halves: a thread's loads are requested in
-// tables_fetch() (put it beside the kernel's other first loads), and tables_store() writes them to LDS once they are needed -
-// the loop above waits for every load in turn, one memory round trip each.
-template <int NTHR>
-struct TableWords {
-    uint32_t w[(NSLM_TAB_WORDS + NTHR - 1) / NTHR];
-};
-template <int NTHR>
-__device__ __forceinline__ TableWords<NTHR> tables_fetch() {
-    TableWords<NTHR> t;
-#pragma unroll
-    for (int j = 0; j < (NSLM_TAB_WORDS + NTHR - 1) / NTHR; ++j) {
-        const int i = min((int) threadIdx.x + NTHR * j, NSLM_TAB_WORDS - 1);   // clamped: the loads stay unconditional
-        t.w[j] = i < 512 ? kBasis.v[i] : kPairs.v[i - 512];
-    }
-    return t;
-}
-template <int NTHR>
-__device__ __forceinline__ void tables_store(uint32_t* tab, const TableWords<NTHR>& t) {
-#pragma unroll
-    for (int j = 0; j < (NSLM_TAB_WORDS + NTHR - 1) / NTHR; ++j) {
-        const int i = (int) threadIdx.x + NTHR * j;
-        if (i < NSLM_TAB_WORDS) tab[i] = t.w[j];
-    }
-}
 // keeps the loads written above this line above it: left alone, the compiler moves a load down to its first use, and a load
 // whose use sits in a conditional block becomes a load, a wait and a branch - one round trip per load instead of one for all
 __device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
@@ -190,60 +165,9 @@ __device__ __forceinline__ void isum_p3(uint32_t up, uint32_t g, uint32_t q01, u
     }
 }
 
-// ---- P = 4 by nibble columns (the matvec's form) -----------------------------------------------------------------------------
-// What a VALU instruction costs on this target was measured (issue slots of a SIMD with two or more waves resident): and / or /
-// xor / shift right / add / mov / f32 mul, fma / int -> f32 convert ~2.5 cycles; everything with three sources or sub-word
-// operands - v_alignbit, v_perm, v_bfe, shift left, the v_dot*, v_mad_* - ~4.3.  The exact decode above spends 47 of the
-// expensive ones a block (15 windows, 16 pairings, 16 dot2).  A matvec does not need the eight sums themselves, only
-// sum_c x_c isum_c, and that can be regrouped so that eleven v_dot8_i32_i4 do the 32 multiply-adds:
-//   state_(4c+1+p) = sum_n 16^n N_p(c + n),  N_p(m) = the nibble at bits [4m+1+p, 4m+5+p) of the 48-bit stream S (m = 0..10);
-//   sum_c x_c isum_c = sum_m Z(m) X(m) - 32768 Q SX,   Z(m) = sum_p q_p N_p(m),  X(m) = sum_n 16^n x_(m-n),  Q = sum_p q_p,  SX = sum_c x_c;
-//   with signed nibbles N' = N - 8 (one xor):  = sum_m Z'(m) X(m) + Q CX,  Z'(m) = sum_p q_p N'_p(m),  CX = (8 * 4369 - 32768) SX = 2184 SX.
-// N_p(m) is nibble m of V_p = S >> (1 + p), so byte j of V_0..V_3, gathered into one register (a 4 x 6 byte transpose: 12 v_perm),
-// holds the columns m = 2j and 2j + 1, and v_dot8_i32_i4 against the coefficient nibbles spread to the even (odd) nibble
-// positions gives Z'(2j) (Z'(2j + 1)).  Z' and Q are exact small integers; X and CX depend on the activations only and are
-// formed once per activation row (xform_block in nslm_mv_dev.h).  The weights are never materialised: kernels that need
-// them (the GEMM's decoder, kc_slice_deq) keep the exact sums above.
-__device__ __forceinline__ int dot8z(uint32_t a, uint32_t b) {
-    int d;
-    asm("v_dot8_i32_i4 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
-    return d;
-}
-// the coefficient nibbles q0..q3 of block `odd` (0 / 1) of a packed pair of coefficient words, one to a byte: the even-column operand
-__device__ __forceinline__ uint32_t coef_bytes(uint32_t cc, int odd) {
-    const uint32_t t = cc & 0x0F0F0F0Fu, u = (cc >> 4) & 0x0F0F0F0Fu;   // (q0, q2 | q0', q2'), (q1, q3 | q1', q3')
-    return __builtin_amdgcn_perm(u, t, odd ? 0x07030602u : 0x05010400u);
-}
-// the sum of the four coefficients of a coefficient operand (even-column form): a dot product with ones, the constant from a scalar register
-__device__ __forceinline__ int dot8ones(uint32_t a) {
-    int d;
-    asm("v_dot8_i32_i4 %0, %1, %2, 0" : "=v"(d) : "v"(a), "s"(0x01010101u));
-    return d;
-}
-// up: any word whose upper 16 bits are the seed, g: stream bits 16..47.  G[j] = byte j of V_0..V_3 with the nibbles made signed:
-// columns 2j (low nibbles) and 2j + 1 (high nibbles).  V_p's bytes 0..3 are one funnel shift of (g : up) by 17 + p, its bytes
-// 4 and 5 one shift of g - no word of the stream's low 32 bits is formed first.
-__device__ __forceinline__ void col_bytes_p4(uint32_t up, uint32_t g, uint32_t (&G)[6]) {
-    uint32_t vl[4], vh[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        vl[p] = __builtin_amdgcn_alignbit(g, up, 17 + p);
-        vh[p] = g >> (17 + p);
-    }
-    const uint32_t a01 = __builtin_amdgcn_perm(vl[1], vl[0], 0x05010400u), b01 = __builtin_amdgcn_perm(vl[1], vl[0], 0x07030602u);
-    const uint32_t a23 = __builtin_amdgcn_perm(vl[3], vl[2], 0x05010400u), b23 = __builtin_amdgcn_perm(vl[3], vl[2], 0x07030602u);
-    const uint32_t h01 = __builtin_amdgcn_perm(vh[1], vh[0], 0x05010400u), h23 = __builtin_amdgcn_perm(vh[3], vh[2], 0x05010400u);
-    G[0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x88888888u;
-    G[1] = __builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x88888888u;
-    G[2] = __builtin_amdgcn_perm(b23, b01, 0x05040100u) ^ 0x88888888u;
-    G[3] = __builtin_amdgcn_perm(b23, b01, 0x07060302u) ^ 0x88888888u;
-    G[4] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x88888888u;
-    G[5] = __builtin_amdgcn_perm(h23, h01, 0x07060302u) ^ 0x88888888u;
-}
-
 #define NSLM_R32 (1.0f / 32767.0f)
 
-// ---- the eight sums by one multiply-add each (the GEMMs' form) -----------------------------------------------------------------
+// ---- the eight sums by one multiply-add each (the matvecs' and the GEMMs' form) -----------------------------------------------------------------
 // The P states of a weight are one window of the stream, shifted: all but the few bits at its two ends are the same bits.  So one state times
 // one multiplier, and two small corrections that depend on the end bits alone, give the whole sum:
 //   P = 4, weight c, T = state_(4c+4), l = the three stream bits below it, h = the three above it:  state_(4c+1+p) = 2^(3-p) T + (l >> p) - 65536 (h >> p), so
@@ -256,7 +180,10 @@ __device__ __forceinline__ void col_bytes_p4(uint32_t up, uint32_t g, uint32_t (
 // The bytes are offset to be positive, so what a multiply-add leaves is an integer 0 < y < 2^24, y = k - isum (P = 3: k + 4 isum):
 //   P = 4: k = 32769 L + 88 * 65537, 1.8e6 <= y <= 9.4e6;   P = 3: k = 32768 L + 40 + 80 * 65536, 0.8e6 <= y <= 9.6e6.
 // Such an integer is a float's bits: y * 2^-149, subnormal or of the first binade, so no convert is needed and k goes by an exact subtraction.
-// A block is about 70 vector instructions as BF16 weights, records and all (four multiply-adds a weight, a convert and a multiply: about 95).
+// A block is about 70 vector instructions as BF16 weights, records and all (four multiply-adds a weight, a convert and a multiply: about 95);
+// as one token's products about 68 (P = 4 by eleven sums of nibble columns, a convert and a multiply-add each: 78; P = 3 by windows paired
+// for dot products: 76).  us a pass, before and after: layer step of 64 tokens (E 128, top-8, d 2048, ff 768, P = 4) 239 -> 200, of 8 tokens
+// 95 -> 86.5, of one 19.7 -> 18.3; of 3 tokens, E 64, top-4, d 2880, ff 2880, P = 3, 147 -> 134; 2880 x 2880, P = 3, 6 tokens 10.9 -> 10.2.
 struct SumTab4 {
     uint32_t v[256];
 };
@@ -291,6 +218,31 @@ template <int P>
 __device__ __forceinline__ void load_sum_tables(uint32_t* tab) {
     for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = kBasis.v[i];
     for (int i = threadIdx.x; i < sum_tab_words<P>() - 512; i += blockDim.x) tab[512 + i] = P == 4 ? kSumTab4.v[i] : kSumTab3.v[i];
+}
+// The same for a workgroup of exactly NTHR threads (256, 512 or 1024), in two halves: a thread's loads are requested in
+// tables_fetch() (put it beside the kernel's other first loads), and tables_store() writes them to LDS once they are needed -
+// the loop above waits for every load in turn, one memory round trip each.
+template <int P>
+__device__ __forceinline__ uint32_t sum_tab_word(int i) { return i < 512 ? kBasis.v[i] : P == 4 ? kSumTab4.v[i - 512] : kSumTab3.v[i - 512]; }
+template <int P, int NTHR>
+struct TableWords {
+    uint32_t w[(sum_tab_words<P>() + NTHR - 1) / NTHR];
+};
+template <int P, int NTHR>
+__device__ __forceinline__ TableWords<P, NTHR> tables_fetch() {
+    TableWords<P, NTHR> t;
+#pragma unroll
+    for (int j = 0; j < (sum_tab_words<P>() + NTHR - 1) / NTHR; ++j)
+        t.w[j] = sum_tab_word<P>(min((int) threadIdx.x + NTHR * j, sum_tab_words<P>() - 1));   // clamped: the loads stay unconditional
+    return t;
+}
+template <int P, int NTHR>
+__device__ __forceinline__ void tables_store(uint32_t* tab, const TableWords<P, NTHR>& t) {
+#pragma unroll
+    for (int j = 0; j < (sum_tab_words<P>() + NTHR - 1) / NTHR; ++j) {
+        const int i = (int) threadIdx.x + NTHR * j;
+        if (i < sum_tab_words<P>()) tab[i] = t.w[j];
+    }
 }
 // half ha of a x half hb of b, int16, + c (ha, hb: constants once unrolled)
 #define NSLM_MAD16(HA, HB) asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[" #HA "," #HB ",0,0]" : "=v"(d) : "v"(a), "v"(b), "v"(c))
@@ -373,6 +325,16 @@ __device__ __forceinline__ void sums_of(uint32_t up, uint32_t g, const SumCoefs&
         hook(3);
     }
 }
+// isum_c 2^-22 (exact): what a matvec multiplies with the activations; a row's sum is then multiplied by R32 2^22
+#define NSLM_SUM_R32 (NSLM_R32 * 4194304.0f)
+template <int P>
+__device__ __forceinline__ void sums_float(const uint32_t (&y)[8], uint32_t k, float (&f)[8]) {
+    const float s = __uint_as_float((P == 4 ? 254u : 252u) << 23), d = __uint_as_float(k) * s;   // 2^127, P = 3: a quarter
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] = P == 4 ? fmaf(__uint_as_float(y[c]), -s, d) : fmaf(__uint_as_float(y[c]), s, -d);
+}
+// 2^eb as f32 bits: a block's scale is this plus its code in the exponent field
+__device__ __forceinline__ uint32_t sums_e2(int eb) { return (uint32_t) (eb + 127) << 23; }
 // The weights times 2^(-eb - 22): y as a float's bits, k off (exact), times the block's scale (one rounding).  The products' sums are these of
 // the weights themselves to the last bit once sums_scale has put the power of two back.
 template <int P>
@@ -384,40 +346,6 @@ __device__ __forceinline__ void sums_scaled(const uint32_t (&y)[8], uint32_t k, 
     for (int c = 0; c < 8; ++c) f[c] *= s;
 }
 __device__ __forceinline__ float sums_scale(float v, int eb) { return ldexpf(v, eb + 22); }
-
-// Two blocks at once, written in phases (all windows, then all sign flips, all pairings, all products) with the
-// scheduler held to that order: a VALU result is not available to the next instruction slots, and a wave that has a SIMD's
-// vector issue to itself loses those slots unless dependent instructions sit far apart.  In phase order every operand is at
-// least a dozen instructions old.
-__device__ __forceinline__ void isum2_p3(const uint32_t (&up)[2], const uint32_t (&g)[2], const uint32_t (&q01)[2],
-                                         const uint32_t (&q2)[2], int (&is)[2][8]) {
-    uint32_t A[2][17], pr[2][8];
-#pragma unroll
-    for (int k = 1; k <= 15; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = __builtin_amdgcn_alignbit(g[h], up[h], 16 + k);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 1; k <= 16; ++k)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) A[h][k] = (k < 16 ? A[h][k] : g[h]) ^ 0x80008000u;
-    __builtin_amdgcn_sched_barrier(0);
-    int t[2][8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k0 = 3 * c + 1, k1 = k0 + 1, k2 = k0 + 2;   // state k lives in A[k] low (k <= 16) or A[k-16] high
-            pr[h][c] = halves(A[h][k0 <= 16 ? k0 : k0 - 16], k0 > 16, A[h][k1 <= 16 ? k1 : k1 - 16], k1 > 16);
-            t[h][c] = k2 <= 16 ? dot2z(A[h][k2], q2[h]) : dot2z(A[h][k2 - 16], q2[h] << 16);
-        }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) is[h][c] = dot2(pr[h][c], q01[h], t[h][c]);
-    __builtin_amdgcn_sched_barrier(0);
-}
 
 // One block of either seed format from its raw fields.  seed16 / word16: the 16-bit seed and coefficient (P = 4) or
 // nibble (P = 3) word, zero-extended.  Returns the integer sums and the block's exponent e = eb + code.

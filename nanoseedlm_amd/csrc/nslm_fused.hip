@@ -58,9 +58,7 @@ __device__ __forceinline__ void rows_pass(Chunk cur, const WSlice& wA, const WSl
         const Chunk nxt = fetch(v + rpi);
         float acc[1] = {0.0f};
         const int eb = (GATEUP && (v & 1)) ? wB.eb : wA.eb;
-        // (two blocks at a time in phase order where three workgroups a CU compute at once; the down pass, whose waves mostly
-        // run alone behind their pair's readiness, keeps the compiler's order)
-        if (active && v < v1) chunk_dot<P, 1, GATEUP>(cur, eb, tab, xl + ch * xpad<P>(), 0, 1, acc);
+        if (active && v < v1) chunk_dot<P, 1>(cur, eb, tab, xl + ch * XPAD, 0, acc);
         if (SHFL) {
             float s = acc[0];
             for (int o = L >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -70,9 +68,9 @@ __device__ __forceinline__ void rows_pass(Chunk cur, const WSlice& wA, const WSl
                 const float other = __shfl_xor(s, L);
                 if (active && ch == 0 && !(v & 1) && v < v1) {
                     if (gu) gu[(v - v0) >> 1] = make_float2(s, other);
-                    else emit(v >> 1, s * NSLM_R32, other * NSLM_R32);
+                    else emit(v >> 1, s * NSLM_SUM_R32, other * NSLM_SUM_R32);
                 }
-            } else if (active && ch == 0 && v < v1) emit(v, s * NSLM_R32, 0.0f);
+            } else if (active && ch == 0 && v < v1) emit(v, s * NSLM_SUM_R32, 0.0f);
         } else {
             part[par][tid] = acc[0];
             __syncthreads();
@@ -82,12 +80,12 @@ __device__ __forceinline__ void rows_pass(Chunk cur, const WSlice& wA, const WSl
                     float gs = 0.0f, us = 0.0f;
                     for (int j = 0; j < L; ++j) gs += part[par][(2 * tid) * L + j];
                     for (int j = 0; j < L; ++j) us += part[par][(2 * tid + 1) * L + j];
-                    emit((vb >> 1) + tid, gs * NSLM_R32, us * NSLM_R32);
+                    emit((vb >> 1) + tid, gs * NSLM_SUM_R32, us * NSLM_SUM_R32);
                 }
             } else if (tid < nrow) {
                 float s = 0.0f;
                 for (int j = 0; j < L; ++j) s += part[par][tid * L + j];
-                emit(vb + tid, s * NSLM_R32, 0.0f);
+                emit(vb + tid, s * NSLM_SUM_R32, 0.0f);
             }
         }
         cur = nxt;
@@ -97,16 +95,14 @@ __device__ __forceinline__ void rows_pass(Chunk cur, const WSlice& wA, const WSl
         __syncthreads();
         for (int i = tid; i < (v1 - v0) >> 1; i += 256) {
             const float2 q = gu[i];
-            emit((v0 >> 1) + i, q.x * NSLM_R32, q.y * NSLM_R32);
+            emit((v0 >> 1) + i, q.x * NSLM_SUM_R32, q.y * NSLM_SUM_R32);
         }
     }
 }
 
-// n floats of a row staged into LDS in the form the format's matvec reads (store_block: chunk-padded, P = 4 as its 12 column
-// values a block) by the whole workgroup; coherent: agent-scope loads (the row was written by other workgroups of this
+// n floats of a row staged into LDS, chunk-padded (store_block), by the whole workgroup; coherent: agent-scope loads (the row was written by other workgroups of this
 // launch).  A thread takes whole blocks, four a round, and requests their 32 words before the first is used (clamped
 // indices, so the loads are unconditional): one load and one LDS store a round is one memory round trip a round.
-template <int P>
 __device__ __forceinline__ void stage_row(const float* src, int n, float* xl, bool coherent) {
     const int nb = n / 8;
     for (int b0 = threadIdx.x; b0 < nb; b0 += 256 * 4) {
@@ -124,13 +120,12 @@ __device__ __forceinline__ void stage_row(const float* src, int n, float* xl, bo
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-            if (b0 + 256 * u < nb) store_block<P>(xl, b0 + 256 * u, v[u]);
+            if (b0 + 256 * u < nb) store_block(xl, b0 + 256 * u, v[u]);
     }
 }
 // an input row, normalised on the way when nw is given: the values kq4_norm1p would have stored
-template <int P>
 __device__ __forceinline__ void stage_input(const float* src, int n, float* xl, const float* nw, float rn) {
-    if (!nw) { stage_row<P>(src, n, xl, false); return; }
+    if (!nw) { stage_row(src, n, xl, false); return; }
     const int nb = n / 8;
     for (int b0 = threadIdx.x; b0 < nb; b0 += 256 * 4) {
         float v[4][8], w[4][8];
@@ -147,7 +142,7 @@ __device__ __forceinline__ void stage_input(const float* src, int n, float* xl, 
             if (b0 + 256 * u < nb) {
 #pragma unroll
                 for (int c = 0; c < 8; ++c) v[u][c] = v[u][c] * rn * (1.0f + w[u][c]);
-                store_block<P>(xl, b0 + 256 * u, v[u]);
+                store_block(xl, b0 + 256 * u, v[u]);
             }
     }
 }
@@ -202,7 +197,7 @@ template <int P, bool SHFL_G, bool SHFL_D, int WAVES>
 __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // WAVES waves a SIMD: five = at most 96 registers
     extern __shared__ float xl[];   // activations of the current pair: max(d, ff) floats, chunk-padded
     float2* const gu_s = (float2*) (xl + a.gu_off);   // behind them: the gate and up row sums of the item in hand
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[sum_tab_words<P>()];
     __shared__ float part[2][256];
     __shared__ __attribute__((aligned(16))) float rv[1024];   // route: the token's logits
     __shared__ float rw_s[33];      // route: weight by rank (+ the shared expert's 1)
@@ -241,11 +236,11 @@ __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // W
     }
     // The decode tables are first needed in phase 2: loaded here, behind the logits (everybody waits for the workgroups
     // that form logits; tables first was one more memory round trip on their way).
-    load_tables(tab);
+    load_sum_tables<P>(tab);
     // the first gate+up item's activations are an input of the launch: staged while the other workgroups' logits arrive
     if ((int) blockIdx.x < items_g) {
         staged = ((int) blockIdx.x / a.ntile_g) / a.kk;
-        stage_input<P>(a.x + (size_t) staged * a.xs, a.d, xl, a.nw, a.nw ? rn_s[staged] : 1.0f);
+        stage_input(a.x + (size_t) staged * a.xs, a.d, xl, a.nw, a.nw ? rn_s[staged] : 1.0f);
     }
     // No grid barrier: what the other workgroups produce here are the logits, and those say themselves when they are there.
     __syncthreads();   // every wave has used its copy of the generation
@@ -321,7 +316,7 @@ __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // W
         route_weights(t);
         if (staged != t) {
             __syncthreads();
-            stage_input<P>(a.x + (size_t) t * a.xs, a.d, xl, a.nw, a.nw ? rn_s[t] : 1.0f);
+            stage_input(a.x + (size_t) t * a.xs, a.d, xl, a.nw, a.nw ? rn_s[t] : 1.0f);
             staged = t;
             __syncthreads();
         }
@@ -373,7 +368,7 @@ __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // W
         }
         __syncthreads();
         wg_acquire();
-        stage_row<P>(a.A + (size_t) p * a.ff, a.ff, xl, true);
+        stage_row(a.A + (size_t) p * a.ff, a.ff, xl, true);
         staged = -1;
         __syncthreads();
         float* Dp = a.D + (size_t) p * a.d;
@@ -437,7 +432,7 @@ __device__ __forceinline__ void rows_pass_n(Chunk cur, const WSlice& wA, const W
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
         const int eb = (GATEUP && (v & 1)) ? wB.eb : wA.eb;
-        if (active && v < v1) chunk_dot<P, NT, true>(cur, eb, tab, xl + ch * xpad<P>(), xstride, nt, acc);
+        if (active && v < v1) chunk_dot<P, NT>(cur, eb, tab, xl + ch * XPAD, xstride, acc);
         if (SHFL) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
@@ -447,9 +442,9 @@ __device__ __forceinline__ void rows_pass_n(Chunk cur, const WSlice& wA, const W
                     const float other = __shfl_xor(s, L);
                     if (t < nt && active && ch == 0 && !(v & 1) && v < v1) {
                         if (gu) gu[t * ((v1 - v0) >> 1) + ((v - v0) >> 1)] = make_float2(s, other);   // (as in rows_pass)
-                        else emit(t, v >> 1, s * NSLM_R32, other * NSLM_R32);
+                        else emit(t, v >> 1, s * NSLM_SUM_R32, other * NSLM_SUM_R32);
                     }
-                } else if (t < nt && active && ch == 0 && v < v1) emit(t, v, s * NSLM_R32, 0.0f);
+                } else if (t < nt && active && ch == 0 && v < v1) emit(t, v, s * NSLM_SUM_R32, 0.0f);
             }
         } else {
             float* pp = part + par * NT * 256;
@@ -464,14 +459,14 @@ __device__ __forceinline__ void rows_pass_n(Chunk cur, const WSlice& wA, const W
                     float gs = 0.0f, us = 0.0f;
                     for (int j = 0; j < L; ++j) gs += pp[t * 256 + (2 * r) * L + j];
                     for (int j = 0; j < L; ++j) us += pp[t * 256 + (2 * r + 1) * L + j];
-                    emit(t, (vb >> 1) + r, gs * NSLM_R32, us * NSLM_R32);
+                    emit(t, (vb >> 1) + r, gs * NSLM_SUM_R32, us * NSLM_SUM_R32);
                 }
             } else {
                 for (int w = tid; w < nrow * nt; w += 256) {
                     const int t = w / nrow, r = w - t * nrow;
                     float sm = 0.0f;
                     for (int j = 0; j < L; ++j) sm += pp[t * 256 + r * L + j];
-                    emit(t, vb + r, sm * NSLM_R32, 0.0f);
+                    emit(t, vb + r, sm * NSLM_SUM_R32, 0.0f);
                 }
             }
         }
@@ -484,7 +479,7 @@ __device__ __forceinline__ void rows_pass_n(Chunk cur, const WSlice& wA, const W
         for (int i = tid; i < nr * nt; i += 256) {
             const int t = i / nr, r = i - t * nr;
             const float2 q = gu[i];
-            emit(t, (v0 >> 1) + r, q.x * NSLM_R32, q.y * NSLM_R32);
+            emit(t, (v0 >> 1) + r, q.x * NSLM_SUM_R32, q.y * NSLM_SUM_R32);
         }
     }
 }
@@ -500,7 +495,7 @@ __global__ void __launch_bounds__(256) k_moe_decode_grouped(FusedArgs a) {
     uint16_t* const gof = (uint16_t*) (xl + 1024);                 // [FG_MAXP] a pair's position among its expert's pairs
     uint16_t* const cnt_s = gof + FG_MAXP;                         // [1024 + 32] per expert: pairs
     uint16_t* const base_s = cnt_s + 1024 + 32;                    // [1024 + 32] per expert: first group
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[sum_tab_words<P>()];
     __shared__ float part[2 * NT * 256];
     __shared__ float rw_s[33];
     __shared__ int ri_s[33];
@@ -513,7 +508,7 @@ __global__ void __launch_bounds__(256) k_moe_decode_grouped(FusedArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const uint32_t G = (uint32_t) a.grid;
     const int P_ = a.T * a.kk, NE = a.E + a.ns;
-    const int xsg = a.Lg * xpad<P>(), xsd = a.Ld * xpad<P>();   // LDS floats between two rows of activations
+    const int xsg = a.Lg * XPAD, xsd = a.Ld * XPAD;   // LDS floats between two rows of activations
     // (fixed places, whatever the launch's rows and widths: launches of different sizes share the area, and every word
     // but the scales is back at zero when a launch ends)
     float* rnpub = (float*) (a.sync + FUSED_SYNC_WORDS);
@@ -524,7 +519,7 @@ __global__ void __launch_bounds__(256) k_moe_decode_grouped(FusedArgs a) {
     const uint32_t tag = my_gen + 1u;
     unsigned long long* lg64 = (unsigned long long*) (a.sync + FUSED_LOGIT_WORDS);
     unsigned long long* ind64 = (unsigned long long*) (a.sync + FUSED_IND_WORDS);
-    load_tables(tab);
+    load_sum_tables<P>(tab);
 
     // ---- phase 1: router logits, one wave per (token, expert) -------------------------------------------------------------
     if (a.nw) {   // the scales of the rows whose logits this workgroup forms (uniform over the workgroup)
@@ -680,7 +675,7 @@ __global__ void __launch_bounds__(256) k_moe_decode_grouped(FusedArgs a) {
         if (staged_g != g) {
             for (int m = 0; m < nt; ++m) {
                 const int t = gm[g * NT + m] / a.kk;
-                stage_input<P>(a.x + (size_t) t * a.xs, a.d, xl + m * xsg, a.nw, a.nw ? rn_s[t] : 1.0f);
+                stage_input(a.x + (size_t) t * a.xs, a.d, xl + m * xsg, a.nw, a.nw ? rn_s[t] : 1.0f);
             }
             staged_g = g;
             __syncthreads();
@@ -721,7 +716,7 @@ __global__ void __launch_bounds__(256) k_moe_decode_grouped(FusedArgs a) {
         }
         __syncthreads();
         wg_acquire();
-        for (int m = 0; m < nt; ++m) stage_row<P>(a.A + (size_t) gm[g * NT + m] * a.ff, a.ff, xl + m * xsd, true);
+        for (int m = 0; m < nt; ++m) stage_row(a.A + (size_t) gm[g * NT + m] * a.ff, a.ff, xl + m * xsd, true);
         staged_g = -1;
         __syncthreads();
         auto put_d = [&](int m, int r, float sm, float) { st_agent(a.D + (size_t) gm[g * NT + m] * a.d + r, bfr(sm)); };
@@ -817,7 +812,7 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     a.gu_off = (int) (lds / sizeof(float));
     lds += GU_ROWS * sizeof(float2);
     // One token is at most a few hundred items more than three workgroups a CU hold (C2: 784): that launch may use the
-    // registers of four waves a SIMD instead of five (107 instead of 96, no spills: 35.0 -> 34.5 us).  With the P = 4 column form the
+    // registers of four waves a SIMD instead of five (no spills: 35.0 -> 34.5 us).  At P = 4 the
     // same holds up to four tokens (C2, four / five waves, us: 2 tokens 41.4 / 45.8, 3: 55.6 / 56.3, 4: 66.4 / 69.8, 5: 85.9 / 80.3,
     // 8: 115.1 / 110.8; P = 3, C3: 2 tokens 166.5 / 157.7, 4: 272.6 / 263.7).
     const bool few = a.T == 1 || (P == 4 && a.T <= 4);
@@ -869,7 +864,7 @@ int launch_grouped(hipStream_t st, FusedArgs& a, bool sg, bool sd) {
     void (*kern)(FusedArgs) = sg ? (sd ? k_moe_decode_grouped<P, NT, true, true> : k_moe_decode_grouped<P, NT, true, false>)
                                  : (sd ? k_moe_decode_grouped<P, NT, false, true> : k_moe_decode_grouped<P, NT, false, false>);
     const int lmax = a.Lg > a.Ld ? a.Lg : a.Ld;
-    size_t lds = (size_t) NT * lmax * xpad<P>() * sizeof(float);
+    size_t lds = (size_t) NT * lmax * XPAD * sizeof(float);
     if (lds < FG_PRE_BYTES) lds = FG_PRE_BYTES;
 
     static int cached[2][2] = {{0, 0}, {0, 0}};   // resident workgroups per CU, by kernel variant, for the largest request seen
@@ -1006,7 +1001,7 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
     const bool cu_two = fmt != MF_SEED4P4 || (sg && (long) top_k * d * ff >= 24L << 20);
     if ((g_kernel_choice == 2 || (g_kernel_choice == 0 && T <= (cu_two ? 2 : 1))) && launch_moe_decode_cu((hipStream_t) s, a, fmt == MF_SEED4P4 ? 4 : 3, sd) == 0) return 0;
     const int kmax = d > ff ? d : ff;
-    size_t lds = (size_t) (kmax / 64) * (fmt == MF_SEED4P4 ? xpad<4>() : xpad<3>()) * sizeof(float);
+    size_t lds = (size_t) (kmax / 64) * XPAD * sizeof(float);
     return fmt == MF_SEED4P4 ? launch_fused<4>((hipStream_t) s, a, sg, sd, lds) : launch_fused<3>((hipStream_t) s, a, sg, sd, lds);
 }
 

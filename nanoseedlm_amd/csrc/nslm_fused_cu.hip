@@ -31,7 +31,7 @@ using namespace nslm;
 
 namespace {
 
-#define CU_LDS_MAX (160 * 1024 - NSLM_TAB_WORDS * 4)   // dynamic LDS: what the kernel's own table leaves of a CU's 160 KB
+#define CU_LDS_MAX (160 * 1024 - sum_tab_words<3>() * 4)   // dynamic LDS: what the kernel's own table leaves of a CU's 160 KB
 #define CU_LDS_MIN (82 * 1024)   // more than half a CU's LDS: two of these workgroups never share a CU
 #define CU_LG 4                  // router logits a CU forms
 #define CU_PRE_MAXE 256          // experts whose slice tables are copied to LDS while the logits are on their way
@@ -45,8 +45,8 @@ __device__ __forceinline__ uint32_t operator/(uint32_t x, FastDiv f) { return f.
 
 // What the host works out once per launch (offsets into the workgroup's dynamic LDS in 4-byte words, each a multiple of 4)
 struct CuParams {
-    int xg;      // [T][Lg * xpad] the tokens' inputs in the form the gate + up matvec reads
-    int xd;      // [kk][Ld * xpad] one token's A, all pairs, in the form the down matvec reads
+    int xg;      // [T][Lg * XPAD] the tokens' inputs in the form the gate + up matvec reads
+    int xd;      // [kk][Ld * XPAD] one token's A, all pairs, in the form the down matvec reads
     int scr;     // [4 NTHR] passes by iterations: the chunks' sums of three iterations, the first iteration's slots twice
     int pk;      // [T][KP] ranking: the logits' keys
     int rv;      // [T][E4] the logits
@@ -77,9 +77,9 @@ struct CuParams {
 // NORM: the launch normalises its input (a.nw); launches that do not are compiled without what that path adds.
 template <int P, bool SHFL_G, bool SHFL_D, int NTHR, bool NORM>
 __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c) {
-    constexpr int NW = NTHR / 64, XP = xpad<P>();
+    constexpr int NW = NTHR / 64, XP = XPAD;
     extern __shared__ __attribute__((aligned(16))) float dyn[];
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    __shared__ __attribute__((aligned(8))) uint32_t tab[sum_tab_words<P>()];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int G = c.G, T = a.T, E = a.E, kk = a.kk, Lg = a.Lg, Ld = a.Ld, E4 = c.E4, rpc = c.rpc;
     float* const xg = dyn + c.xg;
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
 
     // ---- what does not depend on the routing: generation, tables, slice tables, norm scales, the staged input, the logits ----
     const uint32_t gen = ld_agent(a.sync + 32 * (BAR_GROUPS + 1 + blockIdx.x % BAR_GROUPS));
-    const TableWords<NTHR> tw = tables_fetch<NTHR>();
+    const TableWords<P, NTHR> tw = tables_fetch<P, NTHR>();
     // the layer's three slice tables, 16 bytes of each a thread (unconditional: with more experts than the LDS copy takes,
     // pieces that are not kept)
     static_assert(CU_PRE_MAXE * sizeof(WSlice) / 16 <= NTHR, "a thread a piece covers a slice table");
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
                                : router_logit(a.rw + (size_t) e * a.d, a.x + (size_t) t * a.xs, a.d, a.nw, a.nw ? rn_s[t] : 1.0f);
         if (lane == 0) lgs[u] = lv;
     }
-    tables_store<NTHR>(tab, tw);
+    tables_store<P, NTHR>(tab, tw);
     if (preload && tid < per) {
         pre[tid] = pw0;
         pre[per + tid] = pw1;
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
 #pragma unroll
                     for (int cc = 0; cc < 8; ++cc) v[cc] = v[cc] * rn * (1.0f + w[cc]);
                 }
-                store_block<P>(xg + t * (Lg * XP), b, v);
+                store_block(xg + t * (Lg * XP), b, v);
             }
     }
     if (a.ns && tid < 3) {   // the shared expert's slices (field by field: a struct copy of a kernel argument goes through scratch memory)
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             const int qq = q_lo + (u >> c.lgV), jj = (int) ((uint32_t) qq / c.by_tpp);
             const size_t at = (size_t) (t * kk + jj) * a.ff + (size_t) (((qq - jj * c.tpp) << c.lgV) + (u & (c.vpt - 1)));
             const float2 gu = *(const float2*) &avs[2 * (t * nav + u)];
-            const float av = bfr(silu_bf(bfr(gu.x * NSLM_R32)) * bfr(gu.y * NSLM_R32));
+            const float av = bfr(silu_bf(bfr(gu.x * NSLM_SUM_R32)) * bfr(gu.y * NSLM_SUM_R32));
             st_agent(xa16 + at, (uint16_t) (__float_as_uint(av) >> 16));
             a.A[at] = av;
         }
@@ -413,7 +413,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             const Chunk nxt = fetch(tn, inx);
             const int q = q_lo + i, j = (int) ((uint32_t) q / c.by_tpp);
             float acc[1] = {0.0f};
-            chunk_dot<P, 1, true>(cur, slice_gu(t, j).eb, tab, xg + t * (Lg * XP) + ch * XP, 0, 1, acc);
+            chunk_dot<P, 1>(cur, slice_gu(t, j).eb, tab, xg + t * (Lg * XP) + ch * XP, 0, acc);
             float s = acc[0];
             for (int o = Lg >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
             const float other = __shfl_xor(s, Lg);
@@ -461,11 +461,11 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
                 const float* xq = xg + t * (Lg * XP) + q.ch * XP;
                 if (!q.tail) {
                     float acc[1] = {0.0f};
-                    if (q.f < nch) chunk_dot<P, 1, true>(cur, slice(t, j, vc & 1).eb, tab, xq, 0, 1, acc);
+                    if (q.f < nch) chunk_dot<P, 1>(cur, slice(t, j, vc & 1).eb, tab, xq, 0, acc);
                     ring_put(partg, q.f, acc[0]);
                 } else if constexpr (P == 3) {
                     if (q.f < nch) {   // (the lanes of a shared chunk take this branch together)
-                        const float sum = chunk_dot_split(cur, slice(t, j, vc & 1).eb, tab, xq, q.sub, ltg);
+                        const float sum = chunk_dot_split<P>(cur, slice(t, j, vc & 1).eb, tab, xq, q.sub, ltg);
                         if (q.sub == (1 << ltg) - 1) ring_put(partg, q.f, sum);
                     }
                 }
@@ -535,7 +535,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             const unsigned long long lo = ld_agent(src), hi = ld_agent(src + 1);
             const float v[8] = {bf((uint32_t) lo & 0xFFFFu), bf((uint32_t) (lo >> 16) & 0xFFFFu), bf((uint32_t) (lo >> 32) & 0xFFFFu), bf((uint32_t) (lo >> 48)),
                                 bf((uint32_t) hi & 0xFFFFu), bf((uint32_t) (hi >> 16) & 0xFFFFu), bf((uint32_t) (hi >> 32) & 0xFFFFu), bf((uint32_t) (hi >> 48))};
-            store_block<P>(xd, b, v);
+            store_block(xd, b, v);
         }
         __syncthreads();
     };
@@ -546,7 +546,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             float s = acc0;
             for (int o = Ld >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
             if (ok && dch == 0) {
-                const float dv = bfr(s * NSLM_R32);
+                const float dv = bfr(s * NSLM_SUM_R32);
                 dsum[g] = dv;
                 a.D[((size_t) t * kk + j) * a.d + r0 + rr] = dv;
             }
@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
 #pragma unroll
                     for (int cc = 0; cc < 16; ++cc) s += c0 + cc < Ld ? pv[cc] : 0.0f;
                 }
-                const float dv = bfr(s * NSLM_R32);
+                const float dv = bfr(s * NSLM_SUM_R32);
                 dsum[gs] = dv;
                 a.D[((size_t) t * kk + js) * a.d + r0 + rs] = dv;
             }
@@ -598,17 +598,16 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
         }
     };
     if (P == 4 && T == 1 && c.nit == 1) {
-        // One token whose down rows take one iteration: what the chunk can do without A - the streams, the byte transposition,
-        // the twelve exact column sums of every block - is done now, while A is still on its way between the CUs; what remains
-        // behind the exchange is a convert and a multiply-add a column (cols_pre / cols_post: chunk_dot's bits).
+        // One token whose down rows take one iteration: what the chunk can do without A - the streams and its 64 weights - is done now, while
+        // A is still on its way between the CUs; what remains behind the exchange is a multiply-add a weight (chunk_pre / chunk_post: chunk_dot's bits).
         if constexpr (P == 4) {
             const int g = dl, j = min((int) ((uint32_t) g / c.by_rpc), kk - 1), rr = g - (int) ((uint32_t) g / c.by_rpc) * rpc;
             const bool ok = dl < c.rpi && g < c.rows_t && rr < nr;
-            uint32_t zp[8][6];
-            if (ok) cols_pre(dcur, tab, zp);
+            float w8[8][8];
+            if (ok) chunk_pre<P>(dcur, tab, w8);
             wait_stage(0);
             float acc0 = 0.0f;
-            if (ok) cols_post(zp, dcur.codes, slice(0, j, 2).eb, xd + j * (Ld * XP) + dch * XP, acc0);
+            if (ok) chunk_post<P>(dcur, w8, slice(0, j, 2).eb, xd + j * (Ld * XP) + dch * XP, acc0);
             if constexpr (SHFL_D) rows_out(0, 0, acc0, ok, g, j, rr, true, tid);
             else {
                 // (one iteration: the threads' sums side by side, no ring - this path is the C2 step's, and every instruction of it counts)
@@ -624,7 +623,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
 #pragma unroll
                         for (int cc = 0; cc < 8; ++cc) sm += c0 + cc < Ld ? pv[cc] : 0.0f;
                     }
-                    const float dv = bfr(sm * NSLM_R32);
+                    const float dv = bfr(sm * NSLM_SUM_R32);
                     dsum[tid] = dv;
                     a.D[(size_t) js * a.d + r0 + rs] = dv;
                 }
@@ -646,9 +645,9 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             float acc[1] = {0.0f};
             int slot = ok ? q.f : -1;
             if (!q.tail) {
-                if (ok) chunk_dot<P, 1, false>(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, 0, 1, acc);
+                if (ok) chunk_dot<P, 1>(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, 0, acc);
             } else if constexpr (P == 3) {
-                if (ok) acc[0] = chunk_dot_split(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, q.sub, ltd);   // (a chunk's lanes together)
+                if (ok) acc[0] = chunk_dot_split<P>(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, q.sub, ltd);   // (a chunk's lanes together)
                 if (q.sub != (1 << ltd) - 1) slot = -1;
             }
             rows_out(t, it, acc[0], ok, g, j, rr, last, slot);
@@ -754,7 +753,7 @@ int launch_moe_decode_cu(hipStream_t st, FusedArgs& a, int P, bool sd) {
     c.by_Ld = fastdiv_of((uint32_t) a.Ld);
     c.by_nbp = fastdiv_of((uint32_t) c.nbp);
     c.by_kk = fastdiv_of((uint32_t) a.kk);
-    const int xp = P == 4 ? xpad<4>() : xpad<3>(), ws = (int) (sizeof(WSlice) / 4);
+    const int xp = XPAD, ws = (int) (sizeof(WSlice) / 4);
     int o = 0;
     auto take = [&](int words) { const int at = o; o += (words + 3) & ~3; return at; };
     c.xg = take(a.T * a.Lg * xp);

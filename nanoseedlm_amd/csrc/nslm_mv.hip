@@ -7,8 +7,8 @@
 // rpi = 256 / (K/64) rows per iteration; thread t keeps chunk t % (K/64) for the whole kernel, so at one token its 64
 // activations stay in registers and the records of consecutive threads are consecutive 16-byte units of the row-major
 // streams: every load instruction of a wave reads one contiguous kilobyte.  The LFSR stream of a seed comes from two
-// 256-entry LDS lookups (GF(2) linearity), the 32 states are 16-bit windows cut with v_alignbit, and the 8 integer
-// sums of a block are sixteen v_dot2_i32_i16 on packed state pairs: exact integers, one convert and one FMA per weight.
+// 256-entry LDS lookups (GF(2) linearity); a weight's exact integer sum is one multiply-add on a 16-bit window of the stream and two
+// table bytes, and becomes a float by the fma that takes its offset off (sums_of, sums_float): one more FMA a weight and token.
 // Row sums are reduced in a fixed order that depends on K and the entry point only, never on the token count, so a
 // token's rows are bit-identical whether it is computed alone or with others (the reference's batch invariance,
 // engine/kernels_moe.cu:239-240).
@@ -54,13 +54,11 @@ enum { DENSE = 0, GATHER = 1, GATEUP = 2, MULTI = 3 };
 // SHFL: L is a power of two <= 64 (<= 32 for GATEUP): row sums by wave shuffles, no barrier.  Otherwise through LDS.
 // NTHR: threads a workgroup (256; 512 or 1024 for one-token SHFL launches whose rows fill more than four waves a CU - the
 // row and the tables are then fetched once per CU instead of once per four waves).
-// COLS: P = 4 blocks in the column form (one- and two-token passes, and every pass of a launch of up to MV_MAXT tokens, whose
-// tokens get the bits of a one-token call); false: the weights' form (launches of more tokens, four to a pass).
-template <int P, int MODE, int NT, bool SHFL, int NTHR = 256, bool COLS = (P == 4)>
+template <int P, int MODE, int NT, bool SHFL, int NTHR = 256>
 __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
     static_assert(NTHR == 256 || (SHFL && NT == 1), "the LDS row sums and the staged multi-token passes are written for 256 threads");
-    extern __shared__ float xl[];                  // activations as the format reads them (xform_block): [token][chunk][xpad<P>()]
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    extern __shared__ float xl[];                  // activations: [token][chunk][XPAD]
+    __shared__ __attribute__((aligned(8))) uint32_t tab[sum_tab_words<P>()];
     __shared__ float part[SHFL ? 1 : 2][SHFL ? 1 : NT][SHFL ? 1 : 256];
     __shared__ float nred[4];
     // The workgroup's results wait here until the loop is over and leave as coalesced stores.  A store inside the loop costs a
@@ -90,12 +88,10 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
     const float* xrow = a.x + (size_t) (DN ? 0 : pair / a.xdiv) * a.xs;
     // Request order = return order (a wave's loads come back in the order they went out): the tables and the row, which sit in
     // L2 and are needed first, go out before the records, which come from HBM behind everybody else's.
-    const TableWords<NTHR> tw = tables_fetch<NTHR>();
+    const TableWords<P, NTHR> tw = tables_fetch<P, NTHR>();
     const bool prenorm = MODE == MULTI && a.nw != nullptr;   // uniform; the other modes compile without it
-    constexpr int XW = xw<P, COLS>(), XP = xpad<P, COLS>();
-    constexpr bool XREG = NT == 1 && !COLS;   // P = 3 keeps the thread's 64 activations in registers; the 96 column values of
-                                               // P = 4 stay in LDS (three 16-byte reads a block), which leaves the registers for eight waves a SIMD
-    float xreg[XREG ? 8 * XW : 1];
+    constexpr bool XREG = NT == 1 && P == 3;   // P = 3 keeps the thread's 64 activations in registers
+    float xreg[XREG ? 64 : 1];
     constexpr int NXQ = 1024 / NTHR;   // K <= 8192: at most 1024 blocks of a row, a thread takes whole blocks (two 16-byte pieces)
     float4 xq[NT == 1 ? NXQ : 1][2], wq[NT == 1 ? NXQ : 1][2];
     if (NT == 1) {   // clamped, so that the loads stay unconditional
@@ -137,7 +133,7 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
         // first wait, so the kernel starts after one memory round trip.
         // (with a norm: the row's scale, bit for bit as the norm kernel forms it - a second pass over the row, from L2)
         const float rn = (MODE == MULTI && prenorm) ? row_rnorm(xrow, a.K, a.neps, nred) : 1.0f;
-        tables_store<NTHR>(tab, tw);
+        tables_store<P, NTHR>(tab, tw);
 #pragma unroll
         for (int j = 0; j < NXQ; ++j) {
             const int i = tid + NTHR * j;
@@ -148,13 +144,13 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
 #pragma unroll
                     for (int c = 0; c < 8; ++c) x8[c] = x8[c] * rn * (1.0f + w8[c]);
                 }
-                store_block<P, COLS>(xl, i, x8);
+                store_block(xl, i, x8);
             }
         }
     } else {
         // Stage nt rows of K floats: 8 loads in flight a thread before the first store (a loop of load-then-store over a
         // run-time count waits for every load in turn).
-        tables_store<NTHR>(tab, tw);
+        tables_store<P, NTHR>(tab, tw);
         __shared__ float rn_s[NT];
         if (prenorm) {
             for (int t = 0; t < nt_; ++t) {
@@ -185,15 +181,15 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
 #pragma unroll
                     for (int c = 0; c < 8; ++c) x8[c] = x8[c] * rn * (1.0f + w8[c]);
                 }
-                store_block<P, COLS>(xl + (size_t) t * L * XP, i, x8);
+                store_block(xl + (size_t) t * L * XPAD, i, x8);
             }
         }
     }
     __syncthreads();
     if (XREG && active) {
 #pragma unroll
-        for (int i = 0; i < 2 * XW; ++i) {
-            const float4 q = *(const float4*) &xl[ch * XP + 4 * i];
+        for (int i = 0; i < 16; ++i) {
+            const float4 q = *(const float4*) &xl[ch * XPAD + 4 * i];
             xreg[4 * i] = q.x; xreg[4 * i + 1] = q.y; xreg[4 * i + 2] = q.z; xreg[4 * i + 3] = q.w;
         }
     }
@@ -209,8 +205,8 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
         for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
         const int eb = (MODE == GATEUP && (v & 1)) ? eB : eA;
         if (active && v < v1) {
-            if (XREG) chunk_dot<P, NT, false, COLS>(cur, eb, tab, xreg, 0, 1, acc);
-            else chunk_dot<P, NT, false, COLS>(cur, eb, tab, xl + ch * XP, L * XP, nt_, acc);
+            if (XREG) chunk_dot<P, NT, true>(cur, eb, tab, xreg, 0, acc);
+            else chunk_dot<P, NT>(cur, eb, tab, xl + ch * XPAD, L * XPAD, acc);
         }
         if (SHFL) {
 #pragma unroll
@@ -221,13 +217,13 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
                 if (MODE == GATEUP) {
                     const float other = __shfl_xor(s, L);   // rows 2r and 2r+1 sit side by side in the wave
                     if (active && ch == 0 && !(v & 1) && v < v1) {
-                        const float gs = s * NSLM_R32, us = other * NSLM_R32;
+                        const float gs = s * NSLM_SUM_R32, us = other * NSLM_SUM_R32;
                         ybuf[t][(v - v0) >> 1] = a.f32out ? (gs / (1.0f + expf(-gs))) * us : bfr(silu_bf(bfr(gs)) * bfr(us));
                     }
                 } else if (active && ch == 0 && v < v1) {
                     // a workgroup with one iteration has no later wait that a store could hold up: its sums leave at once
-                    if (single) store_y(yb + (size_t) (DN ? t : pair) * ys + v, s * NSLM_R32, add, a.f32out);
-                    else ybuf[t][v - v0] = s * NSLM_R32;
+                    if (single) store_y(yb + (size_t) (DN ? t : pair) * ys + v, s * NSLM_SUM_R32, add, a.f32out);
+                    else ybuf[t][v - v0] = s * NSLM_SUM_R32;
                 }
             }
         } else {
@@ -240,8 +236,8 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
                     float gs = 0.0f, us = 0.0f;
                     for (int j = 0; j < L; ++j) gs += part[par][0][(2 * tid) * L + j];
                     for (int j = 0; j < L; ++j) us += part[par][0][(2 * tid + 1) * L + j];
-                    gs *= NSLM_R32;
-                    us *= NSLM_R32;
+                    gs *= NSLM_SUM_R32;
+                    us *= NSLM_SUM_R32;
                     ybuf[0][((vb - v0) >> 1) + tid] = a.f32out ? (gs / (1.0f + expf(-gs))) * us : bfr(silu_bf(bfr(gs)) * bfr(us));
                 }
             } else {
@@ -249,7 +245,7 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
                     const int t = w / nrow, r = w - t * nrow;
                     float s = 0.0f;
                     for (int j = 0; j < L; ++j) s += part[par][t][r * L + j];
-                    ybuf[t][vb - v0 + r] = s * NSLM_R32;
+                    ybuf[t][vb - v0 + r] = s * NSLM_SUM_R32;
                 }
             }
         }
@@ -267,9 +263,9 @@ __global__ void __launch_bounds__(NTHR) k_mv_seed(MvArgs a) {
 }
 
 // ---- several tokens: the products on the matrix cores, with the one-token pass's bits --------------------------------------------
-// A block's products with 4 tokens are 4 x 8 (P = 4: 4 x 12) multiply-adds beside its 70 to 90 instructions of decode, and they are what
+// A block's products with 4 tokens are 4 x 8 multiply-adds beside its 60 instructions of decode, and they are what
 // grows with the tokens.  v_mfma_f32_4x4x1_16b_f32 is sixteen 4 x 4 outer products, one fused multiply-add an element: with a wave's four
-// adjacent lanes on the same chunk of four rows, A = a lane's own weight (column sum) and B = its token's activation, element (i, j)
+// adjacent lanes on the same chunk of four rows, A = a lane's own weight and B = its token's activation, element (i, j)
 // runs through chunk_dot's chain of multiply-adds for row i and token j, in its order - the same bits as a one-token call - at one
 // instruction a weight for 4 tokens, on a pipe of its own.  Lane j of the quad ends up with token j's sums of the four rows, and
 // takes each row's block scale from the lane that decoded it (a quad permutation inside the multiply-add).
@@ -284,9 +280,9 @@ __device__ __forceinline__ float quad_lane(float v) {   // lane I of the lane's 
 }
 template <int P, int NQ>
 __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, int rb, int tstride, bool shfl) {
-    constexpr int XW = xw<P>(), XP = xpad<P>();
-    extern __shared__ float xl[];   // [tr tokens][chunk][XP], tstride floats a token; then the chunk sums [row][token][L | 1]
-    __shared__ uint32_t tab[NSLM_TAB_WORDS];
+    constexpr int TW = sum_tab_words<P>(), TJ = (TW + 255) / 256;
+    extern __shared__ float xl[];   // [tr tokens][chunk][XPAD], tstride floats a token; then the chunk sums [row][token][L | 1]
+    __shared__ __attribute__((aligned(8))) uint32_t tab[TW];
     const int tid = threadIdx.x, nthr = blockDim.x, L = a.L, LS = L | 1;
     float* const part = xl + tr * tstride;
     const int quad = tid >> 2, ti = tid & 3, nquad = nthr >> 2;
@@ -299,12 +295,9 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
         return load_chunk<P>(a.wd, (uint32_t) row * (uint32_t) L + (uint32_t) (it - rq * L));
     };
     // requested in this order (see k_mv_seed): the tables, the first blocks of the activations, the records
-    uint32_t tw[3];
+    uint32_t tw[TJ];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int i = min(tid + nthr * j, NSLM_TAB_WORDS - 1);
-        tw[j] = i < 512 ? kBasis.v[i] : kPairs.v[i - 512];
-    }
+    for (int j = 0; j < TJ; ++j) tw[j] = sum_tab_word<P>(min(tid + nthr * j, TW - 1));
     const int nb = a.K / 8, tot = nt * nb;
     Chunk cur;
     for (int base = tid; base == tid || base < tot; base += nthr * 4) {   // four blocks a thread and round, their loads in flight together
@@ -320,8 +313,8 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
             cur = fetch(q0, quad);
             loads_issued();
 #pragma unroll
-            for (int j = 0; j < 3; ++j)
-                if (tid + nthr * j < NSLM_TAB_WORDS) tab[tid + nthr * j] = tw[j];
+            for (int j = 0; j < TJ; ++j)
+                if (tid + nthr * j < TW) tab[tid + nthr * j] = tw[j];
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -329,11 +322,11 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
             if (idx >= tot) break;
             const int t = idx / nb, i = idx - t * nb;
             const float x8[8] = {q[j][0].x, q[j][0].y, q[j][0].z, q[j][0].w, q[j][1].x, q[j][1].y, q[j][1].z, q[j][1].w};
-            store_block<P>(xl + t * tstride, i, x8);
+            store_block(xl + t * tstride, i, x8);
         }
     }
     __syncthreads();
-    const uint32_t ebase = (uint32_t) (a.wd.eb + 127) << 23;
+    const uint32_t ebase = sums_e2(a.wd.eb);
     for (int base = q0; base < q1; base += rb) {
         const int nrq = min(rb, q1 - base), items = nrq * L;
         for (int item = quad; item - quad < items; item += nquad) {
@@ -342,36 +335,20 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
             const int it = min(item, items - 1), rq = it / L, ch = it - rq * L;
             const float* xr[NQ];   // (tokens past the run's end: its last one again, never stored)
 #pragma unroll
-            for (int n = 0; n < NQ; ++n) xr[n] = xl + min(4 * n + ti, nt - 1) * tstride + ch * XP;
+            for (int n = 0; n < NQ; ++n) xr[n] = xl + min(4 * n + ti, nt - 1) * tstride + ch * XPAD;
             f32x4 acc[NQ];
 #pragma unroll
             for (int n = 0; n < NQ; ++n) acc[n] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
-                const uint32_t ss = word_of(cur.sd, b >> 1), cc = word_of(cur.cw, b >> 1);
-                const uint32_t g = stream_of(tab, (b & 1) ? ss >> 16 : ss & 0xFFFFu), up = (b & 1) ? ss : ss << 16;
-                float z[XW], e2;
-                if constexpr (P == 4) {
-                    const uint32_t be = coef_bytes(cc, b & 1), bo = be << 4;
-                    uint32_t G[6];
-                    col_bytes_p4(up, g, G);
-#pragma unroll
-                    for (int m = 0; m < 12; ++m) z[m] = (float) (m == 11 ? dot8ones(be) : dot8z(G[m >> 1], (m & 1) ? bo : be));
-                    e2 = __uint_as_float((((cur.codes >> (4 * b)) & 15u) << 23) + ebase);
-                } else {
-                    const uint32_t word = (b & 1) ? cc >> 16 : cc & 0xFFFFu;
-                    int is[8];
-                    isum_p3(up, g, tab[512 + ((word >> 4) & 0xFFu)], tab[512 + (word >> 12)], is);
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) z[c] = (float) is[c];
-                    e2 = __uint_as_float(((word & 15u) << 23) + ebase);
-                }
+                float z[8];
+                const float e2 = block_of<P>(cur, b, ebase, tab, z);
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) {
-                    const float* xt = xr[n] + XW * b;
+                    const float* xt = xr[n] + 8 * b;
                     f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                    for (int m = 0; m < XW; m += 4) {
+                    for (int m = 0; m < 8; m += 4) {
                         const float4 v = *(const float4*) (xt + m);
                         d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m], v.x, d, 0, 0, 0);
                         d = __builtin_amdgcn_mfma_f32_4x4x1f32(z[m + 1], v.y, d, 0, 0, 0);
@@ -402,7 +379,7 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
                 const int wc = min(w, sums - 1), t = wc / (4 * nrq), r = wc - t * 4 * nrq, row = 4 * base + r;
                 float s = part[(r * tr + t) * LS + l];
                 for (int o = L >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
-                if (l == 0 && w < sums && row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_R32, a.add, a.f32out);
+                if (l == 0 && w < sums && row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_SUM_R32, a.add, a.f32out);
             }
         } else {
             for (int w = tid; w < sums; w += nthr) {
@@ -411,7 +388,7 @@ __global__ void __launch_bounds__(1024) k_mv_tok(MvArgs a, int tr, int rq_wg, in
                 float s = 0.0f;
 #pragma unroll 4
                 for (int j = 0; j < L; ++j) s += p[j];
-                if (row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_R32, a.add, a.f32out);
+                if (row < a.R) store_y(yb + (size_t) t * a.ys + row, s * NSLM_SUM_R32, a.add, a.f32out);
             }
         }
         if (base + rb < q1) __syncthreads();
@@ -813,12 +790,6 @@ bool fast_shape(int fmt, int K, int mode, int* L, int* rpi, bool* shfl) {
     return true;
 }
 
-// staged floats per 64-weight chunk; cols: the launch's P = 4 blocks go in the column form
-int xpad_of(int fmt, bool cols = true) { return fmt == MF_SEED4P4 ? (cols ? xpad<4, true>() : xpad<4, false>()) : xpad<3>(); }
-// launches of up to MV_MAXT tokens give every token the bits of a one-token call (the column form); longer ones trade that for
-// the weights' form, which reads a third less LDS a token
-bool cols_for(int T) { return T <= MV_MAXT; }
-
 int cu_count() {
     static int n = 0;
     if (!n) {
@@ -863,31 +834,28 @@ void allow_lds(int bytes) {
 template <auto K>
 void allow_big_lds() { allow_lds<K>(MV_LDS_MAX); }
 #define MV_TOK_LDS (152 * 1024)   // k_mv_tok's, beside its tables
-template <int P, int MODE, int NT, bool COLS>
+template <int P, int MODE, int NT>
 void launch_seed256(hipStream_t st, const MvArgs& a, bool shfl, dim3 grid, size_t lds) {
     if (shfl) {
-        if (lds > 48 * 1024) allow_big_lds<k_mv_seed<P, MODE, NT, true, 256, COLS>>();
-        hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, true, 256, COLS>), grid, dim3(256), lds, st, a);
+        if (lds > 48 * 1024) allow_big_lds<k_mv_seed<P, MODE, NT, true, 256>>();
+        hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, true, 256>), grid, dim3(256), lds, st, a);
     } else {
-        if (lds > 48 * 1024) allow_big_lds<k_mv_seed<P, MODE, NT, false, 256, COLS>>();
-        hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, false, 256, COLS>), grid, dim3(256), lds, st, a);
+        if (lds > 48 * 1024) allow_big_lds<k_mv_seed<P, MODE, NT, false, 256>>();
+        hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, false, 256>), grid, dim3(256), lds, st, a);
     }
 }
 template <int P, int MODE, int NT>
-void launch_seed(hipStream_t st, const MvArgs& a, bool shfl, dim3 grid, size_t lds, int nthr = 256, bool cols = true) {
+void launch_seed(hipStream_t st, const MvArgs& a, bool shfl, dim3 grid, size_t lds, int nthr = 256) {
     if constexpr (NT == 1 && (MODE == DENSE || MODE == MULTI)) {
         if (shfl && nthr == 1024) { hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, true, 1024>), grid, dim3(1024), lds, st, a); return; }
         if (shfl && nthr == 512) { hipLaunchKernelGGL((k_mv_seed<P, MODE, NT, true, 512>), grid, dim3(512), lds, st, a); return; }
     }
-    if constexpr (P == 4 && NT > 2) {
-        if (!cols) { launch_seed256<P, MODE, NT, false>(st, a, shfl, grid, lds); return; }
-    }
-    launch_seed256<P, MODE, NT, P == 4>(st, a, shfl, grid, lds);
+    launch_seed256<P, MODE, NT>(st, a, shfl, grid, lds);
 }
 template <int MODE, int NT>
-void launch_seed_fmt(hipStream_t st, int fmt, const MvArgs& a, bool shfl, dim3 grid, size_t lds, int nthr = 256, bool cols = true) {
-    if (fmt == MF_SEED4P4) launch_seed<4, MODE, NT>(st, a, shfl, grid, lds, nthr, cols);
-    else launch_seed<3, MODE, NT>(st, a, shfl, grid, lds, nthr, cols);
+void launch_seed_fmt(hipStream_t st, int fmt, const MvArgs& a, bool shfl, dim3 grid, size_t lds, int nthr = 256) {
+    if (fmt == MF_SEED4P4) launch_seed<4, MODE, NT>(st, a, shfl, grid, lds, nthr);
+    else launch_seed<3, MODE, NT>(st, a, shfl, grid, lds, nthr);
 }
 
 // the wide path: BF16 / Q8 / Q4, whole blocks, 16-byte aligned activations and weights, staged activations within LDS
@@ -961,7 +929,7 @@ bool launch_tok(hipStream_t st, MvArgs a, int T, bool shfl) {
     const long quads = (long) rq * L;
     if (shfl && L <= 32 && (T == 2 || (T > 4 && quads >= 32L * cu_count() && quads <= 96L * cu_count()))) return false;
     // token stride: 16 banks apart, so that the 16-byte reads of a quad's four tokens do not meet
-    const int tstride = ((L * xpad<P>() + 63) / 64) * 64 + 16;
+    const int tstride = ((L * XPAD + 63) / 64) * 64 + 16;
     const size_t tok = (size_t) tstride * sizeof(float), tok_sums = (size_t) 4 * LS * sizeof(float);   // a token's, of a row quad
     auto held = [&](int tr, size_t lds) { return tr * tok >= lds ? 0 : (int) ((lds - tr * tok) / (tr * tok_sums)); };   // row quads' sums beside a run's tokens
     const int all = (rq + cu_count() - 1) / cu_count();   // row quads a CU
@@ -1045,18 +1013,17 @@ void kc_mv(kc_stream_t s, int fmt, WSlice w, int K, int R, const float* x, int x
             note_launch();
             return;
         }
-        const bool cols = cols_for(T);
-        if (T > 1 && (size_t) MV_TG * L * xpad_of(fmt, cols) * sizeof(float) <= MV_LDS_MAX) {
+        if (T > 1 && (size_t) MV_TG * L * XPAD * sizeof(float) <= MV_LDS_MAX) {
             a.ttot = T;
             launch_seed_fmt<DENSE, MV_TG>(st, fmt, a, shfl, dim3(grid.x, (unsigned) (T + MV_TG - 1) / MV_TG),
-                                          (size_t) MV_TG * L * xpad_of(fmt, cols) * sizeof(float), 256, cols);
+                                          (size_t) MV_TG * L * XPAD * sizeof(float));
         } else {
             for (int t0 = 0; t0 < T; ++t0) {
                 MvArgs b = a1;
                 b.x = x + (size_t) t0 * xs;
                 b.y = y + (size_t) t0 * ys;
                 b.nt = 1;
-                launch_seed_fmt<DENSE, 1>(st, fmt, b, shfl, grid1, (size_t) L * xpad_of(fmt) * sizeof(float), nthr);
+                launch_seed_fmt<DENSE, 1>(st, fmt, b, shfl, grid1, (size_t) L * XPAD * sizeof(float), nthr);
             }
         }
         note_launch();
@@ -1124,7 +1091,7 @@ int kc_mv_multi(kc_stream_t s, int fmt, int n, const WSlice* w, const int* R, fl
     int L, rpi;
     bool shfl;
     if (n < 1 || n > MV_MAXJ || T < 1 || T > MV_MULTI_MAXT || !fast_shape(fmt, K, DENSE, &L, &rpi, &shfl) || !aligned16(x) || xs % 4 ||
-        (size_t) MV_TG * L * xpad_of(fmt, cols_for(T)) * sizeof(float) > MV_LDS_MAX)
+        (size_t) MV_TG * L * XPAD * sizeof(float) > MV_LDS_MAX)
         return -1;
     if (norm_w && (K > 256 * 16 || !aligned16(norm_w))) return -1;
     MvArgs a = {};
@@ -1145,12 +1112,12 @@ int kc_mv_multi(kc_stream_t s, int fmt, int n, const WSlice* w, const int* R, fl
     if (T == 1) {
         a.nt = 1;
         for (int j = 0; j < n; ++j) a.yj[j] = y[j];
-        launch_seed_fmt<MULTI, 1>(st, fmt, a, shfl, grid, (size_t) L * xpad_of(fmt) * sizeof(float), nthr);
+        launch_seed_fmt<MULTI, 1>(st, fmt, a, shfl, grid, (size_t) L * XPAD * sizeof(float), nthr);
     } else {   // runs of MV_TG tokens over grid.y, as kc_mv's
         a.ttot = T;
         for (int j = 0; j < n; ++j) a.yj[j] = y[j];
         launch_seed_fmt<MULTI, MV_TG>(st, fmt, a, shfl, dim3(grid.x, (unsigned) (T + MV_TG - 1) / MV_TG),
-                                      (size_t) MV_TG * L * xpad_of(fmt, cols_for(T)) * sizeof(float), 256, cols_for(T));
+                                      (size_t) MV_TG * L * XPAD * sizeof(float));
     }
     note_launch();
     return 0;
@@ -1170,7 +1137,7 @@ void kc_mv_sel(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const flo
         a.L = L; a.rpi = rpi;
         a.rows_per_wg = pick_rows_per_wg(R, rpi, P);
         const dim3 grid((unsigned) ((R + a.rows_per_wg - 1) / a.rows_per_wg), (unsigned) P);
-        launch_seed_fmt<GATHER, 1>(st, fmt, a, shfl, grid, (size_t) L * xpad_of(fmt) * sizeof(float));
+        launch_seed_fmt<GATHER, 1>(st, fmt, a, shfl, grid, (size_t) L * XPAD * sizeof(float));
         note_launch();
         return;
     }
@@ -1193,7 +1160,7 @@ void kc_mv_gu(kc_stream_t s, int fmt, const WSlice* wg, const WSlice* wu, int K,
         a.L = L; a.rpi = rpi;
         a.rows_per_wg = pick_rows_per_wg(2 * R, rpi, P);
         const dim3 grid((unsigned) ((2 * R + a.rows_per_wg - 1) / a.rows_per_wg), (unsigned) P);
-        launch_seed_fmt<GATEUP, 1>(st, fmt, a, shfl, grid, (size_t) L * xpad_of(fmt) * sizeof(float));
+        launch_seed_fmt<GATEUP, 1>(st, fmt, a, shfl, grid, (size_t) L * XPAD * sizeof(float));
         note_launch();
         return;
     }

@@ -326,10 +326,11 @@ def test_mm_few_tokens(be, oracle, fmt, R, K):
             assert np.array_equal(y[:9].view(np.uint32), y9.view(np.uint32)), (NAMES[fmt], R, K, T)
 
 
-@pytest.mark.parametrize("T", [64, 512])   # 16384 rows: the kernel for few tokens, the streamed one
+# 16384 rows - GEMM: the kernel for few tokens, the streamed one; matvec: one token, a quad of rows a lane group (8), the staged pass
+@pytest.mark.parametrize("call,T", [("mm", 64), ("mm", 512), ("mv", 1), ("mv", 8), ("mv", 64)])
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
-def test_mm_weights_are_the_oracles_bits(be, oracle, fmt, T):
-    """One-hot activations read the weights out of the GEMM: all seeds (0 too), all coefficient words, the words of only the largest and smallest
+def test_one_hot_activations_read_the_oracles_weights(be, oracle, fmt, call, T):
+    """One-hot activations read the weights out of the products: all seeds (0 too), all coefficient words, the words of only the largest and smallest
     coefficients on the seeds with the most extreme states, every exponent code, exponent bases far from the usual one."""
     n = 131072
     rng = np.random.default_rng(fmt)
@@ -337,16 +338,16 @@ def test_mm_weights_are_the_oracles_bits(be, oracle, fmt, T):
     words[65536:65536 + 2048] = np.resize([0x8888, 0x7777, 0x8000, 0x0008, 0x7778, 0x8887, 0x0888, 0x8880], 2048)   # (on seeds 0 .. 2047)
     words[-2048:] = np.resize([0x8888, 0x7777, 0x8000, 0x0007, 0x7778, 0x8887, 0x0777, 0x7770], 2048)                 # (.. 65535)
     R = n // 8
-    x = np.resize(np.eye(64, dtype=np.float32), (T, 64))
+    x = np.resize(np.eye(64, dtype=np.float32)[::-1], (T, 64))
     for eb in (-22, 40, -90):
         p = {"fmt": fmt, "S": 1, "R": R, "K": 64, "seeds": seeds.reshape(1, R, 8), "eb": np.array([eb], dtype=np.int32)}
         p["coefs" if fmt == packs.MF_SEED4P4 else "nibs"] = words.reshape(1, R, 8)
         if fmt == packs.MF_SEED4P4:
             p["codes"] = packs._pack_nibbles(rng.integers(0, 16, size=(1, n), dtype=np.uint8))
         want = packs.bf16_bits_to_f32(oracle.slice_bf16(fmt, slice_of(oracle, p, 0), R, 64)).T
-        got = be.kt_mm_plain(p, x, packed=1)
-        for t in range(0, T, 64):
-            assert np.array_equal(got[t:t + 64], want), (eb, t)
+        got = be.kt_mm_plain(p, x, packed=1) if call == "mm" else be.kt_mv(p, x)
+        for t in range(T):
+            assert np.array_equal(got[t], want[63 - t % 64]), (eb, t)
 
 
 # f32 activations at token counts that the first-generation kernel had (seeds: from 200 tokens; BF16: at 130): the last token tile partial, one row past a tile
