@@ -25,7 +25,7 @@ namespace {
 // Loads in an MFMA operand's layout (consecutive lanes in different rows) cost the address unit a cycle a lane; staged by
 // global_load_lds, consecutive lanes take consecutive 16-byte pieces of a row.  The wave reads a step into registers at once and
 // requests the next one into the same place, so the LDS holds one step a wave and its decode covers the latency.
-//   activations  [16 NT][64] BF16, the 16-byte pieces of a row swizzled (x_swizzle) so that a fragment read spreads over the banks
+//   activations  [16 NT][64] BF16, the 16-byte pieces of a row swizzled (x_swizzle16) so that a fragment read spreads over the banks
 //   seeds        per row tile: 16 rows x 16 bytes of seeds, 16 x 16 of coefficient words; then 16 x 4 of codes
 //   Q4 / Q8      16 rows x 32 / 64 bytes a row tile (Q8: pieces swizzled); scales and biases stay in registers
 //   BF16         like the activations
@@ -102,7 +102,7 @@ struct Weights {
                 pa[i] = ((g & 1) ? stream(rt, 1) : stream(rt, 0)) + (size_t) row_of(16 * rt + t) * (size_t) (K / 4);
             } else {
                 const int at = 1024 * i + 16 * lane, r = min(at / RB, 16 * RT - 1), piece = (at % RB) / 16;
-                const int sw = FMT == MF_BF16 ? piece ^ x_swizzle(r & 15) : FMT == MF_Q8 ? piece ^ ((r >> 2) & 3) : piece;
+                const int sw = FMT == MF_BF16 ? piece ^ x_swizzle16(r & 15) : FMT == MF_Q8 ? piece ^ (r >> 3 & 1) * 3 : piece;
                 pa[i] = stream(r >> 4, 0) + (size_t) row_of(r) * (size_t) (K / 64 * RB) + 16 * sw;
             }
         }
@@ -147,11 +147,11 @@ struct Weights {
                 if (FMT == MF_SEED4P4) s.cd[rt] = ws[CODES + 64 * rt + 4 * t + g];
             } else if constexpr (FMT == MF_BF16) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) s.raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+                for (int h = 0; h < 2; ++h) s.raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle16(t)));
             } else {
                 s.u[rt] = sc[rt];
                 s.v[rt] = bi[rt];
-                if (FMT == MF_Q8) s.raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ ((t >> 2) & 3)));
+                if (FMT == MF_Q8) s.raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ (t >> 3) * 3));
                 else {
                     const uint2 b = *(const uint2*) (ws + 512 * rt + 32 * t + 8 * g);
                     s.raw[rt][0] = make_uint4(b.x, b.y, 0, 0);
@@ -216,7 +216,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
 #pragma unroll
         for (int i = 0; i < 2 * NT; ++i) {
             const int n = 8 * i + (lane >> 3);
-            px[i] = (uint32_t) (src_of(n) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle(n & 15));
+            px[i] = (uint32_t) (src_of(n) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle16(n & 15));
         }
     } else {
 #pragma unroll
@@ -250,7 +250,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 if constexpr (PACKED) {
-                    xb[HALVES ? 0 : h][nt] = *(const bf16x8*) (wx + nt * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t)));
+                    xb[HALVES ? 0 : h][nt] = *(const bf16x8*) (wx + nt * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle16(t)));
                 } else {
                     const NSLM_GLOBAL uint8_t* xp = gp<uint8_t>(X) + (size_t) (px[nt] + 16u * (uint32_t) c + 2u * h) * 16;
                     const uint4 va = ldg16(xp), vb = ldg16(xp + 16);
@@ -346,7 +346,7 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 #pragma unroll
     for (int i = 0; i < NT / 4; ++i) {
         const int n = 64 * i + 8 * w + (lane >> 3);
-        px[i] = (uint32_t) (((size_t) (perm[start + min(n, count - 1)] / a.xdiv) * (size_t) a.xs) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle(n & 15));
+        px[i] = (uint32_t) (((size_t) (perm[start + min(n, count - 1)] / a.xdiv) * (size_t) a.xs) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle16(n & 15));
     }
     auto request_x = [&](int c) {
 #pragma unroll
@@ -362,7 +362,7 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
     typename Weights<FMT, 1>::Step st;
     bf16x8 wb, xq[XD][NG];
     auto half = [&](int c, int h) {   // multiplies (c, h) while the next half's weights are formed
-        const uint8_t* const xt = lds + (c & 1) * NT * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle(t));
+        const uint8_t* const xt = lds + (c & 1) * NT * 2048 + t * 128 + 16 * ((2 * g + h) ^ x_swizzle16(t));
         auto fetch = [&](int i) {
 #pragma unroll
             for (int j = 0; j < NG; ++j)
