@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const 
 //   level 1: a wave ranks each group of 64 consecutive values among themselves (64 compares a lane against keys read as
 //            LDS broadcasts); a value with k or more larger values in its own group cannot be among the k best of the row,
 //   level 2: the survivors (at most k a group) are ranked among themselves; rank r < k is the r-th pick.
-// No serial arg-max rounds: the depth of the computation does not grow with k.  One workgroup of 256 threads a row.
+// No serial arg-max rounds: the depth of the computation does not grow with k.  NTHR threads a row; rows of a workgroup go through the same barriers.
 // MODE 0, the softmax router (engine/kernels_qwen4.cu:385-416 semantics: ties to the higher index, weights = softmax over
 // the k picked, summed in pick order); MODE 1, the sigmoid router's selection (ties to the lowest index, weights =
 // score / sum of the picked scores * scale, engine/kernels_moe.cu:742-772 semantics).
@@ -163,16 +163,17 @@ __device__ __forceinline__ uint32_t float_order(float v) {
     const uint32_t b = __float_as_uint(v + 0.0f);   // -0 ranks as +0
     return b ^ ((uint32_t) ((int32_t) b >> 31) | 0x80000000u);
 }
-// row t of the launch, by a workgroup of NTHR threads (every thread reaches the end: callers may go on with a barrier)
+// row t of the launch, by NTHR threads (every thread reaches the end: callers may go on with a barrier)
 // COH: the selection is stored past the L2 of this workgroup's XCD (agent-scope atomic stores), for a reader in the same launch
+constexpr int topk_lds(int E) { return ((E + 63) & ~63) * 12 + 8 * TK_MAXK + 4 * TK_MAXK + 16; }   // bytes a row
 template <int MODE, int NTHR, bool COH = false>
-__device__ __forceinline__ void topk_row(int t, int E, int k, const float* vals, int ld, const float* score, float scale, int32_t* ind, float* wt) {
-    __shared__ __attribute__((aligned(16))) unsigned long long key[TK_MAXE];   // 0 = no value: below every real key
-    __shared__ unsigned long long skey[TK_MAXE / 2];                           // survivors of level 1 (at most 32 of every 64)
-    __shared__ float pv[TK_MAXK], pw[TK_MAXK];
-    __shared__ int pi[TK_MAXK];
-    __shared__ int nsurv;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+__device__ __forceinline__ void topk_row(int t, int E, int k, const float* vals, int ld, const float* score, float scale, int32_t* ind, float* wt, uint8_t* lds) {
+    const int tid = threadIdx.x % NTHR, lane = tid & 63, wv = tid >> 6;
+    unsigned long long* const key = (unsigned long long*) lds;           // [E64], 0 = no value: below every real key
+    unsigned long long* const skey = key + ((E + 63) & ~63);             // [E64 / 2]: survivors of level 1 (at most 32 of every 64)
+    float* const pv = (float*) (skey + ((E + 63) & ~63) / 2);
+    float* const pw = pv + TK_MAXK;
+    int *const pi = (int*) (pw + TK_MAXK), &nsurv = pi[TK_MAXK];
     const float* row = vals + (size_t) t * ld;
     const int E64 = (E + 63) & ~63;
     for (int e = tid; e < E64; e += NTHR)
@@ -220,7 +221,8 @@ __device__ __forceinline__ void topk_row(int t, int E, int k, const float* vals,
 template <int MODE>
 __global__ void __launch_bounds__(256) k_topk_rank(int E, int k, const float* vals, int ld, const float* score, float scale, int32_t* ind,
                                                    float* wt) {
-    topk_row<MODE, 256>((int) blockIdx.x, E, k, vals, ld, score, scale, ind, wt);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[topk_lds(TK_MAXE)];
+    topk_row<MODE, 256>((int) blockIdx.x, E, k, vals, ld, score, scale, ind, wt, lds);
 }
 
 // ---- elementwise --------------------------------------------------------------------------------------------------------
@@ -314,35 +316,9 @@ __device__ __forceinline__ unsigned long long equal_lanes(int e, int nbits) {
     }
     return m;
 }
-// COH: the selections were stored by other workgroups of this launch (agent-scope atomic loads)
-template <bool COH = false>
-__device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
-    auto sel_at = [&](int i) { return COH ? __hip_atomic_load(inds + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : inds[i]; };
-    extern __shared__ uint32_t hist[];   // [BK_WAVES][n]
-    __shared__ int wsum[2][BK_WAVES];
+// The whole workgroup: thread x < n has the number of expert x's pairs.  Writes the offsets and the expert's tiles, returns its first pair.
+__device__ __forceinline__ int scan_experts(int cnt, int n, int32_t* work, MmTile* tiles, int (*wsum)[BK_WAVES]) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    int nbits = 1;
-    while ((1 << nbits) < n) ++nbits;
-    ++nbits;   // one more bit: lanes past the end of the run hold the value n-or-above 1 << (nbits - 1) and only equal each other
-    const int run = ((count + BK_WAVES - 1) / BK_WAVES + 63) & ~63, i0 = wv * run, i1 = min(count, i0 + run);
-    uint32_t* mine = hist + (size_t) wv * n;
-    for (int i = tid; i < BK_WAVES * n; i += 64 * BK_WAVES) hist[i] = 0;
-    __syncthreads();
-    for (int i = i0; i < i1; i += 64) {
-        int e = i + lane < i1 ? sel_at(i + lane) : -1;
-        const bool live = (unsigned) e < (unsigned) n;   // an index outside the table is left out
-        if (!live) e = 1 << (nbits - 1);
-        const unsigned long long eq = equal_lanes(e, nbits);
-        if (live && (eq & ((1ull << lane) - 1ull)) == 0) mine[e] += (uint32_t) __popcll(eq);
-    }
-    __syncthreads();
-    int cnt = 0;
-    if (tid < n)
-        for (int w = 0; w < BK_WAVES; ++w) {
-            const uint32_t c = hist[(size_t) w * n + tid];
-            hist[(size_t) w * n + tid] = (uint32_t) cnt;
-            cnt += (int) c;
-        }
     const int ntl = (cnt + MMT_BN - 1) / MMT_BN;
     int pin = cnt, tin = ntl;   // inclusive sums over the experts: across the wave, then across the waves
     for (int o = 1; o < 64; o <<= 1) {
@@ -356,7 +332,6 @@ __device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n
     if (tid < n) {
         work[1 + tid] = pofs;
         work[2 + n + tid] = tofs;
-        for (int w = 0; w < BK_WAVES; ++w) hist[(size_t) w * n + tid] += (uint32_t) pofs;
         for (int j = 0; j < ntl; ++j) {
             MmTile tl;
             tl.slice = tid;
@@ -371,33 +346,94 @@ __device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n
             work[0] = tofs + ntl;
         }
     }
-    __syncthreads();
-    for (int i = i0; i < i1; i += 64) {
-        int e = i + lane < i1 ? sel_at(i + lane) : -1;
-        const bool live = (unsigned) e < (unsigned) n;
-        if (!live) e = 1 << (nbits - 1);
-        const unsigned long long eq = equal_lanes(e, nbits), before = eq & ((1ull << lane) - 1ull);
-        if (live) {
-            const uint32_t at = mine[e];   // every lane of the group reads before its first lane moves the mark (LDS in wave order)
-            perm[at + (uint32_t) __popcll(before)] = i + lane;
-            if (before == 0) mine[e] = at + (uint32_t) __popcll(eq);
+    return pofs;
+}
+// COH: the selections were stored by other workgroups of this launch (agent-scope atomic loads).  STEPS steps' selections are requested together, and
+// a run of up to so many keeps them and their equals for the second pass: a load and a wait a step, twice, took two thirds of the launch that groups
+// 2048 rows of 8.
+template <bool COH, int STEPS>
+__device__ __forceinline__ void bucket_steps(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles, int (*wsum)[BK_WAVES]) {
+    auto sel_at = [&](int i) { return COH ? __hip_atomic_load(inds + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : inds[i]; };
+    extern __shared__ uint32_t hist[];   // [BK_WAVES][n]
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    int nbits = 1;
+    while ((1 << nbits) < n) ++nbits;
+    ++nbits;   // one more bit: lanes past the end of the run hold the value n-or-above 1 << (nbits - 1) and only equal each other
+    const int run = ((count + BK_WAVES - 1) / BK_WAVES + 63) & ~63, i0 = wv * run, i1 = min(count, i0 + run);
+    uint32_t* mine = hist + (size_t) wv * n;
+    for (int i = tid; i < BK_WAVES * n; i += 64 * BK_WAVES) hist[i] = 0;
+    int e[STEPS];
+    unsigned long long eq[STEPS];
+    auto load = [&](int i) {
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u) e[u] = sel_at(min(i + 64 * u + lane, count - 1));
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u) {
+            if (i + 64 * u + lane >= i1 || (unsigned) e[u] >= (unsigned) n) e[u] = 1 << (nbits - 1);   // an index outside the table is left out
+            eq[u] = equal_lanes(e[u], nbits);
         }
+    };
+    const bool kept = run <= 64 * STEPS;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    __syncthreads();
+    for (int i = i0; i < i1; i += 64 * STEPS) {
+        load(i);
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u)
+            if (e[u] < n && (eq[u] & below) == 0) mine[e[u]] += (uint32_t) __popcll(eq[u]);
     }
+    __syncthreads();
+    int cnt = 0;
+    if (tid < n)
+        for (int w = 0; w < BK_WAVES; ++w) {
+            const uint32_t c = hist[(size_t) w * n + tid];
+            hist[(size_t) w * n + tid] = (uint32_t) cnt;
+            cnt += (int) c;
+        }
+    const int pofs = scan_experts(cnt, n, work, tiles, wsum);
+    if (tid < n)
+        for (int w = 0; w < BK_WAVES; ++w) hist[(size_t) w * n + tid] += (uint32_t) pofs;
+    __syncthreads();
+    for (int i = i0; i < i1; i += 64 * STEPS) {
+        if (!kept) load(i);
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u)
+            if (e[u] < n) {
+                const uint32_t at = mine[e[u]];   // every lane of the group reads before its first lane moves the mark (LDS in wave order)
+                perm[at + (uint32_t) __popcll(eq[u] & below)] = i + 64 * u + lane;
+                if ((eq[u] & below) == 0) mine[e[u]] = at + (uint32_t) __popcll(eq[u]);
+            }
+    }
+}
+template <bool COH>
+__device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
+    __shared__ int wsum[2][BK_WAVES];
+    if (count <= 64 * BK_WAVES) bucket_steps<COH, 1>(inds, count, n, work, perm, tiles, wsum);
+    else if (count <= 4 * 64 * BK_WAVES) bucket_steps<COH, 4>(inds, count, n, work, perm, tiles, wsum);
+    else if (count <= 8 * 64 * BK_WAVES) bucket_steps<COH, 8>(inds, count, n, work, perm, tiles, wsum);
+    else bucket_steps<COH, 16>(inds, count, n, work, perm, tiles, wsum);
 }
 __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
     bucket_all<false>(inds, count, n, work, perm, tiles);
 }
-// The batched softmax step's routing and grouping in one launch: workgroup t ranks row t (k_topk_rank<0>'s arithmetic), and the
-// workgroup that finishes last - a ticket in the word behind the bucket's work area, back at zero when the launch ends -
-// groups the launch's pairs (k_bucket's).  Nobody waits for anybody.
+// The batched softmax step's routing and grouping in one launch: the workgroups rank the rows (k_topk_rank<0>'s arithmetic; ROWS 1 or 4 a workgroup),
+// and the workgroup that finishes last - a ticket in the word behind the bucket's work area, back at zero when the
+// launch ends - groups the launch's pairs (k_bucket's).  Nobody waits for anybody.
+template <int ROWS>
 __global__ void __launch_bounds__(64 * BK_WAVES) k_route_bucket(int E, int k, const float* logits, int ld, int32_t* ind, float* wt, int T, int32_t* work,
                                                                 int32_t* perm, MmTile* tiles) {
     __shared__ int last;
-    topk_row<0, 64 * BK_WAVES, true>((int) blockIdx.x, E, k, logits, ld, (const float*) 0, 1.0f, ind, wt);
-    if (threadIdx.x == 0) {   // wave 0 stored the row's selection: those stores have left the wave before the ticket is taken
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];   // the rows' ranking, then the grouping
+    const int sub = __builtin_amdgcn_readfirstlane((int) threadIdx.x / (64 * BK_WAVES / ROWS));   // (rows past the end: the last one again, the same values)
+    topk_row<0, 64 * BK_WAVES / ROWS, true>(min(ROWS * (int) blockIdx.x + sub, T - 1), E, k, logits, ld, (const float*) 0, 1.0f, ind, wt, dyn + sub * topk_lds(E));
+    if (ROWS > 1) {   // the selections have left their waves before the workgroup's ticket is taken
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {   // (one row: wave 0 stored its selection)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        last = atomicAdd((unsigned*) &work[2 * E + 3], 1u) == (unsigned) (T - 1);
+        last = atomicAdd((unsigned*) &work[2 * E + 3], 1u) == gridDim.x - 1u;
     }
     __syncthreads();
     if (!last) return;
@@ -716,12 +752,21 @@ void kq4_route_bucket(kc_stream_t s, const Qwen4Cfg* c, const float* logits, int
                       int32_t* ntiles) {
     if (T < 1) return;
     if (c->n_exp < c->top_k || c->n_exp > TK_MAXE || c->top_k < 1 || c->top_k > TK_MAXK || c->n_exp > BUCKET_MAX_EXPERTS) { host_note_unsupported(); return; }
-    const size_t lds = sizeof(uint32_t) * BK_WAVES * (size_t) c->n_exp;
-    static const hipError_t once = hipFuncSetAttribute((const void*) k_route_bucket, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));
-    (void) once;
-    hipLaunchKernelGGL(k_route_bucket, dim3((unsigned) T), dim3(64 * BK_WAVES), lds, (hipStream_t) s, c->n_exp, c->top_k, logits, c->n_exp, ind, wt, T,
-                       ntiles, perm, tiles);
+    // Rows by fours where they are more than a workgroup on every other CU (E 128 / 64, top-8, us a launch by ones and by fours: 32 rows 7.6 and 8.3, 64 rows
+    // 8.1 and 8.5; 200 rows 11.0 and 10.4; 2048 rows, which had taken 54.1, 31.0 by fours).
+    const size_t group = sizeof(uint32_t) * BK_WAVES * (size_t) c->n_exp;
+#define ROUTE(ROWS)                                                                                                                                              \
+    do {                                                                                                                                                         \
+        static const hipError_t once = hipFuncSetAttribute((const void*) k_route_bucket<ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize,                        \
+                                                           (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));                                            \
+        (void) once;                                                                                                                                             \
+        const size_t rows = (size_t) ROWS * topk_lds(c->n_exp), lds = group > rows ? group : rows;                                                               \
+        hipLaunchKernelGGL(k_route_bucket<ROWS>, dim3((unsigned) (T + ROWS - 1) / ROWS), dim3(64 * BK_WAVES), lds, (hipStream_t) s, c->n_exp, c->top_k, logits,   \
+                           c->n_exp, ind, wt, T, ntiles, perm, tiles);                                                                                 \
+    } while (0)
+    if (T > host_cu_count() / 2) ROUTE(4);
+    else ROUTE(1);
+#undef ROUTE
     host_note_launch();
 }
 void kc_cache_admit(kc_stream_t s, const CachePool* p, int sl, const int32_t* inds, int count, int flags) {
