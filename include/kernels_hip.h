@@ -162,6 +162,9 @@ void kc_moe_combine(kc_stream_t s, const float* D, const float* w, const float* 
 /* engine/kernels_qwen4.h:71, engine/kernels_qwen4.cu:514-516 */
 void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* wt, const float* sh, const float* sg,
                      int sgld, float* out, int T);
+/* (ours: the same over D as BF16 bits, kc_mm_grouped_packed_bf16's) */
+void kc_moe_combine_bf16(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T);
+void kq4_moe_combine_bf16(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T);
 
 /* ---- expert slot table (engine/kernels_cuda.h:53-55, engine/kernels_moe.cu:2710-2722) ------------------------------ */
 void kc_cache_admit(kc_stream_t s, const CachePool* p, int sl, const int32_t* inds, int count, int flags);
@@ -187,6 +190,10 @@ void kc_slice_deq(kc_stream_t s, int fmt, WSlice w, int K, int R, uint16_t* out)
 void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, float* y,
                                int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles,
                                int tile_rows);
+/* The same with the results, which are BF16 values, stored as their BF16 bits y [pair][ys], for mostly full tiles (tile_rows above MMT_BN).  -1 (nothing
+ * launched) for any other word, and where K % 64, x or xs is not aligned, the weights are in exact mode or kc_store_f32(1) is set. */
+int kc_mm_grouped_packed_bf16(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, uint16_t* y, int ys, int xdiv,
+                              const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows);
 /* Two grouped GEMMs of one shape over the same tiles and activations in one launch (an expert's gate and up matrices: ya = the
  * ws_a slices' product, yb = the ws_b slices'), each bit for bit what kc_mm_grouped_packed_rows gives alone: one launch's ramp
  * and tail instead of two.  No counterpart in the reference (two launches, engine/mova_cuda.c:1308-1311). */

@@ -29,6 +29,7 @@ struct NslmMoe {
     int32_t *ind, *perm, *ntiles;
     MmTile* tiles;
     int max_tiles;
+    int d16;                    /* the last step left the experts' outputs in D as BF16 bits */
     uint32_t* sync;             /* device: the fused decode kernel's barrier words */
     int fused;                  /* 1: steps of the softmax composition up to kc_moe_decode_max_rows() rows take kc_moe_decode;
                                    2: the same, and every such step is checked and redone by the separate launchers if it failed */
@@ -293,6 +294,7 @@ int nslm_moe_step_layer(NslmMoe* m, kc_stream_t s, int layer, const float* xn, i
                             c->d, m->logit, m->ind, m->wt, m->A, m->D, m->sync, shared, res, norm_w, norm_eps))
         return 1;
     m->fused_steps++;
+    m->d16 = 0;
     return kc_last_error() ? -1 : 0;
 }
 
@@ -321,6 +323,7 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
     const NslmMoeCfg* c = &m->c;
     if (!m->final || T < 1 || T > c->max_rows || layer < 0 || layer >= c->n_layer) return -1;
     const int E = c->n_exp, k = c->top_k, d = c->d, ff = c->ff, P = T * k;
+    m->d16 = 0;
     const WSlice* gate = m->pool.tab + ((size_t) layer * 3 + 0) * E;
     const WSlice* up = m->pool.tab + ((size_t) layer * 3 + 1) * E;
     const WSlice* down = m->pool.tab + ((size_t) layer * 3 + 2) * E;
@@ -411,8 +414,10 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
                 kc_mm_grouped_packed_pair(s, c->fmt, gate, up, d, ff, m->px, d, m->G, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, word);
                 kc_swiglu_pack(s, m->G, m->U, (uint16_t*) m->A, (size_t) P * ff);
             }
-            kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles,
-                                      m->max_tiles, word);
+            /* the experts' outputs are BF16 values; as BF16 bits the combine reads half as much */
+            m->d16 = kc_mm_grouped_packed_bf16(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, (uint16_t*) m->D, d, 1, m->perm, m->tiles, m->ntiles,
+                                            m->max_tiles, word) == 0;
+            if (!m->d16) kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles, m->max_tiles, word);
         } else {
             kc_mm_grouped_dev(s, c->fmt, gate, d, ff, xn, d, m->G, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
             kc_mm_grouped_dev(s, c->fmt, up, d, ff, xn, d, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
@@ -420,8 +425,13 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
             kc_mm_grouped_dev(s, c->fmt, down, ff, d, m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
         }
     }
-    if (c->router == NSLM_ROUTE_SOFTMAX) kq4_moe_combine(s, d, k, m->D, m->wt, NULL, m->zero, 0, io, T);
-    else kc_moe_combine(s, m->D, m->wt, NULL, io, d, k, T);
+    if (c->router == NSLM_ROUTE_SOFTMAX) {
+        if (m->d16) kq4_moe_combine_bf16(s, d, k, (const uint16_t*) m->D, m->wt, NULL, m->zero, 0, io, T);
+        else kq4_moe_combine(s, d, k, m->D, m->wt, NULL, m->zero, 0, io, T);
+    } else {
+        if (m->d16) kc_moe_combine_bf16(s, (const uint16_t*) m->D, m->wt, NULL, io, d, k, T);
+        else kc_moe_combine(s, m->D, m->wt, NULL, io, d, k, T);
+    }
     return kc_last_error() ? -1 : 0;
 }
 
@@ -467,8 +477,18 @@ int nslm_moe_last_logits(NslmMoe* m, int T, float* logits) {
     return nh_memcpy_d2h(logits, m->logit, 4 * (size_t) T * m->c.n_exp) ? -1 : 0;
 }
 int nslm_moe_last_pairs(NslmMoe* m, int pairs, float* A, float* D) {
-    if (nh_device_sync()) return -1;
-    return (nh_memcpy_d2h(A, m->A, 4 * (size_t) pairs * m->c.ff) | nh_memcpy_d2h(D, m->D, 4 * (size_t) pairs * m->c.d)) ? -1 : 0;
+    const size_t n = (size_t) pairs * m->c.d;
+    if (nh_device_sync() || nh_memcpy_d2h(A, m->A, 4 * (size_t) pairs * m->c.ff)) return -1;
+    if (!m->d16) return nh_memcpy_d2h(D, m->D, 4 * n) ? -1 : 0;
+    /* BF16 bits: into the upper half of the caller's array, then widened from the front */
+    if (nh_memcpy_d2h((char*) D + 2 * n, m->D, 2 * n)) return -1;
+    for (size_t i = 0; i < n; ++i) {
+        uint16_t h;
+        memcpy(&h, (char*) D + 2 * n + 2 * i, 2);
+        const uint32_t w = (uint32_t) h << 16;
+        memcpy(D + i, &w, 4);
+    }
+    return 0;
 }
 int nslm_moe_prefetch_stats(NslmMoe* m, uint32_t* hits, uint32_t* misses) {
     uint32_t st[2] = {0, 0};

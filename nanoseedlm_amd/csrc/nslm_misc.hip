@@ -244,16 +244,36 @@ __global__ void k_swiglu_pack(const float* g, const float* u, uint16_t* y, size_
 }
 // x[t][c] = bf16(x + bf16(bf16(sum_j bf16(D[t,j][c] * bf16(w[t,j]))) + shared[t][c]))
 // out[t][i] = sigmoid(sg[t * sgld]) * sh[t][i] + sum_j wt[t][j] D[t,j][i], all f32
-// Bound by the reads of D (k rows of d a token).  V = 4: a thread takes four columns, all its rows' 16-byte loads requested before the
-// first is added (a column a thread, each load behind the last add: 45 us at 2048 tokens, top-8, d = 2048; now 30, where
-// 150 MB at a large copy's rate are 29).  Q4 = false: the first form, with sh = shared, io = x.  sh NULL: zeros, not read.
-template <int V, bool Q4>
-__global__ void __launch_bounds__(256) k_combine(const float* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k) {
+// Bound by the reads of D (k rows of d a token).  A thread takes V columns, all its rows' 16-byte loads requested before the
+// first is added (a column a thread, each load behind the last add: 45 us at 2048 tokens, top-8, d = 2048; four columns of f32 23, where
+// 150 MB at a large copy's rate are 29; of BF16 bits 14).  Q4 = false: the first form, with sh = shared, io = x.  sh NULL: zeros, not read.
+template <int V>
+struct DVec {   // V values of a row of D
+    typedef float type __attribute__((ext_vector_type(V), aligned(V % 4 ? 4 : 16)));
+};
+template <int V>
+__device__ __forceinline__ typename DVec<V>::type load_d(const float* p) { return *(const typename DVec<V>::type*) p; }
+template <int V>
+__device__ __forceinline__ typename DVec<V>::type load_d(const uint16_t* p) {
+    typename DVec<V>::type v;
+    if constexpr (V == 4) {
+        const uint2 q = *(const uint2*) p;
+        const uint32_t w[2] = {q.x, q.y};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { v[2 * i] = bf(w[i] & 0xFFFFu); v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u); }
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = bf(p[i]);
+    }
+    return v;
+}
+template <int V, bool Q4, class D_>
+__global__ void __launch_bounds__(256) k_combine(const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k) {
     const int c = V * (int) (blockIdx.x * blockDim.x + threadIdx.x), t = (int) blockIdx.y;
     if (c >= d) return;
-    typedef float vec __attribute__((ext_vector_type(V)));
+    typedef typename DVec<V>::type vec;
     const size_t at = (size_t) t * d + c;
-    const float* Dt = D + (size_t) t * k * d + c;
+    const D_* Dt = D + (size_t) t * k * d + c;
     vec s = {}, h = {}, x = {};
     if (sh) h = *(const vec*) (sh + at);
     if (!Q4) x = *(const vec*) (io + at);
@@ -267,7 +287,7 @@ __global__ void __launch_bounds__(256) k_combine(const float* D, const float* wt
         float w[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {   // (clamped: the loads stay unconditional)
-            v[j] = *(const vec*) (Dt + (size_t) min(j0 + j, k - 1) * d);
+            v[j] = load_d<V>(Dt + (size_t) min(j0 + j, k - 1) * d);
             w[j] = wt[t * k + min(j0 + j, k - 1)];
         }
 #pragma unroll
@@ -281,12 +301,13 @@ __global__ void __launch_bounds__(256) k_combine(const float* D, const float* wt
     for (int i = 0; i < V; ++i) x[i] = Q4 ? s[i] : bfr(x[i] + bfr(bfr(s[i]) + h[i]));
     *(vec*) (io + at) = x;
 }
-template <bool Q4>
-void combine(hipStream_t st, const float* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, int T) {
-    if (d % 4 == 0 && (((uintptr_t) D | (uintptr_t) sh | (uintptr_t) io) & 15u) == 0)
-        hipLaunchKernelGGL((k_combine<4, Q4>), dim3((unsigned) (d / 4 + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
+template <bool Q4, class D_>
+void combine(hipStream_t st, const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, int T) {
+    constexpr int V = 4;
+    if (d % V == 0 && (((uintptr_t) D | (uintptr_t) sh | (uintptr_t) io) & 15u) == 0)
+        hipLaunchKernelGGL((k_combine<V, Q4, D_>), dim3((unsigned) (d / V + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
     else
-        hipLaunchKernelGGL((k_combine<1, Q4>), dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
+        hipLaunchKernelGGL((k_combine<1, Q4, D_>), dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
 }
 __global__ void k_pack_input_bf16(const float* x, uint16_t* y, size_t n) {
     const size_t b = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -732,6 +753,14 @@ void kc_moe_combine(kc_stream_t s, const float* D, const float* w, const float* 
 }
 void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* wt, const float* sh, const float* sg,
                      int sgld, float* out, int T) {
+    if (T < 1) return;
+    combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T);
+}
+void kc_moe_combine_bf16(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T) {
+    if (T < 1) return;
+    combine<false>((hipStream_t) s, D, w, shared, nullptr, 0, x, d, k, T);
+}
+void kq4_moe_combine_bf16(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T) {
     if (T < 1) return;
     combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T);
 }

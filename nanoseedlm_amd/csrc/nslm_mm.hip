@@ -700,6 +700,14 @@ void kc_mm_grouped_packed_rows(kc_stream_t s, int fmt, const WSlice* ws, int K, 
                                int tile_rows) {
     mm_grouped<true>((hipStream_t) s, fmt, ws, K, R, x, xs, y, ys, xdiv, perm, tiles, nt, max_tiles, tile_rows < 1 ? MMT_BN : tile_rows);
 }
+int kc_mm_grouped_packed_bf16(kc_stream_t s, int fmt, const WSlice* ws, int K, int R, const uint16_t* x, int xs, uint16_t* y, int ys, int xdiv,
+                              const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows) {
+    if (max_tiles < 1 || R < 1) return 0;
+    if (tile_rows <= MMT_BN || !rows_ok<true>(fmt, K, xs, x) || host_store_f32()) return -1;
+    const MmArgs a = {K, R, 0, xs, ys, xdiv, 0, OUT_BF16, 0, MMT_BN, 0, nullptr, nullptr, nullptr};
+    mm_wide_grouped((hipStream_t) s, fmt, a, ws, x, (float*) y, perm, tiles, nt, max_tiles);
+    return 0;
+}
 int kc_mm_grouped_swiglu(kc_stream_t s, int fmt, const WSlice* gate, const WSlice* up, int K, int R, const uint16_t* x, int xs, uint16_t* a16,
                          int ys, int xdiv, const int32_t* perm, const MmTile* tiles, const int32_t* nt, int max_tiles, int tile_rows) {
     if (max_tiles < 1 || R < 1) return 0;

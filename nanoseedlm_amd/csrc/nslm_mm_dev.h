@@ -12,6 +12,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+#define OUT_BF16 2   // f32out: the results as BF16 bits (y is uint16_t [][ys])
 struct MmArgs {
     int K, R, T, xs, ys, xdiv, add, f32out;
     int least, most;     // grouped: a tile of up to `least` pairs, or of more than `most`, is another launch's;

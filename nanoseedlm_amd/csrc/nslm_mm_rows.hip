@@ -179,7 +179,16 @@ __device__ __forceinline__ f32x4 scaled(const f32x4& s, int eb) {
     return (f32x4) {mm_scale<FMT>(s[0], eb), mm_scale<FMT>(s[1], eb), mm_scale<FMT>(s[2], eb), mm_scale<FMT>(s[3], eb)};
 }
 // four sums of pair / token dst, rows orow .. orow + 3 (those below R)
+// BITS: a launch may ask for BF16 bits (k_mm_wide; in the other kernels the branch cost registers, and small launches up to 3 %)
+template <bool BITS = false>
 __device__ __forceinline__ void store_rows(const MmArgs& a, float* Y, int dst, int orow, const f32x4& s) {
+    if (BITS && a.f32out == OUT_BF16) {
+        uint16_t* o = (uint16_t*) Y + (size_t) dst * a.ys + orow;
+        if ((a.ys & 3) == 0 && orow + 4 <= a.R && ((uintptr_t) o & 7u) == 0) *(uint2*) o = make_uint2(pack_bf2(s[0], s[1]), pack_bf2(s[2], s[3]));
+        else
+            for (int j = 0; j < 4 && orow + j < a.R; ++j) o[j] = (uint16_t) tobf(s[j]);
+        return;
+    }
     float* yo = Y + (size_t) dst * a.ys + orow;
     if ((a.ys & 3) == 0 && orow + 4 <= a.R && !a.add && !a.f32out && ((uintptr_t) yo & 15u) == 0) *(f32x4*) yo = (f32x4) {bfr(s[0]), bfr(s[1]), bfr(s[2]), bfr(s[3])};
     else
@@ -413,7 +422,7 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-        if (16 * nt + t < count && orow < a.R) store_rows(a, Y, perm[start + 16 * nt + t], orow, acc[nt]);
+        if (16 * nt + t < count && orow < a.R) store_rows<true>(a, Y, perm[start + 16 * nt + t], orow, acc[nt]);
 }
 
 // Who computes a tile of a grouped launch, whatever table the host made: k_mm_wide takes every tile of more than `least` pairs, alone or together

@@ -829,6 +829,48 @@ def test_mm_grouped_tile_sizes(be, oracle, fmt, tile_rows):
         b.free()
 
 
+# R 150: rows that end inside a lane's four, a stride that leaves them unaligned; 152: aligned
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_Q4])
+@pytest.mark.parametrize("R", [150, 152])
+def test_mm_grouped_packed_bf16_holds_the_f32_results_bits(fmt, R):
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    backend.require_gpu()
+    L = backend.hip()
+    rng = np.random.default_rng(R)
+    counts, tile_rows = [1, 17, 64, 65, 0, 128, 129, 200, 70], 129
+    E, K, P = len(counts), 320, sum(counts)
+    p = make_pack(rng, fmt, E, R, K)
+    arr, keep = (backend.WSlice * E)(), []
+    for name, i in [("seeds", 0), ("coefs", 1), ("codes", 3)] if fmt == packs.MF_SEED4P4 else [("words", 0), ("scales", 1), ("biases", 2)]:
+        keep.append(moe.DevBuf.from_array(np.ascontiguousarray(p[name])))
+        for e in range(E):
+            arr[e].p[i] = keep[-1].ptr.value + e * (keep[-1].nbytes // E)
+    for e in range(E):
+        arr[e].eb, arr[e].gs = (int(p["eb"][e]), 0) if "eb" in p else (0, 6)
+    tab = moe.DevBuf(C.sizeof(arr))
+    backend.check(L.nh_memcpy_h2d(tab.ptr, arr, C.c_size_t(C.sizeof(arr))), "nh_memcpy_h2d")
+    rows = []
+    for e, n in enumerate(counts):
+        rows += [[e, sum(counts[:e]) + j, min(128, n - j), 0] for j in range(0, n, 128)]
+    dx = moe.DevBuf.from_array(packs.f32_to_bf16_bits(rng.standard_normal((P, K)).astype(np.float32)))
+    dperm, dtiles, dn = (moe.DevBuf.from_array(np.array(v, dtype=np.int32)) for v in (rng.permutation(P), rows, [len(rows)]))
+    y, y16 = moe.DevBuf(4 * P * R), moe.DevBuf(2 * P * R)
+    L.kc_mm_grouped_packed_rows(None, fmt, tab.ptr, K, R, dx.ptr, K, y.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, len(rows), tile_rows)
+    assert L.kc_mm_grouped_packed_bf16(None, fmt, tab.ptr, K, R, dx.ptr, K, y16.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, len(rows), tile_rows) == 0
+    moe.device_sync()
+    assert L.kc_last_error() == 0
+    assert np.array_equal(y.to_array(np.uint32, (P, R)) >> 16, y16.to_array(np.uint16, (P, R)))
+    assert L.kc_mm_grouped_packed_bf16(None, fmt, tab.ptr, K, R, dx.ptr, K, y16.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, len(rows), 128) == -1
+    L.kc_store_f32(1)
+    try:   # no BF16 values to store
+        assert L.kc_mm_grouped_packed_bf16(None, fmt, tab.ptr, K, R, dx.ptr, K, y16.ptr, R, 1, dperm.ptr, dtiles.ptr, dn.ptr, len(rows), tile_rows) == -1
+    finally:
+        L.kc_store_f32(0)
+    for b in keep + [tab, dx, dperm, dtiles, dn, y, y16]:
+        b.free()
+
+
 # (slice, pairs) in table order: runs of a slice's adjoining tiles that kc_bucket, which fills a tile before it begins the next, never makes
 HAND_TILES = {
     "small_first": [(0, 20), (0, 20), (1, 20), (1, 100), (2, 32), (2, 32), (2, 32), (2, 64), (3, 1), (3, 33), (3, 33)],
@@ -1141,3 +1183,36 @@ def test_combine_widths(be, oracle, d, k):
     assert np.array_equal(be.kt_combine(D, w, sh, x).view(np.uint32), oracle.moe_combine(D, w, sh, x).view(np.uint32))
     ref = sh.astype(np.float64) / (1 + np.exp(-sg.astype(np.float64))) + (w[:, :, None].astype(np.float64) * D.reshape(T, k, d)).sum(1)
     assert np.allclose(be.kt_q4_combine(D, w, sh, sg), ref, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("d", [6, 24, 2048])   # a column a thread; eight: a part of a workgroup, several workgroups
+@pytest.mark.parametrize("k", [1, 8, 11])
+def test_combines_of_bf16_bits_equal_those_of_f32(d, k):
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    backend.require_gpu()
+    L = backend.hip()
+    rng = np.random.default_rng(d + k)
+    T = 5
+    D = packs.round_bf16(rng.standard_normal((T * k, d)).astype(np.float32))
+    D[0, 0], D[-1, -1] = np.inf, -0.0
+    x = packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32))
+    sh = packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32))
+    b32, b16, w, dsh, sg = (moe.DevBuf.from_array(v) for v in (D, packs.f32_to_bf16_bits(D), rng.random((T, k)).astype(np.float32), sh, rng.standard_normal(T).astype(np.float32)))
+    for shared in (dsh.ptr, None):
+        outs = []
+        for bits in (0, 1):
+            a, b = moe.DevBuf.from_array(x), moe.DevBuf(4 * T * d)
+            if bits:
+                L.kc_moe_combine_bf16(None, b16.ptr, w.ptr, shared, a.ptr, d, k, T)
+                L.kq4_moe_combine_bf16(None, d, k, b16.ptr, w.ptr, shared, sg.ptr, 1, b.ptr, T)
+            else:
+                L.kc_moe_combine(None, b32.ptr, w.ptr, shared, a.ptr, d, k, T)
+                L.kq4_moe_combine(None, d, k, b32.ptr, w.ptr, shared, sg.ptr, 1, b.ptr, T)
+            moe.device_sync()
+            outs.append((a.to_array(np.uint32, (T, d)), b.to_array(np.uint32, (T, d))))
+            a.free(); b.free()
+        assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+    assert L.kc_last_error() == 0
+    for b in (b32, b16, w, dsh, sg):
+        b.free()
