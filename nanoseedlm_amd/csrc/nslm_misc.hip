@@ -79,25 +79,40 @@ __global__ void __launch_bounds__(256) k_router_logits(RouterArgs a, const uint1
 // 1218 us at 512 tokens of 2048, where this launch has 256 workgroups.)  A wave takes two experts at a time and sums all its
 // 2 RM_TOK x 2 partial sums in one folding tree: at each level a lane hands half of its values to its partner and adds the other
 // half - the additions of the xor tree, without forming every sum in every lane (33 exchanges instead of 192).
+// Bound by its own latency: a workgroup's row loads are requested a row of every token at a time, a weight piece one turn ahead.  In the
+// tree a lane's halves are read before one is chosen: written as a choice between elements of the array, the compiler made it a
+// lane's index into the registers, 4392 vector instructions a pair of experts instead of 565.  2048 tokens of 1536, 16 experts
+// 37.8 -> 9.9 us; 500 of 2880, 64 experts 45.4 -> 14.8; 1000 of 2048, 128 experts 80.8 -> 24.7; 100 of 1024, 32 experts 35 -> 7.6.
 #define RM_TOK 8
 #define RM_EXP 16
 __global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const uint16_t* W, const uint16_t* bias, const float* x, int T,
                                                             float* score, float* selout) {
     extern __shared__ __attribute__((aligned(16))) float xs[];   // [RM_TOK][2][d / 8][4]: a piece's first and last four values apart
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, np = a.d / 8, t0 = (int) blockIdx.x * RM_TOK;
-    for (int i = tid; i < RM_TOK * np * 2; i += 256) {
-        const int t = i / (2 * np), q = i - t * 2 * np;   // 16-byte unit q of token t's row
-        const float4 v = *(const float4*) (x + (size_t) min(t0 + t, T - 1) * a.d + 4 * (size_t) q);
-        *(float4*) &xs[((size_t) (t * 2 + (q & 1)) * np + (q >> 1)) * 4] = v;
+    const int eN = min(a.n, ((int) blockIdx.y + 1) * RM_EXP);
+    int e0 = (int) blockIdx.y * RM_EXP + 2 * wv;
+    uint4 nq[2];   // the pieces one turn ahead (indices clamped: the loads stay unconditional)
+    auto request = [&](int e, int c) {
+        const size_t cc = 8 * (size_t) min(c, np - 1);
+        nq[0] = *(const uint4*) (W + (size_t) min(e, a.n - 1) * a.d + cc);
+        nq[1] = *(const uint4*) (W + (size_t) min(e + 1, a.n - 1) * a.d + cc);
+    };
+    request(e0, lane);
+    for (int q = tid; q < 2 * np; q += 256) {   // 16-byte unit q of every token's row, the rows' requests together
+        float4 v[RM_TOK];
+#pragma unroll
+        for (int t = 0; t < RM_TOK; ++t) v[t] = *(const float4*) (x + (size_t) min(t0 + t, T - 1) * a.d + 4 * (size_t) q);
+#pragma unroll
+        for (int t = 0; t < RM_TOK; ++t) *(float4*) &xs[((size_t) (t * 2 + (q & 1)) * np + (q >> 1)) * 4] = v[t];
     }
     __syncthreads();
-    for (int e0 = (int) blockIdx.y * RM_EXP + 2 * wv; e0 < min(a.n, ((int) blockIdx.y + 1) * RM_EXP); e0 += 8) {
-        const int e1 = min(e0 + 1, a.n - 1);
+    for (; e0 < eN; e0 += 8) {
         float lo[2][RM_TOK], hi[2][RM_TOK];
 #pragma unroll
         for (int u = 0; u < RM_TOK; ++u) lo[0][u] = lo[1][u] = hi[0][u] = hi[1][u] = 0.0f;
         for (int c = lane; c < np; c += 64) {
-            const uint4 q[2] = {*(const uint4*) (W + (size_t) e0 * a.d + 8 * (size_t) c), *(const uint4*) (W + (size_t) e1 * a.d + 8 * (size_t) c)};
+            const uint4 q[2] = {nq[0], nq[1]};
+            if (c + 64 < np) request(e0, c + 64);
             float w[2][8];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -119,6 +134,7 @@ __global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const 
                 }
             }
         }
+        request(e0 + 8, lane);
         // value index v = (token, expert half, partition); after the level with stride o a lane holds the half of the values that its bit o picks
         float v[4 * RM_TOK];
 #pragma unroll
@@ -131,7 +147,8 @@ __global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const 
             const bool up = (lane & o) != 0;
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const float give = up ? v[i] : v[i + n], keep = up ? v[i + n] : v[i];
+                const float a0 = v[i], a1 = v[i + n];
+                const float give = up ? +a0 : +a1, keep = up ? +a1 : +a0;
                 v[i] = keep + __shfl_xor(give, o);
             }
         }
