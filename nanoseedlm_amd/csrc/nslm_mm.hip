@@ -553,13 +553,13 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
 #pragma unroll
     for (int m = 0; m < CT; ++m)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
-            const int orow = r0 + 32 * n + (lane & 31);
-            if (orow >= a.R) continue;
+        for (int v = 0; v < 16; ++v) {   // (a token's two runs of 32 columns one after the other: they share its 256 bytes)
+            const int dst = drow[wtok + 32 * m + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
+            if (dst < 0) continue;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int dst = drow[wtok + 32 * m + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
-                if (dst < 0) continue;
+            for (int n = 0; n < 2; ++n) {
+                const int orow = r0 + 32 * n + (lane & 31);
+                if (orow >= a.R) continue;
                 float* yo = Y + (size_t) dst * a.ys + orow;
                 if (plain) __builtin_nontemporal_store(bfr(mm_scale<FMT>(acc[m][n][v], wt.eb)), yo);
                 else store_y(yo, mm_scale<FMT>(acc[m][n][v], wt.eb), a.add, a.f32out);
