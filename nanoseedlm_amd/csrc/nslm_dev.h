@@ -106,6 +106,11 @@ __device__ __forceinline__ void load_tables(uint32_t* tab) {
 // keeps the loads written above this line above it: left alone, the compiler moves a load down to its first use, and a load
 // whose use sits in a conditional block becomes a load, a wait and a branch - one round trip per load instead of one for all
 __device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void to_lds16(const void* src, uint8_t* dst) {   // dst: the wave's base, lane l lands at dst + 16 l
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 16, 0, 0);
+}
 __device__ __forceinline__ uint32_t stream_of(const uint32_t* tab, uint32_t seed16) {
     return tab[seed16 & 0xFFu] ^ tab[256 + (seed16 >> 8)];
 }
@@ -218,6 +223,16 @@ template <int P>
 __device__ __forceinline__ void load_sum_tables(uint32_t* tab) {
     for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = kBasis.v[i];
     for (int i = threadIdx.x; i < sum_tab_words<P>() - 512; i += blockDim.x) tab[512 + i] = P == 4 ? kSumTab4.v[i] : kSumTab3.v[i];
+}
+// The same, requested into the LDS (16-byte aligned) by the workgroup's first four waves: beside the kernel's other first loads they cost no
+// round trip of their own, where the loop above waits for each of its loads.  The waves wait for vmcnt(0) before the workgroup meets.
+// (Grouped GEMM, E 128, top-8, d 2048, ff 768, 64 rows 196 -> 189 us a layer step, 32 rows 172 -> 166; wide, 2048 rows 428 -> 424.  The dense GEMM
+// for few tokens, whose waves went on at once after its loop, lost 2 % by meeting with their first weights.)
+template <int P>
+__device__ __forceinline__ void tables_to_lds(uint32_t* tab) {
+    const int w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t* const rest = P == 4 ? kSumTab4.v : kSumTab3.v;
+    if (256 * w < sum_tab_words<P>()) to_lds16((w < 2 ? kBasis.v + 256 * w : rest + 256 * (w - 2)) + 4 * lane, (uint8_t*) (tab + 256 * w));
 }
 // The same for a workgroup of exactly NTHR threads (256, 512 or 1024), in two halves: a thread's loads are requested in
 // tables_fetch() (put it beside the kernel's other first loads), and tables_store() writes them to LDS once they are needed -

@@ -197,7 +197,7 @@ template <int P, bool SHFL_G, bool SHFL_D, int WAVES>
 __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // WAVES waves a SIMD: five = at most 96 registers
     extern __shared__ float xl[];   // activations of the current pair: max(d, ff) floats, chunk-padded
     float2* const gu_s = (float2*) (xl + a.gu_off);   // behind them: the gate and up row sums of the item in hand
-    __shared__ __attribute__((aligned(8))) uint32_t tab[sum_tab_words<P>()];
+    __shared__ __attribute__((aligned(16))) uint32_t tab[sum_tab_words<P>()];
     __shared__ float part[2][256];
     __shared__ __attribute__((aligned(16))) float rv[1024];   // route: the token's logits
     __shared__ float rw_s[33];      // route: weight by rank (+ the shared expert's 1)
@@ -236,12 +236,16 @@ __global__ void __launch_bounds__(256, WAVES) k_moe_decode(FusedArgs a) {   // W
     }
     // The decode tables are first needed in phase 2: loaded here, behind the logits (everybody waits for the workgroups
     // that form logits; tables first was one more memory round trip on their way).
-    load_sum_tables<P>(tab);
+    // (requested into the LDS: 2 tokens of a layer of 128 experts, top-8, d 2048, ff 768, two layers 66.8 -> 64.9 us, 4 tokens 102.5 -> 99.6.  With five
+    // waves a SIMD the other waves hide the table's loads, and waiting here for the logits' stores, too, costs more: 8 tokens 170.1 -> 172.8.)
+    if constexpr (WAVES == 4) tables_to_lds<P>(tab);
+    else load_sum_tables<P>(tab);
     // the first gate+up item's activations are an input of the launch: staged while the other workgroups' logits arrive
     if ((int) blockIdx.x < items_g) {
         staged = ((int) blockIdx.x / a.ntile_g) / a.kk;
         stage_input(a.x + (size_t) staged * a.xs, a.d, xl, a.nw, a.nw ? rn_s[staged] : 1.0f);
     }
+    if constexpr (WAVES == 4) wait_vm<0>();   // the tables have landed
     // No grid barrier: what the other workgroups produce here are the logits, and those say themselves when they are there.
     __syncthreads();   // every wave has used its copy of the generation
     uint32_t arrived = 0;

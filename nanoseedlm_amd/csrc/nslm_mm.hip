@@ -335,9 +335,6 @@ void launch_mm(hipStream_t st, int fmt, const MmArgs& a, WSlice wd, const WSlice
 #define XCHUNK 2048      // BF16 elements of an activation chunk: 32 tokens x 64 K
 #define RECD 4           // weight steps between a record's request and its decode
 
-template <int N>
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 struct MmRec2 {
     uint4 raw[2];      // BF16: the two blocks; Q8: raw[0]; Q4: raw[0].xy
     uint32_t u, v, c;  // seeds: two seeds, two coefficient words, the codes byte; Q8 / Q4: the group's scale and bias bits
@@ -352,17 +349,18 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
     typedef uint16_t WTile[BM][LDW2];
     WTile* Wsm = (WTile*) (smem + NCW * XCH * XCHUNK);          // [2]
     __shared__ int srow[BN], drow[BN];
-    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
+    __shared__ __attribute__((aligned(16))) uint32_t tab[mm_tab_words<FMT>()];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool producer = wv >= NCW;
     const int r0 = (int) blockIdx.x * BM, start = (int) blockIdx.y * BN, count = min(BN, a.T - start);
     if (count < 1) return;
-    if constexpr (seedf) load_sum_tables<seed_p<FMT>()>(tab);
+    if constexpr (seedf) tables_to_lds<seed_p<FMT>()>(tab);
     for (int i = tid; i < BN; i += NTHR) {
         const bool ok = i < count;
         srow[i] = start + (ok ? i : 0);   // padding rows load the tile's first row; their results are never stored
         drow[i] = ok ? start + i : -1;
     }
+    if constexpr (seedf) wait_vm<0>();
     __syncthreads();
     const int nsteps = a.K / WK;
 

@@ -34,9 +34,6 @@ constexpr int row_bytes() { return seed_fmt<FMT>() || FMT == MF_Q4 ? 32 : FMT ==
 template <int FMT, int RT, int NT, bool PACKED>
 constexpr int step_bytes() { return 16 * RT * (row_bytes<FMT>() + (FMT == MF_SEED4P4 ? 4 : 0)) + (PACKED ? NT * 2048 : 0); }
 
-__device__ __forceinline__ void to_lds16(const void* src, uint8_t* dst) {   // dst: the wave's base, lane l lands at dst + 16 l
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 16, 0, 0);
-}
 __device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
 }
@@ -206,10 +203,10 @@ __device__ __forceinline__ void store_swiglu(const MmArgs& a, int dst, int orow,
 }
 
 // The 16 RT rows from r0 (with a.a16: 8 RT gate rows and the same 8 RT up rows) x the 16 NT tokens n0 .. of a workgroup of NW waves.
-// lds: NW x max(step, RT NT KB).
+// lds: NW x max(step, RT NT KB).  meet: the decode tables are requested, and the workgroup has not met since.
 template <int FMT, int RT, int NT, int NW, bool PACKED, bool GROUPED>
 __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, const WSlice& m1, const void* X, float* Y, const int32_t* perm, int start, int count,
-                                          int n0, int r0, const uint32_t* tab, uint8_t* lds) {
+                                          int n0, int r0, const uint32_t* tab, uint8_t* lds, bool meet) {
     const int tid = threadIdx.x & (64 * NW - 1), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
     const bool gu = GROUPED && a.a16 != nullptr;
     const int nch = a.K / 64;
@@ -251,6 +248,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
     int c = w;
     auto next = [&](int at) { at += 8; if (NW == 4 && at >= nch) at = at % 8 >= 4 ? nch : w + 4; return at; };
     if (n > 0) request(c);
+    if (seed_fmt<FMT>() && meet) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (int s = 0; s < n; ++s) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         constexpr bool HALVES = NW == 4 && NT >= 4;
@@ -389,10 +387,10 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
         });
     };
     W.request(0, ws);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    request_x(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (and the decode tables)
     W.read(ws, st);
     wb = W.block(st, 0, 0, tab, [](int) {});
-    request_x(0);
     if (nch > 1) W.request(1, ws + SB);
     for (int c = 0; c < nch; ++c) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the activations of chunk c have landed, those of c - 1 are read
@@ -478,7 +476,7 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
         load_sum_tables<seed_p<FMT>()>(tab);
         __syncthreads();
     }
-    rows_tile<FMT, RT, NT, 8, PACKED, false>(a, w, w, X, Y, nullptr, 0, a.T, (int) blockIdx.y * 16 * NT, (int) blockIdx.x * 16 * RT, tab, lds);
+    rows_tile<FMT, RT, NT, 8, PACKED, false>(a, w, w, X, Y, nullptr, 0, a.T, (int) blockIdx.y * 16 * NT, (int) blockIdx.x * 16 * RT, tab, lds, false);
 }
 
 #define GRT 2   // row tiles of the grouped kernel's workgroups
@@ -487,7 +485,7 @@ template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
                                                                            const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
+    __shared__ __attribute__((aligned(16))) uint32_t tab[mm_tab_words<FMT>()];
     // The grid has a workgroup row for as many tiles as the host's table holds.  Of fewer than `few` tiles, whose own workgroups do not fill the
     // chip, those past *ntiles take the later passes over 16 MOST pairs: pass 1 of every tile, then pass 2, .. (row nt + e: pass 1 + e / nt of
     // tile e % nt); the passes that they do not reach are the tile's own workgroups', after pass 0.  Tokens that agree on a few experts make
@@ -525,14 +523,11 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
             }
         }
     const int count = min(tl.count, limit);
-    if constexpr (seed_fmt<FMT>()) {
-        load_sum_tables<seed_p<FMT>()>(tab);
-        __syncthreads();
-    }
+    if constexpr (seed_fmt<FMT>()) tables_to_lds<seed_p<FMT>()>(tab);
     for (int n0 = first; n0 < count; n0 = next, next += PASS) {
         if (n0 != first) __syncthreads();   // the sums of the tokens before are read
         const int left = count - n0;
-#define T(NT) rows_tile<FMT, GRT, NT, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds)
+#define T(NT) rows_tile<FMT, GRT, NT, 4, PACKED, true>(a, m0, m1, X, Y, perm, tl.start, count, n0, r0, tab, lds, n0 == first)
         if (left <= 16) T(1);
         else if (MOST == 2 || left <= 32) T(2);
         else if constexpr (MOST == 4) T(4);
@@ -549,7 +544,7 @@ template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ __attribute__((aligned(8))) uint32_t tab[mm_tab_words<FMT>()];
+    __shared__ __attribute__((aligned(16))) uint32_t tab[mm_tab_words<FMT>()];
     const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
     if (y >= nt) return;
     const MmTile tl = tiles[y];
@@ -563,10 +558,7 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     const WSlice m = gu && __builtin_amdgcn_readfirstlane((int) threadIdx.x) >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
     int count = tl.count;
     if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
-    if constexpr (seed_fmt<FMT>()) {
-        load_sum_tables<seed_p<FMT>()>(tab);
-        __syncthreads();
-    }
+    if constexpr (seed_fmt<FMT>()) tables_to_lds<seed_p<FMT>()>(tab);
     const int r0 = (int) blockIdx.x * (gu ? 64 : 128);
 #define W(NT) wide_tile<FMT, NT>(a, m, X, Y, perm, tl.start, count, r0, tab, lds)
     if (count <= 64) W(4);
