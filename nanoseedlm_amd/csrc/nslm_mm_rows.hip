@@ -27,13 +27,23 @@ namespace {
 // requests the next one into the same place, so the LDS holds one step a wave and its decode covers the latency.
 //   activations  [16 NT][64] BF16, the 16-byte pieces of a row swizzled (x_swizzle16) so that a fragment read spreads over the banks
 //   seeds        per row tile: 16 rows x 16 bytes of seeds, 16 x 16 of coefficient words; then 16 x 4 of codes
-//   Q4 / Q8      16 rows x 32 / 64 bytes a row tile (Q8: pieces swizzled); scales and biases stay in registers
+//   Q4 / Q8      16 rows x 32 / 64 bytes a row tile (Q8: pieces swizzled); scales and biases a dword each (SL), or they stay in registers
 //   BF16         like the activations
 template <int FMT>
 constexpr int row_bytes() { return seed_fmt<FMT>() || FMT == MF_Q4 ? 32 : FMT == MF_Q8 ? 64 : 128; }   // of weights, a chunk
-template <int FMT, int RT, int NT, bool PACKED>
-constexpr int step_bytes() { return 16 * RT * (row_bytes<FMT>() + (FMT == MF_SEED4P4 ? 4 : 0)) + (PACKED ? NT * 2048 : 0); }
+// SL: the scales and biases of Q4 / Q8 in the LDS, too.  A load of them by every lane for its own row takes the address unit as many cycles as
+// there are lanes, and 2 RT of them a step were a fifth to a third of the launch; where a chunk has one scale and one bias a row, 16 lanes load
+// those of a row tile, and the others read what they landed.  In registers that gained half as much: the compiler waited for the loads
+// where the two cases met.  Q4, 301 tokens, 2880 x 2880 18.3 -> 16.0 us; 26 tokens, 8513 x 4800 18.3 -> 14.7; Q8, 12 tokens, 6309 x 9792
+// 17.7 -> 14.9.  (Only the dense kernel: the grouped ones have no LDS left for it.)
+template <int FMT, int RT, int NT, bool PACKED, bool SL = false>
+constexpr int step_bytes() {
+    return 16 * RT * (row_bytes<FMT>() + (FMT == MF_SEED4P4 ? 4 : SL && (FMT == MF_Q4 || FMT == MF_Q8) ? 32 : 0)) + (PACKED ? NT * 2048 : 0);
+}
 
+__device__ __forceinline__ void to_lds2(const void* src, uint8_t* dst) {   // two bytes a lane, at dst + 4 l
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 2, 0, 0);
+}
 __device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
 }
@@ -58,10 +68,12 @@ __device__ __forceinline__ bf16x8 seed_weights(uint32_t u, uint32_t v, int odd, 
 // eight Q4 (q.x) or Q8 weights
 template <int FMT>
 __device__ __forceinline__ bf16x8 affine_weights(uint2 q, float scale, float bias) {
+    // (Q4: even and odd nibbles as bytes, which the conversion selects by itself)
+    const uint32_t a = FMT == MF_Q8 ? q.x : q.x & 0x0F0F0F0Fu, b = FMT == MF_Q8 ? q.y : q.x >> 4 & 0x0F0F0F0Fu;
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const uint32_t v = FMT == MF_Q8 ? ((i < 4 ? q.x : q.y) >> (8 * (i & 3))) & 255u : (q.x >> (4 * i)) & 15u;
+        const uint32_t v = FMT == MF_Q8 ? (i < 4 ? a : b) >> (8 * (i & 3)) & 255u : (i & 1 ? b : a) >> (8 * (i >> 1)) & 255u;
         f[i] = scale * (float) v + bias;
     }
     return __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
@@ -69,9 +81,9 @@ __device__ __forceinline__ bf16x8 affine_weights(uint2 q, float scale, float bia
 
 // A wave's weights: 16 RT rows from r0 (with gu: 8 RT gate rows of m0 and the same 8 RT rows of up, m1), a chunk a step, staged in the wave's
 // own part of the LDS.
-template <int FMT, int RT>
+template <int FMT, int RT, bool SL = false>
 struct Weights {
-    static constexpr bool SEED = seed_fmt<FMT>();
+    static constexpr bool SEED = seed_fmt<FMT>(), AFFINE = FMT == MF_Q4 || FMT == MF_Q8;
     static constexpr int RB = row_bytes<FMT>(), CODES = 16 * RT * RB;
     static constexpr int NA = SEED || FMT == MF_Q4 ? (RT + 1) / 2 : FMT == MF_Q8 ? RT : 2 * RT;   // 16-byte loads a step
     const WSlice &m0, &m1;
@@ -79,6 +91,12 @@ struct Weights {
     const int K, R, r0, lane, t, g;
     const uint8_t *pa[NA], *pcode;   // the lane's addresses in chunk 0
     uint32_t sc[RT], bi[RT];         // Q4 / Q8: scale and bias bits of the step that is staged
+    // SL: value k = scales of row tiles 0 .. RT - 1, then biases.  `whole` (groups of 64 or more): 16 lanes a value, four values a load
+    static constexpr int NS = (2 * RT + 3) / 4;
+    const uint8_t* ps[NS];
+    size_t g0;        // the row that the lane loads for, in groups of 64 weights
+    int gsh, read0, read1;   // its matrix's group in those, as a shift; the LDS bytes from a lane's first value, and from a value to the next
+    bool whole;
     bool aligned;
     // what a step's decode reads.  u, v, cd: two seeds, two words, their codes; Q4 / Q8: scale and bias.  raw: BF16: the two blocks; Q8: [0]; Q4: [0].xy
     struct Step {
@@ -107,6 +125,16 @@ struct Weights {
             const int rt = min(g, RT - 1);
             pcode = stream(rt, 3) + (size_t) row_of(16 * rt + t) * (size_t) (K / 16);
         }
+        if constexpr (AFFINE && SL) {
+            const int rt = RT == 4 ? g : RT == 2 ? g & 1 : 0;
+#pragma unroll
+            for (int i = 0; i < NS; ++i) ps[i] = (4 * i + g) / RT & 1 ? stream(rt, 2) : stream(rt, 1);
+            g0 = (size_t) row_of(16 * rt + t) * (size_t) (K / 64);
+            whole = group_shift(m0) >= 6 && group_shift(m1) >= 6;
+            gsh = (second(rt) ? group_shift(m1) : group_shift(m0)) - 6;
+            read0 = CODES + 4 * (whole ? t : lane);
+            read1 = whole ? 64 : 256;
+        }
         // streams may start at any 2-byte (codes: any) boundary; those that are not aligned go through registers
         auto low = [&](const WSlice& m) { return (uintptr_t) m.p[0] | (SEED ? (uintptr_t) m.p[1] : 0) | (FMT == MF_SEED4P4 ? ((uintptr_t) m.p[3] & 3u) << 2 : 0); };
         aligned = ((low(m0) | (gu ? low(m1) : 0)) & 15u) == 0;
@@ -126,12 +154,22 @@ struct Weights {
                 else *(uint32_t*) (ws + CODES + 4 * lane) = *(const NSLM_GLOBAL u32_a1*) (pcode + 4 * (size_t) c);
             }
         }
-        if constexpr (FMT == MF_Q4 || FMT == MF_Q8) {
+        if (AFFINE && SL && whole) {
+            const size_t gi = (g0 + (size_t) c) >> gsh;
+#pragma unroll
+            for (int i = 0; i < NS; ++i)
+                if (RT > 1 || lane < 32) to_lds2(ps[i] + 2 * gi, ws + CODES + 256 * i);
+        } else if constexpr (AFFINE) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const size_t gi = ((size_t) row_of(16 * rt + t) * K + (size_t) c * 64 + 16 * g) >> (second(rt) ? group_shift(m1) : group_shift(m0));
-                sc[rt] = gp<uint16_t>(stream(rt, 1))[gi];
-                bi[rt] = gp<uint16_t>(stream(rt, 2))[gi];
+                if constexpr (SL) {
+                    to_lds2(stream(rt, 1) + 2 * gi, ws + CODES + 256 * rt);
+                    to_lds2(stream(rt, 2) + 2 * gi, ws + CODES + 256 * (RT + rt));
+                } else {
+                    sc[rt] = gp<uint16_t>(stream(rt, 1))[gi];
+                    bi[rt] = gp<uint16_t>(stream(rt, 2))[gi];
+                }
             }
         }
     }
@@ -146,8 +184,8 @@ struct Weights {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) s.raw[rt][h] = *(const uint4*) (ws + 2048 * rt + t * 128 + 16 * ((2 * g + h) ^ x_swizzle16(t)));
             } else {
-                s.u[rt] = sc[rt];
-                s.v[rt] = bi[rt];
+                s.u[rt] = SL ? *(const uint16_t*) (ws + read0 + rt * read1) : sc[rt];
+                s.v[rt] = SL ? *(const uint16_t*) (ws + read0 + (RT + rt) * read1) : bi[rt];
                 if (FMT == MF_Q8) s.raw[rt][0] = *(const uint4*) (ws + 1024 * rt + 64 * t + 16 * (g ^ (t >> 3) * 3));
                 else {
                     const uint2 b = *(const uint2*) (ws + 512 * rt + 32 * t + 8 * g);
@@ -210,9 +248,10 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
     const int tid = threadIdx.x & (64 * NW - 1), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
     const bool gu = GROUPED && a.a16 != nullptr;
     const int nch = a.K / 64;
-    Weights<FMT, RT> W(m0, m1, gu, a.K, a.R, r0, lane);
-    uint8_t* const ws = lds + w * step_bytes<FMT, RT, NT, PACKED>();
-    uint8_t* const wx = ws + step_bytes<FMT, RT, NT, false>();   // activations
+    constexpr bool SL = NW == 8;
+    Weights<FMT, RT, SL> W(m0, m1, gu, a.K, a.R, r0, lane);
+    uint8_t* const ws = lds + w * step_bytes<FMT, RT, NT, PACKED, SL>();
+    uint8_t* const wx = ws + step_bytes<FMT, RT, NT, false, SL>();   // activations
     auto src_of = [&](int i) {   // token i of the tile's 16 NT (past the end: the last one again, never stored)
         const int n = start + min(n0 + i, count - 1);
         return (size_t) (GROUPED ? perm[n] / a.xdiv : n) * (size_t) a.xs;
@@ -270,7 +309,7 @@ __device__ __forceinline__ void rows_tile(const MmArgs& a, const WSlice& m0, con
         };
         read_x(0);
         if (!HALVES) read_x(1);
-        typename Weights<FMT, RT>::Step st;
+        typename Weights<FMT, RT, SL>::Step st;
         W.read(ws, st);
         const int cn = next(c);
         auto go_on = [&]() {
@@ -465,7 +504,7 @@ struct Join {
 
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
 template <int FMT, int RT, int NT, int NW, bool PACKED>
-constexpr size_t rows_lds() { return (size_t) NW * max_of(step_bytes<FMT, RT, NT, PACKED>(), RT * NT * 1024); }
+constexpr size_t rows_lds() { return (size_t) NW * max_of(step_bytes<FMT, RT, NT, PACKED, NW == 8>(), RT * NT * 1024); }
 constexpr size_t MOST_LDS = 156 * 1024;   // beside the decode tables
 
 template <int FMT, int RT, int NT, bool PACKED>

@@ -326,6 +326,20 @@ def test_mm_few_tokens(be, oracle, fmt, R, K):
             assert np.array_equal(y[:9].view(np.uint32), y9.view(np.uint32)), (NAMES[fmt], R, K, T)
 
 
+# (R, T): workgroups of one, two and four row tiles, the last one partial; K 1088: 17 chunks, a wave with three, two and none ahead of it.  A chunk has one
+# scale a row with groups of 64 (loaded 16 lanes a row tile) and two with groups of 32 (every lane its own)
+@pytest.mark.parametrize("R,T", [(70, 9), (4100, 16), (4100, 60), (17000, 33), (2885, 301)])
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("fmt", [packs.MF_Q4, packs.MF_Q8])
+def test_mm_few_tokens_affine_groups(be, oracle, fmt, group, R, T):
+    K = 1088 if R < 4000 else 192
+    rng = np.random.default_rng(R + T + group + fmt)
+    p = make_pack(rng, fmt, 1, R, K, group)
+    x = packs.round_bf16(rng.standard_normal((T, K)).astype(np.float32))
+    ref, mag = ref_mm(oracle, p, 0, x, 0)
+    assert close_bf(be.kt_mm_plain(p, x, packed=1), packs.round_bf16(ref.astype(np.float32)).astype(np.float64), F32B * mag).all()
+
+
 # 16384 rows - GEMM: the kernel for few tokens, the streamed one; matvec: one token, a quad of rows a lane group (8), the staged pass
 @pytest.mark.parametrize("call,T", [("mm", 64), ("mm", 512), ("mv", 1), ("mv", 8), ("mv", 64)])
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
