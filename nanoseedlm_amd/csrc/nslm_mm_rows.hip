@@ -702,11 +702,12 @@ namespace nslm {
 
 // Against the kernel of 64 rows x up to 512 tokens a workgroup - for packed activations the streamed one, for f32 the first-generation one -, which
 // spends on a step, in row decodes, what `step` says: that one wins where its workgroups fill the chip.  The streamed kernel was timed with 64 ..
-// 224 workgroups, one a CU.  f32: 290 matrices of 300 .. 32000 rows at 9 .. 2048 tokens on both kernels; the lines lie where the faster one
-// changes (up to 128 tokens, and for Q4, Q8 and BF16 up to 256, it never does), and the kernel taken is 0.1 % off the faster one on average,
+// 224 workgroups, one a CU; BF16 of more than 128 tokens again, on both and on every shape of this file (521 tokens, 17758 x 8000: 395 us with the
+// line where it was, streamed 276; 415 tokens, 7690 x 768 29.7 and 18.1; 132 tokens, 71938 x 448 69 and 52; none slower).  f32: 290 matrices of
+// 300 .. 32000 rows at 9 .. 2048 tokens on both kernels; the lines lie where the faster one changes (up to 128 tokens, and for Q4, Q8 and BF16 up to 256, it never does), and the kernel taken is 0.1 % off the faster one on average,
 // 16 % at worst (4096 x 4096, 1000 tokens, P = 4: first generation 236 us, this 165; 14336 x 4096, 400 tokens: 216 and 270).
 bool mm_rows_better(int fmt, int R, int T, bool packed) {
-    static const double step[2][3][3] = {{{6.2, 7.5, 8.8}, {8.4, 12.7, 14.5}, {13.7, 23.0, 34.0}},
+    static const double step[2][3][3] = {{{6.2, 7.5, 8.8}, {8.4, 12.7, 14.5}, {13.7, 19.5, 27.0}},
                                          {{16.0, 16.0, 24.0}, {24.0, 24.0, 31.6}, {32.0, 40.0, 60.0}}};
     const int q = T <= 128 ? 0 : T <= 256 ? 1 : 2, f = fmt == MF_BF16 ? 2 : fmt == MF_Q8 || fmt == MF_Q4 ? 1 : 0, cus = host_cu_count();
     const long long wgs = (long long) ((R + 63) / 64) * ((T + 511) / 512);
