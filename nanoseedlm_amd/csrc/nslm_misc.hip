@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(256) k_router_logits_many(RouterArgs a, const 
 //   level 1: a wave ranks each group of 64 consecutive values among themselves (64 compares a lane against keys read as
 //            LDS broadcasts); a value with k or more larger values in its own group cannot be among the k best of the row,
 //   level 2: the survivors (at most k a group) are ranked among themselves; rank r < k is the r-th pick.
-// No serial arg-max rounds: the depth of the computation does not grow with k.  NTHR threads a row; rows of a workgroup go through the same barriers.
+// No serial arg-max rounds: the depth of the computation does not grow with k.  NTHR threads a row.
 // MODE 0, the softmax router (engine/kernels_qwen4.cu:385-416 semantics: ties to the higher index, weights = softmax over
 // the k picked, summed in pick order); MODE 1, the sigmoid router's selection (ties to the lowest index, weights =
 // score / sum of the picked scores * scale, engine/kernels_moe.cu:742-772 semantics).
@@ -180,12 +180,12 @@ __device__ __forceinline__ uint32_t float_order(float v) {
     const uint32_t b = __float_as_uint(v + 0.0f);   // -0 ranks as +0
     return b ^ ((uint32_t) ((int32_t) b >> 31) | 0x80000000u);
 }
-// row t of the launch, by NTHR threads (every thread reaches the end: callers may go on with a barrier)
+// row t of the launch, by a workgroup of NTHR threads (every thread reaches the end: callers may go on with a barrier)
 // COH: the selection is stored past the L2 of this workgroup's XCD (agent-scope atomic stores), for a reader in the same launch
 constexpr int topk_lds(int E) { return ((E + 63) & ~63) * 12 + 8 * TK_MAXK + 4 * TK_MAXK + 16; }   // bytes a row
 template <int MODE, int NTHR, bool COH = false>
 __device__ __forceinline__ void topk_row(int t, int E, int k, const float* vals, int ld, const float* score, float scale, int32_t* ind, float* wt, uint8_t* lds) {
-    const int tid = threadIdx.x % NTHR, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     unsigned long long* const key = (unsigned long long*) lds;           // [E64], 0 = no value: below every real key
     unsigned long long* const skey = key + ((E + 63) & ~63);             // [E64 / 2]: survivors of level 1 (at most 32 of every 64)
     float* const pv = (float*) (skey + ((E + 63) & ~63) / 2);
@@ -335,13 +335,13 @@ __global__ void k_pack_input_bf16(const float* x, uint16_t* y, size_t n) {
 
 // ---- grouping: selections -> pair ids by expert (ascending inside an expert), tiles of <= MMT_BN pairs, ONE launch ------
 // work (= the ntiles buffer, 2n + 3 ints): [0] tile count, [1 .. n+1] pair offsets, [n+2 .. 2n+2] tile offsets.
-// A stable counting sort by one workgroup of 16 waves.  Wave w owns the w-th contiguous run of pairs and a histogram row
+// A stable counting sort by workgroups of 16 waves, 1024 pairs each.  Wave w owns 64 consecutive pairs and a histogram row
 // hist[w][.] of its own in LDS, so nothing is contended and the order inside an expert is the pair order by construction:
-//   count   64 pairs a step; the lanes that hold the same expert find each other with one ballot per index bit (the
-//           intersection of the ballots a lane agrees with is the set of its equals), the first of them adds their number,
+//   count   the lanes that hold the same expert find each other with one ballot per index bit (the
+//           intersection of the ballots a lane agrees with is the set of its equals), the first of them notes their number,
 //   scan    thread x turns column x into running sums over the waves and the workgroup scans the experts' totals
 //           (pairs and tiles); thread x writes expert x's tiles,
-//   place   the count loop again: hist[w][x] now says where wave w's next pair of expert x goes.
+//   place   hist[w][x] now says where wave w's first pair of expert x goes.
 // The reference spends two launches on this (a counting kernel and a one-workgroup-per-expert compaction,
 // engine/kernels_moe.cu:527-573); a launch costs more than the work here.
 #define BK_WAVES 16
@@ -355,7 +355,7 @@ __device__ __forceinline__ unsigned long long equal_lanes(int e, int nbits) {
     return m;
 }
 // The whole workgroup: thread x < n has the number of expert x's pairs.  Writes the offsets and the expert's tiles, returns its first pair.
-__device__ __forceinline__ int scan_experts(int cnt, int n, int32_t* work, MmTile* tiles, int (*wsum)[BK_WAVES]) {
+__device__ __forceinline__ int scan_experts(int cnt, int n, int32_t* work, MmTile* tiles, int (*wsum)[BK_WAVES], bool write = true) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int ntl = (cnt + MMT_BN - 1) / MMT_BN;
     int pin = cnt, tin = ntl;   // inclusive sums over the experts: across the wave, then across the waves
@@ -367,7 +367,7 @@ __device__ __forceinline__ int scan_experts(int cnt, int n, int32_t* work, MmTil
     __syncthreads();
     int pofs = pin - cnt, tofs = tin - ntl;
     for (int w = 0; w < wv; ++w) { pofs += wsum[0][w]; tofs += wsum[1][w]; }
-    if (tid < n) {
+    if (write && tid < n) {
         work[1 + tid] = pofs;
         work[2 + n + tid] = tofs;
         for (int j = 0; j < ntl; ++j) {
@@ -386,89 +386,88 @@ __device__ __forceinline__ int scan_experts(int cnt, int n, int32_t* work, MmTil
     }
     return pofs;
 }
-// COH: the selections were stored by other workgroups of this launch (agent-scope atomic loads).  STEPS steps' selections are requested together, and
-// a run of up to so many keeps them and their equals for the second pass: a load and a wait a step, twice, took two thirds of the launch that groups
-// 2048 rows of 8.
-template <bool COH, int STEPS>
-__device__ __forceinline__ void bucket_steps(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles, int (*wsum)[BK_WAVES]) {
-    auto sel_at = [&](int i) { return COH ? __hip_atomic_load(inds + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : inds[i]; };
-    extern __shared__ uint32_t hist[];   // [BK_WAVES][n]
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+// The bits in which expert indices below n, and the value of a pair left out, can differ
+__device__ __forceinline__ int pair_bits(int n) {
     int nbits = 1;
     while ((1 << nbits) < n) ++nbits;
-    ++nbits;   // one more bit: lanes past the end of the run hold the value n-or-above 1 << (nbits - 1) and only equal each other
-    const int run = ((count + BK_WAVES - 1) / BK_WAVES + 63) & ~63, i0 = wv * run, i1 = min(count, i0 + run);
-    uint32_t* mine = hist + (size_t) wv * n;
-    for (int i = tid; i < BK_WAVES * n; i += 64 * BK_WAVES) hist[i] = 0;
-    int e[STEPS];
-    unsigned long long eq[STEPS];
-    auto load = [&](int i) {
-#pragma unroll
-        for (int u = 0; u < STEPS; ++u) e[u] = sel_at(min(i + 64 * u + lane, count - 1));
-#pragma unroll
-        for (int u = 0; u < STEPS; ++u) {
-            if (i + 64 * u + lane >= i1 || (unsigned) e[u] >= (unsigned) n) e[u] = 1 << (nbits - 1);   // an index outside the table is left out
-            eq[u] = equal_lanes(e[u], nbits);
-        }
-    };
-    const bool kept = run <= 64 * STEPS;
-    const unsigned long long below = (1ull << lane) - 1ull;
+    return nbits + 1;
+}
+// Up to 64 pairs a wave, one a lane, of expert e (1 << (nbits - 1): left out), the workgroup's first one being pair `first`.  hist [BK_WAVES][n], zero;
+// place(cnt): thread x < n with the workgroup's number of expert x's pairs -> where the first of them goes.  All threads come here.
+template <class Place>
+__device__ __forceinline__ void bucket_rank(int e, int nbits, int n, uint32_t* hist, int first, int32_t* perm, Place place) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    uint32_t* const mine = hist + (size_t) wv * n;
+    const unsigned long long eq = equal_lanes(e, nbits), below = (1ull << lane) - 1ull;
+    if (e < n && (eq & below) == 0) mine[e] = (uint32_t) __popcll(eq);
     __syncthreads();
-    for (int i = i0; i < i1; i += 64 * STEPS) {
-        load(i);
-#pragma unroll
-        for (int u = 0; u < STEPS; ++u)
-            if (e[u] < n && (eq[u] & below) == 0) mine[e[u]] += (uint32_t) __popcll(eq[u]);
-    }
-    __syncthreads();
-    int cnt = 0;
+    uint32_t cnt = 0;
+    if (tid < n)
+        for (int w = 0; w < BK_WAVES; ++w) cnt += hist[(size_t) w * n + tid];
+    uint32_t at = place(cnt);
     if (tid < n)
         for (int w = 0; w < BK_WAVES; ++w) {
             const uint32_t c = hist[(size_t) w * n + tid];
-            hist[(size_t) w * n + tid] = (uint32_t) cnt;
-            cnt += (int) c;
+            hist[(size_t) w * n + tid] = at;
+            at += c;
         }
-    const int pofs = scan_experts(cnt, n, work, tiles, wsum);
-    if (tid < n)
-        for (int w = 0; w < BK_WAVES; ++w) hist[(size_t) w * n + tid] += (uint32_t) pofs;
     __syncthreads();
-    for (int i = i0; i < i1; i += 64 * STEPS) {
-        if (!kept) load(i);
-#pragma unroll
-        for (int u = 0; u < STEPS; ++u)
-            if (e[u] < n) {
-                const uint32_t at = mine[e[u]];   // every lane of the group reads before its first lane moves the mark (LDS in wave order)
-                perm[at + (uint32_t) __popcll(eq[u] & below)] = i + 64 * u + lane;
-                if ((eq[u] & below) == 0) mine[e[u]] = at + (uint32_t) __popcll(eq[u]);
-            }
-    }
+    if (e < n) perm[mine[e] + (uint32_t) __popcll(eq & below)] = first + tid;
 }
+// Up to 64 BK_WAVES pairs, by one workgroup.  COH: the selections were stored by other workgroups of this launch (agent-scope atomic loads).
 template <bool COH>
 __device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
     __shared__ int wsum[2][BK_WAVES];
-    if (count <= 64 * BK_WAVES) bucket_steps<COH, 1>(inds, count, n, work, perm, tiles, wsum);
-    else if (count <= 4 * 64 * BK_WAVES) bucket_steps<COH, 4>(inds, count, n, work, perm, tiles, wsum);
-    else if (count <= 8 * 64 * BK_WAVES) bucket_steps<COH, 8>(inds, count, n, work, perm, tiles, wsum);
-    else bucket_steps<COH, 16>(inds, count, n, work, perm, tiles, wsum);
+    extern __shared__ uint32_t hist[];
+    const int tid = threadIdx.x, nbits = pair_bits(n);
+    int e = n;
+    if (tid < count) e = COH ? __hip_atomic_load(inds + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : inds[tid];
+    if ((unsigned) e >= (unsigned) n) e = 1 << (nbits - 1);   // (an index outside the table is left out)
+    for (int j = tid; j < BK_WAVES * n; j += 64 * BK_WAVES) hist[j] = 0;
+    __syncthreads();
+    bucket_rank(e, nbits, n, hist, 0, perm, [&](uint32_t cnt) { return (uint32_t) scan_experts((int) cnt, n, work, tiles, wsum); });
 }
 __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
     bucket_all<false>(inds, count, n, work, perm, tiles);
 }
-// The batched softmax step's routing and grouping in one launch: the workgroups rank the rows (k_topk_rank<0>'s arithmetic; ROWS 1 or 4 a workgroup),
+// More pairs: a workgroup for every 64 BK_WAVES.  Each counts all pairs by expert, those before its own apart, so that it needs nothing of the others, and
+// ranks its own.  One workgroup for all was bound by its CU's vector issue - count / 1024 steps of ranking a wave - and by its scattered stores of
+// the permutation.  E 128, us: 2048 pairs 6.2 -> 5.5, 4096 7.3 -> 5.6, 16384 19.1 -> 6.3, 65536 78.5 -> 11.1; 1024 pairs 4.4 and 5.3.
+#define BM_LOADS 16
+__global__ void __launch_bounds__(64 * BK_WAVES) k_bucket_many(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
+    __shared__ int wsum[2][BK_WAVES];
+    extern __shared__ uint32_t hist[];   // (first its first two rows: the pairs before this workgroup's, the others)
+    const int tid = threadIdx.x, nbits = pair_bits(n), first = (int) blockIdx.x * 64 * BK_WAVES;
+    for (int j = tid; j < 2 * n; j += 64 * BK_WAVES) hist[j] = 0;
+    int e = inds[min(first + tid, count - 1)];
+    if (first + tid >= count || (unsigned) e >= (unsigned) n) e = 1 << (nbits - 1);
+    __syncthreads();
+    for (int i0 = tid; i0 < count; i0 += BM_LOADS * 64 * BK_WAVES) {
+        int x[BM_LOADS];
+#pragma unroll
+        for (int u = 0; u < BM_LOADS; ++u) x[u] = inds[min(i0 + u * 64 * BK_WAVES, count - 1)];
+#pragma unroll
+        for (int u = 0; u < BM_LOADS; ++u) {
+            const int i = i0 + u * 64 * BK_WAVES;
+            if (i < count && (unsigned) x[u] < (unsigned) n) atomicAdd(&hist[(i < first ? 0 : n) + x[u]], 1u);
+        }
+    }
+    __syncthreads();
+    const uint32_t before = tid < n ? hist[tid] : 0u, all = tid < n ? before + hist[n + tid] : 0u;
+    const uint32_t at = before + (uint32_t) scan_experts((int) all, n, work, tiles, wsum, blockIdx.x == 0);   // (its barrier: the counts are read)
+    for (int j = tid; j < BK_WAVES * n; j += 64 * BK_WAVES) hist[j] = 0;
+    __syncthreads();
+    bucket_rank(e, nbits, n, hist, first, perm, [&](uint32_t) { return at; });
+}
+// The batched softmax step's routing and grouping of up to 64 BK_WAVES pairs in one launch: the workgroups rank a row each (k_topk_rank<0>'s arithmetic),
 // and the workgroup that finishes last - a ticket in the word behind the bucket's work area, back at zero when the
 // launch ends - groups the launch's pairs (k_bucket's).  Nobody waits for anybody.
-template <int ROWS>
 __global__ void __launch_bounds__(64 * BK_WAVES) k_route_bucket(int E, int k, const float* logits, int ld, int32_t* ind, float* wt, int T, int32_t* work,
                                                                 int32_t* perm, MmTile* tiles) {
     __shared__ int last;
-    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];   // the rows' ranking, then the grouping
-    const int sub = __builtin_amdgcn_readfirstlane((int) threadIdx.x / (64 * BK_WAVES / ROWS));   // (rows past the end: the last one again, the same values)
-    topk_row<0, 64 * BK_WAVES / ROWS, true>(min(ROWS * (int) blockIdx.x + sub, T - 1), E, k, logits, ld, (const float*) 0, 1.0f, ind, wt, dyn + sub * topk_lds(E));
-    if (ROWS > 1) {   // the selections have left their waves before the workgroup's ticket is taken
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {   // (one row: wave 0 stored its selection)
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];   // the row's ranking, then the grouping
+    topk_row<0, 64 * BK_WAVES, true>((int) blockIdx.x, E, k, logits, ld, (const float*) 0, 1.0f, ind, wt, dyn);
+    if (threadIdx.x == 0) {   // (wave 0 stored the selection)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         last = atomicAdd((unsigned*) &work[2 * E + 3], 1u) == gridDim.x - 1u;
@@ -788,6 +787,15 @@ void kc_pack_input_bf16(kc_stream_t s, const float* x, uint16_t* y, size_t n) {
 void kc_bucket(kc_stream_t s, const int32_t* inds, int count, int n, int32_t* perm, MmTile* tiles, int32_t* ntiles) {
     if (n < 1 || n > BUCKET_MAX_EXPERTS || count < 0) { host_note_unsupported(); return; }
     const size_t lds = sizeof(uint32_t) * BK_WAVES * (size_t) n;
+    if (count > 64 * BK_WAVES) {
+        static const hipError_t once = hipFuncSetAttribute((const void*) k_bucket_many, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                           (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));
+        (void) once;
+        hipLaunchKernelGGL(k_bucket_many, dim3((unsigned) (count + 64 * BK_WAVES - 1) / (64 * BK_WAVES)), dim3(64 * BK_WAVES), lds, (hipStream_t) s, inds, count, n,
+                           ntiles, perm, tiles);
+        host_note_launch();
+        return;
+    }
     static const hipError_t once = hipFuncSetAttribute((const void*) k_bucket, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));
     (void) once;
@@ -798,21 +806,19 @@ void kq4_route_bucket(kc_stream_t s, const Qwen4Cfg* c, const float* logits, int
                       int32_t* ntiles) {
     if (T < 1) return;
     if (c->n_exp < c->top_k || c->n_exp > TK_MAXE || c->top_k < 1 || c->top_k > TK_MAXK || c->n_exp > BUCKET_MAX_EXPERTS) { host_note_unsupported(); return; }
-    // Rows by fours where they are more than a workgroup on every other CU (E 128 / 64, top-8, us a launch by ones and by fours: 32 rows 7.6 and 8.3, 64 rows
-    // 8.1 and 8.5; 200 rows 11.0 and 10.4; 2048 rows, which had taken 54.1, 31.0 by fours).
-    const size_t group = sizeof(uint32_t) * BK_WAVES * (size_t) c->n_exp;
-#define ROUTE(ROWS)                                                                                                                                              \
-    do {                                                                                                                                                         \
-        static const hipError_t once = hipFuncSetAttribute((const void*) k_route_bucket<ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize,                        \
-                                                           (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));                                            \
-        (void) once;                                                                                                                                             \
-        const size_t rows = (size_t) ROWS * topk_lds(c->n_exp), lds = group > rows ? group : rows;                                                               \
-        hipLaunchKernelGGL(k_route_bucket<ROWS>, dim3((unsigned) (T + ROWS - 1) / ROWS), dim3(64 * BK_WAVES), lds, (hipStream_t) s, c->n_exp, c->top_k, logits,   \
-                           c->n_exp, ind, wt, T, ntiles, perm, tiles);                                                                                 \
-    } while (0)
-    if (T > host_cu_count() / 2) ROUTE(4);
-    else ROUTE(1);
-#undef ROUTE
+    // In one launch up to a workgroup's pairs and half as many rows as CUs (E 128, top-8, us in one launch and in two: 64 rows 7.5 and 7.5, 128 rows 8.5 and
+    // 8.0; E 1024 12.6 and 14.5; 200 rows, E 64, top-4, 8.3 and 7.7; 2048 rows 29.6 and 11.1 - the last workgroup grouped all).
+    if (T * c->top_k > 64 * BK_WAVES || T > host_cu_count() / 2) {
+        kq4_route_ld(s, c, logits, c->n_exp, ind, wt, T);
+        kc_bucket(s, ind, T * c->top_k, c->n_exp, perm, tiles, ntiles);
+        return;
+    }
+    static const hipError_t once = hipFuncSetAttribute((const void*) k_route_bucket, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));
+    (void) once;
+    const size_t group = sizeof(uint32_t) * BK_WAVES * (size_t) c->n_exp, rows = (size_t) topk_lds(c->n_exp), lds = group > rows ? group : rows;
+    hipLaunchKernelGGL(k_route_bucket, dim3((unsigned) T), dim3(64 * BK_WAVES), lds, (hipStream_t) s, c->n_exp, c->top_k, logits, c->n_exp, ind, wt, T, ntiles,
+                       perm, tiles);
     host_note_launch();
 }
 void kc_cache_admit(kc_stream_t s, const CachePool* p, int sl, const int32_t* inds, int count, int flags) {

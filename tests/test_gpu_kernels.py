@@ -415,9 +415,9 @@ def test_bucket(be, oracle):
         assert np.array_equal(perm, operm) and np.array_equal(tiles, otiles)
 
 
-@pytest.mark.parametrize("count", [1, 1023, 16384, 16385, 50001])
-def test_bucket_of_long_runs(be, oracle, count):
-    """A wave's run of up to 16 steps of 64 pairs, which it keeps in registers, and longer ones; indices outside the table; a few experts with most pairs."""
+@pytest.mark.parametrize("count", [1, 1024, 1025, 2048, 16384, 16385, 50001])
+def test_bucket_of_many_pairs(be, oracle, count):
+    """A workgroup's 1024 pairs and one more, 16 rounds of them and one more; indices outside the table; a few experts with most pairs."""
     rng = np.random.default_rng(count)
     for n in (3, 128, 1000):
         inds = np.minimum(rng.integers(0, n, count), rng.integers(0, 4 * n, count)).astype(np.int32)
@@ -782,9 +782,9 @@ def test_route_bucket_equals_route_then_bucket(E, k, T):
         b.free()
 
 
-# a row a wave, 16 a workgroup: one row, a workgroup's rows and one more, rows of one to four groups of 64, the most picks, thousands of rows; 257: a row a workgroup
-@pytest.mark.parametrize("E,k,T", [(64, 8, 1), (65, 32, 16), (130, 1, 17), (256, 32, 40), (32, 32, 33), (257, 8, 20), (128, 8, 2100)])
-def test_route_bucket_rows_of_a_wave(be, E, k, T):
+# one launch up to 1024 pairs and half as many rows as CUs, two from there on: one row, both sides of either line, rows of one to five groups of 64, the most picks
+@pytest.mark.parametrize("E,k,T", [(64, 8, 1), (65, 32, 32), (32, 32, 33), (130, 8, 128), (128, 8, 129), (16, 2, 129), (257, 8, 20), (128, 8, 2100)])
+def test_route_bucket_in_one_launch_and_two(be, E, k, T):
     test_route_bucket_equals_route_then_bucket(E, k, T)
 
 
