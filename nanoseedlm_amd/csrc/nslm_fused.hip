@@ -19,6 +19,7 @@
 // Waiting: the grid is sized to the number of workgroups the device can hold at once (occupancy query), because
 // workgroups wait for each other's data; every wait is a bounded poll, and a workgroup that gives up sets an error word
 // and runs on to the end, so every wave always exits.
+#include <limits.h>
 #include <math.h>
 #include <stdlib.h>
 
@@ -774,7 +775,7 @@ bool shape_of(int K, bool gateup, int* L, int* rpi, bool* shfl) {
 }
 
 // Items per pair (or group) of a phase of `iters` iterations, `units` pairs, at most gmax workgroups.
-// one_round: the count that gives the busiest workgroup the least to do when every workgroup takes its items one after the
+// The count that gives the busiest workgroup the least to do when every workgroup takes its items one after the
 // other (an item's set-up priced at a third of an iteration, unequal items at half an iteration: workgroups i, i + 256, ...
 // share a CU, so the long items of a regular pattern meet on the same CUs); up to `slack` items more than the workgroups still
 // count as one round.
@@ -788,21 +789,6 @@ int pick_one_round(int units, int iters, int gmax, int nmax, int slack = 0, int 
     }
     return best;
 }
-// by_cu_load: the count that gives the busiest CU the least to do (items go round the workgroups, the workgroups round the
-// CUs, and a CU's waves share its issue slots, so a CU is as late as the sum of its items, plus one item for the end of
-// the phase, when the CU is no longer full), with fewer than five workgroups a CU priced for the latencies they no longer hide.
-int pick_by_cu_load(int units, int iters, int cus, int nmax) {
-    static const int thin[6] = {200, 160, 130, 115, 103, 100};
-    int best = 1;
-    long best_cost = -1;
-    for (int n = 1; n <= iters && n <= nmax; ++n) {
-        const long items = (long) units * n, per = (iters + n - 1) / n, on_cu = (items + cus - 1) / cus;
-        const long cost = (on_cu * (6 * per + (iters % n ? 3 : 0) + 2) + 2 * per) * thin[items / cus < 5 ? items / cus : 5];
-        if (best_cost < 0 || cost <= best_cost) { best = n; best_cost = cost; }
-    }
-    return best;
-}
-
 #define GU_ROWS 128   // SwiGLU rows of an item whose two sums wait in LDS for the end of the item's row loop (per-item kernel)
 // the fewest items a pair at which an item's rows fit that area
 int gu_min_tiles(const FusedArgs& a) {
@@ -815,15 +801,21 @@ template <int P>
 int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     a.gu_off = (int) (lds / sizeof(float));
     lds += GU_ROWS * sizeof(float2);
-    // One token is at most a few hundred items more than three workgroups a CU hold (C2: 784): that launch may use the
-    // registers of four waves a SIMD instead of five (no spills: 35.0 -> 34.5 us).  At P = 4 the
-    // same holds up to four tokens (C2, four / five waves, us: 2 tokens 41.4 / 45.8, 3: 55.6 / 56.3, 4: 66.4 / 69.8, 5: 85.9 / 80.3,
-    // 8: 115.1 / 110.8; P = 3, C3: 2 tokens 166.5 / 157.7, 4: 272.6 / 263.7).
-    const bool few = a.T == 1 || (P == 4 && a.T <= 4);
+    // Four waves a SIMD, or five, whose registers spill (76 bytes a lane) but which leave shorter items, 1280 workgroups for 1024.  Timed on 122 layers
+    // of 2 .. 8 tokens (us a layer, four / five waves): five where the step is large and the gate + up sums stay in a wave (8 tokens, E 128, top-8,
+    // 2048 x 768 86.0 / 81.9; 6 of top-8, 2048 x 1024 98.8 / 81.7; 5 of top-8, 2048 x 768 59.4 / 61.3), and, where both phases' sums go through
+    // LDS, whose barriers more workgroups cover, from less on (4 tokens of top-4, 2880 x 1408 93.1 / 83.2; 8, 1344 x 704 43.2 / 37.6;
+    // 4, 1344 x 704 26.3 / 29.4).  With the gate + up sums alone there it is four (8 tokens of top-4, 4096 x 512 82.7 / 131; 6 of top-2,
+    // 768 x 2048 31.1 / 36.4; P = 3, 8 of top-4, 2560 x 1024 94.0 / 97.2) but for the large steps of P = 4 whose rows are shorter than 64 chunks (8 of
+    // top-4, 3072 x 1024 122 / 112), and four for every small step (6 tokens of top-4, 1024 x 512 21.9 / 28.8).  The rule is 0.5 % off the
+    // faster of the two on average.
+    const long work = (long) a.T * a.kk * a.d * a.ff;
+    const long large = sg ? 48L << 20 : !sd ? 20L << 20 : P == 4 && a.Lg < 64 ? 40L << 20 : LONG_MAX;
+    const bool few = a.T == 1 || work < large;
     void (*kern)(FusedArgs) = few ? (sg ? (sd ? k_moe_decode<P, true, true, 4> : k_moe_decode<P, true, false, 4>)
                                         : (sd ? k_moe_decode<P, false, true, 4> : k_moe_decode<P, false, false, 4>))
                                   : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
-                                        : (sd ? k_moe_decode<P, false, true, 5> : k_moe_decode<P, false, false, 5>));
+                                        : (sd ? k_moe_decode<P, false, true, P == 4 ? 5 : 4> : k_moe_decode<P, false, false, 5>));
     // resident workgroups per CU, by kernel variant, for the largest LDS request seen (the request grows with max(d, ff): a launch
     // that asks for more than the cached answer covered asks the occupancy calculator again, and raises the kernel's limit above 48 KB)
     static int cached[2][2][2] = {};
@@ -839,15 +831,13 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     }
     // The grid must be resident at once (workgroups wait for each other's data): at most what the device holds, and no more than
     // five workgroups a CU (the most that was tried).  Items per pair (an item = a run of a pair's iterations, as
-    // equal as whole iterations allow).  Down items, and every item of one token: one round (measured on C2, one token: 96 x 2
+    // equal as whole iterations allow): one round (measured on C2, one token: 96 x 2
     // gate+up iterations and 98 x 1 down iterations a pair on 784 workgroups, 40.1 us; 96 unequal down items on 768
     // workgroups: 42.9; 8 tokens with 32 instead of 20 down items a pair: 144 against 131 us - a down item waits for its
-    // pair, and a second round of them waits behind the first).  Gate+up items of several tokens: by the CUs' load, which
-    // takes more, shorter items than one round holds (C2, items a pair -> us; 4 tokens: 24 -> 82.2, 40 -> 79.6, 64 -> 78.0;
-    // 6 tokens: 24 -> 120.2, 32 -> 111.4, 48 -> 115.2; 8 tokens: 20 -> 135.4, 32 -> 131.2, 48 -> 138.9); where the row sums go
-    // through LDS (C3) one round stayed ahead.
+    // pair, and a second round of them waits behind the first).  More, shorter gate+up items by the CUs' load, for several tokens, had been ahead
+    // (by 1 .. 10 %) while a block's decode took a third longer; now they are 3 .. 5 % behind at 7 and 8 tokens of C2 and 3 % ahead at 6.
     const int gmax = (per_cu < 5 ? per_cu : 5) * cu_count(), P_ = a.T * a.kk;
-    a.ntile_g = few || !sg ? pick_one_round(P_, a.it_g, gmax, FUSED_TILES) : pick_by_cu_load(P_, a.it_g, cu_count(), FUSED_TILES);
+    a.ntile_g = pick_one_round(P_, a.it_g, gmax, FUSED_TILES);
     // (a down item's set-up - the wait for its pair, the staging of A - priced at two thirds of an iteration: at a third, six
     // tokens of C2 took two rounds of 49 two-iteration items a pair, 81.6 us, where one round of 26 takes 76.5)
     a.ntile_d = pick_one_round(P_, a.it_d, gmax, FUSED_TILES, 0, 4);

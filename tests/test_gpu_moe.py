@@ -371,6 +371,33 @@ def test_both_step_kernels_give_the_separate_launches_bits(fmt, E, k, d, ff):
         st.close()
 
 
+# the per-pair kernel with four and with five waves a SIMD: either side of T k d ff = 48 Mi with gate + up sums by shuffles (the down ones through LDS, by
+# shuffles), of 20 Mi with both through LDS, of 40 Mi with the gate + up ones there (P = 4)
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (3, 4, 5, 8)), (8, 2048, 512, (5, 6, 8)), (4, 1344, 704, (5, 6)), (4, 3072, 1024, (3, 4))])
+def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows):
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    rng = np.random.default_rng(d + ff + fmt)
+    st = moe.MoeStack(1, 16, k, d, ff, fmt=fmt, router=moe.ROUTE_SOFTMAX, max_rows=8)
+    backend.check(st.L.nslm_moe_fill_random(st.h, C.c_uint64(77), -22, C.c_float(0.035)), "nslm_moe_fill_random")
+    st.finalize()
+    for T in rows:
+        dx = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32)))
+        outs = []
+        for fused in (0, 1):
+            st.set_fused(fused)
+            before = st.fused_steps()
+            dio = moe.DevBuf.from_array(np.zeros((T, d), dtype=np.float32))
+            st.step(None, 0, dx.ptr, T, dio.ptr)
+            outs.append(dio.to_array(np.float32, (T, d)))
+            dio.free()
+            assert st.fused_error() == 0 and st.fused_steps() == before + fused, (T, fused)
+        dx.free()
+        assert np.abs(outs[0]).max() > 0 and np.array_equal(outs[1].view(np.uint32), outs[0].view(np.uint32)), T
+    st.close()
+
+
 def test_steps_issued_by_one_call_equal_single_steps():
     """nslm_moe_step_seq (n steps and the two timing events from one call into the C host) leaves what the same steps leave when
     issued one by one, and its events bracket them; nslm_mv_seq does the same for the dense matvec."""
