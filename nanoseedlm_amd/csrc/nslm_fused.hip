@@ -979,7 +979,8 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
     if (T > MV_MAXT || (shared && T >= FG_MINT_SHARED && sg && T * a.kk <= FG_MAXP)) {
         // More rows than the per-pair kernel takes: pairs grouped by expert, two to a decode.  Measured against the grouped
         // GEMMs of the separate launches (C2, 16 rows: 199 against 268 us; 20 rows: 242 against 295; 24 rows: 278 against 305;
-        // 28 rows: 335 against 327, so the limit is 24); with four to a decode (402 against 338 us at 32 rows) and where the gate+up row sums go through LDS (C3's 45 chunks a row: 1129 against 753 us) the GEMMs
+        // 28 rows: 335 against 327, so the limit is 24; the GEMMs have gained more since, 32 rows
+        // take 171 there and 24 rows 190 here, but they multiply the rows' BF16 values, and these rows are f32); with four to a decode (402 against 338 us at 32 rows) and where the gate+up row sums go through LDS (C3's 45 chunks a row: 1129 against 753 us) the GEMMs
         // win, so those shapes are left to them.  With an always-on expert every row brings a pair on the same expert, and
         // the grouped kernel is already ahead of the per-pair one at 5 rows (whole model, 5 rows: 4.05 against 4.18 ms, 8 rows:
         // 5.37 against 5.70; 4 rows: 3.85 against 3.68); without
@@ -987,13 +988,15 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
         if (!sg) return -1;
         return fmt == MF_SEED4P4 ? launch_grouped<4, 2>((hipStream_t) s, a, sg, sd) : launch_grouped<3, 2>((hipStream_t) s, a, sg, sd);
     }
-    // one workgroup per CU: ahead at one token everywhere, at two where the step is large or P = 3 (us, a workgroup per CU / per
-    // item, records from HBM.  C2: 1 token 19.9 / 25.2, 2: 36.6 / 35.5, 3: 48.4 / 45.5; C2's shape in P = 3: 24.6 / 26.3,
-    // 39.4 / 43.5, 54.7 / 50.9, 4: 70.0 / 63.8; 256 experts of 4096 x 1024: 45.8 / 54.9, 80.7 / 90.6, 168.8 / 168.9; C3, whose rows
-    // of 45 chunks make that kernel's passes go by iterations of the workgroup: 55.0 / 67.3, 100.9 / 104.7, 146.9 / 147.6,
-    // 192.6 / 186.2)
-    const bool cu_two = fmt != MF_SEED4P4 || (sg && (long) top_k * d * ff >= 24L << 20);
-    if ((g_kernel_choice == 2 || (g_kernel_choice == 0 && T <= (cu_two ? 2 : 1))) && launch_moe_decode_cu((hipStream_t) s, a, fmt == MF_SEED4P4 ? 4 : 3, sd) == 0) return 0;
+    // One workgroup per CU: ahead at one token everywhere, and at two to six where rows are long - 44 chunks or more, whose sums the other kernel takes through
+    // LDS with its waves' registers spilled or its workgroups few - and the step large.  (Timed on 28 layers in both formats, us a layer, a workgroup
+    // an item / a CU.  4 experts of 2880 x 2880, P = 3: 2 tokens 94.9 / 78.1, 3: 132.8 / 113.7, 4: 168 / 150, 5: 200 / 185; 8 of 3072 x 1024, P = 4: 2: 67.1 /
+    // 57.4, 6: 168 / 158; 8 of 4096 x 512: 6: 142 / 115; 4 of 2880 x 1408: 2: 53.8 / 48.6, 3: 69.2 / 68.5, 4: 83.2 / 88.6; 2 of 4096 x 512: 3: 30.5 / 33.4.
+    // Shorter rows: C2 2: 32.7 / 34.0, 3: 41.7 / 45.9; 8 of 1536 x 1536, P = 3: 2: 48.4 / 53.1, 3: 63.0 / 76.0; 4 of 2560 x 1024: 2: 36.0 / 37.5, though
+    // 4 of 1536 x 1024 2: 29.3 / 26.4.)
+    const long layer = (long) top_k * d * ff;
+    const bool by_cu = T == 1 || (a.Lg >= 44 && T <= 6 && layer >= (T == 2 ? 6L : T == 3 ? 12L : 16L) << 20);
+    if ((g_kernel_choice == 2 || (g_kernel_choice == 0 && by_cu)) && launch_moe_decode_cu((hipStream_t) s, a, fmt == MF_SEED4P4 ? 4 : 3, sd) == 0) return 0;
     const int kmax = d > ff ? d : ff;
     size_t lds = (size_t) (kmax / 64) * XPAD * sizeof(float);
     return fmt == MF_SEED4P4 ? launch_fused<4>((hipStream_t) s, a, sg, sd, lds) : launch_fused<3>((hipStream_t) s, a, sg, sd, lds);

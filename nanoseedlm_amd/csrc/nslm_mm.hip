@@ -617,7 +617,7 @@ void mm_dense(hipStream_t st, int fmt, WSlice w, int K, int R, const void* x, in
 }
 // Grouped launches, by what the caller says of its tiles (tile_rows, kernels_hip.h):
 //   up to 96 pairs: the kernel for few tokens, which decodes as fast as the chip can but passes over a tile's weights once every 32, 64 or 96
-//   pairs (E 128, top-8, d 2048, ff 768, P = 4, us a layer step against the streamed kernel's workgroups of 128 pairs: 64 rows 304 -> 237,
+//   pairs (E 128, top-8, d 2048, ff 768, P = 4, us a layer step against the streamed kernel's workgroups of 128 pairs: 64 rows 304 -> 237 (now 189),
 //   512 rows - 32 pairs a tile - 387 -> 306);
 //   more than a tile holds: the tiles are mostly full - k_mm_wide, one decode for up to 256 pairs (2048 rows: 641 -> 521);
 //   nothing: both, tiles of up to ROWS_MOST pairs to the first (but for those that join a fuller one: Join), fuller ones to the other.

@@ -11,8 +11,9 @@
 //     y = sum over w < 4 of (segment w + segment w + 4).  So a token's bits depend on K alone, not on the launch's shape, the tile or its
 //     other tokens, in every dense launch of this file and in grouped passes of up to 32 pairs.  Passes of more have no registers for two
 //     sums a pair: a wave's two segments are one chain there, and k_mm_wide's sum is one chain over all of K.
-// Measured (us, streamed kernel -> this one): P = 4, 4096 x 4096: 9 tokens 40.1 -> 9.7, 48 tokens 42.8 -> 11.1, 200 tokens 51.8 -> 23.0;
-// 1024 x 4096, 100 tokens 44.7 -> 11.2; Q4 2880 x 2880, 301 tokens 43.0 -> 17.8; BF16 151936 x 2048, 16 tokens 155.7 -> 115.3 (5.5 TB/s).
+// Measured (us, streamed kernel -> this one, when both decoded by four multiply-adds a weight): P = 4, 4096 x 4096: 9 tokens 40.1 -> 9.7, 48 tokens
+// 42.8 -> 11.1, 200 tokens 51.8 -> 23.0; 1024 x 4096, 100 tokens 44.7 -> 11.2; Q4 2880 x 2880, 301 tokens 43.0 -> 17.8; BF16 151936 x 2048, 16 tokens
+// 155.7 -> 115.3 (5.5 TB/s).  By one multiply-add a weight 48 tokens take 9.4, by Q4's scales 16 lanes a row tile 301 tokens 15.9.
 // What bounds it: vector issue of the decode for the seed formats, the activations' way from L2 for Q4 / Q8 / BF16 at many tokens,
 // HBM for BF16 at few.
 #include "nslm_mm_dev.h"
