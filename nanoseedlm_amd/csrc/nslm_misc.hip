@@ -430,17 +430,17 @@ __device__ __forceinline__ void bucket_all(const int32_t* inds, int count, int n
 __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
     bucket_all<false>(inds, count, n, work, perm, tiles);
 }
-// More pairs: a workgroup for every 64 BK_WAVES.  Each counts all pairs by expert, those before its own apart, so that it needs nothing of the others, and
-// ranks its own.  One workgroup for all was bound by its CU's vector issue - count / 1024 steps of ranking a wave - and by its scattered stores of
+// More pairs: a workgroup for every 64 BK_WAVES, or for an equal run of those (`runs`) - each counts all pairs by expert, those before its own apart, so that
+// it needs nothing of the others, and that makes at most BM_GROUPS times the pairs to count.  Then it ranks its own.  One workgroup for all was bound by its CU's vector issue - count / 1024 steps of ranking a wave - and by its scattered stores of
 // the permutation.  E 128, us: 2048 pairs 6.2 -> 5.5, 4096 7.3 -> 5.6, 16384 19.1 -> 6.3, 65536 78.5 -> 11.1; 1024 pairs 4.4 and 5.3.
 #define BM_LOADS 16
-__global__ void __launch_bounds__(64 * BK_WAVES) k_bucket_many(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles) {
+#define BM_GROUPS 256
+__global__ void __launch_bounds__(64 * BK_WAVES) k_bucket_many(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles, int runs) {
     __shared__ int wsum[2][BK_WAVES];
     extern __shared__ uint32_t hist[];   // (first its first two rows: the pairs before this workgroup's, the others)
-    const int tid = threadIdx.x, nbits = pair_bits(n), first = (int) blockIdx.x * 64 * BK_WAVES;
+    const int tid = threadIdx.x, nbits = pair_bits(n), first = (int) blockIdx.x * runs * 64 * BK_WAVES;
     for (int j = tid; j < 2 * n; j += 64 * BK_WAVES) hist[j] = 0;
     int e = inds[min(first + tid, count - 1)];
-    if (first + tid >= count || (unsigned) e >= (unsigned) n) e = 1 << (nbits - 1);
     __syncthreads();
     for (int i0 = tid; i0 < count; i0 += BM_LOADS * 64 * BK_WAVES) {
         int x[BM_LOADS];
@@ -454,10 +454,22 @@ __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket_many(const int32_t* in
     }
     __syncthreads();
     const uint32_t before = tid < n ? hist[tid] : 0u, all = tid < n ? before + hist[n + tid] : 0u;
-    const uint32_t at = before + (uint32_t) scan_experts((int) all, n, work, tiles, wsum, blockIdx.x == 0);   // (its barrier: the counts are read)
-    for (int j = tid; j < BK_WAVES * n; j += 64 * BK_WAVES) hist[j] = 0;
-    __syncthreads();
-    bucket_rank(e, nbits, n, hist, first, perm, [&](uint32_t) { return at; });
+    uint32_t at = before + (uint32_t) scan_experts((int) all, n, work, tiles, wsum, blockIdx.x == 0);   // (its barrier: the counts are read)
+    const int end = min(count, first + runs * 64 * BK_WAVES);
+    for (int i = first; i < end; i += 64 * BK_WAVES) {
+        if (i != first) {
+            e = inds[min(i + tid, count - 1)];
+            __syncthreads();   // the places of the pairs before are read
+        }
+        if (i + tid >= count || (unsigned) e >= (unsigned) n) e = 1 << (nbits - 1);
+        for (int j = tid; j < BK_WAVES * n; j += 64 * BK_WAVES) hist[j] = 0;
+        __syncthreads();
+        bucket_rank(e, nbits, n, hist, i, perm, [&](uint32_t cnt) {
+            const uint32_t p = at;
+            at += cnt;
+            return p;
+        });
+    }
 }
 // The batched softmax step's routing and grouping of up to 64 BK_WAVES pairs in one launch: the workgroups rank a row each (k_topk_rank<0>'s arithmetic),
 // and the workgroup that finishes last - a ticket in the word behind the bucket's work area, back at zero when the
@@ -791,8 +803,9 @@ void kc_bucket(kc_stream_t s, const int32_t* inds, int count, int n, int32_t* pe
         static const hipError_t once = hipFuncSetAttribute((const void*) k_bucket_many, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                            (int) (sizeof(uint32_t) * BK_WAVES * BUCKET_MAX_EXPERTS));
         (void) once;
-        hipLaunchKernelGGL(k_bucket_many, dim3((unsigned) (count + 64 * BK_WAVES - 1) / (64 * BK_WAVES)), dim3(64 * BK_WAVES), lds, (hipStream_t) s, inds, count, n,
-                           ntiles, perm, tiles);
+        const int steps = (int) (((unsigned) count + 64 * BK_WAVES - 1) / (64 * BK_WAVES)), runs = (steps + BM_GROUPS - 1) / BM_GROUPS;
+        hipLaunchKernelGGL(k_bucket_many, dim3((unsigned) (steps + runs - 1) / (unsigned) runs), dim3(64 * BK_WAVES), lds, (hipStream_t) s, inds, count, n,
+                           ntiles, perm, tiles, runs);
         host_note_launch();
         return;
     }

@@ -415,9 +415,9 @@ def test_bucket(be, oracle):
         assert np.array_equal(perm, operm) and np.array_equal(tiles, otiles)
 
 
-@pytest.mark.parametrize("count", [1, 1024, 1025, 2048, 16384, 16385, 50001])
+@pytest.mark.parametrize("count", [1, 1024, 1025, 2048, 16384, 16385, 50001, 262144, 262145, 700001])
 def test_bucket_of_many_pairs(be, oracle, count):
-    """A workgroup's 1024 pairs and one more, 16 rounds of them and one more; indices outside the table; a few experts with most pairs."""
+    """A workgroup's 1024 pairs and one more, 16 rounds of them and one more, 256 workgroups' and one more (two and three runs a workgroup); indices outside the table; a few experts with most pairs."""
     rng = np.random.default_rng(count)
     for n in (3, 128, 1000):
         inds = np.minimum(rng.integers(0, n, count), rng.integers(0, 4 * n, count)).astype(np.int32)
