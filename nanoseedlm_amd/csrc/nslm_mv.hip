@@ -921,13 +921,16 @@ int wide_run(int fmt, int K, int R, int T) {
 // instead of one (2048 x 2048, P = 3, 8 tokens: 9.5 us in two runs of four, 12.2 in one: what it takes is the staging).  A workgroup's share
 // of the row quads is a CU's, or half or a quarter of it where there is work for so many workgroups and their tokens fit the LDS: one
 // stages while another decodes.  A round is as many row quads as two passes of the threads and the LDS hold.
-// Rows of up to 32 chunks whose sums go by shuffles stay with the staged pass of k_mv_seed where that was as fast or faster: two tokens
-// (8192 x 2048: 11.6 us there, 12.0 here), and 5 to 8 of a matrix near 2048 x 2048 (8.0 and 9.0).
+// Rows of up to 32 chunks whose sums go by shuffles stay with the staged pass of k_mv_seed where that is as fast or faster (us, this kernel / that
+// one, P = 4): two tokens, and, from 32 chunk quads a CU on, more (4 tokens, 2000 x 1024 6.0 / 6.4); of rows of up to 16 chunks (3 tokens, 12000 x 512
+// 7.8 / 6.2; 7 tokens 11.6 / 7.5; 6 tokens, 16384 x 1024 16.1 / 14.4), and of 32 up to a size (2 tokens, 8192 x 2048 11.3 / 10.2, 12000 x 2048
+// 17.7 / 17.1, 16000 x 2048 18.6 / 23.0; 3 tokens 12.9 / 11.8, 19.8 / 24.8; 6 tokens, 2048 x 2048 8.4 / 7.2, 6000 x 2048 16.4 / 17.7).
 template <int P>
 bool launch_tok(hipStream_t st, MvArgs a, int T, bool shfl) {
     const int L = a.L, rq = (a.R + 3) / 4, LS = L | 1;
     const long quads = (long) rq * L;
-    if (shfl && L <= 32 && (T == 2 || (T > 4 && quads >= 32L * cu_count() && quads <= 96L * cu_count()))) return false;
+    const int cus = cu_count();
+    if (shfl && L <= 32 && (T == 2 || quads >= 32L * cus) && (L <= 16 || quads <= (T > 4 ? 96L : T > 2 ? 256L : 400L) * cus)) return false;
     // token stride: 16 banks apart, so that the 16-byte reads of a quad's four tokens do not meet
     const int tstride = ((L * XPAD + 63) / 64) * 64 + 16;
     const size_t tok = (size_t) tstride * sizeof(float), tok_sums = (size_t) 4 * LS * sizeof(float);   // a token's, of a row quad

@@ -403,6 +403,19 @@ def test_mm_few_tokens_streams_at_any_boundary(be, oracle, off):
     assert np.array_equal(ys[0], ys[1])
 
 
+# two to eight tokens of rows whose sums go by shuffles, on either side of the line between the staged pass and the kernel with products on the matrix pipe: 8,
+# 16 and 32 chunks a row, few and many chunk quads a CU (R / 4 K / 64 / 256), a last row quad of one and three rows
+@pytest.mark.parametrize("R,K,T", [(4101, 512, 3), (4003, 512, 8), (2001, 1024, 4), (2051, 1024, 6), (1023, 2048, 3), (3075, 2048, 5), (8195, 2048, 4)])
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+def test_mv_rows_of_either_kernel_have_the_one_token_bits(be, fmt, R, K, T):
+    rng = np.random.default_rng(R + K + T + fmt)
+    p = make_pack(rng, fmt, 1, R, K)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    y = be.kt_mv(p, x)
+    for t in range(T):
+        assert np.array_equal(y[t].view(np.uint32), be.kt_mv(p, x[t:t + 1])[0].view(np.uint32)), t
+
+
 # ---- grouping, routers, elementwise, slot table -------------------------------------------------------------------------------
 
 def test_bucket(be, oracle):
