@@ -797,6 +797,35 @@ int gu_min_tiles(const FusedArgs& a) {
     return n;
 }
 
+// Workgroups of `bytes` of LDS, static and dynamic, that a CU holds at once.  LDS is given out in pieces of 1280 bytes, which
+// hipOccupancyMaxActiveBlocksPerMultiprocessor leaves out of account: of 32736 bytes it counts five to a CU, which holds four.  (Timed with workgroups that
+// wait 50 us, as many as it counts: 54 us at 32000, 53588 and 26792 bytes, 104 at 32256 .. 32768, 53844 .. 54612 and 27048 .. 27304.)
+constexpr int lds_workgroups(size_t bytes) { return bytes ? (int) (160 * 1024 / ((bytes + 1279) / 1280 * 1280)) : INT_MAX; }
+static_assert(lds_workgroups(40960) == 4 && lds_workgroups(32000) == 5 && lds_workgroups(32004) == 4 && lds_workgroups(32736) == 4 &&
+              lds_workgroups(53760) == 3 && lds_workgroups(53764) == 2 && lds_workgroups(160 * 1024) == 1 && lds_workgroups(160 * 1024 + 1) == 0, "LDS pieces");
+// A kernel of 256 threads: the workgroups a CU holds by its registers, its static LDS, and the dynamic LDS it has been prepared for
+struct Residency {
+    int by_registers = 0;
+    size_t fixed = 0, prepared = 48 * 1024;
+};
+// Workgroups of `kern` with `dyn` bytes of dynamic LDS that a CU holds at once; < 1: none, or an error.  These kernels' workgroups wait for each other, so
+// a grid of more than this a CU would wait for workgroups that have not started.
+int resident_workgroups(const void* kern, Residency& r, size_t dyn) {
+    if (!r.by_registers) {
+        hipFuncAttributes at;
+        int n = 0;
+        if (hipFuncGetAttributes(&at, kern) != hipSuccess || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 256, 0) != hipSuccess) return -1;
+        r.fixed = at.sharedSizeBytes;
+        r.by_registers = n;
+    }
+    if (dyn > r.prepared) {   // above 48 KB a kernel has to be asked for
+        if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) dyn) != hipSuccess) return -1;
+        r.prepared = dyn;
+    }
+    const int by_lds = lds_workgroups(r.fixed + dyn);
+    return by_lds < r.by_registers ? by_lds : r.by_registers;
+}
+
 template <int P>
 int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     a.gu_off = (int) (lds / sizeof(float));
@@ -816,19 +845,9 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
                                         : (sd ? k_moe_decode<P, false, true, 4> : k_moe_decode<P, false, false, 4>))
                                   : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
                                         : (sd ? k_moe_decode<P, false, true, P == 4 ? 5 : 4> : k_moe_decode<P, false, false, 5>));
-    // resident workgroups per CU, by kernel variant, for the largest LDS request seen (the request grows with max(d, ff): a launch
-    // that asks for more than the cached answer covered asks the occupancy calculator again, and raises the kernel's limit above 48 KB)
-    static int cached[2][2][2] = {};
-    static size_t cached_lds[2][2][2] = {};
-    int& per_cu = cached[few][sg][sd];
-    if (!per_cu || lds > cached_lds[few][sg][sd]) {
-        if (lds > 48 * 1024 && hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return -1;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds) != hipSuccess || per_cu < 1) {
-            per_cu = 0;
-            return -1;
-        }
-        cached_lds[few][sg][sd] = lds;
-    }
+    static Residency known[2][2][2];
+    const int per_cu = resident_workgroups((const void*) kern, known[few][sg][sd], lds);
+    if (per_cu < 1) return -1;
     // The grid must be resident at once (workgroups wait for each other's data): at most what the device holds, and no more than
     // five workgroups a CU (the most that was tried).  Items per pair (an item = a run of a pair's iterations, as
     // equal as whole iterations allow): one round (measured on C2, one token: 96 x 2
@@ -861,17 +880,10 @@ int launch_grouped(hipStream_t st, FusedArgs& a, bool sg, bool sd) {
     size_t lds = (size_t) NT * lmax * XPAD * sizeof(float);
     if (lds < FG_PRE_BYTES) lds = FG_PRE_BYTES;
 
-    static int cached[2][2] = {{0, 0}, {0, 0}};   // resident workgroups per CU, by kernel variant, for the largest request seen
-    static size_t cached_lds[2][2] = {{0, 0}, {0, 0}};
-    int& per_cu = cached[sg][sd];
-    if (!per_cu || lds > cached_lds[sg][sd]) {
-        if (lds > 48 * 1024 && hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return -1;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds) != hipSuccess || per_cu < 1) {
-            per_cu = 0;
-            return -1;
-        }
-        cached_lds[sg][sd] = lds;
-    }
+    static Residency known[2][2];
+    Residency& kn = known[sg][sd];
+    const int per_cu = resident_workgroups((const void*) kern, kn, lds);
+    if (per_cu < 1) return -1;
     // The groups are formed on the device; the host sizes the items for the number it expects from a uniform routing:
     // the experts that receive a pair at all, plus the always-on experts' runs of NT tokens.  Four workgroups a CU are
     // resident, and items for about five were fastest (C2, 16 rows, 81 groups on 1024 workgroups, gate+up items a group
@@ -893,14 +905,7 @@ int launch_grouped(hipStream_t st, FusedArgs& a, bool sg, bool sd) {
     if (sg) {
         const size_t base = (lds + 15) & ~(size_t) 15;
         const size_t want = base + (size_t) NT * ((a.it_g + a.ntile_g - 1) / a.ntile_g) * (a.rpig / 2) * sizeof(float2);
-        static size_t ok_lds[2] = {0, 0}, bad_lds[2] = {~(size_t) 0, ~(size_t) 0};   // by sd: the largest request known to keep per_cu, the smallest known not to
-        bool fits = want <= ok_lds[sd];
-        if (!fits && want < bad_lds[sd] && want <= 48 * 1024) {
-            int n = 0;
-            fits = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 256, want) == hipSuccess && n >= per_cu;
-            if (fits) ok_lds[sd] = want;
-            else bad_lds[sd] = want;
-        }
+        const bool fits = want <= 48 * 1024 && resident_workgroups((const void*) kern, kn, want) >= per_cu;
         if (fits) {
             a.gu_off = (int) (base / sizeof(float));
             lds = want;

@@ -398,6 +398,30 @@ def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d
     st.close()
 
 
+# workgroups whose LDS, given out in pieces of 1280 bytes, fits a CU once less than 160 KB divided by its bytes says: 64 and 58 chunks with five waves a SIMD (32736
+# and 32128 bytes), 79 chunks in the kernel that groups pairs (54288 bytes).  A grid sized by the bytes would wait for workgroups that have not started.
+@pytest.mark.parametrize("fmt,k,d,ff,T", [(packs.MF_SEED4P4, 4, 4096, 704, 8), (packs.MF_SEED4, 4, 3712, 704, 8), (packs.MF_SEED4P4, 2, 2048, 5056, 12)])
+def test_step_grids_are_resident_at_once(fmt, k, d, ff, T):
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    rng = np.random.default_rng(d + ff)
+    st = moe.MoeStack(1, 8, k, d, ff, fmt=fmt, router=moe.ROUTE_SOFTMAX, max_rows=16)
+    backend.check(st.L.nslm_moe_fill_random(st.h, C.c_uint64(78), -22, C.c_float(0.035)), "nslm_moe_fill_random")
+    st.finalize()
+    dx, dio = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32))), moe.DevBuf(4 * T * d)
+    st.step(None, 0, dx.ptr, T, dio.ptr)
+    got = dio.to_array(np.float32, (T, d))
+    assert st.fused_error() == 0 and st.fused_steps() == 1
+    st.set_fused(0)
+    for t in range(0, T, 8):   # the separate launches' matvecs, eight rows at a time
+        n = min(8, T - t)
+        st.step(None, 0, dx.at(4 * t * d), n, dio.at(4 * t * d))
+    want = dio.to_array(np.float32, (T, d))
+    assert st.fused_steps() == 1 and np.abs(want).max() > 0 and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    dx.free(); dio.free()
+    st.close()
+
+
 def test_steps_issued_by_one_call_equal_single_steps():
     """nslm_moe_step_seq (n steps and the two timing events from one call into the C host) leaves what the same steps leave when
     issued one by one, and its events bracket them; nslm_mv_seq does the same for the dense matvec."""
