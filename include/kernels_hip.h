@@ -165,6 +165,12 @@ void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* w
 /* (ours: the same over D as BF16 bits, kc_mm_grouped_packed_bf16's) */
 void kc_moe_combine_bf16(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T);
 void kq4_moe_combine_bf16(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T);
+/* (the same; mark, 16-byte aligned: its four words become KC_BF16_MARK, + 1, + 2, + 3, so that a host can tell from device memory that it was these sums that ran
+ * last, whatever it has enqueued or captured since.  No four BF16 values widened to f32 have those bits.) */
+#define KC_BF16_MARK 0x42463136u
+void kc_moe_combine_bf16_mark(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T, uint32_t* mark);
+void kq4_moe_combine_bf16_mark(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T,
+                               uint32_t* mark);
 
 /* ---- expert slot table (engine/kernels_cuda.h:53-55, engine/kernels_moe.cu:2710-2722) ------------------------------ */
 void kc_cache_admit(kc_stream_t s, const CachePool* p, int sl, const int32_t* inds, int count, int flags);

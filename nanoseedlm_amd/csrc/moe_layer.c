@@ -29,13 +29,18 @@ struct NslmMoe {
     int32_t *ind, *perm, *ntiles;
     MmTile* tiles;
     int max_tiles;
-    int d16;                    /* the last step left the experts' outputs in D as BF16 bits */
     uint32_t* sync;             /* device: the fused decode kernel's barrier words */
     int fused;                  /* 1: steps of the softmax composition up to kc_moe_decode_max_rows() rows take kc_moe_decode;
                                    2: the same, and every such step is checked and redone by the separate launchers if it failed */
     int fallbacks;              /* checked steps that were redone */
     long fused_steps;           /* steps the persistent kernel took */
 };
+
+/* D holds a step's expert outputs [pair][d]: f32 words from its start, or - steps whose GEMMs take mostly full tiles - BF16 bits from D16_AT on, behind
+ * a mark that the combine writes.  Every f32 step writes over the mark (a pair has at least 8 columns), so D itself says in which form the last step that RAN
+ * left it: what was enqueued or captured last would not, once captured steps of both kinds are replayed. */
+#define D16_AT 256   /* bytes; behind them 2 bytes a value, of the 4 a value that D has: such a step has more than MMT_BN pairs */
+static uint16_t* d16_of(const NslmMoe* m) { return (uint16_t*) ((char*) m->D + D16_AT); }
 
 static uint64_t pad256(uint64_t n) { return (n + 255) & ~(uint64_t) 255; }
 
@@ -294,7 +299,6 @@ int nslm_moe_step_layer(NslmMoe* m, kc_stream_t s, int layer, const float* xn, i
                             c->d, m->logit, m->ind, m->wt, m->A, m->D, m->sync, shared, res, norm_w, norm_eps))
         return 1;
     m->fused_steps++;
-    m->d16 = 0;
     return kc_last_error() ? -1 : 0;
 }
 
@@ -323,7 +327,7 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
     const NslmMoeCfg* c = &m->c;
     if (!m->final || T < 1 || T > c->max_rows || layer < 0 || layer >= c->n_layer) return -1;
     const int E = c->n_exp, k = c->top_k, d = c->d, ff = c->ff, P = T * k;
-    m->d16 = 0;
+    int d16 = 0;   /* the experts' outputs are BF16 bits */
     const WSlice* gate = m->pool.tab + ((size_t) layer * 3 + 0) * E;
     const WSlice* up = m->pool.tab + ((size_t) layer * 3 + 1) * E;
     const WSlice* down = m->pool.tab + ((size_t) layer * 3 + 2) * E;
@@ -415,9 +419,9 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
                 kc_swiglu_pack(s, m->G, m->U, (uint16_t*) m->A, (size_t) P * ff);
             }
             /* the experts' outputs are BF16 values; as BF16 bits the combine reads half as much */
-            m->d16 = kc_mm_grouped_packed_bf16(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, (uint16_t*) m->D, d, 1, m->perm, m->tiles, m->ntiles,
+            d16 = kc_mm_grouped_packed_bf16(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, d16_of(m), d, 1, m->perm, m->tiles, m->ntiles,
                                             m->max_tiles, word) == 0;
-            if (!m->d16) kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles, m->max_tiles, word);
+            if (!d16) kc_mm_grouped_packed_rows(s, c->fmt, down, ff, d, (const uint16_t*) m->A, ff, m->D, d, 1, m->perm, m->tiles, m->ntiles, m->max_tiles, word);
         } else {
             kc_mm_grouped_dev(s, c->fmt, gate, d, ff, xn, d, m->G, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
             kc_mm_grouped_dev(s, c->fmt, up, d, ff, xn, d, m->U, ff, k, m->perm, m->tiles, m->ntiles, m->max_tiles, NULL);
@@ -426,10 +430,10 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
         }
     }
     if (c->router == NSLM_ROUTE_SOFTMAX) {
-        if (m->d16) kq4_moe_combine_bf16(s, d, k, (const uint16_t*) m->D, m->wt, NULL, m->zero, 0, io, T);
+        if (d16) kq4_moe_combine_bf16_mark(s, d, k, d16_of(m), m->wt, NULL, m->zero, 0, io, T, (uint32_t*) m->D);
         else kq4_moe_combine(s, d, k, m->D, m->wt, NULL, m->zero, 0, io, T);
     } else {
-        if (m->d16) kc_moe_combine_bf16(s, (const uint16_t*) m->D, m->wt, NULL, io, d, k, T);
+        if (d16) kc_moe_combine_bf16_mark(s, d16_of(m), m->wt, NULL, io, d, k, T, (uint32_t*) m->D);
         else kc_moe_combine(s, m->D, m->wt, NULL, io, d, k, T);
     }
     return kc_last_error() ? -1 : 0;
@@ -478,10 +482,13 @@ int nslm_moe_last_logits(NslmMoe* m, int T, float* logits) {
 }
 int nslm_moe_last_pairs(NslmMoe* m, int pairs, float* A, float* D) {
     const size_t n = (size_t) pairs * m->c.d;
-    if (nh_device_sync() || nh_memcpy_d2h(A, m->A, 4 * (size_t) pairs * m->c.ff)) return -1;
-    if (!m->d16) return nh_memcpy_d2h(D, m->D, 4 * n) ? -1 : 0;
+    uint32_t mark[4];
+    if (nh_device_sync() || nh_memcpy_d2h(A, m->A, 4 * (size_t) pairs * m->c.ff) || nh_memcpy_d2h(mark, m->D, sizeof mark)) return -1;
+    int d16 = 1;
+    for (uint32_t i = 0; i < 4; ++i) d16 &= mark[i] == KC_BF16_MARK + i;
+    if (!d16) return nh_memcpy_d2h(D, m->D, 4 * n) ? -1 : 0;
     /* BF16 bits: into the upper half of the caller's array, then widened from the front */
-    if (nh_memcpy_d2h((char*) D + 2 * n, m->D, 2 * n)) return -1;
+    if (nh_memcpy_d2h((char*) D + 2 * n, d16_of(m), 2 * n)) return -1;
     for (size_t i = 0; i < n; ++i) {
         uint16_t h;
         memcpy(&h, (char*) D + 2 * n + 2 * i, 2);

@@ -285,7 +285,8 @@ __device__ __forceinline__ typename DVec<V>::type load_d(const uint16_t* p) {
     return v;
 }
 template <int V, bool Q4, class D_>
-__global__ void __launch_bounds__(256) k_combine(const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k) {
+__global__ void __launch_bounds__(256) k_combine(const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, uint32_t* mark) {
+    if (sizeof(D_) == 2 && mark && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 4) mark[threadIdx.x] = KC_BF16_MARK + threadIdx.x;
     const int c = V * (int) (blockIdx.x * blockDim.x + threadIdx.x), t = (int) blockIdx.y;
     if (c >= d) return;
     typedef typename DVec<V>::type vec;
@@ -319,12 +320,12 @@ __global__ void __launch_bounds__(256) k_combine(const D_* D, const float* wt, c
     *(vec*) (io + at) = x;
 }
 template <bool Q4, class D_>
-void combine(hipStream_t st, const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, int T) {
+void combine(hipStream_t st, const D_* D, const float* wt, const float* sh, const float* sg, int sgld, float* io, int d, int k, int T, uint32_t* mark = nullptr) {
     constexpr int V = 4;
     if (d % V == 0 && (((uintptr_t) D | (uintptr_t) sh | (uintptr_t) io) & 15u) == 0)
-        hipLaunchKernelGGL((k_combine<V, Q4, D_>), dim3((unsigned) (d / V + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
+        hipLaunchKernelGGL((k_combine<V, Q4, D_>), dim3((unsigned) (d / V + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k, mark);
     else
-        hipLaunchKernelGGL((k_combine<1, Q4, D_>), dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k);
+        hipLaunchKernelGGL((k_combine<1, Q4, D_>), dim3((unsigned) (d + 255) / 256, (unsigned) T), dim3(256), 0, st, D, wt, sh, sg, sgld, io, d, k, mark);
 }
 __global__ void k_pack_input_bf16(const float* x, uint16_t* y, size_t n) {
     const size_t b = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -784,13 +785,20 @@ void kq4_moe_combine(kc_stream_t s, int d, int k, const float* D, const float* w
     if (T < 1) return;
     combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T);
 }
-void kc_moe_combine_bf16(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T) {
+void kc_moe_combine_bf16_mark(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T, uint32_t* mark) {
     if (T < 1) return;
-    combine<false>((hipStream_t) s, D, w, shared, nullptr, 0, x, d, k, T);
+    combine<false>((hipStream_t) s, D, w, shared, nullptr, 0, x, d, k, T, mark);
+}
+void kq4_moe_combine_bf16_mark(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T,
+                               uint32_t* mark) {
+    if (T < 1) return;
+    combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T, mark);
+}
+void kc_moe_combine_bf16(kc_stream_t s, const uint16_t* D, const float* w, const float* shared, float* x, int d, int k, int T) {
+    kc_moe_combine_bf16_mark(s, D, w, shared, x, d, k, T, nullptr);
 }
 void kq4_moe_combine_bf16(kc_stream_t s, int d, int k, const uint16_t* D, const float* wt, const float* sh, const float* sg, int sgld, float* out, int T) {
-    if (T < 1) return;
-    combine<true>((hipStream_t) s, D, wt, sh, sg, sgld, out, d, k, T);
+    kq4_moe_combine_bf16_mark(s, d, k, D, wt, sh, sg, sgld, out, T, nullptr);
 }
 void kc_pack_input_bf16(kc_stream_t s, const float* x, uint16_t* y, size_t n) {
     if (n < 8) return;

@@ -422,6 +422,44 @@ def test_step_grids_are_resident_at_once(fmt, k, d, ff, T):
     st.close()
 
 
+@pytest.mark.parametrize("router", [0, 1])
+def test_last_pairs_are_those_of_the_step_that_ran_last(router):
+    """A large step leaves the experts' outputs as BF16 bits, a small one as f32: nslm_moe_last_pairs gives the values of the one that ran last, whichever was
+    enqueued or captured last."""
+    from nanoseedlm_amd import backend, moe
+    rng = np.random.default_rng(31 + router)
+    E, k, d, ff, big, small = 4, 2, 256, 128, 300, 3
+    st = moe.MoeStack(1, E, k, d, ff, fmt=packs.MF_SEED4P4, router=router, max_rows=big, route_scale=2.5)
+    mk = lambda R, K: packs.seed4p4(rng, E, R, K, eb=-21)
+    st.set_layer(0, mk(ff, d), mk(ff, d), mk(d, ff), packs.f32_to_bf16_bits((rng.standard_normal((E, d)) * 0.05).astype(np.float32)),
+                 packs.f32_to_bf16_bits(np.zeros(E, dtype=np.float32)))
+    st.finalize()
+    s = moe.new_stream()
+    dx = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((big, d)).astype(np.float32)))
+    dio = moe.DevBuf.from_array(np.zeros((big, d), dtype=np.float32))
+    want = {}
+    for T in (big, small):
+        st.step(s, 0, dx.ptr, T, dio.ptr)
+        want[T] = st.last_pairs(T * k)[1]
+    # the experts' outputs of a token do not depend on the step: the two sizes' agree to BF16 (weights rounded to BF16 and not)
+    assert np.max(np.abs(want[big][:small * k] - want[small])) < 0.02 * np.max(np.abs(want[small])) > 0
+    for rep in range(3):
+        gb = st.graph_of_step(s, 0, dx.ptr, big, dio.ptr)
+        gs = st.graph_of_step(s, 0, dx.ptr, small, dio.ptr)
+        for T in (big, small, big, big, small):
+            st.launch(gb if T == big else gs, s)
+            assert _same(st.last_pairs(T * k)[1], want[T]), (rep, T)
+        st.launch(gb, s)
+        g3 = st.graph_of_step(s, 0, dx.ptr, small, dio.ptr)   # captured, not run
+        assert _same(st.last_pairs(big * k)[1], want[big]), rep
+        st.step(s, 0, dx.ptr, small, dio.ptr)
+        assert _same(st.last_pairs(small * k)[1], want[small]), rep
+        for g in (gb, gs, g3):
+            backend.host().nslm_graph_free(g)
+    dx.free(); dio.free()
+    st.close()
+
+
 def test_steps_issued_by_one_call_equal_single_steps():
     """nslm_moe_step_seq (n steps and the two timing events from one call into the C host) leaves what the same steps leave when
     issued one by one, and its events bracket them; nslm_mv_seq does the same for the dense matvec."""
