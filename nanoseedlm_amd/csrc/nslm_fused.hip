@@ -776,7 +776,7 @@ bool shape_of(int K, bool gateup, int* L, int* rpi, bool* shfl) {
 
 // Items per pair (or group) of a phase of `iters` iterations, `units` pairs, at most gmax workgroups.
 // The count that gives the busiest workgroup the least to do when every workgroup takes its items one after the
-// other (an item's set-up priced at a third of an iteration, unequal items at half an iteration: workgroups i, i + 256, ...
+// other (an item's set-up priced at `setup` sixths of an iteration, unequal items at half an iteration: workgroups i, i + 256, ...
 // share a CU, so the long items of a regular pattern meet on the same CUs); up to `slack` items more than the workgroups still
 // count as one round.
 int pick_one_round(int units, int iters, int gmax, int nmax, int slack = 0, int setup = 2) {
@@ -853,10 +853,13 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     // equal as whole iterations allow): one round (measured on C2, one token: 96 x 2
     // gate+up iterations and 98 x 1 down iterations a pair on 784 workgroups, 40.1 us; 96 unequal down items on 768
     // workgroups: 42.9; 8 tokens with 32 instead of 20 down items a pair: 144 against 131 us - a down item waits for its
-    // pair, and a second round of them waits behind the first).  More, shorter gate+up items by the CUs' load, for several tokens, had been ahead
-    // (by 1 .. 10 %) while a block's decode took a third longer; now they are 3 .. 5 % behind at 7 and 8 tokens of C2 and 3 % ahead at 6.
+    // pair, and a second round of them waits behind the first).
+    // A gate+up item's set-up - the slices, the first records, the arrival at the pair's counter - is priced at five sixths of an iteration: at a third, a pair's
+    // iterations went out as one item each wherever they did not divide evenly, in up to five rounds (us a layer at a third / at five sixths: 5 tokens of
+    // top-8, 2048 x 512 55.2 / 41.5, 3 of them 36.3 / 30.8; 5 of top-4, 1024 x 2048 57.1 / 41.6; 2 of top-4, 1536 x 1024, P = 3, 29.6 / 25.5; 1248
+    // steps of 1 .. 8 tokens: 0.73 to 1.01, four sixths and seven sixths within 0.4 % of five).
     const int gmax = (per_cu < 5 ? per_cu : 5) * cu_count(), P_ = a.T * a.kk;
-    a.ntile_g = pick_one_round(P_, a.it_g, gmax, FUSED_TILES);
+    a.ntile_g = pick_one_round(P_, a.it_g, gmax, FUSED_TILES, 0, 5);
     // (a down item's set-up - the wait for its pair, the staging of A - priced at two thirds of an iteration: at a third, six
     // tokens of C2 took two rounds of 49 two-iteration items a pair, 81.6 us, where one round of 26 takes 76.5)
     a.ntile_d = pick_one_round(P_, a.it_d, gmax, FUSED_TILES, 0, 4);

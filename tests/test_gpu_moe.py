@@ -398,6 +398,13 @@ def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d
     st.close()
 
 
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 512, (3, 5)), (4, 1024, 2048, (5,)), (4, 1536, 1024, (2,))])
+def test_per_pair_steps_of_uneven_items_give_the_separate_launches_bits(fmt, k, d, ff, rows):
+    """A pair's gate + up iterations in one round of items of unequal length (25, 42, 51 or 128 of 128, 256 or 205 iterations)."""
+    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+
+
 # workgroups whose LDS, given out in pieces of 1280 bytes, fits a CU once less than 160 KB divided by its bytes says: 64 and 58 chunks with five waves a SIMD (32736
 # and 32128 bytes), 79 chunks in the kernel that groups pairs (54288 bytes).  A grid sized by the bytes would wait for workgroups that have not started.
 @pytest.mark.parametrize("fmt,k,d,ff,T", [(packs.MF_SEED4P4, 4, 4096, 704, 8), (packs.MF_SEED4, 4, 3712, 704, 8), (packs.MF_SEED4P4, 2, 2048, 5056, 12)])
