@@ -830,22 +830,26 @@ template <int P>
 int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     a.gu_off = (int) (lds / sizeof(float));
     lds += GU_ROWS * sizeof(float2);
-    // Four waves a SIMD, or five, whose registers spill (76 bytes a lane) but which leave shorter items, 1280 workgroups for 1024.  Timed on 122 layers
-    // of 2 .. 8 tokens (us a layer, four / five waves): five where the step is large and the gate + up sums stay in a wave (8 tokens, E 128, top-8,
-    // 2048 x 768 86.0 / 81.9; 6 of top-8, 2048 x 1024 98.8 / 81.7; 5 of top-8, 2048 x 768 59.4 / 61.3), and, where both phases' sums go through
-    // LDS, whose barriers more workgroups cover, from less on (4 tokens of top-4, 2880 x 1408 93.1 / 83.2; 8, 1344 x 704 43.2 / 37.6;
-    // 4, 1344 x 704 26.3 / 29.4).  With the gate + up sums alone there it is four (8 tokens of top-4, 4096 x 512 82.7 / 131; 6 of top-2,
-    // 768 x 2048 31.1 / 36.4; P = 3, 8 of top-4, 2560 x 1024 94.0 / 97.2) but for the large steps of P = 4 whose rows are shorter than 64 chunks (8 of
-    // top-4, 3072 x 1024 122 / 112), and four for every small step (6 tokens of top-4, 1024 x 512 21.9 / 28.8).  The rule is 0.5 % off the
-    // faster of the two on average.
+    // Four waves a SIMD, or five, whose registers spill (up to 76 bytes a lane) but which leave shorter items, 1280 workgroups for 1024.  Timed on 142 layers of
+    // 2 .. 8 tokens, P = 4 where not said (us a layer, four / five waves).  Five where the step is large: from T pairs d ff = 90 Mi on where the gate + up
+    // sums stay in a wave (E 128, top-8, 2048 x 768: 6 tokens, 72 Mi, 65.9 / 71.3, 8 tokens, 96 Mi, 86.2 / 81.3; top-8, 2048 x 1024: 4, 64 Mi, 56.5 / 59.5, 6,
+    // 96 Mi, 94.6 / 81.4), from 22 Mi on where they go through LDS, whose barriers more workgroups cover (top-4, 2880 x 1408: 4, 62 Mi, 92.4 / 83.0; top-4,
+    // 1344 x 704: 6, 21.7 Mi, 32.7 / 38.4, 8, 29 Mi, 38.4 / 37.8; top-4, 1920 x 1152: 3, 25 Mi, 41.4 / 39.6; P = 3,
+    // top-4, 2560 x 1024: 4, 40 Mi, 59.7 / 54.2).  Where rows are so long that a CU's LDS
+    // holds only four workgroups of either, four if the down sums are by shuffles (top-8, 4096 x 512: 4 tokens 83.4 / 84.8); else the five waves' code is
+    // still level or ahead (P = 3, top-4, 4096 x 1408: 8 tokens 224 / 216).
+    // The rule is 0.5 % off the faster of the two on average.
     const long work = (long) a.T * a.kk * a.d * a.ff;
-    const long large = sg ? 48L << 20 : !sd ? 20L << 20 : P == 4 && a.Lg < 64 ? 40L << 20 : LONG_MAX;
-    const bool few = a.T == 1 || work < large;
-    void (*kern)(FusedArgs) = few ? (sg ? (sd ? k_moe_decode<P, true, true, 4> : k_moe_decode<P, true, false, 4>)
-                                        : (sd ? k_moe_decode<P, false, true, 4> : k_moe_decode<P, false, false, 4>))
-                                  : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
-                                        : (sd ? k_moe_decode<P, false, true, P == 4 ? 5 : 4> : k_moe_decode<P, false, false, 5>));
     static Residency known[2][2][2];
+    auto variant = [&](bool few) {
+        return few ? (sg ? (sd ? k_moe_decode<P, true, true, 4> : k_moe_decode<P, true, false, 4>)
+                         : (sd ? k_moe_decode<P, false, true, 4> : k_moe_decode<P, false, false, 4>))
+                   : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
+                         : (sd ? k_moe_decode<P, false, true, 5> : k_moe_decode<P, false, false, 5>));
+    };
+    bool few = a.T == 1 || work < (sg ? 90L : 22L) << 20;
+    if (!few && sd && resident_workgroups((const void*) variant(false), known[0][sg][sd], lds) < 5) few = true;
+    void (*kern)(FusedArgs) = variant(few);
     const int per_cu = resident_workgroups((const void*) kern, known[few][sg][sd], lds);
     if (per_cu < 1) return -1;
     // The grid must be resident at once (workgroups wait for each other's data): at most what the device holds, and no more than

@@ -371,8 +371,8 @@ def test_both_step_kernels_give_the_separate_launches_bits(fmt, E, k, d, ff):
         st.close()
 
 
-# the per-pair kernel with four and with five waves a SIMD: either side of T k d ff = 48 Mi with gate + up sums by shuffles (the down ones through LDS, by
-# shuffles), of 20 Mi with both through LDS, of 40 Mi with the gate + up ones there (P = 4)
+# the per-pair kernel over the sizes of T k d ff where it takes four or five waves a SIMD: gate + up sums by shuffles (the down ones through LDS, by
+# shuffles), both through LDS, the gate + up ones there
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
 @pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (3, 4, 5, 8)), (8, 2048, 512, (5, 6, 8)), (4, 1344, 704, (5, 6)), (4, 3072, 1024, (3, 4))])
 def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows):
@@ -402,6 +402,13 @@ def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d
 @pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 512, (3, 5)), (4, 1024, 2048, (5,)), (4, 1536, 1024, (2,))])
 def test_per_pair_steps_of_uneven_items_give_the_separate_launches_bits(fmt, k, d, ff, rows):
     """A pair's gate + up iterations in one round of items of unequal length (25, 42, 51 or 128 of 128, 256 or 205 iterations)."""
+    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+
+
+# either side of T k d ff = 90 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS; and above it where five workgroups do not fit a CU's LDS
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,))])
+def test_per_pair_steps_of_four_and_five_waves_give_the_separate_launches_bits(fmt, k, d, ff, rows):
     test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
 
 
