@@ -1001,13 +1001,17 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
         return fmt == MF_SEED4P4 ? launch_grouped<4, 2>((hipStream_t) s, a, sg, sd) : launch_grouped<3, 2>((hipStream_t) s, a, sg, sd);
     }
     // One workgroup per CU: ahead at one token everywhere, and at two to six where rows are long - 44 chunks or more, whose sums the other kernel takes through
-    // LDS with its waves' registers spilled or its workgroups few - and the step large.  (Timed on 28 layers in both formats, us a layer, a workgroup
-    // an item / a CU.  4 experts of 2880 x 2880, P = 3: 2 tokens 94.9 / 78.1, 3: 132.8 / 113.7, 4: 168 / 150, 5: 200 / 185; 8 of 3072 x 1024, P = 4: 2: 67.1 /
-    // 57.4, 6: 168 / 158; 8 of 4096 x 512: 6: 142 / 115; 4 of 2880 x 1408: 2: 53.8 / 48.6, 3: 69.2 / 68.5, 4: 83.2 / 88.6; 2 of 4096 x 512: 3: 30.5 / 33.4.
-    // Shorter rows: C2 2: 32.7 / 34.0, 3: 41.7 / 45.9; 8 of 1536 x 1536, P = 3: 2: 48.4 / 53.1, 3: 63.0 / 76.0; 4 of 2560 x 1024: 2: 36.0 / 37.5, though
-    // 4 of 1536 x 1024 2: 29.3 / 26.4.)
-    const long layer = (long) top_k * d * ff;
-    const bool by_cu = T == 1 || (a.Lg >= 44 && T <= 6 && layer >= (T == 2 ? 6L : T == 3 ? 12L : 16L) << 20);
+    // LDS with its waves' registers spilled or its workgroups few - and the step large.  Timed on 142 layers in both formats, us a layer, a workgroup an item (of
+    // four or five waves a SIMD, as launch_fused has it) / a CU; Mi: top_k d ff.
+    //   2 tokens, from 6 Mi on: top-2, 4096 x 1024, 8 Mi, 34.6 / 30.8; 4 of 2880 x 1408 54.2 / 48.7; 4 of 2880 x 2880, P = 3, 93.4 / 77.2; top-2, 3776 x 384, 2.8 Mi, 24.8 / 25.2
+    //   3, from 12 Mi on: 4 of 2880 x 1408, 15 Mi, 69.2 / 68.8; 4 of 2880 x 2880, P = 3, 133 / 113; 4 of 3648 x 1408, 20 Mi, 79.1 / 80.9; top-2, 3136 x 1216, 7 Mi, 42.3 / 43.6
+    //   4 to 6, from 22 Mi on: 4 tokens, 8 of 3072 x 1024, 24 Mi, 115 / 108; 4 of 2880 x 2880, P = 3, 167 / 149; 4 of 3648 x 1408 98.3 / 106; 4 of 3072 x 1536, 18 Mi,
+    //      93.8 / 104; 6 tokens, 8 of 2880 x 1088, 24 Mi, 171 / 164; 4 of 3072 x 1536 132 / 154; but from 16 Mi where rows are so long that a CU's LDS holds four workgroups
+    //      of the other kernel (8 of 4096 x 512: 4 tokens 83.4 / 78.9, 6 135 / 114), and not for 6 tokens from 30 Mi on (4 of 2880 x 2880, P = 3, 238 / 245)
+    // Rows of 36 to 42 chunks, 7 to 36 Mi: 2 tokens 0.88 to 1.08 of the other kernel's time, 3 tokens 0.81 to 1.18, 4 and more 0.94 to 1.36; shorter rows: C2 2: 32.5 / 34.0,
+    // 3: 41.6 / 45.9; 4 of 1536 x 1024 2: 25.4 / 25.9.
+    const long layer = (long) top_k * d * ff, large = (T == 2 ? 6L : T == 3 ? 12L : a.Lg > 60 ? 16L : 22L) << 20;
+    const bool by_cu = T == 1 || (a.Lg >= 44 && T <= 6 && layer >= large && !(T == 6 && layer >= 30L << 20));
     if ((g_kernel_choice == 2 || (g_kernel_choice == 0 && by_cu)) && launch_moe_decode_cu((hipStream_t) s, a, fmt == MF_SEED4P4 ? 4 : 3, sd) == 0) return 0;
     const int kmax = d > ff ? d : ff;
     size_t lds = (size_t) (kmax / 64) * XPAD * sizeof(float);

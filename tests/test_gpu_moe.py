@@ -405,6 +405,14 @@ def test_per_pair_steps_of_uneven_items_give_the_separate_launches_bits(fmt, k, 
     test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
 
 
+# either side of the lines between the kernel of a workgroup an item and the one of a workgroup a CU: rows of 42 and 45 chunks; k d ff = 22 Mi and, at 6 rows, 30 Mi
+# (2880 x 1984, 2112 and 2752); 16 Mi with rows of 64 chunks
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("k,d,ff,rows", [(4, 2688, 2112, (4,)), (4, 2880, 1984, (4, 5)), (4, 2880, 2112, (4, 5, 6)), (4, 2880, 2752, (6,)), (4, 4096, 1024, (4, 6, 7))])
+def test_steps_of_long_rows_by_either_kernel_give_the_separate_launches_bits(fmt, k, d, ff, rows):
+    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+
+
 # either side of T k d ff = 90 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS; and above it where five workgroups do not fit a CU's LDS
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
 @pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,))])
