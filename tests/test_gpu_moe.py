@@ -482,6 +482,66 @@ def test_last_pairs_are_those_of_the_step_that_ran_last(router):
     st.close()
 
 
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("router", [0, 1])
+def test_large_step_and_a_small_one_behind_it(oracle, router, fmt):
+    """600 rows of top-2 on 8 experts: 150 pairs an expert, so that the host groups by many workgroups, the down GEMM leaves BF16 bits and the combine reads
+    them.  Stage by stage: the selection on the GPU's own logits, sampled pairs against the oracle, the sums bit for bit against the f32 combine of the outputs that
+    last_pairs returns.  Then a small step on the same stack, and the large one again.  d = 320: a last row group of 64 of 128."""
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    L = backend.hip()
+    rng = np.random.default_rng(40 + 2 * router + fmt)
+    E, k, d, ff, big = 8, 2, 320, 192, 600
+    mk = packs.seed4p4 if fmt == packs.MF_SEED4P4 else packs.seed4
+    st = moe.MoeStack(1, E, k, d, ff, fmt=fmt, router=router, max_rows=big, route_scale=2.5)
+    gate, up, down = mk(rng, E, ff, d, eb=-21), mk(rng, E, ff, d, eb=-21), mk(rng, E, d, ff, eb=-20)
+    rw = packs.f32_to_bf16_bits((rng.standard_normal((E, d)) * 0.05).astype(np.float32))
+    rb = packs.f32_to_bf16_bits((rng.standard_normal(E) * 0.01).astype(np.float32)) if router else None
+    st.set_layer(0, gate, up, down, rw, rb)
+    st.finalize()
+    r = packs.round_bf16
+    xn, x0 = r(rng.standard_normal((big, d)).astype(np.float32)), r(rng.standard_normal((big, d)).astype(np.float32))
+    dx = moe.DevBuf.from_array(xn)
+    seen = {}
+    for T in (big, 6, big, 40, big):   # 40 rows: the batched launches with f32 outputs
+        dio = moe.DevBuf.from_array(x0[:T])
+        st.step(None, 0, dx.ptr, T, dio.ptr)
+        out, (ind, wt), (A, D) = dio.to_array(np.float32, (T, d)), st.last_routing(T), st.last_pairs(T * k)
+        if router == 0:
+            check_routing_on_gpu_logits(oracle, st, T, k, xn[:T], rw, ind, wt)
+        else:
+            oi = oracle.route_sigmoid(rw, rb, xn[:T], k, d // 2, 2.5)[2]
+            assert np.mean([len(set(ind[t]) & set(oi[t])) / k for t in range(T)]) >= 0.98
+        assert np.array_equal(D, r(D))
+        # sampled pairs: D against the oracle's product with the A that the GPU made (one BF16 unit and f32 sums of 192 products), both against the oracle's own
+        gemm = T > 8
+        a = packs.bf16_bits_to_f32(A.view(np.uint16).reshape(-1)[:T * k * ff].reshape(T * k, ff)) if gemm else A
+        for p in sorted({0, 1, T * k - 1, *rng.integers(0, T * k, 24).tolist()}):
+            e = int(ind[p // k, p % k])
+            wd = oracle.rows_f32(fmt, slice_of(oracle, down, e), d, ff)
+            wd = (r(wd) if gemm else wd).astype(np.float64)
+            ref, mag = wd @ a[p].astype(np.float64), np.abs(wd) @ np.abs(a[p]).astype(np.float64)
+            assert np.all(np.abs(D[p] - ref) <= np.abs(ref) / 128 + 2e-6 * mag), (T, p)
+            want = expert_ref(oracle, gate, up, down, e, xn[p // k], gemm=gemm)
+            assert np.max(np.abs(D[p] - want)) < 1e-2 * np.max(np.abs(want)), (T, p)
+        # the sums, of the same outputs in f32
+        dD, dw, dz, dy = moe.DevBuf.from_array(D), moe.DevBuf.from_array(wt), moe.DevBuf.from_array(np.zeros(T, dtype=np.float32)), moe.DevBuf.from_array(x0[:T])
+        if router == 0:
+            L.kq4_moe_combine(None, d, k, dD.ptr, dw.ptr, None, dz.ptr, 0, dy.ptr, T)
+        else:
+            L.kc_moe_combine(None, dD.ptr, dw.ptr, None, dy.ptr, d, k, T)
+        moe.device_sync()
+        assert np.array_equal(out.view(np.uint32), dy.to_array(np.uint32, (T, d))), T
+        if T in seen:
+            assert _same(out, seen[T][0]) and _same(D, seen[T][1])
+        seen[T] = (out, D)
+        for b in (dio, dD, dw, dz, dy):
+            b.free()
+    dx.free()
+    st.close()
+
+
 def test_steps_issued_by_one_call_equal_single_steps():
     """nslm_moe_step_seq (n steps and the two timing events from one call into the C host) leaves what the same steps leave when
     issued one by one, and its events bracket them; nslm_mv_seq does the same for the dense matvec."""
