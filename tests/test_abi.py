@@ -66,3 +66,15 @@ def test_missing_library_fails_loudly(libs, monkeypatch):
     monkeypatch.setattr(libs, "HIP_SO", "/nonexistent/libnslm_hip.so")
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         libs.hip()
+
+
+def test_device_code_keeps_subnormals_whatever_the_extra_flags():
+    """The decode of the seed formats reads integers as the bits of subnormal f32: EXTRA flags that flush those come before the flag that keeps them."""
+    import subprocess
+    out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "nanoseedlm_amd", "csrc"), "EXTRA=-fgpu-flush-denormals-to-zero", "libs"],
+                         check=True, capture_output=True, text=True).stdout
+    compiles = [l.split() for l in out.splitlines() if " -c " in l and ".hip" in l]
+    assert len(compiles) >= 9
+    for words in compiles:
+        flags = [w for w in words if w.endswith("gpu-flush-denormals-to-zero")]
+        assert len(flags) == 2 and flags[-1] == "-fno-gpu-flush-denormals-to-zero", words
