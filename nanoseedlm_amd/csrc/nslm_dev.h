@@ -62,7 +62,7 @@ __device__ __forceinline__ void store_y(float* yo, float s, int add, int f32out)
 // g(s) = the 32 stream bits that follow seed s: bit k = top bit of state k+1.  g is linear over GF(2), so
 // g(s) = lo[s & 0xFF] ^ hi[s >> 8] with two 256-entry tables, built here at compile time from the LFSR definition
 // (taps 0, 1, 3, 12; shift right; feedback into bit 15).  The P = 3 format reads the low 24 bits of the same table.
-struct StreamBasis {
+struct alignas(16) StreamBasis {
     uint32_t v[512];
 };
 constexpr uint32_t stream32_of(uint32_t s) {
@@ -108,7 +108,7 @@ __device__ __forceinline__ void load_tables(uint32_t* tab) {
 __device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
 template <int N>
 __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void to_lds16(const void* src, uint8_t* dst) {   // dst: the wave's base, lane l lands at dst + 16 l
+__device__ __forceinline__ void to_lds16(const void* src, uint8_t* dst) {   // dst: the wave's base, lane l lands at dst + 16 l; both 16-byte aligned
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 16, 0, 0);
 }
 __device__ __forceinline__ uint32_t stream_of(const uint32_t* tab, uint32_t seed16) {
@@ -189,10 +189,10 @@ __device__ __forceinline__ void isum_p3(uint32_t up, uint32_t g, uint32_t q01, u
 // as one token's products about 68 (P = 4 by eleven sums of nibble columns, a convert and a multiply-add each: 78; P = 3 by windows paired
 // for dot products: 76).  us a pass, before and after: layer step of 64 tokens (E 128, top-8, d 2048, ff 768, P = 4) 239 -> 200, of 8 tokens
 // 95 -> 86.5, of one 19.7 -> 18.3; of 3 tokens, E 64, top-4, d 2880, ff 2880, P = 3, 147 -> 134; 2880 x 2880, P = 3, 6 tokens 10.9 -> 10.2.
-struct SumTab4 {
+struct alignas(16) SumTab4 {
     uint32_t v[256];
 };
-struct SumTab3 {
+struct alignas(16) SumTab3 {
     uint32_t v[512];
 };
 constexpr int sext4(uint32_t n) { return (int) (n & 15u) - (int) ((n & 8u) << 1); }
@@ -215,6 +215,7 @@ constexpr SumTab3 make_sumtab3() {   // entry { q1, q2 }: 40 - H(0..3), 80 + H(0
     }
     return t;
 }
+static_assert(alignof(StreamBasis) >= 16 && alignof(SumTab4) >= 16 && alignof(SumTab3) >= 16, "to_lds16 reads 16 bytes a lane");
 __device__ const SumTab4 kSumTab4 = make_sumtab4();
 __device__ const SumTab3 kSumTab3 = make_sumtab3();
 template <int P>
