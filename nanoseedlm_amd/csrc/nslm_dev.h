@@ -341,7 +341,9 @@ __device__ __forceinline__ void sums_of(uint32_t up, uint32_t g, const SumCoefs&
         hook(3);
     }
 }
-// isum_c 2^-22 (exact): what a matvec multiplies with the activations; a row's sum is then multiplied by R32 2^22
+// isum_c 2^-22 (exact): what a matvec multiplies with the activations; a row's sum is then multiplied by R32 2^22.  So a sum of blocks is kept 2^-22 low:
+// where base + code lie below about -120 it is subnormal, and an addition to it rounds by up to 2^-150, 2^-143 of the row's sum (at -126, the lowest, about one
+// part in 2^18 of a block's; bases of real packs are about -22).  Kept 22 binades higher it would leave the f32 range at the other end.
 #define NSLM_SUM_R32 (NSLM_R32 * 4194304.0f)
 template <int P>
 __device__ __forceinline__ void sums_float(const uint32_t (&y)[8], uint32_t k, float (&f)[8]) {

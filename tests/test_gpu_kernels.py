@@ -364,6 +364,26 @@ def test_one_hot_activations_read_the_oracles_weights(be, oracle, fmt, call, T):
             assert np.array_equal(got[t], want[63 - t % 64]), (eb, t)
 
 
+@pytest.mark.parametrize("T", [1, 3, 8])
+@pytest.mark.parametrize("K", [512, 2880])
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+def test_mv_at_the_lowest_exponents(be, oracle, fmt, K, T):
+    """A base of -126, the lowest whose 2^(base + code) are normal f32: the sums of blocks, which are kept 2^-22 low, are subnormal there.  Each addition of a
+    block then rounds by at most 2^-150, which is 2^-143 once the row's sum is multiplied by 2^22 / 32767."""
+    rng = np.random.default_rng(K + T + fmt)
+    p = packs.seed4p4(rng, 1, 40, K, eb=-22) if fmt == packs.MF_SEED4P4 else packs.seed4(rng, 1, 40, K, eb=-22)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    ref, mag = ref_mv(oracle, p, 0, x)
+    p["eb"] = np.array([-126], dtype=np.int32)
+    be.kt().kt_store_f32(1)
+    try:
+        y = be.kt_mv(p, x)
+    finally:
+        be.kt().kt_store_f32(0)
+    scale = 2.0 ** -104
+    assert np.abs(y).max() > 0 and np.all(np.abs(y - ref * scale) <= F32B * mag * scale + K / 8 * 2.0 ** -143)
+
+
 # f32 activations at token counts that the first-generation kernel had (seeds: from 200 tokens; BF16: at 130): the last token tile partial, one row past a tile
 @pytest.mark.parametrize("T,R", [(130, 16385), (1000, 2881)])
 @pytest.mark.parametrize("fmt", ALL_FMT)
