@@ -830,15 +830,16 @@ template <int P>
 int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     a.gu_off = (int) (lds / sizeof(float));
     lds += GU_ROWS * sizeof(float2);
-    // Four waves a SIMD, or five, whose registers spill (up to 76 bytes a lane) but which leave shorter items, 1280 workgroups for 1024.  Timed on 142 layers of
-    // 2 .. 8 tokens, P = 4 where not said (us a layer, four / five waves).  Five where the step is large: from T pairs d ff = 90 Mi on where the gate + up
-    // sums stay in a wave (E 128, top-8, 2048 x 768: 6 tokens, 72 Mi, 65.9 / 71.3, 8 tokens, 96 Mi, 86.2 / 81.3; top-8, 2048 x 1024: 4, 64 Mi, 56.5 / 59.5, 6,
-    // 96 Mi, 94.6 / 81.4), from 22 Mi on where they go through LDS, whose barriers more workgroups cover (top-4, 2880 x 1408: 4, 62 Mi, 92.4 / 83.0; top-4,
-    // 1344 x 704: 6, 21.7 Mi, 32.7 / 38.4, 8, 29 Mi, 38.4 / 37.8; top-4, 1920 x 1152: 3, 25 Mi, 41.4 / 39.6; P = 3,
-    // top-4, 2560 x 1024: 4, 40 Mi, 59.7 / 54.2).  Where rows are so long that a CU's LDS
-    // holds only four workgroups of either, four if the down sums are by shuffles (top-8, 4096 x 512: 4 tokens 83.4 / 84.8); else the five waves' code is
-    // still level or ahead (P = 3, top-4, 4096 x 1408: 8 tokens 224 / 216).
-    // The rule is 0.5 % off the faster of the two on average.
+    // Four waves a SIMD, or five, whose registers spill (up to 76 bytes a lane) but which leave shorter items, 1280 workgroups for 1024: five where the
+    // step is large, by T pairs d ff.  Timed on 240 layers of 2 .. 8 tokens in both formats, each step both ways (us a layer, four / five waves, P = 4):
+    //   gate + up sums in a wave, from 80 Mi on: top-8, 2048 x 768: 6 tokens, 72 Mi, 65.9 / 71.3, 8, 96 Mi, 86.2 / 81.3; top-8, 2048 x 1024: 5, 80 Mi, 71.0 / 68.2
+    //   through LDS, whose barriers more workgroups cover:
+    //     from 22 Mi on: top-2, 2240 x 2688: 3, 34 Mi, 58.2 / 54.9; top-4, 1216 x 1024: 8, 38 Mi, 49.6 / 47.0 (but 7, 33 Mi, 43.5 / 45.7); top-4, 1344 x 704: 6, 21.7 Mi, 32.7 / 38.4, 8, 29 Mi, 38.4 / 37.8
+    //     from 32 Mi where the down sums stay in a wave: top-4, 1280 x 2048: 3, 30 Mi, 41.4 / 43.7; top-8, 1280 x 512: 8, 40 Mi, 49.7 / 47.0 (but 7, 35 Mi, 43.4 / 46.5)
+    //     from 16 Mi on rows of 44 chunks or more, of which four fill at most 250 of a workgroup's lanes: top-2, 2816 x 448: 6, 14 Mi, 35.0 / 37.1, 8, 19 Mi, 44.1 / 38.8;
+    //     top-2, 3200 x 640, P = 3: 5, 20 Mi, 46.1 / 40.2
+    // Where rows are so long that a CU's LDS holds only four workgroups of either, four if the down sums are by shuffles (top-8, 4096 x 512: 4 tokens 83.4 / 84.8);
+    // else the five waves' code is still level or ahead (P = 3, top-4, 4096 x 1408: 8 tokens 224 / 216).  The rule is 0.5 % off the faster of the two on average.
     const long work = (long) a.T * a.kk * a.d * a.ff;
     static Residency known[2][2][2];
     auto variant = [&](bool few) {
@@ -847,7 +848,7 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
                    : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
                          : (sd ? k_moe_decode<P, false, true, 5> : k_moe_decode<P, false, false, 5>));
     };
-    bool few = a.T == 1 || work < (sg ? 90L : 22L) << 20;
+    bool few = a.T == 1 || work < (sg ? 80L : a.Lg >= 44 ? 16L : sd ? 32L : 22L) << 20;
     if (!few && sd && resident_workgroups((const void*) variant(false), known[0][sg][sd], lds) < 5) few = true;
     void (*kern)(FusedArgs) = variant(few);
     const int per_cu = resident_workgroups((const void*) kern, known[few][sg][sd], lds);
@@ -1000,18 +1001,21 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
         if (!sg) return -1;
         return fmt == MF_SEED4P4 ? launch_grouped<4, 2>((hipStream_t) s, a, sg, sd) : launch_grouped<3, 2>((hipStream_t) s, a, sg, sd);
     }
-    // One workgroup per CU: ahead at one token everywhere, and at two to six where rows are long - 44 chunks or more, whose sums the other kernel takes through
-    // LDS with its waves' registers spilled or its workgroups few - and the step large.  Timed on 142 layers in both formats, us a layer, a workgroup an item (of
-    // four or five waves a SIMD, as launch_fused has it) / a CU; Mi: top_k d ff.
-    //   2 tokens, from 6 Mi on: top-2, 4096 x 1024, 8 Mi, 34.6 / 30.8; 4 of 2880 x 1408 54.2 / 48.7; 4 of 2880 x 2880, P = 3, 93.4 / 77.2; top-2, 3776 x 384, 2.8 Mi, 24.8 / 25.2
-    //   3, from 12 Mi on: 4 of 2880 x 1408, 15 Mi, 69.2 / 68.8; 4 of 2880 x 2880, P = 3, 133 / 113; 4 of 3648 x 1408, 20 Mi, 79.1 / 80.9; top-2, 3136 x 1216, 7 Mi, 42.3 / 43.6
-    //   4 to 6, from 22 Mi on: 4 tokens, 8 of 3072 x 1024, 24 Mi, 115 / 108; 4 of 2880 x 2880, P = 3, 167 / 149; 4 of 3648 x 1408 98.3 / 106; 4 of 3072 x 1536, 18 Mi,
-    //      93.8 / 104; 6 tokens, 8 of 2880 x 1088, 24 Mi, 171 / 164; 4 of 3072 x 1536 132 / 154; but from 16 Mi where rows are so long that a CU's LDS holds four workgroups
-    //      of the other kernel (8 of 4096 x 512: 4 tokens 83.4 / 78.9, 6 135 / 114), and not for 6 tokens from 30 Mi on (4 of 2880 x 2880, P = 3, 238 / 245)
-    // Rows of 36 to 42 chunks, 7 to 36 Mi: 2 tokens 0.88 to 1.08 of the other kernel's time, 3 tokens 0.81 to 1.18, 4 and more 0.94 to 1.36; shorter rows: C2 2: 32.5 / 34.0,
-    // 3: 41.6 / 45.9; 4 of 1536 x 1024 2: 25.4 / 25.9.
-    const long layer = (long) top_k * d * ff, large = (T == 2 ? 6L : T == 3 ? 12L : a.Lg > 60 ? 16L : 22L) << 20;
-    const bool by_cu = T == 1 || (a.Lg >= 44 && T <= 6 && layer >= large && !(T == 6 && layer >= 30L << 20));
+    // One workgroup per CU: ahead at one token everywhere, and at two to six where rows are 44 chunks or longer, whose sums the other kernel takes through LDS,
+    // and the step large.  Timed on 240 layers in both formats, us a layer, a workgroup an item (the better of its two) / a CU; Mi: top_k d ff.
+    //   2 tokens, from 3 Mi on (132 steps, 0.74 to 1.04 of the other kernel's time, 0.92 on average): 4 of 2816 x 320, 3.4 Mi, 27.3 / 24.4; 2 of 3072 x 1088 36.3 / 30.3; 4 of
+    //      2880 x 2880 92.5 / 77.8; 2 of 2816 x 448, 2.4 Mi, 23.8 / 24.0
+    //   3 tokens, from 12 Mi on (0.95): 4 of 2880 x 1920, 21 Mi, 94.8 / 81.8; 4 of 2880 x 2880, P = 3, 132 / 113; 8 of 3456 x 448, 12 Mi, 57.8 / 58.2; 2 of 3072 x 1088, 6.4 Mi, 40.7 / 41.1
+    //   4 and more: where the other kernel is short of lanes - of rows of up to 51 chunks four go to an iteration, which leaves it 176 to 204 of 256 - from 28 Mi on, at 4 tokens and up to 47
+    //      chunks from 20 Mi: 4 tokens, 4 of 2880 x 1920 110 / 106, of 2880 x 2880 162 / 147, 8 of 3200 x 1536 174 / 164, 4 of 3072 x 2176, 26 Mi, 127 / 128; 5 tokens, 4 of
+    //      2880 x 2880 194 / 182, 8 of 3200 x 1536 208 / 202; but 4 tokens, 8 of 3520 x 896 114 / 127; 6 tokens, 4 of 2880 x 1920 155 / 154.
+    //      And, up to 6 tokens, from 12 Mi on where a CU's LDS holds only four of its workgroups, rows of 62 chunks or more: 8 of 4096 x 512 4 tokens 83.4 / 78.9, 6 135 / 114
+    // Shorter rows: C2 2 tokens 32.5 / 34.0, 3: 41.6 / 45.9; 4 of 2176 x 2816 2: 67.2 / 61.0, 3: 93.6 / 86.8, 4: 114 / 113, but 8 of 1536 x 2688 2: 73.5 / 73.5; 4 of 1536 x 1024 25.4 / 25.9.
+    const long layer = (long) top_k * d * ff;
+    const bool by_cu = T == 1 || (a.Lg >= 44 && (T == 2   ? layer >= 3L << 20
+                                                 : T == 3 ? layer >= 12L << 20
+                                                 : T <= 6 && a.Lg >= 62 ? layer >= 12L << 20
+                                                                        : T <= 5 && a.Lg < 52 && layer >= (T == 4 && a.Lg < 48 ? 20L : 28L) << 20));
     if ((g_kernel_choice == 2 || (g_kernel_choice == 0 && by_cu)) && launch_moe_decode_cu((hipStream_t) s, a, fmt == MF_SEED4P4 ? 4 : 3, sd) == 0) return 0;
     const int kmax = d > ff ? d : ff;
     size_t lds = (size_t) (kmax / 64) * XPAD * sizeof(float);

@@ -376,48 +376,61 @@ def test_both_step_kernels_give_the_separate_launches_bits(fmt, E, k, d, ff):
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
 @pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (3, 4, 5, 8)), (8, 2048, 512, (5, 6, 8)), (4, 1344, 704, (5, 6)), (4, 3072, 1024, (3, 4))])
 def test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows):
+    steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 1)
+
+
+def steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, kernel):
+    """kernel: the step kernel that the steps are forced to (kc_moe_decode_kernel), 0: the library's choice."""
     import ctypes as C
     from nanoseedlm_amd import backend, moe
     rng = np.random.default_rng(d + ff + fmt)
     st = moe.MoeStack(1, 16, k, d, ff, fmt=fmt, router=moe.ROUTE_SOFTMAX, max_rows=8)
     backend.check(st.L.nslm_moe_fill_random(st.h, C.c_uint64(77), -22, C.c_float(0.035)), "nslm_moe_fill_random")
     st.finalize()
-    for T in rows:
-        dx = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32)))
-        outs = []
-        for fused in (0, 1):
-            st.set_fused(fused)
-            before = st.fused_steps()
-            dio = moe.DevBuf.from_array(np.zeros((T, d), dtype=np.float32))
-            st.step(None, 0, dx.ptr, T, dio.ptr)
-            outs.append(dio.to_array(np.float32, (T, d)))
-            dio.free()
-            assert st.fused_error() == 0 and st.fused_steps() == before + fused, (T, fused)
-        dx.free()
-        assert np.abs(outs[0]).max() > 0 and np.array_equal(outs[1].view(np.uint32), outs[0].view(np.uint32)), T
-    st.close()
+    backend.hip().kc_moe_decode_kernel(kernel)
+    try:
+        for T in rows:
+            dx = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, d)).astype(np.float32)))
+            outs = []
+            for fused in (0, 1):
+                st.set_fused(fused)
+                before = st.fused_steps()
+                dio = moe.DevBuf.from_array(np.zeros((T, d), dtype=np.float32))
+                st.step(None, 0, dx.ptr, T, dio.ptr)
+                outs.append(dio.to_array(np.float32, (T, d)))
+                dio.free()
+                assert st.fused_error() == 0 and st.fused_steps() == before + fused, (T, fused)
+            dx.free()
+            assert np.abs(outs[0]).max() > 0 and np.array_equal(outs[1].view(np.uint32), outs[0].view(np.uint32)), T
+    finally:
+        backend.hip().kc_moe_decode_kernel(0)
+        st.close()
 
 
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
 @pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 512, (3, 5)), (4, 1024, 2048, (5,)), (4, 1536, 1024, (2,))])
 def test_per_pair_steps_of_uneven_items_give_the_separate_launches_bits(fmt, k, d, ff, rows):
     """A pair's gate + up iterations in one round of items of unequal length (25, 42, 51 or 128 of 128, 256 or 205 iterations)."""
-    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+    steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 1)
 
 
-# either side of the lines between the kernel of a workgroup an item and the one of a workgroup a CU: rows of 42 and 45 chunks; k d ff = 22 Mi and, at 6 rows, 30 Mi
-# (2880 x 1984, 2112 and 2752); 16 Mi with rows of 64 chunks
+# either side of the lines between the kernel of a workgroup an item and the one of a workgroup a CU, and sizes between: rows of 42, 45, 48 and 64 chunks; k d ff = 3 Mi
+# (2 rows: 2880 x 256 and 320), 12 Mi (3 rows: 2880 x 1088 and 1152; 64 chunks: 4096 x 704 and 768), 20 Mi (4 rows: 2880 x 1792 and 1856) and 28 Mi (5 rows: 2880 x 2496 and 2560;
+# 51 chunks: 3264 x 2240 and 2304)
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
-@pytest.mark.parametrize("k,d,ff,rows", [(4, 2688, 2112, (4,)), (4, 2880, 1984, (4, 5)), (4, 2880, 2112, (4, 5, 6)), (4, 2880, 2752, (6,)), (4, 4096, 1024, (4, 6, 7))])
+@pytest.mark.parametrize("k,d,ff,rows", [(4, 2688, 2112, (4,)), (4, 2880, 1984, (4, 5)), (4, 2880, 2112, (4, 5, 6)), (4, 2880, 2752, (6,)), (4, 4096, 1024, (4, 6, 7)),
+                                         (4, 2880, 256, (2,)), (4, 2880, 320, (2,)), (4, 2880, 1088, (3,)), (4, 2880, 1152, (3,)), (4, 4096, 704, (4, 5)), (4, 4096, 768, (4, 5, 6)),
+                                         (4, 2880, 1792, (4,)), (4, 2880, 1856, (4,)), (4, 2880, 2496, (5,)), (4, 2880, 2560, (5,)), (4, 3072, 2176, (4, 5)), (4, 3264, 2240, (4, 5)), (4, 3264, 2304, (4, 5))])
 def test_steps_of_long_rows_by_either_kernel_give_the_separate_launches_bits(fmt, k, d, ff, rows):
-    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+    steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 0)
 
 
-# either side of T k d ff = 90 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS; and above it where five workgroups do not fit a CU's LDS
+# either side of T k d ff = 80 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS, of 32 Mi with the down ones by shuffles, of 16 Mi with rows of 44 chunks; and
+# above it where five workgroups do not fit a CU's LDS
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
-@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,))])
+@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,)), (8, 2048, 1024, (4, 5)), (4, 1280, 2048, (3, 4)), (2, 2816, 448, (6, 7))])
 def test_per_pair_steps_of_four_and_five_waves_give_the_separate_launches_bits(fmt, k, d, ff, rows):
-    test_per_pair_steps_of_either_size_give_the_separate_launches_bits(fmt, k, d, ff, rows)
+    steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 1)
 
 
 # workgroups whose LDS, given out in pieces of 1280 bytes, fits a CU once less than 160 KB divided by its bytes says: 64 and 58 chunks with five waves a SIMD (32736
