@@ -37,9 +37,9 @@ struct NslmMoe {
 };
 
 /* D holds a step's expert outputs [pair][d]: f32 words from its start, or - steps whose GEMMs take mostly full tiles - BF16 bits from D16_AT on, behind
- * a mark that the combine writes.  Every f32 step writes over the mark (a pair has at least 8 columns), so D itself says in which form the last step that RAN
- * left it: what was enqueued or captured last would not, once captured steps of both kinds are replayed. */
-#define D16_AT 256   /* bytes; behind them 2 bytes a value, of the 4 a value that D has: such a step has more than MMT_BN pairs */
+ * a mark that the combine writes.  Every f32 step writes over the mark (a pair has at least 8 columns), so D itself says in
+ * which form the last step that RAN left it: what was enqueued or captured last would not, once captured steps of both kinds are replayed. */
+#define D16_AT 256   /* bytes; behind them 2 bytes a value, of the 4 a value that D has: such a step has more than 32 pairs of 8 columns or more */
 static uint16_t* d16_of(const NslmMoe* m) { return (uint16_t*) ((char*) m->D + D16_AT); }
 
 static uint64_t pad256(uint64_t n) { return (n + 255) & ~(uint64_t) 255; }
@@ -363,7 +363,7 @@ int nslm_moe_step(NslmMoe* m, kc_stream_t s, int layer, const float* xn, int T, 
             /* The batched path: the logits by the decode path's row sums over the input rounded to BF16, as the GEMM
                multiplies it (a 128-row GEMM is two workgroups: 16 us where this takes 5), the BF16 view of xn that the
                three GEMMs read made by the same launch;
-               then routing and grouping in one launch.  Shapes the folded launches do not take go the reference's way
+               then routing and grouping (in one launch up to 1024 pairs).  Shapes the folded launches do not take go the reference's way
                (engine/qwen4_cuda.c:1033-1034, 1058-1061: router matvec or GEMM, route, bucket). */
             const int packed = d % 8 == 0 && ff % 8 == 0;
             if (!(packed && T <= 64 && !kc_mv_pack(s, MF_BF16, rw, d, E, xn, d, m->logit, E, T, m->px))) {

@@ -834,7 +834,8 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     // step is large, by T pairs d ff.  Timed on 240 layers of 2 .. 8 tokens in both formats, each step both ways (us a layer, four / five waves, P = 4):
     //   gate + up sums in a wave, from 80 Mi on: top-8, 2048 x 768: 6 tokens, 72 Mi, 65.9 / 71.3, 8, 96 Mi, 86.2 / 81.3; top-8, 2048 x 1024: 5, 80 Mi, 71.0 / 68.2
     //   through LDS, whose barriers more workgroups cover:
-    //     from 22 Mi on: top-2, 2240 x 2688: 3, 34 Mi, 58.2 / 54.9; top-4, 1216 x 1024: 8, 38 Mi, 49.6 / 47.0 (but 7, 33 Mi, 43.5 / 45.7); top-4, 1344 x 704: 6, 21.7 Mi, 32.7 / 38.4, 8, 29 Mi, 38.4 / 37.8
+    //     from 22 Mi on: top-2, 2240 x 2688: 3, 34 Mi, 58.2 / 54.9; top-4, 1216 x 1024: 8, 38 Mi, 49.6 / 47.0 (but 7, 33 Mi, 43.5 / 45.7);
+    //     top-4, 1344 x 704: 6, 21.7 Mi, 32.7 / 38.4, 8, 29 Mi, 38.4 / 37.8
     //     from 32 Mi where the down sums stay in a wave: top-4, 1280 x 2048: 3, 30 Mi, 41.4 / 43.7; top-8, 1280 x 512: 8, 40 Mi, 49.7 / 47.0 (but 7, 35 Mi, 43.4 / 46.5)
     //     from 16 Mi on rows of 44 chunks or more, of which four fill at most 250 of a workgroup's lanes: top-2, 2816 x 448: 6, 14 Mi, 35.0 / 37.1, 8, 19 Mi, 44.1 / 38.8;
     //     top-2, 3200 x 640, P = 3: 5, 20 Mi, 46.1 / 40.2
@@ -992,9 +993,9 @@ int kc_moe_decode_layer(kc_stream_t s, int fmt, const uint16_t* router_w, const 
     if (T > MV_MAXT || (shared && T >= FG_MINT_SHARED && sg && T * a.kk <= FG_MAXP)) {
         // More rows than the per-pair kernel takes: pairs grouped by expert, two to a decode.  Measured against the grouped
         // GEMMs of the separate launches (C2, 16 rows: 199 against 268 us; 20 rows: 242 against 295; 24 rows: 278 against 305;
-        // 28 rows: 335 against 327, so the limit is 24; the GEMMs have gained more since, 32 rows
-        // take 171 there and 24 rows 190 here, but they multiply the rows' BF16 values, and these rows are f32); with four to a decode (402 against 338 us at 32 rows) and where the gate+up row sums go through LDS (C3's 45 chunks a row: 1129 against 753 us) the GEMMs
-        // win, so those shapes are left to them.  With an always-on expert every row brings a pair on the same expert, and
+        // 28 rows: 335 against 327, so the limit is 24; the GEMMs have gained more since, 32 rows take 171 there and 24 rows 190 here, but they
+        // multiply the rows' BF16 values, and these rows are f32); with four to a decode (402 against 338 us at 32 rows) and where the gate+up row sums
+        // go through LDS (C3's 45 chunks a row: 1129 against 753 us) the GEMMs win, so those shapes are left to them.  With an always-on expert every row brings a pair on the same expert, and
         // the grouped kernel is already ahead of the per-pair one at 5 rows (whole model, 5 rows: 4.05 against 4.18 ms, 8 rows:
         // 5.37 against 5.70; 4 rows: 3.85 against 3.68); without
         // one the two are level at 8 rows (130 us) and the per-pair kernel is ahead below.

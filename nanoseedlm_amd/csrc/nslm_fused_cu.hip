@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
                     ring_put(partg, q.f, acc[0]);
                 } else if constexpr (P == 3) {
                     if (q.f < nch) {   // (the lanes of a shared chunk take this branch together)
-                        const float sum = chunk_dot_split<P>(cur, slice(t, j, vc & 1).eb, tab, xq, q.sub, ltg);
+                        const float sum = chunk_dot_split(cur, slice(t, j, vc & 1).eb, tab, xq, q.sub, ltg);
                         if (q.sub == (1 << ltg) - 1) ring_put(partg, q.f, sum);
                     }
                 }
@@ -647,7 +647,7 @@ __global__ void __launch_bounds__(NTHR) k_moe_decode_cu(FusedArgs a, CuParams c)
             if (!q.tail) {
                 if (ok) chunk_dot<P, 1>(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, 0, acc);
             } else if constexpr (P == 3) {
-                if (ok) acc[0] = chunk_dot_split<P>(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, q.sub, ltd);   // (a chunk's lanes together)
+                if (ok) acc[0] = chunk_dot_split(dcur, slice(t, j, 2).eb, tab, xd + j * (Ld * XP) + q.ch * XP, q.sub, ltd);   // (a chunk's lanes together)
                 if (q.sub != (1 << ltd) - 1) slot = -1;
             }
             rows_out(t, it, acc[0], ok, g, j, rr, last, slot);

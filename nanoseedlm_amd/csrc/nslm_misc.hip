@@ -262,8 +262,9 @@ __global__ void k_swiglu_pack(const float* g, const float* u, uint16_t* y, size_
 // x[t][c] = bf16(x + bf16(bf16(sum_j bf16(D[t,j][c] * bf16(w[t,j]))) + shared[t][c]))
 // out[t][i] = sigmoid(sg[t * sgld]) * sh[t][i] + sum_j wt[t][j] D[t,j][i], all f32
 // Bound by the reads of D (k rows of d a token).  A thread takes V columns, all its rows' 16-byte loads requested before the
-// first is added (a column a thread, each load behind the last add: 45 us at 2048 tokens, top-8, d = 2048; four columns of f32 23, where
-// 150 MB at a large copy's rate are 29; of BF16 bits 14).  Q4 = false: the first form, with sh = shared, io = x.  sh NULL: zeros, not read.
+// first is added (a column a thread, each load behind the last add: 45 us at 2048 tokens, top-8, d = 2048; four columns of f32 23, of
+// BF16 bits 14; 150 MB at a large copy's 5.2 TB/s are 29, but D, which the launch before has just written, is in part still in the 256 MB cache).
+// Q4 = false: the first form, with sh = shared, io = x.  sh NULL: zeros, not read.
 template <int V>
 struct DVec {   // V values of a row of D
     typedef float type __attribute__((ext_vector_type(V), aligned(V % 4 ? 4 : 16)));
@@ -337,7 +338,7 @@ __global__ void k_pack_input_bf16(const float* x, uint16_t* y, size_t n) {
 // ---- grouping: selections -> pair ids by expert (ascending inside an expert), tiles of <= MMT_BN pairs, ONE launch ------
 // work (= the ntiles buffer, 2n + 3 ints): [0] tile count, [1 .. n+1] pair offsets, [n+2 .. 2n+2] tile offsets.
 // A stable counting sort by workgroups of 16 waves, 1024 pairs each.  Wave w owns 64 consecutive pairs and a histogram row
-// hist[w][.] of its own in LDS, so nothing is contended and the order inside an expert is the pair order by construction:
+// hist[w][.] of its own in LDS, so here nothing is contended and the order inside an expert is the pair order by construction:
 //   count   the lanes that hold the same expert find each other with one ballot per index bit (the
 //           intersection of the ballots a lane agrees with is the set of its equals), the first of them notes their number,
 //   scan    thread x turns column x into running sums over the waves and the workgroup scans the experts' totals
@@ -432,8 +433,10 @@ __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket(const int32_t* inds, i
     bucket_all<false>(inds, count, n, work, perm, tiles);
 }
 // More pairs: a workgroup for every 64 BK_WAVES, or for an equal run of those (`runs`) - each counts all pairs by expert, those before its own apart, so that
-// it needs nothing of the others, and that makes at most BM_GROUPS times the pairs to count.  Then it ranks its own.  One workgroup for all was bound by its CU's vector issue - count / 1024 steps of ranking a wave - and by its scattered stores of
-// the permutation.  E 128, us: 2048 pairs 6.2 -> 5.5, 4096 7.3 -> 5.6, 16384 19.1 -> 6.3, 65536 78.5 -> 11.1; 1024 pairs 4.4 and 5.3.
+// it needs nothing of the others, and that makes at most BM_GROUPS times the pairs to count.  Then it ranks its own.  One workgroup for all was bound by its CU's
+// vector issue - count / 1024 steps of ranking a wave - and by its scattered stores of the permutation.  E 128, us: 2048 pairs 6.2 -> 5.5, 4096 8.7 -> 5.8, 16384
+// 24.6 -> 6.4, 65536 87.8 -> 11.5; 1024 pairs 4.4 and 5.3.  The counting is by LDS atomics, which take lanes of the same expert in turn: Zipf's selections (1 / rank)
+// 16384 24.3 -> 7.7, 65536 87.1 -> 18.4, all pairs on two experts 25.5 -> 12.8, 91.6 -> 40.3, on one 27.1 -> 21.6, 98.8 -> 75.2.
 #define BM_LOADS 16
 #define BM_GROUPS 256
 __global__ void __launch_bounds__(64 * BK_WAVES) k_bucket_many(const int32_t* inds, int count, int n, int32_t* work, int32_t* perm, MmTile* tiles, int runs) {

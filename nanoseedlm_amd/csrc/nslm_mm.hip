@@ -410,7 +410,7 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
         auto produce = [&](int s, const MmRec2& r, const Look& k) {
             float f[2][8];
             {
-                if constexpr (seedf) {   // (both blocks phase by phase: a decoder wave has a SIMD's vector issue to itself and waits for every result)
+                if constexpr (seedf) {   // (both blocks in one run of instructions: a decoder wave has a SIMD's vector issue to itself, and one block's fill the other's waits)
                     constexpr int P = seed_p<FMT>();
                     const SumCoefs sc[2] = {sum_coefs<P>(r.v, 0, k.t[0]), sum_coefs<P>(r.v, 1, k.t[1])};
                     uint32_t y[2][8];

@@ -49,7 +49,7 @@ __device__ __forceinline__ void to_lds4(const void* src, uint8_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) src, (__attribute__((address_space(3))) void*) dst, 4, 0, 0);
 }
 
-// Block `odd` of the pair of seeds u and words v as BF16 weights.  hook(0 .. 7) is called between the phases (sums_of).
+// Block `odd` of the pair of seeds u and words v as BF16 weights.  hook(0 .. 5) is called between the phases (sums_of), hook(6) and hook(7) behind the last.
 template <int FMT, class Hook>
 __device__ __forceinline__ bf16x8 seed_weights(uint32_t u, uint32_t v, int odd, uint32_t codes, const uint32_t* tab, Hook hook) {
     constexpr int P = seed_p<FMT>();
@@ -520,7 +520,8 @@ __global__ void __launch_bounds__(512, 2) k_mm_rows(MmArgs a, WSlice w, const vo
 }
 
 #define GRT 2   // row tiles of the grouped kernel's workgroups
-// MOST: token tiles a pass.  Two (or four): four waves a SIMD.  Six: three, what their LDS leaves.
+// MOST: token tiles a pass.  Two or four: four waves a SIMD, with four tiles also what the LDS holds.  Six: registers for three; the LDS
+// holds three workgroups a CU of Q4 (52 KB), two of the other formats (56 to 64 KB).
 template <int FMT, int MOST, bool PACKED>
 __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArgs a, const WSlice* ws, const void* X, float* Y, const int32_t* perm,
                                                                            const MmTile* tiles, const int32_t* ntiles, int limit, int few) {
@@ -660,7 +661,8 @@ void grouped(hipStream_t st, const MmArgs& a, const WSlice* ws, const void* X, f
     const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
     constexpr size_t lds = rows_lds<FMT, GRT, MOST, 4, PACKED>();
     allow_big_lds<k_mm_rows_grouped<FMT, MOST, PACKED>>(lds);
-    // Four workgroups a CU run at once.  (Passes of 32: half of that; most tiles there have one pass, and the rows that find none cost small matrices
+    // Passes of 64: four workgroups a CU run at once; passes of 96, of which a CU holds two or three, have the same line.
+    // (Passes of 32: half of that; most tiles there have one pass, and the rows that find none cost small matrices
     // more than they give: E 128, top-2, d 512, ff 256, 96 rows 28 -> 32 us.  Passes of 64, E 16, top-2, d 2688, ff 384, 1010 rows: 135 and 121.)
     const int few = (limit < a.most ? limit : a.most) > 16 * MOST ? (MOST > 2 ? 4 : 2) * host_cu_count() / (int) (grid.x * grid.z) + 1 : 0;
     hipLaunchKernelGGL((k_mm_rows_grouped<FMT, MOST, PACKED>), grid, dim3(256), lds, st, a, ws, X, Y, perm, tiles, ntiles, limit, few);
@@ -705,8 +707,9 @@ namespace nslm {
 // spends on a step, in row decodes, what `step` says: that one wins where its workgroups fill the chip.  The streamed kernel was timed with 64 ..
 // 224 workgroups, one a CU; BF16 of more than 128 tokens again, on both and on every shape of this file (521 tokens, 17758 x 8000: 395 us with the
 // line where it was, streamed 276; 415 tokens, 7690 x 768 29.7 and 18.1; 132 tokens, 71938 x 448 69 and 52; none slower).  f32: 290 matrices of
-// 300 .. 32000 rows at 9 .. 2048 tokens on both kernels; the lines lie where the faster one changes (up to 128 tokens, and for Q4, Q8 and BF16 up to 256, it never does), and the kernel taken is 0.1 % off the faster one on average,
-// 16 % at worst (4096 x 4096, 1000 tokens, P = 4: first generation 236 us, this 165; 14336 x 4096, 400 tokens: 216 and 270).
+// 300 .. 32000 rows at 9 .. 2048 tokens on both kernels; the lines lie where the faster one changes (up to 128 tokens, and for Q4, Q8 and BF16 up to
+// 256, it never does), and the kernel taken is 0.1 % off the faster one on average, 16 % at worst
+// (4096 x 4096, 1000 tokens, P = 4: first generation 236 us, this 165; 14336 x 4096, 400 tokens: 216 and 270).
 bool mm_rows_better(int fmt, int R, int T, bool packed) {
     static const double step[2][3][3] = {{{6.2, 7.5, 8.8}, {8.4, 12.7, 14.5}, {13.7, 19.5, 27.0}},
                                          {{16.0, 16.0, 24.0}, {24.0, 24.0, 31.6}, {32.0, 40.0, 60.0}}};

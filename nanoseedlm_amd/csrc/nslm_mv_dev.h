@@ -118,9 +118,9 @@ __device__ __forceinline__ void chunk_post(const Chunk& ck, const float (&w)[8][
 
 // A chunk's sum by 2^ls adjacent lanes (ls = 1 .. 3), lane s of the group taking blocks [s nb, (s + 1) nb), nb = 8 >> ls: each
 // block's product with the activations as chunk_dot forms it, then its chain of multiply-adds over the blocks in block
-// order, handed from lane to lane (lane s holds its final value after step s).  The group's last lane returns chunk_dot's bits.
-template <int P>
+// order, handed from lane to lane (lane s holds its final value after step s).  The group's last lane returns chunk_dot's bits.  P = 3.
 __device__ __forceinline__ float chunk_dot_split(const Chunk& ck, int eb, const uint32_t* tab, const float* xr, int s, int ls) {
+    constexpr int P = 3;
     const int nb = 8 >> ls, b0 = s * nb;
     const uint32_t ebase = sums_e2(eb);
     float d[4] = {0.0f, 0.0f, 0.0f, 0.0f}, e2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -136,7 +136,7 @@ __device__ __forceinline__ float chunk_dot_split(const Chunk& ck, int eb, const 
             float w[8];
             sums_float<P>(y, sc.k, w);
             d[i] = block_dot(w, xr + 8 * b);
-            e2[i] = __uint_as_float(((P == 4 ? (ck.codes >> (4 * b)) & 15u : cc & 15u) << 23) + ebase);
+            e2[i] = __uint_as_float(((cc & 15u) << 23) + ebase);
         }
     }
     float acc = 0.0f;

@@ -678,10 +678,9 @@ def test_mv_multi_affine_and_bf16_equal_separate_matvecs(fmt, T):
 @pytest.mark.parametrize("T", [5, 16, 23, 64])
 def test_mv_many_tokens_equal_single_token_calls(fmt, K, R, T):
     """kc_mv over T tokens (runs of four tokens dealt to grid.y).  Up to 8 tokens every token gets the bits of a one-token call,
-    the reference's batch invariance (engine/kernels_moe.cu:239-240).  Launches of more tokens may use another order of
-    operations (P = 4: the weights' form instead of the column form) but stay invariant among themselves: a token's bits
-    depend neither on its place nor on the others, checked against 9-token calls over shifted windows; P = 3 has one form
-    and equals the one-token calls at any T.  K = 768: 12 chunks a row, row sums through LDS with more (token, row) sums
+    the reference's batch invariance (engine/kernels_moe.cu:239-240).  Launches of more tokens stay invariant among themselves: a
+    token's bits depend neither on its place nor on the others, checked for P = 4 against 9-token calls over shifted windows, for P = 3
+    against one-token calls.  K = 768: 12 chunks a row, row sums through LDS with more (token, row) sums
     than threads at four tokens; add = 1 accumulates into y."""
     import ctypes as C
     from nanoseedlm_amd import backend, moe
@@ -1232,7 +1231,7 @@ def test_combine_widths(be, oracle, d, k):
     assert np.allclose(be.kt_q4_combine(D, w, sh, sg), ref, rtol=1e-5, atol=1e-5)
 
 
-@pytest.mark.parametrize("d", [6, 24, 2048])   # a column a thread; eight: a part of a workgroup, several workgroups
+@pytest.mark.parametrize("d", [6, 24, 2048])   # a column a thread; four: a part of a workgroup, several workgroups
 @pytest.mark.parametrize("k", [1, 8, 11])
 def test_combines_of_bf16_bits_equal_those_of_f32(d, k):
     import ctypes as C
