@@ -24,6 +24,7 @@
 #include <stdlib.h>
 
 #include <atomic>
+#include <mutex>
 
 #include "nslm_fused_dev.h"
 
@@ -811,6 +812,8 @@ struct Residency {
 // Workgroups of `kern` with `dyn` bytes of dynamic LDS that a CU holds at once; < 1: none, or an error.  These kernels' workgroups wait for each other, so
 // a grid of more than this a CU would wait for workgroups that have not started.
 int resident_workgroups(const void* kern, Residency& r, size_t dyn) {
+    static std::mutex one;   // (threads that launch at once: what a kernel is prepared for only grows)
+    const std::lock_guard<std::mutex> hold(one);
     if (!r.by_registers) {
         hipFuncAttributes at;
         int n = 0;
