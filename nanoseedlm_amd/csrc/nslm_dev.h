@@ -305,41 +305,70 @@ __device__ __forceinline__ SumCoefs sum_coefs(uint32_t cc, int odd, const uint32
     }
     return s;
 }
-// A block's eight y.  up: any word whose upper 16 bits are the seed; g: the 32 stream bits that follow.  hook(0 .. 3) is called between the phases:
-// a caller with matrix instructions to issue puts them there, where the vector ALU has work beside them.
-template <int P, class Hook>
-__device__ __forceinline__ void sums_of(uint32_t up, uint32_t g, const SumCoefs& s, uint32_t (&y)[8], Hook hook) {
+// The eight y of N blocks.  up: any word whose upper 16 bits are the seed; g: the 32 stream bits that follow.  hook(0 .. 3) is called between the phases: a
+// caller with matrix instructions to issue puts them there, where the vector ALU has work beside them, and one whose wave has a SIMD's vector issue to itself
+// holds the scheduler to the phases, in which every operand of several blocks is a dozen instructions old.
+template <int P, int N, class Hook>
+__device__ __forceinline__ void sums_of(const uint32_t (&up)[N], const uint32_t (&g)[N], const SumCoefs (&s)[N], uint32_t (&y)[N][8], Hook hook) {
     if constexpr (P == 4) {
-        const uint32_t le = __builtin_amdgcn_alignbit(g, up, 17), lo = __builtin_amdgcn_alignbit(g, up, 21);   // bits 1 .., 5 ..: fields 0, 2, 4, 6; 1, 3, 5, 7
-        const uint32_t he = g >> 1, ho = g >> 5;                                                             // bits 17 .., 21 ..: fields 4, 6, 8, 10; 5, 7, 9, 11
-        const uint32_t xl[2] = {__builtin_amdgcn_perm(s.hi, s.lo, ~le & 0x07070707u), __builtin_amdgcn_perm(s.hi, s.lo, ~lo & 0x07070707u)};
-        const uint32_t xh[2] = {__builtin_amdgcn_perm(s.hi, s.lo, he & 0x07070707u), __builtin_amdgcn_perm(s.hi, s.lo, ho & 0x07070707u)};
-        hook(0);
-        uint32_t A[4];
+        uint32_t xl[N][2], xh[N][2], A[N][4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) A[c] = (c < 3 ? __builtin_amdgcn_alignbit(g, up, 20 + 4 * c) : g) ^ 0x80008000u;   // states 4c + 4, 4c + 20
+        for (int n = 0; n < N; ++n) {
+            const uint32_t le = __builtin_amdgcn_alignbit(g[n], up[n], 17), lo = __builtin_amdgcn_alignbit(g[n], up[n], 21);   // bits 1 .., 5 ..: fields 0, 2, 4, 6; 1, 3, 5, 7
+            const uint32_t he = g[n] >> 1, ho = g[n] >> 5;                                                                   // bits 17 .., 21 ..: fields 4, 6, 8, 10; 5, 7, 9, 11
+            xl[n][0] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, ~le & 0x07070707u);
+            xl[n][1] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, ~lo & 0x07070707u);
+            xh[n][0] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, he & 0x07070707u);
+            xh[n][1] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, ho & 0x07070707u);
+        }
+        hook(0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) A[n][c] = (c < 3 ? __builtin_amdgcn_alignbit(g[n], up[n], 20 + 4 * c) : g[n]) ^ 0x80008000u;   // states 4c + 4, 4c + 20
         hook(1);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = __builtin_amdgcn_perm(xh[c & 1], xl[c & 1], 0x0C040C00u + 0x00010001u * (uint32_t) (c >> 1));
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) y[n][c] = __builtin_amdgcn_perm(xh[n][c & 1], xl[n][c & 1], 0x0C040C00u + 0x00010001u * (uint32_t) (c >> 1));
         hook(2);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = (uint32_t) mad16(A[c & 3], c >> 2, s.m, 0, (int) y[c]);
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) y[n][c] = (uint32_t) mad16(A[n][c & 3], c >> 2, s[n].m, 0, (int) y[n][c]);
         hook(3);
     } else {
-        uint32_t W[8];
+        uint32_t W[N][8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) W[c] = c < 5 ? __builtin_amdgcn_alignbit(g, up, 17 + 3 * c) : g >> (3 * c - 15);   // state 3c + 1 and the bits above it
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) W[n][c] = c < 5 ? __builtin_amdgcn_alignbit(g[n], up[n], 17 + 3 * c) : g[n] >> (3 * c - 15);   // state 3c + 1 and the bits above it
         hook(0);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = __builtin_amdgcn_perm(s.hi, s.lo, (W[c] & 0x00030003u) | 0x0C040C00u);
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) y[n][c] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, (W[n][c] & 0x00030003u) | 0x0C040C00u);
         hook(1);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) W[c] ^= 0x8000u;
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) W[n][c] ^= 0x8000u;
         hook(2);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = (uint32_t) mad16(W[c], 0, s.m, 0, (int) y[c]);
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int n = 0; n < N; ++n) y[n][c] = (uint32_t) mad16(W[n][c], 0, s[n].m, 0, (int) y[n][c]);
         hook(3);
     }
+}
+template <int P, class Hook>
+__device__ __forceinline__ void sums_of(uint32_t up, uint32_t g, const SumCoefs& s, uint32_t (&y)[8], Hook hook) {
+    const uint32_t u1[1] = {up}, g1[1] = {g};
+    const SumCoefs s1[1] = {s};
+    uint32_t y1[1][8];
+    sums_of<P, 1>(u1, g1, s1, y1, hook);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) y[c] = y1[0][c];
 }
 // isum_c 2^-22 (exact): what a matvec multiplies with the activations; a row's sum is then multiplied by R32 2^22.  So a sum of blocks is kept 2^-22 low:
 // where base + code lie below about -120 it is subnormal, and an addition to it rounds by up to 2^-150, 2^-143 of the row's sum (at -126, the lowest, about one

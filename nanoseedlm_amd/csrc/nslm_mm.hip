@@ -407,15 +407,18 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                 if (FMT == MF_SEED4) k.t[h][1] = e[1];
             }
         };
-        auto produce = [&](int s, const MmRec2& r, const Look& k) {
+        auto produce = [&](int s, const MmRec2& r, const Look& k, auto phased) {
             float f[2][8];
             {
-                if constexpr (seedf) {   // (both blocks in one run of instructions: a decoder wave has a SIMD's vector issue to itself, and one block's fill the other's waits)
+                if constexpr (seedf) {
                     constexpr int P = seed_p<FMT>();
                     const SumCoefs sc[2] = {sum_coefs<P>(r.v, 0, k.t[0]), sum_coefs<P>(r.v, 1, k.t[1])};
                     uint32_t y[2][8];
-                    sums_of<P>(r.u << 16, k.g[0], sc[0], y[0], [](int) {});
-                    sums_of<P>(r.u, k.g[1], sc[1], y[1], [](int) {});
+                    if constexpr (decltype(phased)::value) sums_of<P, 2>({r.u << 16, r.u}, k.g, sc, y, [](int) { __builtin_amdgcn_sched_barrier(0); });
+                    else {
+                        sums_of<P>(r.u << 16, k.g[0], sc[0], y[0], [](int) {});
+                        sums_of<P>(r.u, k.g[1], sc[1], y[1], [](int) {});
+                    }
 #pragma unroll
                     for (int h = 0; h < 2; ++h) sums_scaled<P>(y[h], sc[h].k, FMT == MF_SEED4P4 ? (r.c >> (4 * h)) & 15u : (r.v >> (16 * h)) & 15u, f[h]);
                 } else if (FMT == MF_BF16) {
@@ -442,31 +445,47 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                 *(uint4*) &Wsm[s & 1][rr][16 * jb + 8 * h] = make_uint4(cvt_pk_bf16(f[h][0], f[h][1]), cvt_pk_bf16(f[h][2], f[h][3]),
                                                                        cvt_pk_bf16(f[h][4], f[h][5]), cvt_pk_bf16(f[h][6], f[h][7]));
         };
-        MmRec2 rec[RECD] = {};
-        Look look[2] = {};
+        // The steps, with both blocks' decode phase by phase and the next step's table reads behind it, or in the compiler's order with the reads before.  A
+        // decoder wave has a SIMD's vector issue to itself, but for that SIMD's consumers: phase by phase its instructions wait for no result, and with six or
+        // more consumer waves at work, where the decode is what a step waits for, a launch takes 2 to 12 % less (us in the compiler's order, phase by phase:
+        // 11572 x 11712, P = 3, 384 tokens 178 / 158, 512 197 / 183; P = 4 176 / 169, 201 / 193; 6000 x 3008, P = 4, 448 tokens 54 / 49).  With five or fewer, up
+        // to 320 tokens of a tile, up to 8 % more (9000 x 14336, P = 4, 264 tokens 181 / 194; 16384 x 2048, P = 3 38.8 / 40.8).
+        auto all = [&](auto phased) {
+            MmRec2 rec[RECD] = {};
+            Look look[2] = {};
 #pragma unroll
-        for (int u = 0; u < RECD; ++u) load_rec(u, rec[u]);
-        lookup(rec[0], look[0]);
-        auto one = [&](int s, auto uc) {
-            constexpr int u = decltype(uc)::value;
-            lookup(rec[(u + 1) % RECD], look[(u + 1) & 1]);   // the next step's table reads travel under this step's decode
-            produce(s, rec[u], look[u & 1]);
-            load_rec(s + RECD, rec[u]);
-            lds_barrier();
+            for (int u = 0; u < RECD; ++u) load_rec(u, rec[u]);
+            lookup(rec[0], look[0]);
+            auto one = [&](int s, auto uc) {
+                constexpr int u = decltype(uc)::value;
+                if (!phased) lookup(rec[(u + 1) % RECD], look[(u + 1) & 1]);   // the next step's table reads travel under this step's decode
+                produce(s, rec[u], look[u & 1], phased);
+                if (phased) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    lookup(rec[(u + 1) % RECD], look[(u + 1) & 1]);   // .. under the barrier
+                }
+                load_rec(s + RECD, rec[u]);
+                lds_barrier();
+            };
+            // whole rounds of the record ring in a loop with one way out (a conditional exit per step costs the loop a
+            // register move per record word and step), the steps left over after it
+            int s0 = 0;
+            for (; s0 + RECD <= nsteps; s0 += RECD) {
+                one(s0, std::integral_constant<int, 0>{});
+                one(s0 + 1, std::integral_constant<int, 1>{});
+                one(s0 + 2, std::integral_constant<int, 2>{});
+                one(s0 + 3, std::integral_constant<int, 3>{});
+            }
+            static_assert(RECD == 4, "the unrolling above");
+            if (s0 < nsteps) one(s0, std::integral_constant<int, 0>{});
+            if (s0 + 1 < nsteps) one(s0 + 1, std::integral_constant<int, 1>{});
+            if (s0 + 2 < nsteps) one(s0 + 2, std::integral_constant<int, 2>{});
         };
-        // whole rounds of the record ring in a loop with one way out (a conditional exit per step costs the loop a
-        // register move per record word and step), the steps left over after it
-        int s0 = 0;
-        for (; s0 + RECD <= nsteps; s0 += RECD) {
-            one(s0, std::integral_constant<int, 0>{});
-            one(s0 + 1, std::integral_constant<int, 1>{});
-            one(s0 + 2, std::integral_constant<int, 2>{});
-            one(s0 + 3, std::integral_constant<int, 3>{});
+        if (seedf && NCW > 5 && count > 5 * 32 * CT) all(std::true_type{});
+        else {
+            asm volatile("");   // (what both begin with stays in both: moved before the branch it cost up to 2 %)
+            all(std::false_type{});
         }
-        static_assert(RECD == 4, "the unrolling above");
-        if (s0 < nsteps) one(s0, std::integral_constant<int, 0>{});
-        if (s0 + 1 < nsteps) one(s0 + 1, std::integral_constant<int, 1>{});
-        if (s0 + 2 < nsteps) one(s0 + 2, std::integral_constant<int, 2>{});
         return;
     }
 

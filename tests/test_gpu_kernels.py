@@ -384,6 +384,19 @@ def test_mv_at_the_lowest_exponents(be, oracle, fmt, K, T):
     assert np.abs(y).max() > 0 and np.all(np.abs(y - ref * scale) <= F32B * mag * scale + K / 8 * 2.0 ** -143)
 
 
+# the streamed kernel's two orders of the decode: tiles of up to 320 tokens and of more, a second tile of either kind; one to seven weight steps (a ring of four records)
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
+@pytest.mark.parametrize("T,K", [(320, 64), (321, 64), (320, 448), (321, 448), (352, 128), (512, 192), (513, 256), (832, 320), (833, 384)])
+def test_streamed_decode_in_either_order_reads_the_oracles_weights(be, oracle, fmt, T, K):
+    R = 16384 - 15   # 256 workgroups, the last of 49 rows
+    rng = np.random.default_rng(T + K)
+    p = make_pack(rng, fmt, 1, R, K)
+    want = packs.bf16_bits_to_f32(oracle.slice_bf16(fmt, slice_of(oracle, p, 0), R, K)).T
+    k = (7 * np.arange(T)) % K
+    got = be.kt_mm_plain(p, np.eye(K, dtype=np.float32)[k], packed=1)
+    assert np.array_equal(got, want[k])
+
+
 # f32 activations at token counts that the first-generation kernel had (seeds: from 200 tokens; BF16: at 130): the last token tile partial, one row past a tile
 @pytest.mark.parametrize("T,R", [(130, 16385), (1000, 2881)])
 @pytest.mark.parametrize("fmt", ALL_FMT)
