@@ -780,13 +780,19 @@ bool shape_of(int K, bool gateup, int* L, int* rpi, bool* shfl) {
 // other (an item's set-up priced at `setup` sixths of an iteration, unequal items at half an iteration: workgroups i, i + 256, ...
 // share a CU, so the long items of a regular pattern meet on the same CUs); up to `slack` items more than the workgroups still
 // count as one round.
-int pick_one_round(int units, int iters, int gmax, int nmax, int slack = 0, int setup = 2) {
-    int best = 1;
-    long best_cost = -1;
+struct Split {
+    int n;       // items a unit
+    long cost;   // sixths of an iteration of the busiest workgroup
+};
+Split pick_one_round(int units, int iters, int gmax, int nmax, int slack = 0, int setup = 2) {
+    Split best = {1, -1};
+    long over = -slack, rounds = 1;   // (counted up: a division an n is what the loop takes)
     for (int n = 1; n <= iters && n <= nmax; ++n) {
-        const long over = (long) units * n - slack, rounds = over <= gmax ? 1 : (over + gmax - 1) / gmax, per = (iters + n - 1) / n;
-        const long cost = rounds * (6 * per + (iters % n ? 3 : 0) + setup);
-        if (best_cost < 0 || cost <= best_cost) { best = n; best_cost = cost; }   // ties: more, shorter items
+        over += units;
+        while (over > rounds * gmax) ++rounds;
+        const int q = (iters - 1) / n;   // an item has q + 1 iterations, or some have q
+        const long cost = rounds * (6 * (q + 1) + (iters != (q + 1) * n ? 3 : 0) + setup);
+        if (best.cost < 0 || cost <= best.cost) best = {n, cost};   // ties: more, shorter items
     }
     return best;
 }
@@ -843,7 +849,10 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     //     from 16 Mi on rows of 44 chunks or more, of which four fill at most 250 of a workgroup's lanes: top-2, 2816 x 448: 6, 14 Mi, 35.0 / 37.1, 8, 19 Mi, 44.1 / 38.8;
     //     top-2, 3200 x 640, P = 3: 5, 20 Mi, 46.1 / 40.2
     // Where rows are so long that a CU's LDS holds only four workgroups of either, four if the down sums are by shuffles (top-8, 4096 x 512: 4 tokens 83.4 / 84.8);
-    // else the five waves' code is still level or ahead (P = 3, top-4, 4096 x 1408: 8 tokens 224 / 216).  The rule is 0.5 % off the faster of the two on average.
+    // else the five waves' code is still level or ahead (P = 3, top-4, 4096 x 1408: 8 tokens 224 / 216).
+    // Within a factor of two of its line the items decide where they say more: five where the busiest workgroup of four has more than 1.25 times the iterations, as
+    // many as five share a SIMD by (top-2, 2688 x 960, 4 tokens, P = 3, 38.5 / 34.7), four where it has hardly more (top-4, 2048 x 960, 8 tokens, P = 3, 57.4 / 59.7).
+    // On 2240 steps of other sizes the choice is 0.2 % off the faster of the two on average (by the lines alone 0.5 %), 14 by more than 5 % (75), 12 % at worst.
     const long work = (long) a.T * a.kk * a.d * a.ff;
     static Residency known[2][2][2];
     auto variant = [&](bool few) {
@@ -852,11 +861,27 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
                    : (sg ? (sd ? k_moe_decode<P, true, true, 5> : k_moe_decode<P, true, false, 5>)
                          : (sd ? k_moe_decode<P, false, true, 5> : k_moe_decode<P, false, false, 5>));
     };
-    bool few = a.T == 1 || work < (sg ? 80L : a.Lg >= 44 ? 16L : sd ? 32L : 22L) << 20;
-    if (!few && sd && resident_workgroups((const void*) variant(false), known[0][sg][sd], lds) < 5) few = true;
+    const int P_ = a.T * a.kk;
+    auto grid_of = [&](bool few) {   // the most workgroups of a variant; < 1: an error
+        const int n = resident_workgroups((const void*) variant(few), known[few][sg][sd], lds);
+        return (n < 5 ? n : 5) * cu_count();
+    };
+    auto split_g = [&](int gmax) { return pick_one_round(P_, a.it_g, gmax, FUSED_TILES, 0, 5); };
+    auto split_d = [&](int gmax) { return pick_one_round(P_, a.it_d, gmax, FUSED_TILES, 0, 4); };
+    const long line = (sg ? 80L : a.Lg >= 44 ? 16L : sd ? 32L : 22L) << 20;
+    bool few = a.T == 1 || work < line;
+    if (a.T > 1 && 2 * work >= line) {
+        const int g4 = grid_of(true), g5 = grid_of(false);
+        if (g4 < 1 || g5 < 1) return -1;
+        if (sd && g5 < 5 * cu_count()) few = true;
+        else if (work < 2 * line) {
+            const long c4 = split_g(g4).cost + split_d(g4).cost, c5 = split_g(g5).cost + split_d(g5).cost;
+            few = few ? 4 * c4 <= 5 * c5 : 20 * c4 < 21 * c5;
+        }
+    }
     void (*kern)(FusedArgs) = variant(few);
-    const int per_cu = resident_workgroups((const void*) kern, known[few][sg][sd], lds);
-    if (per_cu < 1) return -1;
+    const int gmax = grid_of(few);
+    if (gmax < 1) return -1;
     // The grid must be resident at once (workgroups wait for each other's data): at most what the device holds, and no more than
     // five workgroups a CU (the most that was tried).  Items per pair (an item = a run of a pair's iterations, as
     // equal as whole iterations allow): one round (measured on C2, one token: 96 x 2
@@ -867,11 +892,10 @@ int launch_fused(hipStream_t st, FusedArgs& a, bool sg, bool sd, size_t lds) {
     // iterations went out as one item each wherever they did not divide evenly, in up to five rounds (us a layer at a third / at five sixths: 5 tokens of
     // top-8, 2048 x 512 55.2 / 41.5, 3 of them 36.3 / 30.8; 5 of top-4, 1024 x 2048 57.1 / 41.6; 2 of top-4, 1536 x 1024, P = 3, 29.6 / 25.5; 1248
     // steps of 1 .. 8 tokens: 0.73 to 1.01, four sixths and seven sixths within 0.4 % of five).
-    const int gmax = (per_cu < 5 ? per_cu : 5) * cu_count(), P_ = a.T * a.kk;
-    a.ntile_g = pick_one_round(P_, a.it_g, gmax, FUSED_TILES, 0, 5);
+    a.ntile_g = split_g(gmax).n;
     // (a down item's set-up - the wait for its pair, the staging of A - priced at two thirds of an iteration: at a third, six
     // tokens of C2 took two rounds of 49 two-iteration items a pair, 81.6 us, where one round of 26 takes 76.5)
-    a.ntile_d = pick_one_round(P_, a.it_d, gmax, FUSED_TILES, 0, 4);
+    a.ntile_d = split_d(gmax).n;
     if (a.ntile_g < gu_min_tiles(a)) a.ntile_g = gu_min_tiles(a);
     if ((long) ((a.it_g + a.ntile_g - 1) / a.ntile_g) * a.rpig / 2 > GU_ROWS) return -1;
     const long items = (long) P_ * (a.ntile_g > a.ntile_d ? a.ntile_g : a.ntile_d);
@@ -905,8 +929,8 @@ int launch_grouped(hipStream_t st, FusedArgs& a, bool sg, bool sd) {
     int groups = (int) (a.E * (1.0 - pow(1.0 - 1.0 / a.E, pairs)) + 0.5) + a.ns * ((a.T + NT - 1) / NT);
     if (groups < 1) groups = 1;
     const int gmax = (per_cu < 5 ? per_cu : 5) * cu_count();
-    a.ntile_g = pick_one_round(groups, a.it_g, gmax, a.it_g, 3 * gmax / 8);
-    a.ntile_d = pick_one_round(groups, a.it_d, gmax, a.it_d, 3 * gmax / 8);
+    a.ntile_g = pick_one_round(groups, a.it_g, gmax, a.it_g, 3 * gmax / 8).n;
+    a.ntile_d = pick_one_round(groups, a.it_d, gmax, a.it_d, 3 * gmax / 8).n;
     const long items = (long) groups * (a.ntile_g > a.ntile_d ? a.ntile_g : a.ntile_d);
     int grid = items < gmax ? (int) items : gmax;
     if (grid < a.T) grid = a.T < gmax ? a.T : gmax;

@@ -425,10 +425,11 @@ def test_steps_of_long_rows_by_either_kernel_give_the_separate_launches_bits(fmt
     steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 0)
 
 
-# either side of T k d ff = 80 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS, of 32 Mi with the down ones by shuffles, of 16 Mi with rows of 44 chunks; and
-# above it where five workgroups do not fit a CU's LDS
+# either side of T k d ff = 80 Mi with gate + up sums by shuffles, of 22 Mi with those through LDS, of 32 Mi with the down ones by shuffles, of 16 Mi with rows of 44 chunks;
+# above it where five workgroups do not fit a CU's LDS; and near it where the items say otherwise
 @pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_SEED4])
-@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,)), (8, 2048, 1024, (4, 5)), (4, 1280, 2048, (3, 4)), (2, 2816, 448, (6, 7))])
+@pytest.mark.parametrize("k,d,ff,rows", [(8, 2048, 768, (7,)), (8, 2048, 1024, (5, 6)), (4, 1344, 704, (6, 7)), (4, 2560, 1024, (2, 3)), (4, 4096, 512, (4,)), (4, 4096, 704, (3,)), (8, 2048, 1024, (4, 5)), (4, 1280, 2048, (3, 4)), (2, 2816, 448, (6, 7)),
+                                         (2, 2688, 960, (4,)), (4, 2048, 960, (8,)), (2, 3392, 320, (4,))])
 def test_per_pair_steps_of_four_and_five_waves_give_the_separate_launches_bits(fmt, k, d, ff, rows):
     steps_give_the_separate_launches_bits(fmt, k, d, ff, rows, 1)
 
