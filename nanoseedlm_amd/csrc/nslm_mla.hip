@@ -252,21 +252,26 @@ __global__ void __launch_bounds__(256) k_qmaps_rope(MlaArgs a, int rope, HmvArgs
 //            the quarters: GA_KT scores a wave are ready at once (no wave-wide reduction per key);
 //   softmax  the tile's maximum and its sum of exp over the 16 quads: four shuffles each, once a tile;
 //   P c      lane l owns latent dims l, l + 64, ...; exp(s_u - m) reaches it as the broadcast of lane 4 u.
-// n_splits > 1: partials [row][head][split] = (m, l, acc[r]) for the reduce; n_splits == 1: olat[row][head] = bf16(acc / l).
+// n_splits > 1: partials (m, l, acc[r]) for the reduce; n_splits == 1: olat[row][head] = bf16(acc / l).
 #define GA_KT 16
 #define GA_HW 4
 #define MLA_MAXL 16    // latent dims a lane (r <= 1024)
 #define MLA_SPLITS_SHORT 32
-__device__ __forceinline__ int mla_row_splits(const MlaArgs& a, int pos) {
-    (void) pos;
-    return a.pad[2] > 0 && a.n_splits > MLA_SPLITS_SHORT ? MLA_SPLITS_SHORT : a.n_splits;
+// a row at position pos: the number of splits that have keys, and the keys of each (the row's own 0..pos in equal runs, as few as `chunk` keys a run allow)
+__device__ __forceinline__ int mla_row_splits(const MlaArgs& a, int pos, int* run) {
+    const int ns = a.pad[2] > 0 && a.n_splits > MLA_SPLITS_SHORT ? MLA_SPLITS_SHORT : a.n_splits, want = (pos + a.chunk) / a.chunk;
+    const int used = max(ns < want ? ns : want, 1);
+    *run = max((pos + used) / used, 1);
+    return (pos + *run) / *run;
 }
-// the keys [p0, p1) of split `split` of a row at position pos: the row's own 0..pos in equal runs, as few as `chunk` keys a run allow
 __device__ __forceinline__ void split_range(const MlaArgs& a, int pos, int split, int* p0, int* p1) {
-    const int ns = mla_row_splits(a, pos), want = (pos + a.chunk) / a.chunk, used = ns < want ? ns : want, run = (pos + used) / used;
+    int run;
+    const int used = mla_row_splits(a, pos, &run);
     *p0 = split * run;
     *p1 = split < used ? min(pos + 1, *p0 + run) : *p0;
 }
+// part: [row][head][split][r] accumulators, then [row][head][split] (m, l); splits without keys are neither written nor read
+__device__ __forceinline__ size_t part_ml(const MlaArgs& a, int T) { return (size_t) T * a.n_head * a.n_splits * a.r; }
 __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope, const float* ql, const float* qr, KvView kv, const RowInfo* ri,
                                                             float* out) {
     extern __shared__ __attribute__((aligned(16))) float sm[];   // [GA_KT keys][ld] then [GA_HW queries][ld]
@@ -282,6 +287,7 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
     }
     int p0, p1;
     split_range(a, ri[t].pos, split, &p0, &p1);
+    if (p0 >= p1) return;   // uniform
     const int q0 = qt * (kw / 4), q1 = q0 + kw / 4;   // kw % 8 == 0: whole pairs
     float acc[MLA_MAXL];
 #pragma unroll
@@ -341,11 +347,12 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
         for (int j = 0; j < MLA_MAXL; ++j)
             if (j < nl && lane + 64 * j < r) o[lane + 64 * j] = bfr(acc[j] / l);
     } else {
-        float* pp = out + (((size_t) t * a.n_head + h) * a.n_splits + split) * (r + 2);
-        if (lane == 0) { pp[0] = m; pp[1] = l; }
+        const size_t at = ((size_t) t * a.n_head + h) * a.n_splits + split;
+        float *pp = out + at * r, *ml = out + part_ml(a, (int) gridDim.z) + 2 * at;
+        if (lane == 0) { ml[0] = m; ml[1] = l; }
 #pragma unroll
         for (int j = 0; j < MLA_MAXL; ++j)
-            if (j < nl && lane + 64 * j < r) pp[2 + lane + 64 * j] = acc[j];
+            if (j < nl && lane + 64 * j < r) pp[lane + 64 * j] = acc[j];
     }
 }
 
@@ -354,251 +361,261 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
 // one MFMA operand for all of them (the reference's default path does the same on its tensor cores,
 // engine/kernels_moe.cu:1388-1397, with the same rounding points: queries are BF16 values, products exact, f32 sums,
 // f32 online softmax, P entering the second product as two BF16 terms hi + lo).
-// Workgroup (split, group of 16 heads, row) of 4 waves; tile = 32 keys.  Per tile:
-//   decode  the tile's cache rows -> BF16 in LDS twice: Ks[key][r + rope] (rows padded by 8) for the scores and
-//           Vt[latent dim][key] for P c (MFMA contracts over the index that is contiguous in a lane's fragment).  A thread
-//           owns 8 latent dims x 8 keys, so the transposition is 32 v_perm in registers.  FP8 -> BF16 is
-//           v_cvt_scalef32_pk_bf16_fp8 (E4M3 code x E8M0 scale, exact); the codes 0x7F / 0xFF (never written by the
-//           encoder; the reference's decoder reads them as +-480, the instruction as NaN) and scales outside 2^+-95
-//           take the arithmetic decoder, so every byte decodes as in nslm/kvq.h.
-//   scores  S^T[key][head] = Ks Q^T by v_mfma_f32_16x16x32_bf16, 18 k-slices x 2 key tiles; Q fragments stay in registers.
-//           Wave w sums half of the k-slices of key tile w & 1; the four partial tiles meet in LDS (a third barrier, but a
-//           quarter of the LDS reads of every wave computing all of S^T, which is what bounded the tile).
-//   softmax lane (head l % 16, keys {4g .. 4g + 3, 16 + 4g .. 16 + 4g + 3}, g = l / 16): two shuffles for the tile's max.
-//   P c     O^T[dim][head] += Vt P^T, wave w owns latent dims 128 w .. 128 w + 127 (8 accumulator tiles); the lane's P
-//           values are already the B fragment when Vt holds key (16 u + 4 g + i) at column 8 g + 4 u + i.
-// The next tile's cache bytes are loaded into registers before the current tile's MFMAs.
+// Workgroup (split, group of 16 heads, row) of 8 waves, a round = 128 keys, 16 a wave.  Per round:
+//   keys    a wave's cache bytes come by loads of whole 128-byte lines (8 lanes a key FP8, 16 BF16: a load whose adjacent lanes are 16 keys, as the MFMA
+//           wants them, saves the way through LDS but costs a look-up a lane: one BF16 row of 12 k positions 27.0 us, this way 19.9), are decoded in
+//           registers and go to LDS once, key by key;
+//   scores  S^T[key][head] = K Q^T by v_mfma_f32_16x16x32_bf16, the wave's own 16 keys, all r + rope dims: no barrier; Q fragments stay in registers;
+//   softmax the waves' maxima meet in LDS (barrier), every wave forms the same reference score and its own keys' P, hi + lo terms, to LDS (barrier);
+//   P c     O^T[dim][head] += V P^T, wave w owns latent dims 64 w .. 64 w + 63 over the round's 128 keys.  MFMA contracts over the index that is
+//           contiguous in a lane's fragment, here the keys: ds_read_b64_tr_b16 hands a lane four keys of one latent dim, so the same LDS copy serves.
+// The next round's cache bytes are requested as soon as this round's are decoded.  FP8 -> BF16 is v_cvt_scalef32_pk_bf16_fp8 (E4M3 code x
+// E8M0 scale, exact); the codes 0x7F / 0xFF (never written by the encoder; the reference's decoder reads them as +-480, the instruction as
+// NaN) show as a NaN score of their key, and with scales outside [2^-95, 2^96] they send the wave's keys through the arithmetic decoder, so
+// every byte decodes as in nslm/kvq.h.
+// What bounds it: with all CUs at work the first rounds' bytes come at the rate of a large copy; then a round is 7000 clocks of phases (writes to LDS 1500,
+// the scores' chain of reads and MFMAs 1500, two barriers with the softmax 1000, P c 1500), none of the units a third busy.  Tried: workgroups of four
+// waves, two a CU (16 rows of 2 to 4 k positions + 6 %, one row of 12 k + 23 %); two rounds' bytes in registers (they spill).  us with the reduce, FP8 / BF16, against tiles of 32 keys
+// decoded twice into LDS by four waves: 16 rows of 2 to 4 k positions 22.6 -> 16.8 / 21.8 -> 19.6, one of 12 k 31.0 -> 19.5 / 28.1 -> 19.9, 32 of 3 to 6 k 46.0 -> 30.6 /
+// 46.9 -> 38.0, 32 of 0.5 to 1 k 37.2 -> 14.8 / 34.3 -> 17.5, one of 75 13.1 -> 10.0 / 12.3 -> 10.3.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-#define MA_KB 32
-template <int R, int ROPE>
-constexpr int mla_mfma_lds() { return (MA_KB * (R + ROPE + 8) + R * MA_KB) * 2 + 4 * 64 * 16; }   // Vt (R x 32) also stages the 16 query rows
-
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // partial results: the caller's buffer promises no more
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(1)));   // cache rows and scales: at whatever address the caller's views have them
+typedef short i16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint32_t bf2(float lo, float hi) {   // v_cvt_pk_bf16_f32: both round to nearest even
     const f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
+#define MA_NW 8
+#define MA_KEYS (16 * MA_NW)
+// A wave's keys in LDS: 16 rows of r values, then 16 of the RoPE key.  A key's 16-byte slots are permuted by exclusive or with mla_swz(key): the 16 lanes that
+// a 16-byte access serves together ({0-3, 12-15, 20-23, 24-27} and so on) and the 8 keys x 32 bytes of a transposing read then fall on distinct banks.
+__device__ __forceinline__ int mla_swz(int key) { return 2 * (key & 7) + (key >> 3); }
+template <int R, int ROPE>
+constexpr int mla_mfma_lds() { return MA_NW * 16 * 2 * (R + ROPE) + (MA_NW / 2) * 2048 + 2 * 16 * MA_NW * 4; }
 
-// NG = 2 (launches that leave most of the chip idle: a workgroup a CU or fewer): two groups of four waves, each with tiles of its
-// own in LDS, take the split's key tiles alternately - the chain of tiles a workgroup walks is half as long - and group 1's running
-// maximum, sum and accumulators are merged into group 0's through LDS before the split's partial result leaves, as two splits'
-// would be by the reduce.  The groups meet at the same workgroup barriers (a group without a tile in an iteration only waits).
-template <int R, int ROPE, int FMT, int NG>
-__global__ void __launch_bounds__(256 * NG) k_mla_attn_mfma(MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* out) {
-    static_assert(R == 512 && ROPE == 64, "the thread mapping of the decode covers 64 latent dim groups and 8 RoPE dim groups");
-    static_assert(NG == 1 || NG == 2, "one group of four waves, or two");
-    constexpr int KW = R + ROPE, KLD = KW + 8, NKS = KW / 32, MT = R / 64, NW = FMT == KV_FP8 ? 2 : 4;
+template <int R, int ROPE, int FMT>
+__global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* __restrict__ ri, float* out,
+                                                             int partial) {
+    static_assert(R == 512 && ROPE == 64, "eight 64-dim slices of the latent, one of the RoPE key, four dim tiles a wave");
+    constexpr int KW = R + ROPE, QLD = KW + 8, NS = R / 64, MT = R / 16 / MA_NW, ES = FMT == KV_FP8 ? 1 : 2;
+    constexpr int LK = FMT == KV_FP8 ? 8 : 16, KL = 16 * LK / 64, NL = R * ES / (16 * LK);   // lanes a key, keys a lane, 16-byte loads a key and lane
     extern __shared__ __attribute__((aligned(16))) uint8_t mla_lds[];
-    const int grp = NG > 1 ? (int) threadIdx.x >> 8 : 0;
-    uint16_t* Ks = (uint16_t*) (mla_lds + grp * mla_mfma_lds<R, ROPE>());
-    uint16_t* Vt = Ks + MA_KB * KLD;
-    f32x4* Sx = (f32x4*) (Vt + R * MA_KB);   // [wave][lane]: the waves' partial score tiles
-    const int tid = (int) threadIdx.x & 255, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;   // (tid, w: within the group)
+    uint32_t* const Ps = (uint32_t*) (mla_lds + MA_NW * 32 * KW);   // [pair of waves][hi, lo][lane][4]
+    float* const mxs = (float*) (Ps + MA_NW / 2 * 512);             // [head][wave]
+    float* const ls = mxs + 16 * MA_NW;
+    const int tid = (int) threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int split = (int) blockIdx.x, t = (int) blockIdx.z, h = (int) blockIdx.y * 16 + c;
     const int pos = ri[t].pos, kv0 = ri[t].kv0;
-    int p0, p1;
-    split_range(a, pos, split, &p0, &p1);
-    const bool live = h < a.n_head;
 
-    // The group's queries, staged once for the four waves: thread e loads 4 consecutive values of head e / 128 (latent) or
-    // e / 16 (RoPE part); heads past n_head read head 0 and are zeroed.  The loads are issued here and converted after the
-    // first tile's loads are in flight.
-    constexpr int QV = 16 * KW / 4 / 256;   // float4 a thread
+    // the group's queries: heads past n_head read head 0 and are zeroed
+    constexpr int NQ4 = 16 * KW / 4, QV = (NQ4 + 64 * MA_NW - 1) / (64 * MA_NW);   // float4 in all, and a thread
     u32x4 qv[QV];
 #pragma unroll
     for (int i = 0; i < QV; ++i) {
-        const int e = tid + 256 * i, hh = e < 16 * R / 4 ? e / (R / 4) : (e - 16 * R / 4) / (ROPE / 4);
+        const int e = min(tid + 64 * MA_NW * i, NQ4 - 1), hh = e < 16 * R / 4 ? e / (R / 4) : (e - 16 * R / 4) / (ROPE / 4);
         const int hq = (int) blockIdx.y * 16 + hh;
         const size_t th = (size_t) t * a.n_head + (hq < a.n_head ? hq : 0);
         const NSLM_GLOBAL uint32_t* src = e < 16 * R / 4 ? gp<uint32_t>(ql) + th * R + 4 * (e % (R / 4)) : gp<uint32_t>(qr) + th * ROPE + 4 * ((e - 16 * R / 4) % (ROPE / 4));
         qv[i] = *(const NSLM_GLOBAL u32x4*) src;
     }
-    // decode roles: latent dims 8 dg .. + 7 of keys {4 kap + j, 16 + 4 kap + j}; RoPE dims rd .. + 7 of key rkey
-    constexpr int ES = FMT == KV_FP8 ? 1 : 2;   // bytes a cached value
-    const int dgl = lane & 15, kap = lane >> 4, dg = 16 * w + dgl, par = dgl & 1, rkey = tid >> 3, rd = 8 * (tid & 7);
-    const uint32_t selA = par ? 0x07060302u : 0x05040100u, selB = par ? 0x05040100u : 0x07060302u;
-    uint32_t raw[8][NW] = {}, rraw[NW] = {}, rsc[8] = {127u, 127u, 127u, 127u, 127u, 127u, 127u, 127u}, rrsc = 127u;
-    auto fetch = [&](const void* codes, const void* scales, int row, int n, int d, uint32_t (&x)[NW], uint32_t& sc) {
-        if (FMT == KV_FP8) {
-            const uint2 q = ldg8(gp<uint8_t>(codes) + (size_t) row * n + d);
-            x[0] = q.x; x[1] = q.y;
-            sc = gp<uint8_t>(scales)[(size_t) row * (n / 32) + d / 32];
-        } else {
-            const uint4 q = ldg16(gp<uint16_t>(codes) + (size_t) row * n + d);
-            x[0] = q.x; x[1] = q.y; x[NW - 2] = q.z; x[NW - 1] = q.w;
-        }
-    };
-    // Keys past the split's end read its last key (finite values; their scores are masked), so no load is conditional.
-    auto load_tile = [&](int p) {
-        const int rb = kv0 + p, last = p1 - 1 - p;
-        if (rb + MA_KB <= kv.nv || rb >= kv.nv) {   // the tile lies in one segment of the view (uniform): 32-bit offsets from its first row
-            const bool first = rb < kv.nv;
-            const KvSeg sg = first ? kv.a : kv.b;
-            const size_t r0 = (size_t) (first ? rb : rb - kv.nv);
-            const NSLM_GLOBAL uint8_t* vb = gp<uint8_t>(sg.v) + r0 * (R * ES);
-            const NSLM_GLOBAL uint8_t* kb = gp<uint8_t>(sg.k) + r0 * (ROPE * ES);
-            const NSLM_GLOBAL uint8_t* vsb = gp<uint8_t>(sg.vs) + r0 * (R / 32);
-            const NSLM_GLOBAL uint8_t* ksb = gp<uint8_t>(sg.ks) + r0 * (ROPE / 32);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t kj = (uint32_t) min(j < 4 ? 4 * kap + j : 12 + 4 * kap + j, last);
-                if (FMT == KV_FP8) {
-                    const uint2 q = ldg8(vb + (kj * (uint32_t) R + 8u * (uint32_t) dg));
-                    raw[j][0] = q.x; raw[j][1] = q.y;
-                    rsc[j] = vsb[kj * (uint32_t) (R / 32) + (uint32_t) (dg >> 2)];
-                } else {
-                    const uint4 q = ldg16(vb + (kj * (uint32_t) (2 * R) + 16u * (uint32_t) dg));
-                    raw[j][0] = q.x; raw[j][1] = q.y; raw[j][NW - 2] = q.z; raw[j][NW - 1] = q.w;
-                }
-            }
-            const uint32_t kr = (uint32_t) min(rkey, last);
-            if (FMT == KV_FP8) {
-                const uint2 q = ldg8(kb + (kr * (uint32_t) ROPE + (uint32_t) rd));
-                rraw[0] = q.x; rraw[1] = q.y;
-                rrsc = ksb[kr * (uint32_t) (ROPE / 32) + (uint32_t) (rd >> 5)];
-            } else {
-                const uint4 q = ldg16(kb + (kr * (uint32_t) (2 * ROPE) + 2u * (uint32_t) rd));
-                rraw[0] = q.x; rraw[1] = q.y; rraw[NW - 2] = q.z; rraw[NW - 1] = q.w;
-            }
-        } else {   // the tile straddles the view's two segments: each key finds its own
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                int row;
-                const KvSeg sg = kv_seg(kv, rb + min(j < 4 ? 4 * kap + j : 12 + 4 * kap + j, last), &row);
-                fetch(sg.v, sg.vs, row, R, 8 * dg, raw[j], rsc[j]);
-            }
-            int row;
-            const KvSeg sg = kv_seg(kv, rb + min(rkey, last), &row);
-            fetch(sg.k, sg.ks, row, ROPE, rd, rraw, rrsc);
-        }
-    };
-    // FP8 words that v_cvt_scalef32_pk_bf16_fp8 reads as the codec does: no all-ones magnitude (bit 7 of a byte of the
-    // result set otherwise); a scale byte in [32, 222] keeps code x scale a normal BF16 value
-    auto odd_codes = [](uint32_t x0, uint32_t x1) { return ((x0 & 0x7F7F7F7Fu) + 0x01010101u) | ((x1 & 0x7F7F7F7Fu) + 0x01010101u); };
-    auto decode8 = [&](const uint32_t (&x)[NW], uint32_t sc, bool exact, uint32_t (&d)[4]) {
-        if (FMT != KV_FP8) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) d[i] = x[i * NW / 4];
-        } else if (!exact) {
-            const float f = __uint_as_float(sc << 23);
-            d[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x[0], f, false));
-            d[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x[0], f, true));
-            d[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x[1], f, false));
-            d[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x[1], f, true));
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t wd = x[i >> 1] >> (16 * (i & 1));
-                d[i] = (__float_as_uint(fp8_value(wd & 255u, sc)) >> 16) | (__float_as_uint(fp8_value((wd >> 8) & 255u, sc)) & 0xFFFF0000u);
-            }
-        }
-    };
-    auto store_tile = [&]() {
-        uint32_t D[8][4], dr[4];
-        bool exact = false;
-        if (FMT == KV_FP8) {
-            uint32_t odd = odd_codes(rraw[0], rraw[1]), far = rrsc - 32u;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                odd |= odd_codes(raw[j][0], raw[j][1]);
-                far = max(far, rsc[j] - 32u);
-            }
-            exact = (odd & 0x80808080u) != 0u || far > 190u;
-        }
-        if (!exact) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) decode8(raw[j], rsc[j], false, D[j]);
-            decode8(rraw, rrsc, false, dr);
-        } else {   // the arithmetic decoder for this lane's whole share
-#pragma unroll 1
-            for (int rep = 0; rep < 1; ++rep) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) decode8(raw[j], rsc[j], true, D[j]);
-                decode8(rraw, rrsc, true, dr);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int key = j < 4 ? 4 * kap + j : 12 + 4 * kap + j;
-            *(u32x4*) &Ks[key * KLD + 8 * dg] = u32x4{D[j][0], D[j][1], D[j][2], D[j][3]};
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {   // latent dims 8 dg + 2 q (+ 1): 8 keys each = one 16-byte block of a Vt row
-            u32x4 oa, ob;
-#pragma unroll
-            for (int jp = 0; jp < 4; ++jp) {
-                oa[jp] = __builtin_amdgcn_perm(D[2 * jp + 1][q], D[2 * jp][q], selA);
-                ob[jp] = __builtin_amdgcn_perm(D[2 * jp + 1][q], D[2 * jp][q], selB);
-            }
-            const int blk = kap ^ (q & 3) ^ ((dg >> 1) & 3), row = 8 * dg + 2 * q;
-            *(u32x4*) &Vt[(row + par) * MA_KB + 8 * blk] = oa;
-            *(u32x4*) &Vt[(row + 1 - par) * MA_KB + 8 * blk] = ob;
-        }
-        *(u32x4*) &Ks[rkey * KLD + R + rd] = u32x4{dr[0], dr[1], dr[2], dr[3]};
-    };
+    int p0, p1;
+    split_range(a, pos, split, &p0, &p1);
+    if (p0 >= p1) return;   // a split without keys (uniform over the workgroup): the reduce does not read it
 
-    // Online softmax against a reference score m per head that is raised only when a tile's maximum exceeds it by more than
-    // MLA_LAZY (so P <= e^MLA_LAZY and the accumulators are rescaled on few tiles); l and acc are in the scale e^-m.
-    constexpr float MLA_LAZY = 8.0f;
+    // the keys of a lane's loads, i < KL (of its RoPE loads, i < 2); keys 8 apart lie on adjacent lanes
+    const int kr = lane / LK, kj = lane % LK, rr = lane >> 3, rj = lane & 7;
+    auto key_of = [&](int i) { return FMT == KV_FP8 ? 8 * (kr & 1) + (kr >> 1) + 4 * i : kr + 4 * i; };
+    auto rkey_of = [&](int i) { return 8 * (rr & 1) + (rr >> 1) + 4 * i; };
+    struct Raw {
+        u32x4 v[KL][NL], vs[2], k[2];   // (k, FP8: two words)
+        uint32_t ks[2];
+    } raw;
+    // Keys past the split's end read its last key (finite values; their scores are masked), so no load is conditional.  A split inside one of the
+    // view's segments reads at 32-bit offsets from its first row (two instructions an address), one across both by each key's own segment.
+    const bool first = kv0 + p0 < kv.nv, one = first == (kv0 + p1 <= kv.nv) && p1 - p0 <= 1 << 21;
+    const size_t row0 = (size_t) (first ? kv0 + p0 : kv0 + p0 - kv.nv);
+    const NSLM_GLOBAL uint8_t* const vb0 = gp<uint8_t>(first ? kv.a.v : kv.b.v) + row0 * (R * ES);
+    const NSLM_GLOBAL uint8_t* const kb0 = gp<uint8_t>(first ? kv.a.k : kv.b.k) + row0 * (ROPE * ES);
+    const NSLM_GLOBAL uint8_t* const vsb0 = gp<uint8_t>(first ? kv.a.vs : kv.b.vs) + row0 * (R / 32);
+    const NSLM_GLOBAL uint8_t* const ksb0 = gp<uint8_t>(first ? kv.a.ks : kv.b.ks) + row0 * (ROPE / 32);
+    auto row_at = [&](int p, int key, const void* pa, const void* pb, int bytes) {
+        const int at = kv0 + min(p + 16 * w + key, p1 - 1);
+        const bool f = at < kv.nv;
+        return gp<uint8_t>(f ? pa : pb) + (size_t) (f ? at : at - kv.nv) * bytes;
+    };
+    auto load_keys = [&](Raw& r, int p) {
+        if (one) {
+            auto row = [&](int key) { return (uint32_t) min(p - p0 + 16 * w + key, p1 - p0 - 1); };
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t u = row(rkey_of(i));
+                if constexpr (FMT == KV_FP8) {
+                    const u32x2 x = *(const NSLM_GLOBAL u32x2u*) (kb0 + (u * (uint32_t) ROPE + 8u * (uint32_t) rj));
+                    r.k[i][0] = x[0];
+                    r.k[i][1] = x[1];
+                    r.ks[i] = ksb0[u * (uint32_t) (ROPE / 32) + (uint32_t) (rj >> 2)];
+                    r.vs[i] = *(const NSLM_GLOBAL u32x4u*) (vsb0 + u * (uint32_t) (R / 32));   // (FP8: the same keys)
+                } else r.k[i] = *(const NSLM_GLOBAL u32x4u*) (kb0 + (u * (uint32_t) (2 * ROPE) + 16u * (uint32_t) rj));
+            }
+#pragma unroll
+            for (int i = 0; i < KL; ++i) {
+                const uint32_t o = row(key_of(i)) * (uint32_t) (R * ES) + 16u * (uint32_t) kj;
+#pragma unroll
+                for (int s = 0; s < NL; ++s) r.v[i][s] = *(const NSLM_GLOBAL u32x4u*) (vb0 + (size_t) o + 16 * LK * s);
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const NSLM_GLOBAL uint8_t* kb = row_at(p, rkey_of(i), kv.a.k, kv.b.k, ROPE * ES) + 8 * ES * rj;
+            if constexpr (FMT == KV_FP8) {
+                const u32x2 x = *(const NSLM_GLOBAL u32x2u*) kb;
+                r.k[i][0] = x[0];
+                r.k[i][1] = x[1];
+                r.ks[i] = row_at(p, rkey_of(i), kv.a.ks, kv.b.ks, ROPE / 32)[rj >> 2];
+                r.vs[i] = *(const NSLM_GLOBAL u32x4u*) row_at(p, key_of(i), kv.a.vs, kv.b.vs, R / 32);
+            } else r.k[i] = *(const NSLM_GLOBAL u32x4u*) kb;
+        }
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            const NSLM_GLOBAL uint8_t* vb = row_at(p, key_of(i), kv.a.v, kv.b.v, R * ES) + 16 * kj;
+#pragma unroll
+            for (int s = 0; s < NL; ++s) r.v[i][s] = *(const NSLM_GLOBAL u32x4u*) (vb + 16 * LK * s);
+        }
+    };
+    auto cvt8 = [&](uint32_t x0, uint32_t x1, float f) {   // 8 codes x the scale
+        return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x0, f, false)), __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x0, f, true)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x1, f, false)), __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x1, f, true))};
+    };
+    auto cvt8_exact = [&](uint32_t x0, uint32_t x1, uint32_t sc) {
+        u32x4 d;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t wd = (i < 2 ? x0 : x1) >> (16 * (i & 1));
+            d[i] = (__float_as_uint(fp8_value(wd & 255u, sc)) >> 16) | (__float_as_uint(fp8_value((wd >> 8) & 255u, sc)) & 0xFFFF0000u);
+        }
+        return d;
+    };
+    uint8_t *const Vw = mla_lds + w * 32 * R, *const Kw = mla_lds + MA_NW * 32 * R + w * 32 * ROPE;   // the wave's keys
+    // (a latent slot's low four bits and the sixteens of slots apart: the permutation reaches the first alone, the second is an instruction's offset)
+    auto vslot = [&](int key, int low, int high) { return (u32x4*) (Vw + 2 * R * key + 16 * (low ^ mla_swz(key)) + 256 * high); };
+    auto kslot = [&](int key, int slot) { return (u32x4*) (Kw + 2 * ROPE * key + 16 * (slot ^ (key & 7))); };
+
     f32x4 acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;
-    if (p0 + grp * MA_KB < p1) load_tile(p0 + grp * MA_KB);
-    // scores: wave w sums k-slices [9 (w >> 1), + 9) of key tile w & 1
-    constexpr int KH = NKS / 2;
-    const int su = w & 1, sk = (w >> 1) * KH;
-    bf16x8 qf[KH];
-    {   // queries -> BF16 rows in LDS (over Vt, which the first tile fills after the barrier below) -> the wave's B fragments
-        uint16_t* Qs = Vt;
+    load_keys(raw, p0);
+    bf16x8 qf[NS + 1][2];
+    {   // queries -> BF16 rows in LDS (over the keys, which the first round stores after the barrier below) -> the wave's B fragments
+        uint16_t* Qs = (uint16_t*) mla_lds;
 #pragma unroll
         for (int i = 0; i < QV; ++i) {
-            const int e = tid + 256 * i, hh = e < 16 * R / 4 ? e / (R / 4) : (e - 16 * R / 4) / (ROPE / 4);
+            const int e = tid + 64 * MA_NW * i, hh = e < 16 * R / 4 ? e / (R / 4) : (e - 16 * R / 4) / (ROPE / 4);
             const int d = e < 16 * R / 4 ? 4 * (e % (R / 4)) : R + 4 * ((e - 16 * R / 4) % (ROPE / 4));
             const uint32_t keep = (int) blockIdx.y * 16 + hh < a.n_head ? 0xFFFFFFFFu : 0u;
-            *(u32x2*) &Qs[hh * KLD + d] = u32x2{bf2(__uint_as_float(qv[i][0]), __uint_as_float(qv[i][1])) & keep,
-                                                bf2(__uint_as_float(qv[i][2]), __uint_as_float(qv[i][3])) & keep};
+            if (e < NQ4)
+                *(u32x2*) &Qs[hh * QLD + d] = u32x2{bf2(__uint_as_float(qv[i][0]), __uint_as_float(qv[i][1])) & keep,
+                                                    bf2(__uint_as_float(qv[i][2]), __uint_as_float(qv[i][3])) & keep};
         }
         __syncthreads();
 #pragma unroll
-        for (int ks = 0; ks < KH; ++ks) qf[ks] = *(const bf16x8*) &Qs[c * KLD + 32 * (sk + ks) + 8 * g];
+        for (int s = 0; s <= NS; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) qf[s][i] = *(const bf16x8*) &Qs[c * QLD + 64 * s + 16 * g + 8 * i];
         __syncthreads();
     }
-    for (int pb = p0; pb < p1; pb += MA_KB * NG) {
-        const int p = pb + grp * MA_KB;
-        const bool mine = NG == 1 || p < p1;   // (uniform over the group)
-        if (mine) store_tile();
-        __syncthreads();
-        if (p + MA_KB * NG < p1) load_tile(p + MA_KB * NG);
-        f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;   // two chains over the wave's 9 k-slices
+    // the wave's 16 keys x 16 heads, from its own rows in LDS; dims 64 s + 16 g + 8 i of key c are lane (c, g)'s
+    auto scores = [&]() {
+        f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;   // two chains
+#pragma unroll
+        for (int s = 0; s <= NS; ++s) {
+            const bf16x8 k0 = *(const bf16x8*) (s < NS ? vslot(c, 8 * (s & 1) + 2 * g, s >> 1) : kslot(c, 2 * g));
+            const bf16x8 k1 = *(const bf16x8*) (s < NS ? vslot(c, 8 * (s & 1) + 2 * g + 1, s >> 1) : kslot(c, 2 * g + 1));
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qf[s][0], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qf[s][1], s1, 0, 0, 0);
+        }
+        return s0 + s1;
+    };
+    // Online softmax against a reference score m per head that is raised only when a round's maximum exceeds it by more than
+    // MLA_LAZY (so P <= e^MLA_LAZY and the accumulators are rescaled on few rounds); l and acc are in the scale e^-m.
+    constexpr float MLA_LAZY = 8.0f;
+    // lane (c, g) of a transposing read: key 4 g + c / 4, four dims from 4 (c % 4) of a tile
+    const int vkey = 4 * g + (c >> 2), vx = ((c >> 1) & 1) ^ mla_swz(vkey);
+    const uint8_t* const vrow = mla_lds + 2 * R * vkey + 8 * (c & 1) + 256 * (w >> 1);   // (tile 4 w + mt: slots 8 w + 2 mt, + 1)
+    for (int p = p0; p < p1; p += MA_KEYS) {
+        Raw& r = raw;
+        const int n = p1 - p;                       // keys left
+        const bool mine = 32 * (w >> 1) < n;        // (a pair of waves shares a fragment of P: both or none)
+        float sv[4], mx = -INFINITY;
         if (mine) {
+            bool odd = false;
+            if constexpr (FMT == KV_FP8) {   // scale bytes in [32, 223]: b + 32 has one of its two top bits (a byte that overflows shows itself)
+                uint32_t ok = 0x80808080u;
 #pragma unroll
-            for (int ks = 0; ks < KH; ++ks) {
-                const bf16x8 a0 = *(const bf16x8*) &Ks[(16 * su + c) * KLD + 32 * (sk + ks) + 8 * g];
-                if (ks & 1) s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[ks], s1, 0, 0, 0);
-                else s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[ks], s0, 0, 0, 0);
+                for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                    for (int j = 0; j < 5; ++j) {
+                        const uint32_t x = (j < 4 ? r.vs[i][j & 3] : r.ks[i] | 0x7F7F7F00u) + 0x20202020u;
+                        ok &= x | (x << 1);
+                    }
+                }
+                odd = (ok & 0x80808080u) != 0x80808080u;
             }
-            Sx[tid] = s0 + s1;
-        }
-        __syncthreads();
-        if (!mine) {   // no tile of this group's in the split's last iteration: the third barrier, nothing else
-            __syncthreads();
-            continue;
-        }
-        s0 = Sx[lane] + Sx[128 + lane];        // key tile 0: waves 0 and 2
-        s1 = Sx[64 + lane] + Sx[192 + lane];   // key tile 1: waves 1 and 3
-        float sv[8], mx = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int key = j < 4 ? 4 * g + j : 12 + 4 * g + j;
-            sv[j] = p + key < p1 ? (j < 4 ? s0[j] : s1[j - 4]) * a.scale : -INFINITY;
-            mx = fmaxf(mx, sv[j]);
+            for (int i = 0; i < 2; ++i)
+                *kslot(rkey_of(i), rj) = FMT == KV_FP8 ? cvt8(r.k[i][0], r.k[i][1], __uint_as_float(r.ks[i] << 23)) : r.k[i];
+#pragma unroll
+            for (int i = 0; i < KL; ++i)
+#pragma unroll
+                for (int s = 0; s < NL; ++s) {
+                    if constexpr (FMT == KV_FP8) {   // dims 128 s + 16 kj ..: scale byte 4 s + kj / 2
+                        const float f = __uint_as_float(r.vs[i][s] >> (8 * (kj >> 1)) << 23 & 0x7F800000u);
+                        *vslot(key_of(i), 2 * kj, s) = cvt8(r.v[i][s][0], r.v[i][s][1], f);
+                        *vslot(key_of(i), 2 * kj + 1, s) = cvt8(r.v[i][s][2], r.v[i][s][3], f);
+                    } else *vslot(key_of(i), kj, s) = r.v[i][s];
+                }
+            load_keys(r, p + MA_KEYS);
+            f32x4 s0 = scores();
+            if constexpr (FMT == KV_FP8) {
+                odd |= s0[0] != s0[0] || s0[1] != s0[1] || s0[2] != s0[2] || s0[3] != s0[3];
+                if (__any(odd)) {   // the arithmetic decoder for the wave's keys
+#pragma unroll 1
+                    for (int i = 0; i < 2; ++i) {
+                        const u32x2 x = *(const NSLM_GLOBAL u32x2u*) (row_at(p, rkey_of(i), kv.a.k, kv.b.k, ROPE) + 8 * rj);
+                        *kslot(rkey_of(i), rj) = cvt8_exact(x[0], x[1], row_at(p, rkey_of(i), kv.a.ks, kv.b.ks, ROPE / 32)[rj >> 2]);
+#pragma unroll 1
+                        for (int s = 0; s < NL; ++s) {
+                            const u32x4 y = *(const NSLM_GLOBAL u32x4u*) (row_at(p, key_of(i), kv.a.v, kv.b.v, R) + 16 * kj + 128 * s);
+                            const uint32_t sc = row_at(p, key_of(i), kv.a.vs, kv.b.vs, R / 32)[4 * s + (kj >> 1)];
+                            *vslot(key_of(i), 2 * kj, s) = cvt8_exact(y[0], y[1], sc);
+                            *vslot(key_of(i), 2 * kj + 1, s) = cvt8_exact(y[2], y[3], sc);
+                        }
+                    }
+                    s0 = scores();
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                sv[j] = 16 * w + 4 * g + j < n ? s0[j] * a.scale : -INFINITY;
+                mx = fmaxf(mx, sv[j]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool up = mx > m + MLA_LAZY;   // true on the first tile (m = -inf; every tile has a key, so mx is finite)
+        if (g == 0) mxs[c * MA_NW + w] = mx;
+        __syncthreads();
+        {
+            const f32x4 a0 = *(const f32x4*) (mxs + c * MA_NW), a1 = *(const f32x4*) (mxs + c * MA_NW + 4);
+            mx = fmaxf(fmaxf(fmaxf(a0[0], a0[1]), fmaxf(a0[2], a0[3])), fmaxf(fmaxf(a1[0], a1[1]), fmaxf(a1[2], a1[3])));
+        }
+        const bool up = mx > m + MLA_LAZY;   // true on the first round (m = -inf; every round has a key, so mx is finite); the same in every wave
         if (__any(up)) {
             const float cor = up ? __expf(m - mx) : 1.0f;
             m = up ? mx : m;
@@ -606,135 +623,154 @@ __global__ void __launch_bounds__(256 * NG) k_mla_attn_mfma(MlaArgs a, const flo
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) acc[mt] *= cor;
         }
-        u32x4 bh, bl;
+        if (mine) {
+            uint32_t* const pd = Ps + (w >> 1) * 512 + 4 * lane + 2 * (w & 1);
+            u32x2 bh, bl;
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-            const float e0 = __expf(sv[j] - m), e1 = __expf(sv[j + 1] - m);   // masked keys: exp(-inf) = 0
-            l += e0 + e1;
-            bh[j >> 1] = bf2(e0, e1);
-            bl[j >> 1] = bf2(e0 - __uint_as_float(bh[j >> 1] << 16), e1 - __uint_as_float(bh[j >> 1] & 0xFFFF0000u));
-        }
-        const bf16x8 ph = __builtin_bit_cast(bf16x8, bh), pl = __builtin_bit_cast(bf16x8, bl);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int tile = w * MT + mt;
-            const bf16x8 vt = *(const bf16x8*) &Vt[(16 * tile + c) * MA_KB + 8 * (g ^ ((c >> 1) & 3) ^ (tile & 3))];
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, ph, acc[mt], 0, 0, 0);
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pl, acc[mt], 0, 0, 0);
+            for (int j = 0; j < 4; j += 2) {
+                const float e0 = __expf(sv[j] - m), e1 = __expf(sv[j + 1] - m);   // masked keys: exp(-inf) = 0
+                l += e0 + e1;
+                bh[j >> 1] = bf2(e0, e1);
+                bl[j >> 1] = bf2(e0 - __uint_as_float(bh[j >> 1] << 16), e1 - __uint_as_float(bh[j >> 1] & 0xFFFF0000u));
+            }
+            *(u32x2*) pd = bh;
+            *(u32x2*) (pd + 256) = bl;
         }
         __syncthreads();
+#pragma unroll
+        for (int q = 0; q < MA_NW / 2; ++q) {
+            if (32 * q >= n) break;   // uniform
+            const bf16x8 ph = *(const bf16x8*) (Ps + q * 512 + 4 * lane), pl = *(const bf16x8*) (Ps + q * 512 + 256 + 4 * lane);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const uint8_t* const v = vrow + 2 * q * 32 * R + 16 * ((8 * (w & 1) + 2 * mt) ^ vx);
+                const i16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*) v);
+                const i16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*) (v + 32 * R));
+                const bf16x8 vt = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, ph, acc[mt], 0, 0, 0);
+                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pl, acc[mt], 0, 0, 0);
+            }
+        }
+        if (n > MA_KEYS) __syncthreads();   // the next round writes V
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    if (NG > 1) {   // group 1's state into group 0's, thread by thread (the same head, the same latent dims), as two splits merge
-        float* mg = (float*) (mla_lds + mla_mfma_lds<R, ROPE>()) + tid * (4 * MT + 2);   // (group 1's tiles: read for the last time before the loop's last barrier)
-        if (grp == 1) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) mg[4 * mt + i] = acc[mt][i];
-            mg[4 * MT] = m;
-            mg[4 * MT + 1] = l;
-        }
-        __syncthreads();
-        if (grp == 1) return;
-        const float m1 = mg[4 * MT], l1 = mg[4 * MT + 1], mn = fmaxf(m, m1);
-        const float f0 = m == mn ? 1.0f : __expf(m - mn), f1 = m1 == mn ? 1.0f : __expf(m1 - mn);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[mt][i] = acc[mt][i] * f0 + mg[4 * mt + i] * f1;
-        l = l * f0 + l1 * f1;
-        m = mn;
+    if (g == 0) ls[c * MA_NW + w] = l;
+    __syncthreads();
+    {
+        const f32x4 a0 = *(const f32x4*) (ls + c * MA_NW), a1 = *(const f32x4*) (ls + c * MA_NW + 4);
+        l = ((a0[0] + a0[1]) + (a0[2] + a0[3])) + ((a1[0] + a1[1]) + (a1[2] + a1[3]));
     }
-    if (!live) return;
-    if (a.n_splits == 1) {
-        float* o = out + ((size_t) t * a.n_head + h) * R;
+    if (h >= a.n_head) return;
+    const size_t th = (size_t) t * a.n_head + h;
+    if (!partial) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[16 * (w * MT + mt) + 4 * g + i] = bfr(acc[mt][i] / l);
+        for (int mt = 0; mt < MT; ++mt) {
+            const int d = 16 * (MT * w + mt) + 4 * g;
+            *(f32x4u*) (out + th * R + d) = f32x4u{bfr(acc[mt][0] / l), bfr(acc[mt][1] / l), bfr(acc[mt][2] / l), bfr(acc[mt][3] / l)};
+        }
     } else {
-        float* pp = out + (((size_t) t * a.n_head + h) * a.n_splits + split) * (R + 2);
-        if (w == 0 && g == 0) { pp[0] = m; pp[1] = l; }
+        const size_t at = th * a.n_splits + split;
+        if (w == 0 && g == 0) *(f32x2u*) (out + part_ml(a, (int) gridDim.z) + 2 * at) = f32x2u{m, l};
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) pp[2 + 16 * (w * MT + mt) + 4 * g + i] = acc[mt][i];
+        for (int mt = 0; mt < MT; ++mt) {
+            const int d = 16 * (MT * w + mt) + 4 * g;
+            *(f32x4u*) (out + at * R + d) = acc[mt];
+        }
     }
 }
 
-// Reduce the splits: olat[t][h][d] = bf16(acc / l).  Workgroup (head, row, 128 latent dims): the splits' maxima and
-// weights exp(m_s - m) once per workgroup (threads stride the splits, so their loads are in flight together), then each
-// thread sums its dim over the splits.
+// The splits of a (row, head) summed, a workgroup of 256 threads: o[i] = bf16(acc / l) of latent dims d0 + i, i < 256 NQ, as far as r reaches.  Wave w takes
+// splits w, w + 4, ... (of whole quads of dims, 16 bytes a load) and the four sums meet in LDS; every wave forms the splits' weights exp(m_s - m) itself, a
+// split a lane, and takes them from there by v_readlane.  The loads of the first 32 splits are requested before anything waits, the row's position included:
+// what a split without keys left in the buffer is not used.
 #define MLA_RED_MAXS 256
-__global__ void __launch_bounds__(128) k_mla_reduce(MlaArgs a, const RowInfo* ri, const float* part, float* olat) {
-    __shared__ float wts[MLA_RED_MAXS], red[4];
-    const int h = (int) blockIdx.x, t = (int) blockIdx.y, r = a.r, w = r + 2, ns = mla_row_splits(a, ri[t].pos), tid = threadIdx.x;
-    const NSLM_GLOBAL float* pp = gp<float>(part) + ((size_t) t * a.n_head + h) * a.n_splits * w;
-    float ms[MLA_RED_MAXS / 128], m = -INFINITY;
+template <int NQ>
+__device__ __forceinline__ void mla_reduce(const MlaArgs& a, int T, int t, int h, int d0, const RowInfo* ri, const float* part, f32x4 (&sum)[4][64 * NQ], float* o) {
+    constexpr int PF = 8, NM = MLA_RED_MAXS / 64;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = a.r;
+    const size_t th = (size_t) t * a.n_head + h;
+    const NSLM_GLOBAL float* pa = gp<float>(part) + th * a.n_splits * r;
+    const NSLM_GLOBAL float* pm = gp<float>(part) + part_ml(a, T) + 2 * th * a.n_splits;
+    const int pos = ri[t].pos;
+    int q[NQ];
 #pragma unroll
-    for (int i = 0; i < MLA_RED_MAXS / 128; ++i) {
-        const int s = tid + 128 * i;
-        ms[i] = s < ns ? pp[(size_t) s * w] : -INFINITY;
-        m = fmaxf(m, ms[i]);
+    for (int k = 0; k < NQ; ++k) q[k] = min(d0 + 4 * (lane + 64 * k), r - 4);
+    f32x2 ml[NM];
+    f32x4 pv[NQ][PF];
+#pragma unroll
+    for (int i = 0; i < NM; ++i) ml[i] = *(const NSLM_GLOBAL f32x2u*) (pm + 2 * min(lane + 64 * i, a.n_splits - 1));
+#pragma unroll
+    for (int j = 0; j < PF; ++j)
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) pv[k][j] = *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) min(w + 4 * j, a.n_splits - 1) * r + q[k]);
+    loads_issued();
+    int run;
+    const int ns = mla_row_splits(a, pos, &run);
+    float m = -INFINITY, l = 0.0f, c[NM];
+#pragma unroll
+    for (int i = 0; i < NM; ++i) m = fmaxf(m, lane + 64 * i < ns ? ml[i][0] : -INFINITY);
+    for (int s = 32; s > 0; s >>= 1) m = fmaxf(m, __shfl_xor(m, s));
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+        const bool on = lane + 64 * i < ns;
+        c[i] = on && ml[i][0] != -INFINITY ? expf(ml[i][0] - m) : 0.0f;
+        l = on ? fmaf(ml[i][1], c[i], l) : l;
     }
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((tid & 63) == 0) red[tid >> 6] = m;
-    __syncthreads();
-    m = fmaxf(red[0], red[1]);
-    float l = 0.0f;
+    for (int s = 32; s > 0; s >>= 1) l += __shfl_xor(l, s);
+    f32x4 acc[NQ];
 #pragma unroll
-    for (int i = 0; i < MLA_RED_MAXS / 128; ++i) {
-        const int s = tid + 128 * i;
-        if (s < ns) {
-            const float c = ms[i] == -INFINITY ? 0.0f : expf(ms[i] - m);
-            wts[s] = c;
-            l = fmaf(pp[(size_t) s * w + 1], c, l);
+    for (int k = 0; k < NQ; ++k) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](const f32x4 (&v)[NQ], float wt) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[k][i] = fmaf(v[k][i], wt, acc[k][i]);
+    };
+#pragma unroll
+    for (int i = 0; i < NM; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int s = 64 * i + w + 4 * j;
+            if (s >= ns) break;   // uniform
+            const float wt = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c[i]), s & 63));
+            f32x4 v[NQ];
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) v[k] = i == 0 && j < PF ? pv[k][j < PF ? j : 0] : *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) s * r + q[k]);
+            add(v, wt);
         }
-    }
-    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-    if ((tid & 63) == 0) red[2 + (tid >> 6)] = l;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) sum[w][lane + 64 * k] = acc[k];
     __syncthreads();
-    l = red[2] + red[3];
-    const int d = (int) blockIdx.z * 128 + tid;
-    if (d >= r) return;
-    float acc = 0.0f;
-#pragma unroll 8
-    for (int s = 0; s < ns; ++s) acc = fmaf(pp[(size_t) s * w + 2 + d], wts[s], acc);
-    olat[((size_t) t * a.n_head + h) * r + d] = bfr(acc / l);
+    const float* sf = (const float*) sum;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+        const int i = tid + 256 * k;
+        const float v = (sf[i] + sf[256 * NQ + i]) + (sf[512 * NQ + i] + sf[768 * NQ + i]);
+        if (d0 + i < r) o[i] = bfr(v / l);
+    }
+}
+// olat[t][h][d] = bf16(acc / l).  Workgroup (head, row, 256 latent dims).
+__global__ void __launch_bounds__(256) k_mla_reduce(MlaArgs a, const RowInfo* ri, const float* part, float* olat) {
+    __shared__ f32x4 sum[4][64];
+    const int h = (int) blockIdx.x, t = (int) blockIdx.y, d0 = (int) blockIdx.z * 256;
+    mla_reduce<1>(a, (int) gridDim.y, t, h, d0, ri, part, sum, olat + ((size_t) t * a.n_head + h) * a.r + d0);
 }
 
 // The splits' reduce and the value-up map of a head in ONE launch: workgroup (row group, head, row) reduces the head's
-// latent output into LDS (k_mla_reduce's arithmetic, all r dims: the map needs them all) and computes rows
+// latent output into LDS (k_mla_reduce's arithmetic, 512 dims a pass: the map needs them all) and computes rows
 // [RG g, RG (g + 1)) of y[t][h] = bf16(W_h . olat[t][h]) (k_heads_mv's arithmetic).  The same bits as the two kernels.
 #define MLA_RV_GROUPS 16   // row groups a head at most: fewer when there are many (row, head) pairs, each group re-reads the partials
 __global__ void __launch_bounds__(256) k_mla_reduce_vup(MlaArgs a, const RowInfo* ri, const float* part, HmvArgs hv, int fmt, WSlice W, float* y,
                                                        int lpr) {
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
-    __shared__ float wts[MLA_RED_MAXS], red[4];
+    __shared__ f32x4 sum[4][128];
     __shared__ __attribute__((aligned(16))) float ol[64 * MLA_MAXL];
-    constexpr int PF = 32, NP = 2;   // splits / map passes whose loads are issued before anything waits
-    const int g = (int) blockIdx.x, h = (int) blockIdx.y, t = (int) blockIdx.z, r = a.r, w = r + 2, ns = mla_row_splits(a, ri[t].pos), tid = threadIdx.x;
-    const NSLM_GLOBAL float* pp = gp<float>(part) + ((size_t) t * a.n_head + h) * a.n_splits * w;
+    constexpr int NP = 2;   // map passes whose loads are issued before anything waits
+    const int g = (int) blockIdx.x, h = (int) blockIdx.y, t = (int) blockIdx.z, r = a.r, tid = threadIdx.x;
     const int rg = (hv.O + (int) gridDim.x - 1) / (int) gridDim.x, o0 = g * rg, o1 = min(o0 + rg, hv.O);
     const int rpw = 64 / lpr, sub = (tid & 63) / lpr, ln = tid & (lpr - 1);
-    // Every load whose address is known now is in flight before the first wait: the splits' (m, l), this thread's two
-    // output dims of the first PF splits, and (BF16 maps, one block a lane) the map rows of the first NP passes.
-    // (loads are unconditional on clamped indices: a conditional load waits for the ones before it)
-    float msv[MLA_RED_MAXS / 128], lsv[MLA_RED_MAXS / 128], pv[2][PF];
-#pragma unroll
-    for (int i = 0; i < MLA_RED_MAXS / 128; ++i) {
-        const int s = tid + 128 * i, sc = min(s, ns - 1);
-        const bool ok = tid < 128 && s < ns;
-        const float mv = pp[(size_t) sc * w], lv = pp[(size_t) sc * w + 1];
-        msv[i] = ok ? mv : -INFINITY;
-        lsv[i] = ok ? lv : 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int s = 0; s < PF; ++s) pv[k][s] = pp[(size_t) min(s, ns - 1) * w + 2 + min(tid + 256 * k, r - 1)];
+    // BF16 maps, one block a lane: the map rows of the first NP passes are in flight beside the splits
     const bool pre = fmt == MF_BF16 && hv.I / 8 == lpr && (((uintptr_t) W.p[0] | (uintptr_t) (2 * hv.I)) & 15u) == 0;
     uint4 wq[NP];
     if (pre) {
@@ -745,47 +781,10 @@ __global__ void __launch_bounds__(256) k_mla_reduce_vup(MlaArgs a, const RowInfo
         }
     }
     if (fmt == MF_SEED4P4 || fmt == MF_SEED4) load_tables(tab);
-    // the splits' maximum and the sum of l exactly as k_mla_reduce forms them: its two waves, splits tid and tid + 128
-    float m = -INFINITY, l = 0.0f;
-    if (tid < 128) {
-#pragma unroll
-        for (int i = 0; i < MLA_RED_MAXS / 128; ++i) m = fmaxf(m, msv[i]);
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-        if ((tid & 63) == 0) red[tid >> 6] = m;
+    for (int d0 = 0; d0 < r; d0 += 512) {
+        mla_reduce<2>(a, (int) gridDim.z, t, h, d0, ri, part, sum, ol + d0);
+        __syncthreads();
     }
-    __syncthreads();
-    m = fmaxf(red[0], red[1]);
-    if (tid < 128) {
-#pragma unroll
-        for (int i = 0; i < MLA_RED_MAXS / 128; ++i) {
-            const int s = tid + 128 * i;
-            if (s < ns) {
-                const float c = msv[i] == -INFINITY ? 0.0f : expf(msv[i] - m);
-                wts[s] = c;
-                l = fmaf(lsv[i], c, l);
-            } else if (s < PF) wts[s] = 0.0f;   // the prefetched terms past the last split add x * 0
-        }
-        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-        if ((tid & 63) == 0) red[2 + (tid >> 6)] = l;
-    }
-    __syncthreads();
-    l = red[2] + red[3];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int d = tid + 256 * k;
-        if (d >= r) break;
-        float acc = 0.0f;
-#pragma unroll
-        for (int s = 0; s < PF; ++s) acc = fmaf(pv[k][s], wts[s], acc);
-        for (int s = PF; s < ns; ++s) acc = fmaf(pp[(size_t) s * w + 2 + d], wts[s], acc);
-        ol[d] = bfr(acc / l);
-    }
-    for (int d = tid + 512; d < r; d += 256) {   // latent widths above 512
-        float acc = 0.0f;
-        for (int s = 0; s < ns; ++s) acc = fmaf(pp[(size_t) s * w + 2 + d], wts[s], acc);
-        ol[d] = bfr(acc / l);
-    }
-    __syncthreads();
     WSlice ws = W;
     if (fmt == MF_SEED4P4) ws.eb = gp<int32_t>(W.p[2])[h];
     auto finish = [&](int o, bool live, float acc) {
@@ -877,32 +876,33 @@ int kc_mla_qmaps_rope(kc_stream_t s, MlaArgs a, HmvArgs hq, HmvArgs hl, int fmt,
     host_note_launch();
     return 0;
 }
-// attention into the partials (n_splits > 1) or olat; the reduce when `reduce`.  false: unsupported, nothing launched
-static bool mla_attn_launch(kc_stream_t s, MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, float* olat,
+// attention into the partials (n_splits > 1) or olat; the reduce when `reduce`.  a.n_splits becomes the number the launch takes (the partials' layout).
+// false: unsupported, nothing launched
+static bool mla_attn_launch(kc_stream_t s, MlaArgs& a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, float* olat,
                             int T, bool reduce) {
     const int rope = rope_of(a);
     if (T < 1 || (kv.fmt != KV_BF16 && kv.fmt != KV_FP8) || (rope != 64 && rope != 128) || a.r % 8 || a.r > 64 * MLA_MAXL || a.n_splits < 1) {
         host_note_unsupported();
         return false;
     }
-    float* o = a.n_splits > 1 ? part : olat;
     if (a.n_splits > MLA_RED_MAXS) { host_note_unsupported(); return false; }
     if (a.r == 512 && rope == 64 && (((uintptr_t) ql | (uintptr_t) qr) & 15u) == 0) {   // the matrix-core kernel: 16 heads a workgroup
         constexpr int lds = mla_mfma_lds<512, 64>();
-        static const hipError_t once[4] = {
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * lds),
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * lds)};
+        static const hipError_t once[2] = {
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8>, hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
         (void) once;
-        const dim3 grid((unsigned) a.n_splits, (unsigned) (a.n_head + 15) / 16, (unsigned) T);
-        // a workgroup a CU or fewer: two groups of waves a workgroup walk a split's tiles (a step of a few rows is a chain of tiles)
-        const bool two = (long) grid.x * grid.y * grid.z <= 256;
-        if (two && kv.fmt == KV_FP8) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_FP8, 2>), grid, dim3(512), 2 * lds, (hipStream_t) s, a, ql, qr, kv, ri, o);
-        else if (two) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_BF16, 2>), grid, dim3(512), 2 * lds, (hipStream_t) s, a, ql, qr, kv, ri, o);
-        else if (kv.fmt == KV_FP8) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_FP8, 1>), grid, dim3(256), lds, (hipStream_t) s, a, ql, qr, kv, ri, o);
-        else hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_BF16, 1>), grid, dim3(256), lds, (hipStream_t) s, a, ql, qr, kv, ri, o);
+        // A workgroup fills a CU: more splits than fill the chip only add partials (2 KB a head and split, written and read again).  (Splits dealt to the rows by
+        // their lengths: 20 rows of 4 to 8 k positions 28.4 -> 25.8, but 32 of 0.5 to 1 k 14.8 -> 18.0 and 16 of 2 to 4 k 16.8 -> 17.2.)
+        const int groups = (a.n_head + 15) / 16, fill = host_cu_count() / (groups * T), least = reduce ? 1 : 2;
+        if (a.n_splits > 1) a.n_splits = a.n_splits < fill ? a.n_splits : fill < least ? least : fill;
+        const dim3 grid((unsigned) a.n_splits, (unsigned) groups, (unsigned) T);
+        const int partial = a.n_splits > 1;
+        float* o = partial ? part : olat;
+        if (kv.fmt == KV_FP8) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_FP8>), grid, dim3(64 * MA_NW), lds, (hipStream_t) s, a, ql, qr, kv, ri, o, partial);
+        else hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_BF16>), grid, dim3(64 * MA_NW), lds, (hipStream_t) s, a, ql, qr, kv, ri, o, partial);
     } else {
+        float* o = a.n_splits > 1 ? part : olat;
         const size_t lds = sizeof(float) * (size_t) (GA_KT + GA_HW) * (size_t) (a.r + rope + 4);
         static const hipError_t once = hipFuncSetAttribute((const void*) k_mla_attn_any, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                            (int) (sizeof(float) * (GA_KT + GA_HW) * (64 * MLA_MAXL + ATT_HD + 4)));
@@ -911,7 +911,7 @@ static bool mla_attn_launch(kc_stream_t s, MlaArgs a, const float* ql, const flo
                            (hipStream_t) s, a, rope, ql, qr, kv, ri, o);
     }
     if (a.n_splits > 1 && reduce)
-        hipLaunchKernelGGL(k_mla_reduce, dim3((unsigned) a.n_head, (unsigned) T, (unsigned) (a.r + 127) / 128), dim3(128), 0, (hipStream_t) s, a, ri,
+        hipLaunchKernelGGL(k_mla_reduce, dim3((unsigned) a.n_head, (unsigned) T, (unsigned) (a.r + 255) / 256), dim3(256), 0, (hipStream_t) s, a, ri,
                            part, olat);
     host_note_launch();
     return true;

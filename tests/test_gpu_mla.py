@@ -165,6 +165,55 @@ def test_latent_attention_long_context_fp8(be, oracle):
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 127, 128, 129, 300])
+@pytest.mark.parametrize("fmt,ns", [("fp8", 1), ("fp8", 3), ("bf16", 1), ("bf16", 3)])
+def test_latent_attention_at_the_edges_of_a_round(be, oracle, fmt, n, ns):
+    """n keys where a round is 128 of 16 a wave: against the oracle; and the same bits over a view whose two segments meet inside a wave's keys, its scale
+    bytes at odd addresses."""
+    import ctypes as C
+    from nanoseedlm_amd import moe
+    L = be.hip()
+    rng = np.random.default_rng(n + ns)
+    H, r, rope, kv0, T = 18, 512, 64, 3, 2          # (row 1: one key less, or the same one)
+    pos = [n - 1, max(n - 2, 0)]
+    ql = packs.round_bf16((rng.standard_normal((T, H, r)) * 0.3).astype(np.float32))
+    qr = packs.round_bf16(rng.standard_normal((T, H, rope)).astype(np.float32))
+    lat = packs.round_bf16(rng.standard_normal((n + kv0, r)).astype(np.float32))
+    kr = packs.round_bf16(rng.standard_normal((n + kv0, rope)).astype(np.float32))
+    fp8, scale = fmt == "fp8", float(1 / np.sqrt(192.0))
+    if fp8:
+        (kc, ksc), (vc, vsc) = oracle.fp8_row(kr), oracle.fp8_row(lat)
+        lat, kr = oracle.fp8_decode(vc, vsc), oracle.fp8_decode(kc, ksc)
+    else:
+        kc, vc = packs.f32_to_bf16_bits(kr), packs.f32_to_bf16_bits(lat)
+        ksc = vsc = np.zeros((n + kv0, 16), np.uint8)
+    a = be.MlaArgs(H, r, 32, ns, scale)
+    a.pad[0] = rope
+    ri = (be.RowInfo * T)()
+    for t in range(T):
+        ri[t].pos, ri[t].kv0 = pos[t], kv0
+    rib = moe.DevBuf.from_array(np.frombuffer(bytes(ri), dtype=np.uint8))
+    qlb, qrb = moe.DevBuf.from_array(ql), moe.DevBuf.from_array(qr)
+    part, olat = moe.DevBuf(4 * T * H * ns * (r + 2)), moe.DevBuf(4 * T * H * r)
+    outs = []
+    for cut, off in ((n + kv0, 0), (kv0 + n // 2, 1)):
+        def dev(x, shift):
+            b = moe.DevBuf.from_array(np.concatenate([np.zeros(shift, np.uint8), np.frombuffer(x.tobytes(), np.uint8), np.zeros(16, np.uint8)]))
+            return b, b.ptr.value + shift
+        segs = [[dev(x[s], sh) for x, sh in ((kc, 0), (vc, 0), (ksc, off), (vsc, 3 * off))] for s in (slice(0, cut), slice(cut, None))]
+        kv = be.KvView(*[be.KvSeg(*[p for _, p in sg]) for sg in segs], cut, be.KV_FP8 if fp8 else be.KV_BF16)
+        L.kc_mla_attn.argtypes = [C.c_void_p, be.MlaArgs, C.c_void_p, C.c_void_p, be.KvView, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]
+        L.kc_mla_attn(None, a, qlb.ptr, qrb.ptr, kv, rib.ptr, part.ptr, olat.ptr, T)
+        moe.device_sync()
+        assert L.kc_last_error() == 0
+        outs.append(olat.to_array(np.float32, (T, H, r)))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    for t in range(T):
+        for h in (0, 15, 17):
+            want = oracle.mla_attn(ql[t, h], qr[t, h], lat[kv0:], kr[kv0:], pos[t], scale)
+            assert np.all(close_bf(outs[0][t, h], want.astype(np.float64), 2e-6)), (t, h)
+
+
 @pytest.mark.parametrize("kvf", ["bf16", "fp8"])
 @pytest.mark.parametrize("H,hd,r,rope,T", [(16, 128, 512, 64, 3), (5, 64, 128, 128, 2)])
 def test_query_maps_rope_and_cache_write_in_one_launch(be, kvf, H, hd, r, rope, T):
