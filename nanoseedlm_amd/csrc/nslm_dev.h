@@ -74,11 +74,11 @@ constexpr uint32_t stream32_of(uint32_t s) {
     }
     return g;
 }
-constexpr StreamBasis make_basis() {
+constexpr StreamBasis make_basis(uint32_t flip) {   // flip: exclusive-or on the sum
     StreamBasis b{};
     for (uint32_t i = 0; i < 256; ++i) {
         b.v[i] = stream32_of(i);
-        b.v[256 + i] = stream32_of(i << 8);
+        b.v[256 + i] = stream32_of(i << 8) ^ flip;
     }
     return b;
 }
@@ -94,7 +94,7 @@ constexpr CoefPairs make_pairs() {
     }
     return t;
 }
-__device__ const StreamBasis kBasis = make_basis();
+__device__ const StreamBasis kBasis = make_basis(0);
 __device__ const CoefPairs kPairs = make_pairs();
 
 // LDS copy of both tables: [0,512) stream basis, [512,768) coefficient pairs
@@ -216,13 +216,16 @@ constexpr SumTab3 make_sumtab3() {   // entry { q1, q2 }: 40 - H(0..3), 80 + H(0
     return t;
 }
 static_assert(alignof(StreamBasis) >= 16 && alignof(SumTab4) >= 16 && alignof(SumTab3) >= 16, "to_lds16 reads 16 bytes a lane");
+__device__ const StreamBasis kBasis3 = make_basis(0x8000u);   // sums_of's for P = 3: bit 15 flipped
 __device__ const SumTab4 kSumTab4 = make_sumtab4();
 __device__ const SumTab3 kSumTab3 = make_sumtab3();
+template <int P>
+__device__ __forceinline__ const uint32_t* sum_basis() { return P == 4 ? kBasis.v : kBasis3.v; }
 template <int P>
 constexpr int sum_tab_words() { return P == 4 ? 768 : 1024; }   // LDS: [0, 512) the stream basis, then the table above
 template <int P>
 __device__ __forceinline__ void load_sum_tables(uint32_t* tab) {
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = kBasis.v[i];
+    for (int i = threadIdx.x; i < 512; i += blockDim.x) tab[i] = sum_basis<P>()[i];
     for (int i = threadIdx.x; i < sum_tab_words<P>() - 512; i += blockDim.x) tab[512 + i] = P == 4 ? kSumTab4.v[i] : kSumTab3.v[i];
 }
 // The same, requested into the LDS (16-byte aligned) by the workgroup's first four waves: beside the kernel's other first loads they cost no
@@ -233,13 +236,13 @@ template <int P>
 __device__ __forceinline__ void tables_to_lds(uint32_t* tab) {
     const int w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t* const rest = P == 4 ? kSumTab4.v : kSumTab3.v;
-    if (256 * w < sum_tab_words<P>()) to_lds16((w < 2 ? kBasis.v + 256 * w : rest + 256 * (w - 2)) + 4 * lane, (uint8_t*) (tab + 256 * w));
+    if (256 * w < sum_tab_words<P>()) to_lds16((w < 2 ? sum_basis<P>() + 256 * w : rest + 256 * (w - 2)) + 4 * lane, (uint8_t*) (tab + 256 * w));
 }
 // The same for a workgroup of exactly NTHR threads (256, 512 or 1024), in two halves: a thread's loads are requested in
 // tables_fetch() (put it beside the kernel's other first loads), and tables_store() writes them to LDS once they are needed -
 // the loop above waits for every load in turn, one memory round trip each.
 template <int P>
-__device__ __forceinline__ uint32_t sum_tab_word(int i) { return i < 512 ? kBasis.v[i] : P == 4 ? kSumTab4.v[i - 512] : kSumTab3.v[i - 512]; }
+__device__ __forceinline__ uint32_t sum_tab_word(int i) { return i < 512 ? sum_basis<P>()[i] : P == 4 ? kSumTab4.v[i - 512] : kSumTab3.v[i - 512]; }
 template <int P, int NTHR>
 struct TableWords {
     uint32_t w[(sum_tab_words<P>() + NTHR - 1) / NTHR];
@@ -277,6 +280,15 @@ __device__ __forceinline__ int dot8c(uint32_t w) {
     asm("v_dot8_i32_i4 %0, %1, %2, 0" : "=v"(d) : "v"(w), "s"(C));
     return d;
 }
+// A block's exponent code: nibble n of w (constant once unrolled).  P = 3: spelled out, for left to itself the compiler moves the shift by 23 in front, and
+// code << 23 plus a constant is three instructions instead of two.
+template <int P>
+__device__ __forceinline__ uint32_t code_of(uint32_t w, int n) {
+    if constexpr (P == 4) return (w >> (4 * n)) & 15u;
+    uint32_t c;
+    asm("v_bfe_u32 %0, %1, %2, 4" : "=v"(c) : "v"(w), "n"(4 * n));
+    return c;
+}
 struct SumCoefs {
     uint32_t lo, hi;   // the tables
     uint32_t m;        // the multiplier, int16
@@ -305,7 +317,19 @@ __device__ __forceinline__ SumCoefs sum_coefs(uint32_t cc, int odd, const uint32
     }
     return s;
 }
-// The eight y of N blocks.  up: any word whose upper 16 bits are the seed; g: the 32 stream bits that follow.  hook(0 .. 3) is called between the phases: a
+// A constant that the compiler keeps in a vector register: an instruction of three operands takes one scalar of them, and with both constants known the
+// compiler makes two instructions of it instead.  (P = 3: a window's selector in one instruction instead of two, 78 -> 68.5 a block in the GEMMs with the flipped
+// bit and the code below.  us a layer step: 3 tokens, E 64, top-4, d 2880, ff 2880 115.3 -> 109.3; 4 tokens, E 128, top-8, d 2048, ff 768 52.7 -> 48.8; 106, E 64, top-2,
+// d 3840, ff 576 155.8 -> 147.6; dense, 6 tokens, 2880 x 2880 10.2 -> 9.9.  The same for P = 4, one instruction of 69 less, is no gain: grouped GEMMs
+// - 1.5 %, dense matrices of few tokens + 1 to + 4 %.)
+template <uint32_t C>
+__device__ __forceinline__ uint32_t vconst() {
+    uint32_t v;
+    asm("v_mov_b32 %0, %1" : "=v"(v) : "i"(C));
+    return v;
+}
+// The eight y of N blocks.  up: any word whose upper 16 bits are the seed; g: stream_of its table (the 32 stream bits that follow; P = 3: bit 15 flipped, as a
+// signed product wants the top bit of one of its windows).  hook(0 .. 3) is called between the phases: a
 // caller with matrix instructions to issue puts them there, where the vector ALU has work beside them, and one whose wave has a SIMD's vector issue to itself
 // holds the scheduler to the phases, in which every operand of several blocks is a dozen instructions old.
 template <int P, int N, class Hook>
@@ -339,20 +363,24 @@ __device__ __forceinline__ void sums_of(const uint32_t (&up)[N], const uint32_t 
         hook(3);
     } else {
         uint32_t W[N][8];
+        const uint32_t q = vconst<0x0C040C00u>();
 #pragma unroll
         for (int c = 0; c < 8; ++c)
 #pragma unroll
             for (int n = 0; n < N; ++n) W[n][c] = c < 5 ? __builtin_amdgcn_alignbit(g[n], up[n], 17 + 3 * c) : g[n] >> (3 * c - 15);   // state 3c + 1 and the bits above it
         hook(0);
+        // (state - 32768: bit 15 flipped.  In g it comes flipped, which is window 5's, bit 12 of window 6 and bit 9 of window 7; bits 18 and up of the others,
+        // where nothing reads it)
 #pragma unroll
         for (int c = 0; c < 8; ++c)
 #pragma unroll
-            for (int n = 0; n < N; ++n) y[n][c] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, (W[n][c] & 0x00030003u) | 0x0C040C00u);
+            for (int n = 0; n < N; ++n)
+                if (c != 5) W[n][c] ^= c < 5 ? 0x8000u : c == 6 ? 0x9000u : 0x8200u;
         hook(1);
 #pragma unroll
         for (int c = 0; c < 8; ++c)
 #pragma unroll
-            for (int n = 0; n < N; ++n) W[n][c] ^= 0x8000u;
+            for (int n = 0; n < N; ++n) y[n][c] = __builtin_amdgcn_perm(s[n].hi, s[n].lo, __builtin_amdgcn_bitop3_b32(W[n][c], 0x00030003u, q, 0xEA));   // (W & ..) | q
         hook(2);
 #pragma unroll
         for (int c = 0; c < 8; ++c)

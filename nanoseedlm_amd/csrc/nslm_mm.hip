@@ -420,7 +420,7 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                         sums_of<P>(r.u, k.g[1], sc[1], y[1], [](int) {});
                     }
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) sums_scaled<P>(y[h], sc[h].k, FMT == MF_SEED4P4 ? (r.c >> (4 * h)) & 15u : (r.v >> (16 * h)) & 15u, f[h]);
+                    for (int h = 0; h < 2; ++h) sums_scaled<P>(y[h], sc[h].k, FMT == MF_SEED4P4 ? code_of<P>(r.c, h) : code_of<P>(r.v, 4 * h), f[h]);
                 } else if (FMT == MF_BF16) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {

@@ -59,7 +59,7 @@ __device__ __forceinline__ bf16x8 seed_weights(uint32_t u, uint32_t v, int odd, 
     uint32_t y[8];
     sums_of<P>(odd ? u : u << 16, g, sc, y, [&](int i) { hook(1 + i); });
     float f[8];
-    sums_scaled<P>(y, sc.k, P == 4 ? (codes >> (4 * odd)) & 15u : (v >> (16 * odd)) & 15u, f);
+    sums_scaled<P>(y, sc.k, P == 4 ? code_of<P>(codes, odd) : code_of<P>(v, 4 * odd), f);
     hook(5);
     bf16x8 w = __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
     hook(6);

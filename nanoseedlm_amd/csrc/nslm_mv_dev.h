@@ -62,7 +62,7 @@ __device__ __forceinline__ float block_of(const Chunk& ck, int b, uint32_t ebase
     uint32_t y[8];
     sums_of<P>((b & 1) ? ss : ss << 16, g, sc, y, [](int) {});
     sums_float<P>(y, sc.k, w);
-    const uint32_t code = P == 4 ? (ck.codes >> (4 * b)) & 15u : (cc >> (16 * (b & 1))) & 15u;
+    const uint32_t code = P == 4 ? code_of<P>(ck.codes, b) : code_of<P>(cc, 4 * (b & 1));
     return __uint_as_float((code << 23) + ebase);
 }
 // a block's products with 8 activations, in order.  REGS: they are in registers, else in LDS
@@ -111,7 +111,7 @@ __device__ __forceinline__ void chunk_post(const Chunk& ck, const float (&w)[8][
     const uint32_t ebase = sums_e2(eb);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-        const uint32_t code = P == 4 ? (ck.codes >> (4 * b)) & 15u : (word_of(ck.cw, b >> 1) >> (16 * (b & 1))) & 15u;
+        const uint32_t code = P == 4 ? code_of<P>(ck.codes, b) : code_of<P>(word_of(ck.cw, b >> 1), 4 * (b & 1));
         acc = fmaf(block_dot(w[b], xr + 8 * b), __uint_as_float((code << 23) + ebase), acc);
     }
 }
