@@ -215,16 +215,7 @@ __device__ __forceinline__ f32x4 scaled(const f32x4& s, int eb) {
     return (f32x4) {mm_scale<FMT>(s[0], eb), mm_scale<FMT>(s[1], eb), mm_scale<FMT>(s[2], eb), mm_scale<FMT>(s[3], eb)};
 }
 // four sums of pair / token dst, rows orow .. orow + 3 (those below R)
-// BITS: a launch may ask for BF16 bits (k_mm_wide; in the other kernels the branch cost registers, and small launches up to 3 %)
-template <bool BITS = false>
 __device__ __forceinline__ void store_rows(const MmArgs& a, float* Y, int dst, int orow, const f32x4& s) {
-    if (BITS && a.f32out == OUT_BF16) {
-        uint16_t* o = (uint16_t*) Y + (size_t) dst * a.ys + orow;
-        if ((a.ys & 3) == 0 && orow + 4 <= a.R && ((uintptr_t) o & 7u) == 0) *(uint2*) o = make_uint2(pack_bf2(s[0], s[1]), pack_bf2(s[2], s[3]));
-        else
-            for (int j = 0; j < 4 && orow + j < a.R; ++j) o[j] = (uint16_t) tobf(s[j]);
-        return;
-    }
     float* yo = Y + (size_t) dst * a.ys + orow;
     if ((a.ys & 3) == 0 && orow + 4 <= a.R && !a.add && !a.f32out && ((uintptr_t) yo & 15u) == 0) *(f32x4*) yo = (f32x4) {bfr(s[0]), bfr(s[1]), bfr(s[2]), bfr(s[3])};
     else
@@ -383,28 +374,32 @@ constexpr int wide_lds() { return 2 * (NT * 2048 + 8 * step_bytes<FMT, 1, NT, fa
 template <int FMT, int NT>
 __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, const uint16_t* X, float* Y, const int32_t* perm, int start, int count,
                                           int r0, const uint32_t* tab, uint8_t* lds) {
-    constexpr int SB = step_bytes<FMT, 1, NT, false>();
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
+    static_assert(NT % 2 == 0, "half the sums fit the activations' LDS");
+    constexpr int SB = step_bytes<FMT, 1, NT, false>(), NS = (NT + 3) / 4;   // NS: 64 pairs each
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // (an item's own: kept out of the loop over items, whose registers it would take)
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, g = lane >> 4;
     const bool gu = a.a16 != nullptr;   // waves 0 - 3: gate rows, 4 - 7: the same rows of up
     const int nch = a.K / 64, rw = r0 + 16 * (gu ? w & 3 : w);
     Weights<FMT, 1> W(m, m, false, a.K, a.R, rw, lane);
     uint8_t* const ws = lds + 2 * NT * 2048 + w * 2 * SB;
-    uint32_t px[NT / 4];   // in 16-byte pieces: the wave stages eight pairs' rows of every 64
+    uint32_t px[NS];   // in 16-byte pieces: the wave stages eight pairs' rows of every 64
 #pragma unroll
-    for (int i = 0; i < NT / 4; ++i) {
+    for (int i = 0; i < NS; ++i) {
         const int n = 64 * i + 8 * w + (lane >> 3);
         px[i] = (uint32_t) (((size_t) (perm[start + min(n, count - 1)] / a.xdiv) * (size_t) a.xs) >> 3) + (uint32_t) ((lane & 7) ^ x_swizzle16(n & 15));
     }
     auto request_x = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < NT / 4; ++i) to_lds16((const uint8_t*) X + (size_t) (px[i] + 8u * (uint32_t) c) * 16, lds + (c & 1) * NT * 2048 + 1024 * (8 * i + w));
+        for (int i = 0; i < NS; ++i)
+            if (NT % 4 == 0 || i + 1 < NS || w < 2 * (NT % 4)) to_lds16((const uint8_t*) X + (size_t) (px[i] + 8u * (uint32_t) c) * 16, lds + (c & 1) * NT * 2048 + 1024 * (8 * i + w));
     };
     f32x4 acc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[nt] = (f32x4) {0.0f, 0.0f, 0.0f, 0.0f};
     // The matrix instructions of half a chunk are issued among the vector instructions that decode the next half.  A wave's records run a chunk
     // ahead of its activations.
-    constexpr int NG = (NT + 7) / 8;   // token tiles a hook
+    constexpr int NG = (NT + 7) / 8;   // token tiles a hook, at most: hook i has tiles i NT / 8 and up
     constexpr int XD = 2;               // hooks a fragment is read ahead of its use
     typename Weights<FMT, 1>::Step st;
     bf16x8 wb, xq[XD][NG];
@@ -413,15 +408,17 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
         auto fetch = [&](int i) {
 #pragma unroll
             for (int j = 0; j < NG; ++j)
-                if (i < 8 && NG * i + j < NT) xq[i % XD][j] = *(const bf16x8*) (xt + (NG * i + j) * 2048);
+                if (i < 8 && i * NT / 8 + j < (i + 1) * NT / 8) xq[i % XD][j] = *(const bf16x8*) (xt + (i * NT / 8 + j) * 2048);
         };
 #pragma unroll
         for (int i = 0; i < XD; ++i) fetch(i);
         wb = W.block(st, 0, h ^ 1, tab, [&](int i) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < NG; ++j)
-                if (NG * i + j < NT) acc[NG * i + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, xq[i % XD][j], acc[NG * i + j], 0, 0, 0);
+            for (int j = 0; j < NG; ++j) {
+                const int nt = i * NT / 8 + j;
+                if (nt < (i + 1) * NT / 8) acc[nt < NT ? nt : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, xq[i % XD][j], acc[nt < NT ? nt : 0], 0, 0, 0);
+            }
             fetch(i + XD);
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -441,26 +438,57 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
         loads_issued();
         half(c, 1);   // (past the end: some block again)
     }
-    const int orow = rw + 4 * g;
+    // The sums go to the LDS of the activations, and from there to their pairs in a loop: 64 or 128 rows of a pair side by side, by all waves.  (Out of
+    // the registers, a pass's code was 10 to 50 KB that ran once an item, as fast as it could be fetched: 13K of an item's 120K clocks; 1917 rows, E 16,
+    // top-8, d 1792, ff 384, P = 3: 181 -> 168 us.)  Row group q of four, token t: slot t ^ mix(q) of the group's 16, so that the reads, of many groups'
+    // same token, reach all banks as the writes do.
+    auto mix = [](int q) { return (q ^ (q >> 4)) & 15; };
+    const int q = 4 * (gu ? w & 3 : w) + g, slot = 16 * g + (t ^ mix(q));
+    __syncthreads();
+    if (gu || a.f32out == OUT_BF16) {   // as the BF16 that is stored, or that SwiGLU reads
+        uint2* const red = (uint2*) lds;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = scaled<FMT>(acc[nt], m.eb);
-    if (gu) {   // the up sums meet the gate sums in LDS
-        f32x4* const red = (f32x4*) lds;
-        __syncthreads();
-        if (w >= 4) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) red[((w - 4) * NT + nt) * 64 + lane] = acc[nt];
+        for (int nt = 0; nt < NT; ++nt) {
+            const f32x4 s = scaled<FMT>(acc[nt], m.eb);
+            red[(w * NT + nt) * 64 + slot] = make_uint2(pack_bf2(s[0], s[1]), pack_bf2(s[2], s[3]));
         }
         __syncthreads();
-        if (w >= 4) return;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            if (16 * nt + t < count && orow < a.R) store_swiglu(a, perm[start + 16 * nt + t], orow, acc[nt], red[(w * NT + nt) * 64 + lane]);
+        const int lg = gu ? 4 : 5, oq = tid & ((1 << lg) - 1), orow = r0 + 4 * oq, step = 512 >> lg;
+        if (orow >= a.R) return;
+        const uint2* const own = red + (oq >> 2) * NT * 64 + 16 * (oq & 3);
+        int n = tid >> lg, dst = perm[start + min(n, count - 1)];
+#pragma unroll 1
+        for (; n < count; n += step) {
+            const int next = perm[start + min(n + step, count - 1)], at = (n >> 4) * 64 + ((n & 15) ^ mix(oq));
+            const uint2 v = own[at];
+            const f32x4 s = {bf(v.x & 0xFFFFu), bf(v.x >> 16), bf(v.y & 0xFFFFu), bf(v.y >> 16)};
+            if (gu) {
+                const uint2 u = own[4 * NT * 64 + at];
+                store_swiglu(a, dst, orow, s, (f32x4) {bf(u.x & 0xFFFFu), bf(u.x >> 16), bf(u.y & 0xFFFFu), bf(u.y >> 16)});
+            } else {
+                uint16_t* const o = (uint16_t*) Y + (size_t) dst * a.ys + orow;
+                if ((a.ys & 3) == 0 && orow + 4 <= a.R && ((uintptr_t) o & 7u) == 0) *(uint2*) o = v;
+                else
+                    for (int j = 0; j < 4 && orow + j < a.R; ++j) o[j] = (uint16_t) (__float_as_uint(s[j]) >> 16);
+            }
+            dst = next;
+        }
         return;
     }
+    f32x4* const red = (f32x4*) lds;
+    const int oq = tid & 31, orow = r0 + 4 * oq;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-        if (16 * nt + t < count && orow < a.R) store_rows<true>(a, Y, perm[start + 16 * nt + t], orow, acc[nt]);
+    for (int part = 0; part < 2; ++part) {   // (half the pairs' fit)
+        if (8 * NT * part >= count) return;
+        if (part) __syncthreads();
+#pragma unroll
+        for (int nt = 0; nt < NT / 2; ++nt) red[(w * (NT / 2) + nt) * 64 + slot] = scaled<FMT>(acc[part * (NT / 2) + nt], m.eb);
+        __syncthreads();
+#pragma unroll 1
+        for (int n = tid >> 5; n < min(8 * NT, count - 8 * NT * part); n += 16)
+            if (orow < a.R)
+                store_rows(a, Y, perm[start + 8 * NT * part + n], orow, red[((oq >> 2) * (NT / 2) + (n >> 4)) * 64 + 16 * (oq & 3) + ((n & 15) ^ mix(oq))]);
+    }
 }
 
 // Who computes a tile of a grouped launch, whatever table the host made: k_mm_wide takes every tile of more than `least` pairs, alone or together
@@ -580,33 +608,78 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     }
 }
 
-// A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join)
+// A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join).  The grid is what runs at once, two workgroups a CU, and a
+// workgroup takes items blockIdx.x, + gridDim.x, .. of (matrix, tile, block of rows): with a workgroup an item, the ones that found nothing to do between
+// them, they were started in turn over the shader engines, and an engine that was full kept the free places of the others waiting, 20 to 40 us of an
+// item's 75 (2048 rows, E 128, top-8, d 2048, ff 768: 54 to 58 of an XCD's 64 places taken; 435 us a
+// layer step, 415 so).  Its tiles are found 64 a wave at once and listed in LDS: an item is then two dependent loads from its slice, as it was.
+// Passes of 64, 96, 128, 160, 192 and 256 pairs: an expert's share of a step spreads round its mean, and of 128 pairs on average half have a few more,
+// joined to the full tile (in passes of 64, 128, 192 and 256, of which the middle two met: 6 % of that step).  Passes of 144 and 224 gave nothing more.
+#define WIDE_TILES 1024   // of the table, looked at together
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ __attribute__((aligned(16))) uint32_t tab[mm_tab_words<FMT>()];
-    const int nt = ntiles ? *ntiles : grid_tiles, y = (int) blockIdx.y;
-    if (y >= nt) return;
-    const MmTile tl = tiles[y];
+    __shared__ uint16_t list[WIDE_TILES];
+    __shared__ uint64_t cans[WIDE_TILES / 64], large[WIDE_TILES / 64];
+    __shared__ int found;
+    const int nt = ntiles ? min(*ntiles, grid_tiles) : grid_tiles;
     const Join join = {a.least, a.least > 0 || at.pairs(nt) ? MMT_BN : FEW};
-    if (tl.count <= a.least || join.joins(tiles, y)) return;
-    if (blockIdx.z) {   // the launch's second matrix: same tiles and activations, its own slices and output
-        ws = a.ws2;
-        Y = a.y2;
-    }
     const bool gu = a.a16 != nullptr;
-    const WSlice m = gu && __builtin_amdgcn_readfirstlane((int) threadIdx.x) >= 256 ? a.ws2[tl.slice] : ws[tl.slice];
-    int count = tl.count;
-    if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
+    const int blocks = (a.R + (gu ? 63 : 127)) / (gu ? 64 : 128);
     if constexpr (seed_fmt<FMT>()) tables_to_lds<seed_p<FMT>()>(tab);
-    const int r0 = (int) blockIdx.x * (gu ? 64 : 128);
-#define W(NT) wide_tile<FMT, NT>(a, m, X, Y, perm, tl.start, count, r0, tab, lds)
-    if (count <= 64) W(4);
-    else if (count <= 128) W(8);
-    else if (count <= 192) W(12);
-    else W(16);
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    const WSlice* const mine_ws = gu && wave >= 4 ? a.ws2 : ws;   // waves 4 - 7: up
+    int run = 0;   // (wave 0) of tiles that can join the one before them, up to the last one looked at
+    for (int base = 0;; base += WIDE_TILES) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));   // (as in wide_tile: nothing of this is kept)
+        for (int g = wave; g < WIDE_TILES / 64 && base + 64 * g < grid_tiles; g += 8) {   // (their loads do not wait for *ntiles)
+            const int y = base + 64 * g + lane, at_y = min(y, grid_tiles - 1);
+            const MmTile t = tiles[at_y], before = tiles[max(at_y - 1, 0)];
+            const uint64_t c = __ballot(y > 0 && join.can(t, before)), l = __ballot(y < nt && t.count > a.least);
+            if (lane == 0) {
+                cans[g] = c;
+                large[g] = l;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {   // this launch's tiles
+            int n = 0;
+            for (int g = 0; g < WIDE_TILES / 64 && base + 64 * g < nt; ++g) {
+                const uint64_t stop = ~cans[g] & (~0ull >> (63 - lane));
+                const int len = stop ? lane - (63 - __clzll((long long) stop)) : run + lane + 1;
+                const bool mine = ((large[g] >> lane) & 1) && !(len & 1);
+                const uint64_t m = __ballot(mine);
+                if (mine) list[n + __popcll(m & ~(~0ull << lane))] = (uint16_t) (64 * g + lane);
+                n += __popcll(m);
+                run = __builtin_amdgcn_readlane(len, 63);
+            }
+            if (lane == 0) found = n;
+        }
+        __syncthreads();
+        const int n = __builtin_amdgcn_readfirstlane(found), items = n * blocks * (a.ws2 && !gu ? 2 : 1);
+        for (int item = (int) blockIdx.x; item < items; item += (int) gridDim.x) {
+            const int ti = item / blocks, second = ti >= n;   // second: the launch's second matrix: same tiles and activations, its own slices and output
+            const int y = base + __builtin_amdgcn_readfirstlane((int) list[second ? ti - n : ti]);
+            const MmTile tl = tiles[y];
+            const WSlice m = (second ? a.ws2 : mine_ws)[tl.slice];
+            int count = tl.count;
+            if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
+            const int r0 = (item - ti * blocks) * (gu ? 64 : 128);
+            __syncthreads();   // the item before has read the LDS
+#define W(NT) wide_tile<FMT, NT>(a, m, X, second ? a.y2 : Y, perm, tl.start, count, r0, tab, lds)
+            if (count <= 64) W(4);
+            else if (count <= 96) W(6);
+            else if (count <= 128) W(8);
+            else if (count <= 160) W(10);
+            else if (count <= 192) W(12);
+            else W(16);
 #undef W
+        }
+        if (base + WIDE_TILES >= nt) return;
+    }
 }
 
 template <int FMT, int RT, int NT, bool PACKED>
@@ -683,7 +756,8 @@ template <int FMT>
 void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
           int grid_tiles) {
     const int rows = a.a16 ? 64 : 128;
-    const dim3 grid((unsigned) (a.R + rows - 1) / rows, (unsigned) grid_tiles, a.ws2 && !a.a16 ? 2u : 1u);
+    const long long most = (long long) ((a.R + rows - 1) / rows) * grid_tiles * (a.ws2 && !a.a16 ? 2 : 1), once = 2 * host_cu_count();
+    const dim3 grid((unsigned) (most < once ? most : once));
     constexpr size_t lds = wide_lds<FMT, 16>();
     allow_big_lds<k_mm_wide<FMT>>(lds);
     hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(a));

@@ -1037,6 +1037,67 @@ def test_mm_grouped_every_tile_of_any_table(be, oracle, fmt, table):
         b.free()
 
 
+@pytest.mark.parametrize("fmt", [packs.MF_SEED4P4, packs.MF_BF16])
+@pytest.mark.parametrize("times", [1, 42])
+def test_mm_grouped_wide_passes_and_long_tables(be, oracle, fmt, times):
+    """Pair counts on both sides of every pass of the kernel of full tiles, alone and joined; 42 times over, more work than workgroups and a run of
+    tiles that can join across row 1024 of the table.  Values to ref_mm's bound, BF16 results and SwiGLU bit for bit."""
+    import ctypes as C
+    from nanoseedlm_amd import backend, moe
+    L = backend.hip()
+    rng = np.random.default_rng(times)
+    E, R, K = 4, 76, 64
+    runs = [[n] for n in (1, 64, 65, 96, 97, 128)] + [[128, n - 128] for n in (129, 160, 161, 192, 193, 256)] + [[128, 0], [3]]
+    runs = runs * times
+    cut = next((i for i in range(len(runs)) if sum(map(len, runs[:i])) >= 1021), 0)
+    runs.insert(cut, [40, 128, 128, 64, 70, 33, 2])
+    tl = [(i % E, n) for i, run in enumerate(runs) for n in run]
+    P, mt, tile_rows = sum(n for _, n in tl), len(tl) + 3, 129
+    pk = [make_pack(rng, fmt, E, R, K) for _ in range(2)]
+    keep, tabs = [], []
+    for p in pk:
+        arr = (backend.WSlice * E)()
+        for name, i in [("seeds", 0), ("coefs", 1), ("codes", 3)] if fmt == packs.MF_SEED4P4 else [("w", 0)]:
+            buf = moe.DevBuf.from_array(np.ascontiguousarray(p[name]))
+            keep.append(buf)
+            for e in range(E):
+                arr[e].p[i] = buf.ptr.value + e * (buf.nbytes // E)
+        for e in range(E):
+            arr[e].eb, arr[e].gs = (int(p["eb"][e]), 0) if "eb" in p else (0, 6)
+        tabs.append(moe.DevBuf(C.sizeof(arr)))
+        backend.check(L.nh_memcpy_h2d(tabs[-1].ptr, arr, C.c_size_t(C.sizeof(arr))), "nh_memcpy_h2d")
+    start = np.concatenate([[0], np.cumsum([n for _, n in tl])])
+    tiles = np.array([[s, start[i], n, 0] for i, (s, n) in enumerate(tl)], dtype=np.int32)
+    perm = rng.permutation(P).astype(np.int32)
+    slc = np.empty(P, dtype=np.int32)
+    slc[perm] = np.repeat([s for s, _ in tl], [n for _, n in tl])
+    x = packs.round_bf16(rng.standard_normal((P, K)).astype(np.float32))
+    dx = moe.DevBuf.from_array(packs.f32_to_bf16_bits(x))
+    dperm, dtiles, dn = (moe.DevBuf.from_array(np.ascontiguousarray(v, dtype=np.int32)) for v in (perm, tiles, [len(tiles)]))
+    y = [moe.DevBuf.from_array(np.full((P, R), np.nan, dtype=np.float32)) for _ in range(3)]
+    b16 = [moe.DevBuf.from_array(np.full((P, R), 0x7FC0, dtype=np.uint16)) for _ in range(3)]
+    more = (R, 1, dperm.ptr, dtiles.ptr, dn.ptr, mt, tile_rows)
+    L.kc_mm_grouped_packed_pair(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, y[0].ptr, y[1].ptr, *more)
+    L.kc_mm_grouped_packed_rows(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, y[2].ptr, *more)
+    assert L.kc_mm_grouped_packed_bf16(None, fmt, tabs[0].ptr, K, R, dx.ptr, K, b16[0].ptr, *more) == 0
+    assert L.kc_mm_grouped_swiglu(None, fmt, tabs[0].ptr, tabs[1].ptr, K, R, dx.ptr, K, b16[1].ptr, *more) == 0
+    n = P * R // 8 * 8
+    L.kc_swiglu_pack(None, y[0].ptr, y[1].ptr, b16[2].ptr, C.c_size_t(n))
+    moe.device_sync()
+    got = [b.to_array(np.float32, (P, R)) for b in y]
+    for j in range(2):
+        for e in range(E):
+            ref, mag = ref_mm(oracle, pk[j], e, x[slc == e], 0)
+            assert close_bf(got[j][slc == e], packs.round_bf16(ref.astype(np.float32)), F32B * mag).all(), (j, e)
+    assert np.array_equal(got[0].view(np.uint32), got[2].view(np.uint32))
+    bits = [b.to_array(np.uint16, (P, R)) for b in b16]
+    assert np.array_equal(bits[0], got[0].view(np.uint32) >> 16)
+    assert np.array_equal(bits[1].ravel()[:n], bits[2].ravel()[:n])
+    assert L.kc_last_error() == 0
+    for b in keep + tabs + y + b16 + [dx, dperm, dtiles, dn]:
+        b.free()
+
+
 def _grouped_rows_case(fmt, T, ind, rng):
     """kc_bucket on ind [T][4] of 9 experts, then kc_mm_grouped_packed and kc_mm_grouped_packed_rows(tile_rows = T) on the same
     tiles (R 72: not a multiple of a tile): both results as uint32 [P][R], and the permutation."""
