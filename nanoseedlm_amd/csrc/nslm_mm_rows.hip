@@ -497,22 +497,20 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 // join another itself: the parity of the run of tiles that can, up to the last one that cannot.  A wave looks at 64 tiles at once (a
 // token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile is a chain of as many loads).
 // Beside k_mm_rows_grouped every tile can join: which kernel computes a tile, and with it its sums' order, is then a matter of the table alone,
-// not of the matrices in the launch.  Alone k_mm_wide pairs full tiles only where the pairs fill the chip: a pair saves a decode and leaves half
-// the workgroups.  Two a CU run at once (512).  Up to so many, and in a second round that they fill, full tiles are faster alone; us a layer
-// step, P = 4, full tiles alone and in pairs, with the workgroups of tiles alone: E 16, top-2, d 2048, ff 1024, 2048 rows on the same two
-// experts (512) 171 and 222; E 32, top-4, d 512, ff 256, 2048 rows (312) 95 and 120; E 64, top-8, d 640, ff 384, 1531 rows (768 and 640) 131
-// and 144; just past a round: E 16, top-2, d 4096, ff 2048, 512 rows (576) 299 and 269; E 128, top-8, d 2048, ff 768, 2048 rows (2292 and
-// 3056) 580 and 543.  A tile of up to FEW pairs joins at any number: with a full one it fits the 192 pairs of a smaller pass (E 16, top-8,
-// d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138; E 16, top-2, d 2048, ff 1024, 2048 rows, one expert
-// in all: 215, 179, 179; 138 cases of 60 to 600 pairs an expert, geometric mean against no rule: 0.944, 0.943, 0.941).
+// not of the matrices in the launch.  Alone k_mm_wide pairs full tiles where their workgroups are more than 5/8 of the two a CU that run at once: a
+// pair saves a decode and leaves half the workgroups.  us for so many workgroups of a full tile, and for half as many of a pair (K 2048, P = 4):
+// 256 44 and 56, 320 63 and 57, 512 69 and 64, 768 97 and 94, 1024 134 and 105, 1536 210 and 149.  36 layer steps of 140 to 620 pairs an expert:
+// geometric mean 0.917 of the time of a workgroup a tile, with one round as the line 0.925, with two 0.941.  A tile of up to FEW pairs joins at any number: it adds a pass's step to a full one's, no decode (E 16, top-8,
+// d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138).
+// Where workgroups are started a tile each (Q8) a pair's second one is an empty one: there full tiles stay alone up to a round and in a second that they
+// fill (E 16, top-2, d 2048, ff 1024, 2048 rows on the same two experts, 512 workgroups: 171 alone, 222 in pairs; 576: 299 and 269).
 #define FEW 64
 struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and between [0] and [1]
     int n[3];
-    explicit JoinAt(const MmArgs& a) {
-        const int blocks = a.a16 ? (a.R + 63) / 64 : (a.R + 127) / 128 * (a.ws2 ? 2 : 1), round = 2 * host_cu_count();   // a tile's workgroups; at once
-        n[0] = round / blocks;
-        n[1] = (5 * round / 4 + blocks - 1) / blocks;
-        n[2] = (2 * round + blocks - 1) / blocks;
+    JoinAt(int blocks, int round, bool dealt) {   // a tile's workgroups; those that run at once
+        n[0] = dealt ? 0 : round / blocks;
+        n[1] = dealt ? 0 : (5 * round / 4 + blocks - 1) / blocks;
+        n[2] = dealt ? 5 * round / 8 / blocks + 1 : (2 * round + blocks - 1) / blocks;
     }
     __device__ __forceinline__ bool pairs(int nt) const { return nt >= n[2] || (nt > n[0] && nt < n[1]); }
 };
@@ -615,15 +613,16 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
 // layer step, 415 so).  Its tiles are found 64 a wave at once and listed in LDS: an item is then two dependent loads from its slice, as it was.
 // Passes of 64, 96, 128, 160, 192 and 256 pairs: an expert's share of a step spreads round its mean, and of 128 pairs on average half have a few more,
 // joined to the full tile (in passes of 64, 128, 192 and 256, of which the middle two met: 6 % of that step).  Passes of 144 and 224 gave nothing more.
+// Fuller items come first: what a workgroup has more than another is then one of the smallest (E 16, top-4, d 2048, ff 1600, 1152 rows, experts of
+// 256 and 32 pairs: 259 us a layer step in the table's order, 229 so).  Two workgroups' LDS of Q8 leave no room for the list: there a workgroup has the tile of its row.
 #define WIDE_TILES 1024   // of the table, looked at together
+template <int FMT>
+constexpr bool wide_deals() { return FMT != MF_Q8; }
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles, JoinAt at) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ __attribute__((aligned(16))) uint32_t tab[mm_tab_words<FMT>()];
-    __shared__ uint16_t list[WIDE_TILES];
-    __shared__ uint64_t cans[WIDE_TILES / 64], large[WIDE_TILES / 64];
-    __shared__ int found;
     const int nt = ntiles ? min(*ntiles, grid_tiles) : grid_tiles;
     const Join join = {a.least, a.least > 0 || at.pairs(nt) ? MMT_BN : FEW};
     const bool gu = a.a16 != nullptr;
@@ -631,6 +630,29 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     if constexpr (seed_fmt<FMT>()) tables_to_lds<seed_p<FMT>()>(tab);
     const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const WSlice* const mine_ws = gu && wave >= 4 ? a.ws2 : ws;   // waves 4 - 7: up
+    auto item = [&](int y, bool second, int r0) {   // second: the launch's second matrix: same tiles and activations, its own slices and output
+        const MmTile tl = tiles[y];
+        const WSlice m = (second ? a.ws2 : mine_ws)[tl.slice];
+        int count = tl.count;
+        if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
+        __syncthreads();   // the item before has read the LDS
+#define W(NT) wide_tile<FMT, NT>(a, m, X, second ? a.y2 : Y, perm, tl.start, count, r0, tab, lds)
+        if (count <= 64) W(4);
+        else if (count <= 96) W(6);
+        else if (count <= 128) W(8);
+        else if (count <= 160) W(10);
+        else if (count <= 192) W(12);
+        else W(16);
+#undef W
+    };
+    if constexpr (!wide_deals<FMT>()) {
+        const int y = (int) blockIdx.y;
+        if (y < nt && tiles[y].count > a.least && !join.joins(tiles, y)) item(y, blockIdx.z, (int) blockIdx.x * (gu ? 64 : 128));
+        return;
+    }
+    __shared__ uint16_t list[WIDE_TILES];   // the launch's tiles: those of more than 64 pairs from the front, the others from the back
+    __shared__ uint64_t cans[WIDE_TILES / 64], large[WIDE_TILES / 64], fuller[WIDE_TILES / 64];
+    __shared__ int2 found;
     int run = 0;   // (wave 0) of tiles that can join the one before them, up to the last one looked at
     for (int base = 0;; base += WIDE_TILES) {
         int lane = threadIdx.x & 63;
@@ -638,45 +660,34 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
         for (int g = wave; g < WIDE_TILES / 64 && base + 64 * g < grid_tiles; g += 8) {   // (their loads do not wait for *ntiles)
             const int y = base + 64 * g + lane, at_y = min(y, grid_tiles - 1);
             const MmTile t = tiles[at_y], before = tiles[max(at_y - 1, 0)];
-            const uint64_t c = __ballot(y > 0 && join.can(t, before)), l = __ballot(y < nt && t.count > a.least);
+            const uint64_t c = __ballot(y > 0 && y < nt && join.can(t, before)), l = __ballot(y < nt && t.count > a.least), f = __ballot(t.count > 64);
             if (lane == 0) {
                 cans[g] = c;
                 large[g] = l;
+                fuller[g] = f;
             }
         }
         __syncthreads();
-        if (wave == 0) {   // this launch's tiles
-            int n = 0;
+        if (wave == 0) {
+            int n = 0, few = 0;
             for (int g = 0; g < WIDE_TILES / 64 && base + 64 * g < nt; ++g) {
-                const uint64_t stop = ~cans[g] & (~0ull >> (63 - lane));
+                const uint64_t can = cans[g], stop = ~can & (~0ull >> (63 - lane));
+                const uint64_t next = can >> 1 | (g + 1 < WIDE_TILES / 64 && base + 64 * (g + 1) < nt ? cans[g + 1] << 63 : 0);   // (the tile after it can join it)
                 const int len = stop ? lane - (63 - __clzll((long long) stop)) : run + lane + 1;
-                const bool mine = ((large[g] >> lane) & 1) && !(len & 1);
-                const uint64_t m = __ballot(mine);
-                if (mine) list[n + __popcll(m & ~(~0ull << lane))] = (uint16_t) (64 * g + lane);
+                const uint64_t mine = large[g] & __ballot(!(len & 1)), m = mine & (fuller[g] | next), under = ~(~0ull << lane);
+                if ((m >> lane) & 1) list[n + __popcll(m & under)] = (uint16_t) (64 * g + lane);
+                else if ((mine >> lane) & 1) list[WIDE_TILES - 1 - (few + __popcll(mine & ~m & under))] = (uint16_t) (64 * g + lane);
                 n += __popcll(m);
+                few += __popcll(mine & ~m);
                 run = __builtin_amdgcn_readlane(len, 63);
             }
-            if (lane == 0) found = n;
+            if (lane == 0) found = make_int2(n, few);
         }
         __syncthreads();
-        const int n = __builtin_amdgcn_readfirstlane(found), items = n * blocks * (a.ws2 && !gu ? 2 : 1);
-        for (int item = (int) blockIdx.x; item < items; item += (int) gridDim.x) {
-            const int ti = item / blocks, second = ti >= n;   // second: the launch's second matrix: same tiles and activations, its own slices and output
-            const int y = base + __builtin_amdgcn_readfirstlane((int) list[second ? ti - n : ti]);
-            const MmTile tl = tiles[y];
-            const WSlice m = (second ? a.ws2 : mine_ws)[tl.slice];
-            int count = tl.count;
-            if (y + 1 < nt && join.can(tiles[y + 1], tl)) count += tiles[y + 1].count;
-            const int r0 = (item - ti * blocks) * (gu ? 64 : 128);
-            __syncthreads();   // the item before has read the LDS
-#define W(NT) wide_tile<FMT, NT>(a, m, X, second ? a.y2 : Y, perm, tl.start, count, r0, tab, lds)
-            if (count <= 64) W(4);
-            else if (count <= 96) W(6);
-            else if (count <= 128) W(8);
-            else if (count <= 160) W(10);
-            else if (count <= 192) W(12);
-            else W(16);
-#undef W
+        const int full = __builtin_amdgcn_readfirstlane(found.x), n = full + __builtin_amdgcn_readfirstlane(found.y), items = n * blocks * (a.ws2 && !gu ? 2 : 1);
+        for (int i = (int) blockIdx.x; i < items; i += (int) gridDim.x) {
+            const int ti = i / blocks, second = ti >= n, of = second ? ti - n : ti;
+            item(base + __builtin_amdgcn_readfirstlane((int) list[of < full ? of : WIDE_TILES - 1 - (of - full)]), second, (i - ti * blocks) * (gu ? 64 : 128));
         }
         if (base + WIDE_TILES >= nt) return;
     }
@@ -756,11 +767,12 @@ template <int FMT>
 void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
           int grid_tiles) {
     const int rows = a.a16 ? 64 : 128;
-    const long long most = (long long) ((a.R + rows - 1) / rows) * grid_tiles * (a.ws2 && !a.a16 ? 2 : 1), once = 2 * host_cu_count();
-    const dim3 grid((unsigned) (most < once ? most : once));
+    const int blocks = (a.R + rows - 1) / rows, mats = a.ws2 && !a.a16 ? 2 : 1, once = 2 * host_cu_count();
+    const long long most = (long long) blocks * grid_tiles * mats;
+    const dim3 grid = wide_deals<FMT>() ? dim3((unsigned) (most < once ? most : once)) : dim3((unsigned) blocks, (unsigned) grid_tiles, (unsigned) mats);
     constexpr size_t lds = wide_lds<FMT, 16>();
     allow_big_lds<k_mm_wide<FMT>>(lds);
-    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(a));
+    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(blocks * mats, once, wide_deals<FMT>()));
     host_note_launch();
 }
 
