@@ -46,6 +46,19 @@ __device__ __forceinline__ uint32_t tobf(float x) {
     return u >> 16;
 }
 __device__ __forceinline__ float bf(uint32_t h) { return __uint_as_float(h << 16); }
+// Eight Q4 (x) or Q8 weights, unrounded.  Q4: even and odd nibbles as bytes, which the conversion selects by itself; the compiler, left to it, takes
+// each nibble out of x first, an instruction of half rate a weight (301 tokens, 2880 x 2880: 17.2 -> 16.5 us; 12, 6309 x 9792: 14.2 -> 13.0;
+// one, 14336 x 4096: 12.0 -> 11.4).
+template <int FMT>
+__device__ __forceinline__ void affine8(uint32_t x, uint32_t y, float scale, float bias, float (&f)[8]) {
+    uint32_t a = FMT == MF_Q8 ? x : x & 0x0F0F0F0Fu, b = FMT == MF_Q8 ? y : x >> 4 & 0x0F0F0F0Fu;
+    if constexpr (FMT == MF_Q4) asm("" : "+v"(a), "+v"(b));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t v = FMT == MF_Q8 ? (i < 4 ? a : b) >> (8 * (i & 3)) & 255u : (i & 1 ? b : a) >> (8 * (i >> 1)) & 255u;
+        f[i] = scale * (float) v + bias;
+    }
+}
 __device__ __forceinline__ uint32_t pack_bf2(float a, float b) { return tobf(a) | (tobf(b) << 16); }
 // nn.silu on a BF16 tensor: the sigmoid and the product are each rounded to BF16
 __device__ __forceinline__ float silu_bf(float g) {

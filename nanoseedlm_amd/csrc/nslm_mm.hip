@@ -430,14 +430,8 @@ __global__ void __launch_bounds__(64 * (NCW + 4)) k_mm_stream(MmArgs a, WSlice w
                     }
                 } else {
                     const float sc = bf(r.u), b = bf(r.v);
-                    const uint32_t u[4] = {r.raw[0].x, r.raw[0].y, r.raw[0].z, r.raw[0].w};
-                    if (FMT == MF_Q8) {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) f[i >> 3][i & 7] = bfr(sc * (float) ((u[i >> 2] >> (8 * (i & 3))) & 255u) + b);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) f[i >> 3][i & 7] = bfr(sc * (float) ((u[i >> 3] >> (4 * (i & 7))) & 15u) + b);
-                    }
+                    affine8<FMT>(r.raw[0].x, r.raw[0].y, sc, b, f[0]);   // (rounded below, by one instruction a pair: 900 tokens, 12894 x 5120, Q4: 173 -> 163 us)
+                    affine8<FMT>(FMT == MF_Q8 ? r.raw[0].z : r.raw[0].y, r.raw[0].w, sc, b, f[1]);
                 }
             }
 #pragma unroll

@@ -69,14 +69,8 @@ __device__ __forceinline__ bf16x8 seed_weights(uint32_t u, uint32_t v, int odd, 
 // eight Q4 (q.x) or Q8 weights
 template <int FMT>
 __device__ __forceinline__ bf16x8 affine_weights(uint2 q, float scale, float bias) {
-    // (Q4: even and odd nibbles as bytes, which the conversion selects by itself)
-    const uint32_t a = FMT == MF_Q8 ? q.x : q.x & 0x0F0F0F0Fu, b = FMT == MF_Q8 ? q.y : q.x >> 4 & 0x0F0F0F0Fu;
     float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t v = FMT == MF_Q8 ? (i < 4 ? a : b) >> (8 * (i & 3)) & 255u : (i & 1 ? b : a) >> (8 * (i >> 1)) & 255u;
-        f[i] = scale * (float) v + bias;
-    }
+    affine8<FMT>(q.x, q.y, scale, bias, f);
     return __builtin_bit_cast(bf16x8, make_uint4(cvt_pk_bf16(f[0], f[1]), cvt_pk_bf16(f[2], f[3]), cvt_pk_bf16(f[4], f[5]), cvt_pk_bf16(f[6], f[7])));
 }
 

@@ -512,8 +512,7 @@ __device__ __forceinline__ void wide_weights(const WideRaw<FMT>& v, float (&o)[8
 #pragma unroll
             for (int c = 0; c < 8; ++c) o[c] = bfr(s * (float) (((c < 4 ? v.q.x : v.q.y) >> (8 * (c & 3))) & 255u) + b);
         } else {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) o[c] = s * (float) ((v.q.x >> (4 * c)) & 15u) + b;
+            affine8<MF_Q4>(v.q.x, 0, s, b, o);
         }
     }
 }
