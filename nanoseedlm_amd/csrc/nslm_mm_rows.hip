@@ -651,8 +651,8 @@ __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, 
     for (int base = 0;; base += WIDE_TILES) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));   // (as in wide_tile: nothing of this is kept)
-        for (int g = wave; g < WIDE_TILES / 64 && base + 64 * g < grid_tiles; g += 8) {   // (their loads do not wait for *ntiles)
-            const int y = base + 64 * g + lane, at_y = min(y, grid_tiles - 1);
+        for (int g = wave; g < WIDE_TILES / 64 && base + 64 * g < nt; g += 8) {   // (the table need not have grid_tiles rows: none past *ntiles is read)
+            const int y = base + 64 * g + lane, at_y = min(y, nt - 1);
             const MmTile t = tiles[at_y], before = tiles[max(at_y - 1, 0)];
             const uint64_t c = __ballot(y > 0 && y < nt && join.can(t, before)), l = __ballot(y < nt && t.count > a.least), f = __ballot(t.count > 64);
             if (lane == 0) {
