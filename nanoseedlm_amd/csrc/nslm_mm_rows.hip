@@ -13,7 +13,8 @@
 //     sums a pair: a wave's two segments are one chain there, and k_mm_wide's sum is one chain over all of K.
 // Measured (us, streamed kernel -> this one, when both decoded by four multiply-adds a weight): P = 4, 4096 x 4096: 9 tokens 40.1 -> 9.7, 48 tokens
 // 42.8 -> 11.1, 200 tokens 51.8 -> 23.0; 1024 x 4096, 100 tokens 44.7 -> 11.2; Q4 2880 x 2880, 301 tokens 43.0 -> 17.8; BF16 151936 x 2048, 16 tokens
-// 155.7 -> 115.3 (5.5 TB/s).  By one multiply-add a weight 48 tokens take 9.4, by Q4's scales 16 lanes a row tile 301 tokens 15.9.
+// 155.7 -> 115.3 (5.5 TB/s).  By one multiply-add a weight 48 tokens take 9.4, by Q4's scales 16 lanes a row tile 301 tokens 15.9, by bytes that
+// the conversion selects 15.2.
 // What bounds it: vector issue of the decode for the seed formats, the activations' way from L2 for Q4 / Q8 / BF16 at many tokens,
 // HBM for BF16 at few.
 #include "nslm_mm_dev.h"
@@ -394,7 +395,9 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
     // The matrix instructions of half a chunk are issued among the vector instructions that decode the next half.  A wave's records run a chunk
     // ahead of its activations.
     constexpr int NG = (NT + 7) / 8;   // token tiles a hook, at most: hook i has tiles i NT / 8 and up
-    constexpr int XD = 2;               // hooks a fragment is read ahead of its use
+    // Hooks a fragment is read ahead of its use.  P = 3 at 256 pairs has registers for one: with two the loop kept values in scratch memory, whose loads wait
+    // for all of the wave's requests (757 rows, E 16, top-4, d 2752, ff 1984 223 -> 213 us; P = 4, with fewer such loads, gains nothing).
+    constexpr int XD = NT > 12 && FMT == MF_SEED4 ? 1 : 2;
     typename Weights<FMT, 1>::Step st;
     bf16x8 wb, xq[XD][NG];
     auto half = [&](int c, int h) {   // multiplies (c, h) while the next half's weights are formed
