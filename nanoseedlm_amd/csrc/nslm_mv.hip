@@ -508,11 +508,17 @@ __device__ __forceinline__ void wide_weights(const WideRaw<FMT>& v, float (&o)[8
         for (int i = 0; i < 4; ++i) { o[2 * i] = __uint_as_float(u[i] << 16); o[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
     } else {
         const float s = bf(v.s), b = bf(v.b);
-        if (FMT == MF_Q8) {
+        affine8<FMT == MF_Q8 ? MF_Q8 : MF_Q4>(v.q.x, v.q.y, s, b, o);
+        if (FMT == MF_Q8) {   // rounded to BF16, a pair an instruction (one token, 14336 x 4096: 18.6 -> 16.4 us with three a weight taken out)
+            typedef float f32x2 __attribute__((ext_vector_type(2)));
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-            for (int c = 0; c < 8; ++c) o[c] = bfr(s * (float) (((c < 4 ? v.q.x : v.q.y) >> (8 * (c & 3))) & 255u) + b);
-        } else {
-            affine8<MF_Q4>(v.q.x, 0, s, b, o);
+            for (int i = 0; i < 4; ++i) {
+                const f32x2 f = {o[2 * i], o[2 * i + 1]};
+                const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+                o[2 * i] = __uint_as_float(u << 16);
+                o[2 * i + 1] = __uint_as_float(u & 0xFFFF0000u);
+            }
         }
     }
 }
