@@ -894,8 +894,9 @@ static bool mla_attn_launch(kc_stream_t s, MlaArgs& a, const float* ql, const fl
         (void) once;
         // A workgroup fills a CU: more splits than fill the chip only add partials (2 KB a head and split, written and read again).  (Splits dealt to the rows by
         // their lengths: 20 rows of 4 to 8 k positions 28.4 -> 25.8, but 32 of 0.5 to 1 k 14.8 -> 18.0 and 16 of 2 to 4 k 16.8 -> 17.2.)
-        const int groups = (a.n_head + 15) / 16, fill = host_cu_count() / (groups * T), least = reduce ? 1 : 2;
-        if (a.n_splits > 1) a.n_splits = a.n_splits < fill ? a.n_splits : fill < least ? least : fill;
+        // At least two, with the reduce or without: kc_mla_attn and kc_mla_attn_vup split alike, and a call that asks for splits goes by way of the partials.
+        const int groups = (a.n_head + 15) / 16, fill = host_cu_count() / (groups * T);
+        if (a.n_splits > 1) a.n_splits = a.n_splits < fill ? a.n_splits : fill < 2 ? 2 : fill;
         const dim3 grid((unsigned) a.n_splits, (unsigned) groups, (unsigned) T);
         const int partial = a.n_splits > 1;
         float* o = partial ? part : olat;

@@ -165,6 +165,33 @@ def test_latent_attention_long_context_fp8(be, oracle):
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
 
 
+@pytest.mark.parametrize("fmt", ["fp8", "bf16"])
+@pytest.mark.parametrize("T,H", [(60, 16), (129, 16), (257, 16), (129, 20)])
+def test_latent_attention_of_more_rows_than_the_chip_has_workgroups(be, oracle, fmt, T, H):
+    """32 splits asked for at row counts where the chip holds four, one or none a row; most rows short, some at the edges of a split, one of 1500 positions."""
+    rng = np.random.default_rng(T + H)
+    r, rope, NP = 512, 64, 1600
+    pos = [int(p) for p in rng.integers(0, 200, T)]
+    pos[0], pos[1], pos[T // 2], pos[T - 2], pos[T - 1] = 0, 127, 1499, 128, 640
+    kv0 = [int(rng.integers(0, NP - p)) for p in pos]
+    ql = packs.round_bf16((rng.standard_normal((T, H, r)) * 0.3).astype(np.float32))
+    qr = packs.round_bf16(rng.standard_normal((T, H, rope)).astype(np.float32))
+    lat = packs.round_bf16(rng.standard_normal((NP, r)).astype(np.float32))
+    kr = packs.round_bf16(rng.standard_normal((NP, rope)).astype(np.float32))
+    scale = float(1 / np.sqrt(192.0))
+    if fmt == "fp8":
+        (kc, ksc), (vc, vsc) = oracle.fp8_row(kr), oracle.fp8_row(lat)
+        cache, kvf = dict(k=kc, v=vc, ks=ksc, vs=vsc), be.KV_FP8
+        lat, kr = oracle.fp8_decode(vc, vsc), oracle.fp8_decode(kc, ksc)
+    else:
+        cache, kvf = dict(k=packs.f32_to_bf16_bits(kr), v=packs.f32_to_bf16_bits(lat)), be.KV_BF16
+    o = be.kt_mla_attn(H, r, rope, kvf, ql, qr, cache, pos, kv0, scale, 128, 32)
+    for t in sorted({0, 1, T // 2, T - 2, T - 1, *range(2, T, 7)}):
+        for h in (0, H - 1):
+            want = oracle.mla_attn(ql[t, h], qr[t, h], lat[kv0[t]:], kr[kv0[t]:], pos[t], scale)
+            assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
+
+
 @pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 127, 128, 129, 300])
 @pytest.mark.parametrize("fmt,ns", [("fp8", 1), ("fp8", 3), ("bf16", 1), ("bf16", 3)])
 def test_latent_attention_at_the_edges_of_a_round(be, oracle, fmt, n, ns):
@@ -268,14 +295,15 @@ def test_query_maps_rope_and_cache_write_in_one_launch(be, kvf, H, hd, r, rope, 
         assert np.array_equal(x, y)
 
 
-@pytest.mark.parametrize("kvf,H,hd,r,rope,ns", [("fp8", 16, 128, 512, 64, 32), ("bf16", 16, 128, 512, 64, 5), ("bf16", 6, 64, 128, 128, 3)])
-def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, hd, r, rope, ns):
-    """kc_mla_attn_vup == kc_mla_attn + kc_heads_mv (latent -> value): the same bits."""
+@pytest.mark.parametrize("kvf,H,hd,r,rope,ns,T", [("fp8", 16, 128, 512, 64, 32, 3), ("bf16", 16, 128, 512, 64, 5, 3), ("bf16", 6, 64, 128, 128, 3, 3),
+                                                  ("fp8", 16, 128, 512, 64, 32, 60), ("fp8", 16, 64, 512, 64, 32, 129), ("bf16", 20, 64, 512, 64, 4, 257)])
+def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, hd, r, rope, ns, T):
+    """kc_mla_attn_vup == kc_mla_attn + kc_heads_mv (latent -> value): the same bits, at few rows and at more than the chip has workgroups for."""
     import ctypes as C
     from nanoseedlm_amd import moe
     L = be.hip()
     rng = np.random.default_rng(H + r + ns)
-    T, NP = 3, 700
+    NP = 700
     fmt = be.KV_FP8 if kvf == "fp8" else be.KV_BF16
     lat = packs.round_bf16(rng.standard_normal((NP, r)).astype(np.float32))
     krr = packs.round_bf16(rng.standard_normal((NP, rope)).astype(np.float32))
@@ -290,8 +318,8 @@ def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, h
     qr = moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, H, rope)).astype(np.float32)))
     wv = moe.DevBuf.from_array(packs.f32_to_bf16_bits((rng.standard_normal((H, hd, r)) / np.sqrt(r)).astype(np.float32)))
     ri = (be.RowInfo * T)()
-    for t, (p, k0) in enumerate(((650, 0), (37, 20), (300, 310))):
-        ri[t].pos, ri[t].kv0 = p, k0
+    for t in range(T):
+        ri[t].pos, ri[t].kv0 = ((650, 0), (37, 20), (300, 310))[t % 3]
     rib = moe.DevBuf(C.sizeof(ri))
     be.check(L.nh_memcpy_h2d(rib.ptr, ri, C.c_size_t(C.sizeof(ri))), "h2d")
     a = be.MlaArgs(H, r, 128, ns, float(1 / np.sqrt(hd + rope)))
@@ -307,6 +335,8 @@ def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, h
                                   C.c_void_p, C.c_int]
     L.kc_mla_attn(None, a, ql.ptr, qr.ptr, kv, rib.ptr, part.ptr, olat.ptr, T)
     L.kc_heads_mv(None, hv, packs.MF_BF16, W, None, olat.ptr, None, ya.ptr, T)
+    moe.device_sync()
+    be.check(L.nh_memset(part.ptr, 0xFF, C.c_size_t(part.nbytes)), "memset")
     assert L.kc_mla_attn_vup(None, a, ql.ptr, qr.ptr, kv, rib.ptr, part.ptr, hv, packs.MF_BF16, W, yb.ptr, T) == 0
     moe.device_sync()
     assert L.kc_last_error() == 0
