@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
     }
     int p0, p1;
     split_range(a, ri[t].pos, split, &p0, &p1);
-    if (p0 >= p1) return;   // uniform
+    if (p0 >= p1 && a.n_splits > 1) return;   // uniform; nobody reads its partials (one split: a row without keys is written, as 0 / 0)
     const int q0 = qt * (kw / 4), q1 = q0 + kw / 4;   // kw % 8 == 0: whole pairs
     float acc[MLA_MAXL];
 #pragma unroll
@@ -426,7 +426,11 @@ __global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const f
     }
     int p0, p1;
     split_range(a, pos, split, &p0, &p1);
-    if (p0 >= p1) return;   // a split without keys (uniform over the workgroup): the reduce does not read it
+    if (p0 >= p1) {   // a split without keys (uniform over the workgroup): the reduce does not read it; a row without any is 0 / 0
+        if (!partial && h < a.n_head)
+            for (int d = 4 * w + g; d < R / 4; d += 4 * MA_NW) *(f32x4u*) (out + ((size_t) t * a.n_head + h) * R + 4 * d) = f32x4u{NAN, NAN, NAN, NAN};
+        return;
+    }
 
     // the keys of a lane's loads, i < KL (of its RoPE loads, i < 2); keys 8 apart lie on adjacent lanes
     const int kr = lane / LK, kj = lane % LK, rr = lane >> 3, rj = lane & 7;

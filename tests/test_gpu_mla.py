@@ -192,6 +192,37 @@ def test_latent_attention_of_more_rows_than_the_chip_has_workgroups(be, oracle, 
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
 
 
+@pytest.mark.parametrize("H,r,rope,T,ns", [(18, 512, 64, 3, 1), (18, 512, 64, 3, 4), (16, 512, 64, 129, 4), (6, 96, 128, 3, 1), (6, 96, 128, 3, 4)])
+def test_latent_attention_of_a_row_without_positions(be, H, r, rope, T, ns):
+    """A row at position -1 has no keys: its result is written, as the 0 / 0 of the sums, not left as it was; the rows beside it are their own."""
+    import ctypes as C
+    from nanoseedlm_amd import moe
+    L = be.hip()
+    rng = np.random.default_rng(H + ns)
+    NP = 60
+    kr, lat = (packs.f32_to_bf16_bits(rng.standard_normal((NP, n)).astype(np.float32)) for n in (rope, r))
+    bufs = [moe.DevBuf.from_array(x) for x in (kr, lat)] + [moe.DevBuf(16), moe.DevBuf(16)]
+    kv = be.KvView(be.KvSeg(*[b.ptr for b in bufs]), be.KvSeg(None, None, None, None), NP, be.KV_BF16)
+    a = be.MlaArgs(H, r, 16 if T < 100 else 64, ns, 0.1)
+    a.pad[0] = rope
+    ql, qr = (moe.DevBuf.from_array(packs.round_bf16(rng.standard_normal((T, H, n)).astype(np.float32))) for n in (r, rope))
+    part, olat = moe.DevBuf(4 * T * H * ns * (r + 2)), moe.DevBuf(4 * T * H * r)
+    L.kc_mla_attn.argtypes = [C.c_void_p, be.MlaArgs, C.c_void_p, C.c_void_p, be.KvView, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]
+    got = []
+    for pos in ([49] * T, [49] + [-1] * (T - 2) + [49]):
+        ri = (be.RowInfo * T)()
+        for t in range(T):
+            ri[t].pos, ri[t].kv0 = pos[t], 10
+        rib = moe.DevBuf.from_array(np.frombuffer(bytes(ri), dtype=np.uint8))
+        be.check(L.nh_memset(olat.ptr, 0x3F, C.c_size_t(olat.nbytes)), "memset")
+        L.kc_mla_attn(None, a, ql.ptr, qr.ptr, kv, rib.ptr, part.ptr, olat.ptr, T)
+        moe.device_sync()
+        assert L.kc_last_error() == 0
+        got.append(olat.to_array(np.float32, (T, H, r)))
+    assert np.isfinite(got[0]).all() and np.isnan(got[1][1:-1]).all()
+    assert np.array_equal(got[0][[0, -1]].view(np.uint32), got[1][[0, -1]].view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 127, 128, 129, 300])
 @pytest.mark.parametrize("fmt,ns", [("fp8", 1), ("fp8", 3), ("bf16", 1), ("bf16", 3)])
 def test_latent_attention_at_the_edges_of_a_round(be, oracle, fmt, n, ns):
