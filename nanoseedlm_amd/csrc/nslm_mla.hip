@@ -257,18 +257,52 @@ __global__ void __launch_bounds__(256) k_qmaps_rope(MlaArgs a, int rope, HmvArgs
 #define GA_HW 4
 #define MLA_MAXL 16    // latent dims a lane (r <= 1024)
 #define MLA_SPLITS_SHORT 32
-// a row at position pos: the number of splits that have keys, and the keys of each (the row's own 0..pos in equal runs, as few as `chunk` keys a run allow)
-__device__ __forceinline__ int mla_row_splits(const MlaArgs& a, int pos, int* run) {
-    const int ns = a.pad[2] > 0 && a.n_splits > MLA_SPLITS_SHORT ? MLA_SPLITS_SHORT : a.n_splits, want = (pos + a.chunk) / a.chunk;
-    const int used = max(ns < want ? ns : want, 1);
-    *run = max((pos + used) / used, 1);
-    return (pos + *run) / *run;
+// The splits of a row at position pos: the keys of 0..pos in `first` equal runs at most, as few as `chunk` keys a run allow.  Where first is less than the caller's
+// n_splits (k_mla_attn_mfma: as many as fill the chip) and a run would be twice cap() or longer, it is cap() keys, and the rest goes in further splits of `rest` keys.
+struct MlaSplits {
+    int n, first, run, rest;   // (n: splits with keys; run, rest: keys)
+    __device__ __forceinline__ void range(int split, int pos, int* p0, int* p1) const {
+        *p0 = split < first ? split * run : first * run + (split - first) * rest;
+        *p1 = split < n ? min(pos + 1, *p0 + (split < first ? run : rest)) : *p0;
+    }
+};
+#define MLA_REST 512   // keys of a further split, and of a cut run, at least
+__device__ __forceinline__ int mla_most(const MlaArgs& a) { return a.pad[2] > 0 && a.n_splits > MLA_SPLITS_SHORT ? MLA_SPLITS_SHORT : a.n_splits; }
+template <class Cap>
+__device__ __forceinline__ MlaSplits mla_splits(const MlaArgs& a, int first, int pos, Cap cap) {
+    const int most = mla_most(a), want = (pos + a.chunk) / a.chunk;
+    const int used = max(min(min(first, most), want), 1);
+    MlaSplits s = {0, first, max((pos + used) / used, 1), 0};
+    s.n = (pos + s.run) / s.run;
+    if (__builtin_expect(first < most && s.run >= 2 * MLA_REST, 0)) {
+        const int c = cap();
+        if (s.run >= 2 * c) {   // (used is first: no run is longer than chunk otherwise)
+            const int left = pos + 1 - first * c;   // (at least as long as the cut runs)
+            s.run = c;
+            s.rest = max(MLA_REST, (left + most - first - 1) / (most - first));
+            s.n = first + (left + s.rest - 1) / s.rest;
+        }
+    }
+    return s;
 }
-__device__ __forceinline__ void split_range(const MlaArgs& a, int pos, int split, int* p0, int* p1) {
-    int run;
-    const int used = mla_row_splits(a, pos, &run);
-    *p0 = split * run;
-    *p1 = split < used ? min(pos + 1, *p0 + run) : *p0;
+// Inclusive sums over the lanes
+__device__ __forceinline__ int wave_scan(int v) {
+#define STEP(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xF, false)
+    STEP(0x111, 0xF);   // from the lane before, 2, 4, 8 before, of 16
+    STEP(0x112, 0xF);
+    STEP(0x114, 0xF);
+    STEP(0x118, 0xF);
+    STEP(0x142, 0xA);   // lane 15 to lanes 16 - 31, 47 to 48 - 63
+    STEP(0x143, 0xC);   // lane 31 to lanes 32 - 63
+#undef STEP
+    return v;
+}
+// What a run may be twice of before it is cut: the rows' mean length over `first`, doubled; the mean of 64 rows spread over the launch where it has more.
+// mla_sample: a lane's one of them, its position, requested before anything else
+__device__ __forceinline__ int mla_sample(const RowInfo* ri, int T, int lane) { return ri[T > 64 ? (int) ((long long) lane * T >> 6) : min(lane, T - 1)].pos; }
+__device__ __forceinline__ int mla_cap(const MlaArgs& a, int first, int sample, int T, int lane) {
+    const int rows = min(T, 64), sum = __builtin_amdgcn_readlane(wave_scan(lane < rows ? max(sample + 1, 0) >> 5 : 0), 63);
+    return max(max(MLA_REST, a.chunk), (int) (64.0f * (float) sum / (float) (rows * first)));
 }
 // part: [row][head][split][r] accumulators, then [row][head][split] (m, l); splits without keys are neither written nor read
 __device__ __forceinline__ size_t part_ml(const MlaArgs& a, int T) { return (size_t) T * a.n_head * a.n_splits * a.r; }
@@ -286,7 +320,7 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
         qs[i] = a.scale * (i < r ? ql[((size_t) t * a.n_head + hh) * r + i] : qr[((size_t) t * a.n_head + hh) * rope + (i - r)]);
     }
     int p0, p1;
-    split_range(a, ri[t].pos, split, &p0, &p1);
+    mla_splits(a, a.n_splits, ri[t].pos, [] { return 0; }).range(split, ri[t].pos, &p0, &p1);
     if (p0 >= p1 && a.n_splits > 1) return;   // uniform; nobody reads its partials (one split: a row without keys is written, as 0 / 0)
     const int q0 = qt * (kw / 4), q1 = q0 + kw / 4;   // kw % 8 == 0: whole pairs
     float acc[MLA_MAXL];
@@ -399,19 +433,20 @@ __device__ __forceinline__ int mla_swz(int key) { return 2 * (key & 7) + (key >>
 template <int R, int ROPE>
 constexpr int mla_mfma_lds() { return MA_NW * 16 * 2 * (R + ROPE) + (MA_NW / 2) * 2048 + 2 * 16 * MA_NW * 4; }
 
-template <int R, int ROPE, int FMT>
-__global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* __restrict__ ri, float* out,
-                                                             int partial) {
+template <int R, int ROPE, int FMT, bool CUT, bool AGAIN>
+__device__ __forceinline__ void mla_run(const MlaArgs& a, int first, const float* ql, const float* qr, const KvView& kv, const RowInfo* __restrict__ ri, float* part,
+                                        float* olat, int T, uint8_t* mla_lds, int t, int split, int sample) {
     static_assert(R == 512 && ROPE == 64, "eight 64-dim slices of the latent, one of the RoPE key, four dim tiles a wave");
     constexpr int KW = R + ROPE, QLD = KW + 8, NS = R / 64, MT = R / 16 / MA_NW, ES = FMT == KV_FP8 ? 1 : 2;
     constexpr int LK = FMT == KV_FP8 ? 8 : 16, KL = 16 * LK / 64, NL = R * ES / (16 * LK);   // lanes a key, keys a lane, 16-byte loads a key and lane
-    extern __shared__ __attribute__((aligned(16))) uint8_t mla_lds[];
     uint32_t* const Ps = (uint32_t*) (mla_lds + MA_NW * 32 * KW);   // [pair of waves][hi, lo][lane][4]
     float* const mxs = (float*) (Ps + MA_NW / 2 * 512);             // [head][wave]
     float* const ls = mxs + 16 * MA_NW;
-    const int tid = (int) threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4;
-    const int split = (int) blockIdx.x, t = (int) blockIdx.z, h = (int) blockIdx.y * 16 + c;
+    int tid = (int) threadIdx.x;
+    if (AGAIN) asm volatile("" : "+v"(tid));   // (a run's own: kept out of the loop over runs, whose registers it would take)
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4, h = (int) blockIdx.y * 16 + c;
     const int pos = ri[t].pos, kv0 = ri[t].kv0;
+    const size_t th = (size_t) t * a.n_head + h;
 
     // the group's queries: heads past n_head read head 0 and are zeroed
     constexpr int NQ4 = 16 * KW / 4, QV = (NQ4 + 64 * MA_NW - 1) / (64 * MA_NW);   // float4 in all, and a thread
@@ -420,15 +455,17 @@ __global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const f
     for (int i = 0; i < QV; ++i) {
         const int e = min(tid + 64 * MA_NW * i, NQ4 - 1), hh = e < 16 * R / 4 ? e / (R / 4) : (e - 16 * R / 4) / (ROPE / 4);
         const int hq = (int) blockIdx.y * 16 + hh;
-        const size_t th = (size_t) t * a.n_head + (hq < a.n_head ? hq : 0);
-        const NSLM_GLOBAL uint32_t* src = e < 16 * R / 4 ? gp<uint32_t>(ql) + th * R + 4 * (e % (R / 4)) : gp<uint32_t>(qr) + th * ROPE + 4 * ((e - 16 * R / 4) % (ROPE / 4));
+        const size_t tq = (size_t) t * a.n_head + (hq < a.n_head ? hq : 0);
+        const NSLM_GLOBAL uint32_t* src = e < 16 * R / 4 ? gp<uint32_t>(ql) + tq * R + 4 * (e % (R / 4)) : gp<uint32_t>(qr) + tq * ROPE + 4 * ((e - 16 * R / 4) % (ROPE / 4));
         qv[i] = *(const NSLM_GLOBAL u32x4*) src;
     }
     int p0, p1;
-    split_range(a, pos, split, &p0, &p1);
+    const MlaSplits sp = mla_splits(a, CUT ? first : a.n_splits, pos, [&] { return mla_cap(a, first, sample, T, lane); });
+    sp.range(split, pos, &p0, &p1);
+    const bool partial = !olat || sp.n > 1 || (a.n_splits > 1 && first > 1);   // (else the row's one split writes its result)
     if (p0 >= p1) {   // a split without keys (uniform over the workgroup): the reduce does not read it; a row without any is 0 / 0
         if (!partial && h < a.n_head)
-            for (int d = 4 * w + g; d < R / 4; d += 4 * MA_NW) *(f32x4u*) (out + ((size_t) t * a.n_head + h) * R + 4 * d) = f32x4u{NAN, NAN, NAN, NAN};
+            for (int d = 4 * w + g; d < R / 4; d += 4 * MA_NW) *(f32x4u*) (olat + th * R + 4 * d) = f32x4u{NAN, NAN, NAN, NAN};
         return;
     }
 
@@ -442,12 +479,12 @@ __global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const f
     } raw;
     // Keys past the split's end read its last key (finite values; their scores are masked), so no load is conditional.  A split inside one of the
     // view's segments reads at 32-bit offsets from its first row (two instructions an address), one across both by each key's own segment.
-    const bool first = kv0 + p0 < kv.nv, one = first == (kv0 + p1 <= kv.nv) && p1 - p0 <= 1 << 21;
-    const size_t row0 = (size_t) (first ? kv0 + p0 : kv0 + p0 - kv.nv);
-    const NSLM_GLOBAL uint8_t* const vb0 = gp<uint8_t>(first ? kv.a.v : kv.b.v) + row0 * (R * ES);
-    const NSLM_GLOBAL uint8_t* const kb0 = gp<uint8_t>(first ? kv.a.k : kv.b.k) + row0 * (ROPE * ES);
-    const NSLM_GLOBAL uint8_t* const vsb0 = gp<uint8_t>(first ? kv.a.vs : kv.b.vs) + row0 * (R / 32);
-    const NSLM_GLOBAL uint8_t* const ksb0 = gp<uint8_t>(first ? kv.a.ks : kv.b.ks) + row0 * (ROPE / 32);
+    const bool front = kv0 + p0 < kv.nv, one = front == (kv0 + p1 <= kv.nv) && p1 - p0 <= 1 << 21;
+    const size_t row0 = (size_t) (front ? kv0 + p0 : kv0 + p0 - kv.nv);
+    const NSLM_GLOBAL uint8_t* const vb0 = gp<uint8_t>(front ? kv.a.v : kv.b.v) + row0 * (R * ES);
+    const NSLM_GLOBAL uint8_t* const kb0 = gp<uint8_t>(front ? kv.a.k : kv.b.k) + row0 * (ROPE * ES);
+    const NSLM_GLOBAL uint8_t* const vsb0 = gp<uint8_t>(front ? kv.a.vs : kv.b.vs) + row0 * (R / 32);
+    const NSLM_GLOBAL uint8_t* const ksb0 = gp<uint8_t>(front ? kv.a.ks : kv.b.ks) + row0 * (ROPE / 32);
     auto row_at = [&](int p, int key, const void* pa, const void* pb, int bytes) {
         const int at = kv0 + min(p + 16 * w + key, p1 - 1);
         const bool f = at < kv.nv;
@@ -666,37 +703,81 @@ __global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, const f
         l = ((a0[0] + a0[1]) + (a0[2] + a0[3])) + ((a1[0] + a1[1]) + (a1[2] + a1[3]));
     }
     if (h >= a.n_head) return;
-    const size_t th = (size_t) t * a.n_head + h;
     if (!partial) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int d = 16 * (MT * w + mt) + 4 * g;
-            *(f32x4u*) (out + th * R + d) = f32x4u{bfr(acc[mt][0] / l), bfr(acc[mt][1] / l), bfr(acc[mt][2] / l), bfr(acc[mt][3] / l)};
+            *(f32x4u*) (olat + th * R + d) = f32x4u{bfr(acc[mt][0] / l), bfr(acc[mt][1] / l), bfr(acc[mt][2] / l), bfr(acc[mt][3] / l)};
         }
     } else {
         const size_t at = th * a.n_splits + split;
-        if (w == 0 && g == 0) *(f32x2u*) (out + part_ml(a, (int) gridDim.z) + 2 * at) = f32x2u{m, l};
+        if (w == 0 && g == 0) *(f32x2u*) (part + part_ml(a, T) + 2 * at) = f32x2u{m, l};
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int d = 16 * (MT * w + mt) + 4 * g;
-            *(f32x4u*) (out + at * R + d) = acc[mt];
+            *(f32x4u*) (part + at * R + d) = acc[mt];
         }
+    }
+}
+// Workgroup (split of the first ones, 16 heads, row).  CUT: where first is less than n_splits, the further splits of rows much longer than the others are then dealt
+// to all workgroups of a head group, one after the other.  The host does not know the rows' lengths; the kernel looks for such rows behind a workgroup's own
+// run, which is another copy of the code: in one loop with the further ones it took 11 % longer, and a list of all the launch's keys dealt evenly,
+// made before the first load, 1.6 us (16 rows of 2 to 4 k positions 17.3 -> 19.3).  us with as many splits of every row -> this, FP8: one row of 16 k positions
+// among 31 of 200 55 -> 34 (BF16 59 -> 35), among 128 of 500 357 -> 54; 4 of 8 k among 60 of 300 57 -> 44, 20 among 180 of 500 186 -> 124.  Rows alike: the same,
+// but where there are more than half as many as CUs (first 1) the reduce, with nothing to do, adds 3 us: 129 of 2 to 4 k 95 -> 98.
+template <int R, int ROPE, int FMT, bool CUT>
+__global__ void __launch_bounds__(64 * MA_NW) k_mla_attn_mfma(MlaArgs a, int first, const float* ql, const float* qr, KvView kv, const RowInfo* __restrict__ ri,
+                                                             float* part, float* olat, int T) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t mla_lds[];
+    const int tid = (int) threadIdx.x, lane = tid & 63, sample = CUT ? mla_sample(ri, T, lane) : 0;
+    int t = (int) blockIdx.z, split = (int) blockIdx.x, pos = CUT ? ri[min(T > 64 ? tid : lane, T - 1)].pos : 0;   // (no branch: it would wait for the loads)
+    mla_run<R, ROPE, FMT, CUT, false>(a, first, ql, qr, kv, ri, part, olat, T, mla_lds, t, split, sample);
+    if constexpr (!CUT) return;
+    if (T <= 64 && !__any(pos >= (2 * MLA_REST - 1) * first)) return;
+    const int cap = mla_cap(a, first, sample, T, lane), from = (2 * cap - 1) * first;   // (where runs of 2 cap keys begin)
+    if (T <= 64) {
+        if (!__any(pos >= from)) return;
+    } else {
+        bool some = pos >= from;
+        for (int i = tid + 64 * MA_NW; i < T; i += 64 * MA_NW) some |= ri[i].pos >= from;
+        int* const flags = (int*) mla_lds;   // (the keys: read for the last time before a run's last barrier)
+        if (lane == 0) flags[tid >> 6] = 0;
+        if (__any(some) && lane == 0) flags[tid >> 6] = 1;
+        __syncthreads();
+        if (!__any(flags[lane & 7])) return;
+        __syncthreads();
+    }
+    for (int blk = 0, base = 0, item = first * t + split; blk < T;) {   // rows blk + lane; the further splits of the rows before; the next to do
+        pos = ri[min(blk + lane, T - 1)].pos;
+        const MlaSplits s = mla_splits(a, first, pos, [&] { return cap; });
+        const int more = blk + lane < T ? max(s.n - first, 0) : 0, upto = base + wave_scan(more);
+        const uint64_t past = __ballot(upto > item);
+        if (!past) {
+            base = __builtin_amdgcn_readlane(upto, 63);
+            blk += 64;
+            continue;
+        }
+        const int l = __builtin_ctzll(past);
+        t = blk + l;
+        split = first + item - __builtin_amdgcn_readlane(upto - more, l);
+        item += (int) gridDim.x * T;
+        mla_run<R, ROPE, FMT, true, true>(a, first, ql, qr, kv, ri, part, olat, T, mla_lds, t, split, sample);
     }
 }
 
 // The splits of a (row, head) summed, a workgroup of 256 threads: o[i] = bf16(acc / l) of latent dims d0 + i, i < 256 NQ, as far as r reaches.  Wave w takes
 // splits w, w + 4, ... (of whole quads of dims, 16 bytes a load) and the four sums meet in LDS; every wave forms the splits' weights exp(m_s - m) itself, a
-// split a lane, and takes them from there by v_readlane.  The loads of the first 32 splits are requested before anything waits, the row's position included:
-// what a split without keys left in the buffer is not used.
+// split a lane, and takes them from there by v_readlane.  The loads of the first 32 splits, as far as every row may have
+// them, are requested before anything waits, the row's position included: what a split without keys left in the buffer is not used.
 #define MLA_RED_MAXS 256
-template <int NQ>
-__device__ __forceinline__ void mla_reduce(const MlaArgs& a, int T, int t, int h, int d0, const RowInfo* ri, const float* part, f32x4 (&sum)[4][64 * NQ], float* o) {
+template <int NQ, bool CUT>
+__device__ __forceinline__ void mla_reduce(const MlaArgs& a, int n1, int T, int t, int h, int d0, const RowInfo* ri, int sample, const float* part, f32x4 (&sum)[4][64 * NQ], float* o) {
     constexpr int PF = 8, NM = MLA_RED_MAXS / 64;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = a.r;
     const size_t th = (size_t) t * a.n_head + h;
     const NSLM_GLOBAL float* pa = gp<float>(part) + th * a.n_splits * r;
     const NSLM_GLOBAL float* pm = gp<float>(part) + part_ml(a, T) + 2 * th * a.n_splits;
-    const int pos = ri[t].pos;
+    const int pos = ri[t].pos, first = CUT ? n1 : a.n_splits;
     int q[NQ];
 #pragma unroll
     for (int k = 0; k < NQ; ++k) q[k] = min(d0 + 4 * (lane + 64 * k), r - 4);
@@ -707,10 +788,9 @@ __device__ __forceinline__ void mla_reduce(const MlaArgs& a, int T, int t, int h
 #pragma unroll
     for (int j = 0; j < PF; ++j)
 #pragma unroll
-        for (int k = 0; k < NQ; ++k) pv[k][j] = *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) min(w + 4 * j, a.n_splits - 1) * r + q[k]);
+        for (int k = 0; k < NQ; ++k) pv[k][j] = *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) min(w + 4 * j, first - 1) * r + q[k]);
     loads_issued();
-    int run;
-    const int ns = mla_row_splits(a, pos, &run);
+    const int ns = mla_splits(a, first, pos, [&] { return mla_cap(a, first, sample, T, lane); }).n;
     float m = -INFINITY, l = 0.0f, c[NM];
 #pragma unroll
     for (int i = 0; i < NM; ++i) m = fmaxf(m, lane + 64 * i < ns ? ml[i][0] : -INFINITY);
@@ -740,7 +820,8 @@ __device__ __forceinline__ void mla_reduce(const MlaArgs& a, int T, int t, int h
             const float wt = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c[i]), s & 63));
             f32x4 v[NQ];
 #pragma unroll
-            for (int k = 0; k < NQ; ++k) v[k] = i == 0 && j < PF ? pv[k][j < PF ? j : 0] : *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) s * r + q[k]);
+            for (int k = 0; k < NQ; ++k)
+                v[k] = i == 0 && j < PF && (!CUT || s < first) ? pv[k][j < PF ? j : 0] : *(const NSLM_GLOBAL f32x4u*) (pa + (size_t) s * r + q[k]);
             add(v, wt);
         }
 #pragma unroll
@@ -754,24 +835,33 @@ __device__ __forceinline__ void mla_reduce(const MlaArgs& a, int T, int t, int h
         if (d0 + i < r) o[i] = bfr(v / l);
     }
 }
-// olat[t][h][d] = bf16(acc / l).  Workgroup (head, row, 256 latent dims).
-__global__ void __launch_bounds__(256) k_mla_reduce(MlaArgs a, const RowInfo* ri, const float* part, float* olat) {
+// olat[t][h][d] = bf16(acc / l).  Workgroup (head, row, 256 latent dims).  FEW (first 1: most rows' one split has written their results): heads blockIdx.x, + gridDim.x, ..
+template <bool CUT, bool FEW>
+__global__ void __launch_bounds__(256) k_mla_reduce(MlaArgs a, int first, const RowInfo* ri, const float* part, float* olat) {
     __shared__ f32x4 sum[4][64];
-    const int h = (int) blockIdx.x, t = (int) blockIdx.y, d0 = (int) blockIdx.z * 256;
-    mla_reduce<1>(a, (int) gridDim.y, t, h, d0, ri, part, sum, olat + ((size_t) t * a.n_head + h) * a.r + d0);
+    int h = (int) blockIdx.x;
+    const int t = (int) blockIdx.y, d0 = (int) blockIdx.z * 256, T = (int) gridDim.y, lane = (int) threadIdx.x & 63, sample = CUT ? mla_sample(ri, T, lane) : 0;
+    if (FEW && mla_splits(a, first, ri[t].pos, [&] { return mla_cap(a, first, sample, T, lane); }).n <= 1) return;
+    for (;;) {
+        mla_reduce<1, CUT>(a, first, T, t, h, d0, ri, sample, part, sum, olat + ((size_t) t * a.n_head + h) * a.r + d0);
+        h += (int) gridDim.x;
+        if (!FEW || h >= a.n_head) return;
+        __syncthreads();
+    }
 }
 
 // The splits' reduce and the value-up map of a head in ONE launch: workgroup (row group, head, row) reduces the head's
 // latent output into LDS (k_mla_reduce's arithmetic, 512 dims a pass: the map needs them all) and computes rows
 // [RG g, RG (g + 1)) of y[t][h] = bf16(W_h . olat[t][h]) (k_heads_mv's arithmetic).  The same bits as the two kernels.
 #define MLA_RV_GROUPS 16   // row groups a head at most: fewer when there are many (row, head) pairs, each group re-reads the partials
-__global__ void __launch_bounds__(256) k_mla_reduce_vup(MlaArgs a, const RowInfo* ri, const float* part, HmvArgs hv, int fmt, WSlice W, float* y,
+template <bool CUT>
+__global__ void __launch_bounds__(256) k_mla_reduce_vup(MlaArgs a, int first, const RowInfo* ri, const float* part, HmvArgs hv, int fmt, WSlice W, float* y,
                                                        int lpr) {
     __shared__ uint32_t tab[NSLM_TAB_WORDS];
     __shared__ f32x4 sum[4][128];
     __shared__ __attribute__((aligned(16))) float ol[64 * MLA_MAXL];
     constexpr int NP = 2;   // map passes whose loads are issued before anything waits
-    const int g = (int) blockIdx.x, h = (int) blockIdx.y, t = (int) blockIdx.z, r = a.r, tid = threadIdx.x;
+    const int g = (int) blockIdx.x, h = (int) blockIdx.y, t = (int) blockIdx.z, r = a.r, tid = threadIdx.x, sample = CUT ? mla_sample(ri, (int) gridDim.z, tid & 63) : 0;
     const int rg = (hv.O + (int) gridDim.x - 1) / (int) gridDim.x, o0 = g * rg, o1 = min(o0 + rg, hv.O);
     const int rpw = 64 / lpr, sub = (tid & 63) / lpr, ln = tid & (lpr - 1);
     // BF16 maps, one block a lane: the map rows of the first NP passes are in flight beside the splits
@@ -786,7 +876,7 @@ __global__ void __launch_bounds__(256) k_mla_reduce_vup(MlaArgs a, const RowInfo
     }
     if (fmt == MF_SEED4P4 || fmt == MF_SEED4) load_tables(tab);
     for (int d0 = 0; d0 < r; d0 += 512) {
-        mla_reduce<2>(a, (int) gridDim.z, t, h, d0, ri, part, sum, ol + d0);
+        mla_reduce<2, CUT>(a, first, (int) gridDim.z, t, h, d0, ri, sample, part, sum, ol + d0);
         __syncthreads();
     }
     WSlice ws = W;
@@ -880,32 +970,34 @@ int kc_mla_qmaps_rope(kc_stream_t s, MlaArgs a, HmvArgs hq, HmvArgs hl, int fmt,
     host_note_launch();
     return 0;
 }
-// attention into the partials (n_splits > 1) or olat; the reduce when `reduce`.  a.n_splits becomes the number the launch takes (the partials' layout).
-// false: unsupported, nothing launched
-static bool mla_attn_launch(kc_stream_t s, MlaArgs& a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, float* olat,
-                            int T, bool reduce) {
+// Attention into the partials or olat, and the reduce; olat NULL: into the partials alone.  *first: the launch's first splits.  false: unsupported, nothing launched
+static bool mla_attn_launch(kc_stream_t s, const MlaArgs& a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, float* olat,
+                            int T, int* first) {
     const int rope = rope_of(a);
     if (T < 1 || (kv.fmt != KV_BF16 && kv.fmt != KV_FP8) || (rope != 64 && rope != 128) || a.r % 8 || a.r > 64 * MLA_MAXL || a.n_splits < 1) {
         host_note_unsupported();
         return false;
     }
     if (a.n_splits > MLA_RED_MAXS) { host_note_unsupported(); return false; }
+    *first = a.n_splits;
     if (a.r == 512 && rope == 64 && (((uintptr_t) ql | (uintptr_t) qr) & 15u) == 0) {   // the matrix-core kernel: 16 heads a workgroup
         constexpr int lds = mla_mfma_lds<512, 64>();
-        static const hipError_t once[2] = {
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8>, hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
+        static const hipError_t once[4] = {
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_BF16, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+            hipFuncSetAttribute((const void*) k_mla_attn_mfma<512, 64, KV_FP8, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
         (void) once;
-        // A workgroup fills a CU: more splits than fill the chip only add partials (2 KB a head and split, written and read again).  (Splits dealt to the rows by
-        // their lengths: 20 rows of 4 to 8 k positions 28.4 -> 25.8, but 32 of 0.5 to 1 k 14.8 -> 18.0 and 16 of 2 to 4 k 16.8 -> 17.2.)
-        // At least two, with the reduce or without: kc_mla_attn and kc_mla_attn_vup split alike, and a call that asks for splits goes by way of the partials.
+        // A workgroup fills a CU: more splits of every row than fill the chip only add partials (2 KB a head and split, written and read again).  (Two or three where two
+        // do not fit, by the chip's turns at them: 129 rows of 2 to 4 k positions 98 -> 84 us, 160 of 0.5 to 1 k 33 -> 43, 300 of 128 to 256 26 -> 48.)
         const int groups = (a.n_head + 15) / 16, fill = host_cu_count() / (groups * T);
-        if (a.n_splits > 1) a.n_splits = a.n_splits < fill ? a.n_splits : fill < 2 ? 2 : fill;
-        const dim3 grid((unsigned) a.n_splits, (unsigned) groups, (unsigned) T);
-        const int partial = a.n_splits > 1;
-        float* o = partial ? part : olat;
-        if (kv.fmt == KV_FP8) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_FP8>), grid, dim3(64 * MA_NW), lds, (hipStream_t) s, a, ql, qr, kv, ri, o, partial);
-        else hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, KV_BF16>), grid, dim3(64 * MA_NW), lds, (hipStream_t) s, a, ql, qr, kv, ri, o, partial);
+        *first = a.n_splits < fill ? a.n_splits : fill < 1 ? 1 : fill;
+        const bool cut = *first < a.n_splits;
+        const dim3 grid((unsigned) *first, (unsigned) groups, (unsigned) T);
+#define LAUNCH(FMT, CUT) hipLaunchKernelGGL((k_mla_attn_mfma<512, 64, FMT, CUT>), grid, dim3(64 * MA_NW), lds, (hipStream_t) s, a, *first, ql, qr, kv, ri, part, olat, T)
+        if (kv.fmt == KV_FP8) { if (cut) LAUNCH(KV_FP8, true); else LAUNCH(KV_FP8, false); }
+        else { if (cut) LAUNCH(KV_BF16, true); else LAUNCH(KV_BF16, false); }
+#undef LAUNCH
     } else {
         float* o = a.n_splits > 1 ? part : olat;
         const size_t lds = sizeof(float) * (size_t) (GA_KT + GA_HW) * (size_t) (a.r + rope + 4);
@@ -915,28 +1007,39 @@ static bool mla_attn_launch(kc_stream_t s, MlaArgs& a, const float* ql, const fl
         hipLaunchKernelGGL(k_mla_attn_any, dim3((unsigned) a.n_splits, (unsigned) (a.n_head + GA_HW - 1) / GA_HW, (unsigned) T), dim3(64 * GA_HW), lds,
                            (hipStream_t) s, a, rope, ql, qr, kv, ri, o);
     }
-    if (a.n_splits > 1 && reduce)
-        hipLaunchKernelGGL(k_mla_reduce, dim3((unsigned) a.n_head, (unsigned) T, (unsigned) (a.r + 255) / 256), dim3(256), 0, (hipStream_t) s, a, ri,
-                           part, olat);
+    if (a.n_splits > 1 && olat) {
+        const bool few = *first == 1;
+        const int at_once = few && T < 1024 ? 1024 / T : few ? 1 : a.n_head;   // (few: as many workgroups as the chip holds, most of them to end at once)
+        const dim3 grid((unsigned) (at_once < a.n_head ? at_once : a.n_head), (unsigned) T, (unsigned) (a.r + 255) / 256);
+#define LAUNCH(CUT, FEW) hipLaunchKernelGGL((k_mla_reduce<CUT, FEW>), grid, dim3(256), 0, (hipStream_t) s, a, *first, ri, part, olat)
+        if (few) LAUNCH(true, true);
+        else if (*first < a.n_splits) LAUNCH(true, false);
+        else LAUNCH(false, false);
+#undef LAUNCH
+    }
     host_note_launch();
     return true;
 }
 void kc_mla_attn(kc_stream_t s, MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, float* olat,
                  int T) {
-    (void) mla_attn_launch(s, a, ql, qr, kv, ri, part, olat, T, true);
+    int first;
+    (void) mla_attn_launch(s, a, ql, qr, kv, ri, part, olat, T, &first);
 }
 int kc_mla_attn_vup(kc_stream_t s, MlaArgs a, const float* ql, const float* qr, KvView kv, const RowInfo* ri, float* part, HmvArgs hv, int fmt,
                     WSlice W, float* y, int T) {
-    int lpr = 1;
+    int lpr = 1, first;
     while (lpr < 64 && lpr < hv.I / 8) lpr <<= 1;
     if (a.n_splits < 2 || a.n_splits > MLA_RED_MAXS || hv.I != a.r || a.r % 8 || a.r > 64 * MLA_MAXL || hv.H != a.n_head || hv.gate ||
         (lpr != hv.I / 8 && hv.I / 8 <= 64) || hv.O < 1)
         return -1;
-    if (!mla_attn_launch(s, a, ql, qr, kv, ri, part, NULL, T, false)) return -1;
+    if (!mla_attn_launch(s, a, ql, qr, kv, ri, part, NULL, T, &first)) return -1;
     int groups = 1024 / (a.n_head * T);   // about a thousand workgroups
     groups = groups < 1 ? 1 : groups > MLA_RV_GROUPS ? MLA_RV_GROUPS : groups;
-    hipLaunchKernelGGL(k_mla_reduce_vup, dim3((unsigned) groups, (unsigned) a.n_head, (unsigned) T), dim3(256), 0, (hipStream_t) s, a, ri, part, hv, fmt,
-                       W, y, lpr);
+#define LAUNCH(CUT)                                                                                                                                              \
+    hipLaunchKernelGGL(k_mla_reduce_vup<CUT>, dim3((unsigned) groups, (unsigned) a.n_head, (unsigned) T), dim3(256), 0, (hipStream_t) s, a, first, ri, part, hv, \
+                       fmt, W, y, lpr)
+    if (first < a.n_splits) LAUNCH(true); else LAUNCH(false);
+#undef LAUNCH
     host_note_launch();
     return 0;
 }

@@ -192,6 +192,36 @@ def test_latent_attention_of_more_rows_than_the_chip_has_workgroups(be, oracle, 
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
 
 
+# first splits of every row, and the further ones of the long row, with 256 CUs: 8 and 16 (32 rows), 3 and the one that is left of four (70), one and up to 23 (300), up to 7 (520: the
+# long row past the first 512), one and 15 for either of two groups of heads (90 rows of 20), seven and as many as the keys make (33); a row without positions among them
+@pytest.mark.parametrize("fmt", ["fp8", "bf16"])
+@pytest.mark.parametrize("T,H,ns,short,chunk", [(32, 16, 32, 200, 128), (70, 16, 4, 300, 128), (300, 16, 32, 150, 128), (520, 16, 8, 120, 128), (90, 20, 16, 600, 128),
+                                                (33, 16, 256, 140, 300)])
+def test_latent_attention_of_a_long_row_among_short_ones(be, oracle, fmt, T, H, ns, short, chunk):
+    rng = np.random.default_rng(T + H)
+    r, rope, NP, long = 512, 64, 12100, T - 5
+    pos = [int(p) for p in rng.integers(0, short, T)]
+    pos[long], pos[3], pos[T - 1] = 11999, -1, 0
+    kv0 = [int(rng.integers(0, NP - p)) for p in pos]
+    ql = packs.round_bf16((rng.standard_normal((T, H, r)) * 0.3).astype(np.float32))
+    qr = packs.round_bf16(rng.standard_normal((T, H, rope)).astype(np.float32))
+    lat = packs.round_bf16(rng.standard_normal((NP, r)).astype(np.float32))
+    kr = packs.round_bf16(rng.standard_normal((NP, rope)).astype(np.float32))
+    scale = float(1 / np.sqrt(192.0))
+    if fmt == "fp8":
+        (kc, ksc), (vc, vsc) = oracle.fp8_row(kr), oracle.fp8_row(lat)
+        cache, kvf = dict(k=kc, v=vc, ks=ksc, vs=vsc), be.KV_FP8
+        lat, kr = oracle.fp8_decode(vc, vsc), oracle.fp8_decode(kc, ksc)
+    else:
+        cache, kvf = dict(k=packs.f32_to_bf16_bits(kr), v=packs.f32_to_bf16_bits(lat)), be.KV_BF16
+    o = be.kt_mla_attn(H, r, rope, kvf, ql, qr, cache, pos, kv0, scale, chunk, ns)
+    assert np.isnan(o[3]).all()
+    for t in sorted({0, 1, 2, 4, 64 % T, long - 1, long, long + 1, T - 1, *range(5, T, 11)}):
+        for h in (0, H - 1):
+            want = oracle.mla_attn(ql[t, h], qr[t, h], lat[kv0[t]:], kr[kv0[t]:], pos[t], scale)
+            assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
+
+
 @pytest.mark.parametrize("H,r,rope,T,ns", [(18, 512, 64, 3, 1), (18, 512, 64, 3, 4), (16, 512, 64, 129, 4), (6, 96, 128, 3, 1), (6, 96, 128, 3, 4)])
 def test_latent_attention_of_a_row_without_positions(be, H, r, rope, T, ns):
     """A row at position -1 has no keys: its result is written, as the 0 / 0 of the sums, not left as it was; the rows beside it are their own."""
@@ -334,7 +364,7 @@ def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, h
     from nanoseedlm_amd import moe
     L = be.hip()
     rng = np.random.default_rng(H + r + ns)
-    NP = 700
+    NP = 700 if T < 100 else 5000
     fmt = be.KV_FP8 if kvf == "fp8" else be.KV_BF16
     lat = packs.round_bf16(rng.standard_normal((NP, r)).astype(np.float32))
     krr = packs.round_bf16(rng.standard_normal((NP, rope)).astype(np.float32))
@@ -351,6 +381,8 @@ def test_attention_with_reduce_and_value_map_in_one_launch(be, oracle, kvf, H, h
     ri = (be.RowInfo * T)()
     for t in range(T):
         ri[t].pos, ri[t].kv0 = ((650, 0), (37, 20), (300, 310))[t % 3]
+    if T > 100:   # (a row that is cut)
+        ri[100].pos, ri[100].kv0 = 4980, 10
     rib = moe.DevBuf(C.sizeof(ri))
     be.check(L.nh_memcpy_h2d(rib.ptr, ri, C.c_size_t(C.sizeof(ri))), "h2d")
     a = be.MlaArgs(H, r, 128, ns, float(1 / np.sqrt(hd + rope)))
