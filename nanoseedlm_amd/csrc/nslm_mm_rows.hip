@@ -494,17 +494,19 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 // join another itself: the parity of the run of tiles that can, up to the last one that cannot.  A wave looks at 64 tiles at once (a
 // token's experts by the thousand make runs of hundreds of tiles, and a walk tile by tile is a chain of as many loads).
 // Beside k_mm_rows_grouped every tile can join: which kernel computes a tile, and with it its sums' order, is then a matter of the table alone,
-// not of the matrices in the launch.  Alone k_mm_wide pairs full tiles where their workgroups are more than 5/8 of the two a CU that run at once: a
+// not of the matrices in the launch.  Alone k_mm_wide pairs full tiles where their workgroups are more than 5/8 of two a CU, of which P = 3, P = 4 and Q4 run as many at once: a
 // pair saves a decode and leaves half the workgroups.  us for so many workgroups of a full tile, and for half as many of a pair (K 2048, P = 4):
 // 256 44 and 56, 320 63 and 57, 512 69 and 64, 768 97 and 94, 1024 134 and 105, 1536 210 and 149.  36 layer steps of 140 to 620 pairs an expert:
-// geometric mean 0.917 of the time of a workgroup a tile, with one round as the line 0.925, with two 0.941.  A tile of up to FEW pairs joins at any number: it adds a pass's step to a full one's, no decode (E 16, top-8,
+// geometric mean 0.917 of the time of a workgroup a tile, with one round as the line 0.925, with two 0.941.  (BF16, with the line at 5/16, 5/8, one and two
+// times two a CU: E 32, top-4, d 512, ff 256, 2048 rows 36.6, 31.0, 31.2, 31.4; E 16, top-2, d 2048, ff 1024, two experts in all 83, 84, 107, 107; E 16, top-4, d 2048,
+// ff 1024, 1024 rows 120, 119, 119, 112.)  A tile of up to FEW pairs joins at any number: it adds a pass's step to a full one's, no decode (E 16, top-8,
 // d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138).
 // Where workgroups are started a tile each (Q8) a pair's second one is an empty one: there full tiles stay alone up to a round and in a second that they
 // fill (E 16, top-2, d 2048, ff 1024, 2048 rows on the same two experts, 512 workgroups: 171 alone, 222 in pairs; 576: 299 and 269).
 #define FEW 64
 struct JoinAt {   // tile counts: full tiles go in pairs from [2] on, and between [0] and [1]
     int n[3];
-    JoinAt(int blocks, int round, bool dealt) {   // a tile's workgroups; those that run at once
+    JoinAt(int blocks, int round, bool dealt) {   // a tile's workgroups; two a CU
         n[0] = dealt ? 0 : round / blocks;
         n[1] = dealt ? 0 : (5 * round / 4 + blocks - 1) / blocks;
         n[2] = dealt ? 5 * round / 8 / blocks + 1 : (2 * round + blocks - 1) / blocks;
@@ -603,7 +605,8 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
     }
 }
 
-// A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join).  The grid is what runs at once, two workgroups a CU, and a
+// A grouped launch's tiles of more than a.least pairs, each with the tile that joins it (Join).  The grid is what runs at once, two workgroups a CU (of BF16, whose steps take
+// more LDS, one: in a grid of two the second half began behind the first one's lists; 1762 rows, E 128, top-4, d 512, ff 256: 44.8 -> 41.6 us, geometric mean of 25 steps 0.978), and a
 // workgroup takes items blockIdx.x, + gridDim.x, .. of (matrix, tile, block of rows): with a workgroup an item, the ones that found nothing to do between
 // them, they were started in turn over the shader engines, and an engine that was full kept the free places of the others waiting, 20 to 40 us of an
 // item's 75 (2048 rows, E 128, top-8, d 2048, ff 768: 54 to 58 of an XCD's 64 places taken; 435 us a
@@ -615,6 +618,8 @@ __global__ void __launch_bounds__(256, MOST > 4 ? 3 : 4) k_mm_rows_grouped(MmArg
 #define WIDE_TILES 1024   // of the table, looked at together
 template <int FMT>
 constexpr bool wide_deals() { return FMT != MF_Q8; }
+template <int FMT>
+constexpr int wide_at_once() { return FMT == MF_BF16 ? 1 : 2; }   // workgroups a CU
 template <int FMT>
 __global__ void __launch_bounds__(512, 4) k_mm_wide(MmArgs a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles,
                                                     const int32_t* ntiles, int grid_tiles, JoinAt at) {
@@ -764,12 +769,14 @@ template <int FMT>
 void wide(hipStream_t st, const MmArgs& a, const WSlice* ws, const uint16_t* X, float* Y, const int32_t* perm, const MmTile* tiles, const int32_t* ntiles,
           int grid_tiles) {
     const int rows = a.a16 ? 64 : 128;
-    const int blocks = (a.R + rows - 1) / rows, mats = a.ws2 && !a.a16 ? 2 : 1, once = 2 * host_cu_count();
+    const int blocks = (a.R + rows - 1) / rows, mats = a.ws2 && !a.a16 ? 2 : 1, once = wide_at_once<FMT>() * host_cu_count();
     const long long most = (long long) blocks * grid_tiles * mats;
     const dim3 grid = wide_deals<FMT>() ? dim3((unsigned) (most < once ? most : once)) : dim3((unsigned) blocks, (unsigned) grid_tiles, (unsigned) mats);
     constexpr size_t lds = wide_lds<FMT, 16>();
+    constexpr size_t all = lds + (seed_fmt<FMT>() ? 4 * mm_tab_words<FMT>() : 0) + (wide_deals<FMT>() ? 2 * WIDE_TILES + 3 * WIDE_TILES / 8 + 16 : 0);
+    static_assert(wide_at_once<FMT>() == 160 * 1024 / ((all + 1279) / 1280 * 1280), "as many fit a CU's LDS, given out in pieces of 1280 bytes");
     allow_big_lds<k_mm_wide<FMT>>(lds);
-    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(blocks * mats, once, wide_deals<FMT>()));
+    hipLaunchKernelGGL((k_mm_wide<FMT>), grid, dim3(512), lds, st, a, ws, X, Y, perm, tiles, ntiles, grid_tiles, JoinAt(blocks * mats, 2 * host_cu_count(), wide_deals<FMT>()));
     host_note_launch();
 }
 
