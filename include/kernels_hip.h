@@ -250,7 +250,7 @@ typedef struct {
 typedef struct { int pos, kv0; int pad[2]; } RowInfo; /* kv0: the cache row of the sequence slot's position 0 (kernels_moe.metal:86) */
 #define ATT_HD 128
 /* engine/kernels_moe.metal:100-104.  chunk: target keys per split; each row splits its own 0..pos into
- * min(n_splits, ceil((pos + 1) / chunk)) parts.  pad[0] (ours; the reference leaves it 0): the RoPE key's width, 64 or 128,
+ * min(n_splits, ceil((pos + 1) / chunk)) parts (kc_mla_attn says where into fewer).  pad[0] (ours; the reference leaves it 0): the RoPE key's width, 64 or 128,
  * 0 = 128 (the reference hard-codes ATT_HD).  pad[2] > 0: at most 32 splits, as the reference's one-pass kernel takes it. */
 typedef struct {
     int n_head, r, chunk, n_splits;

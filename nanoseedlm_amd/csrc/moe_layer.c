@@ -306,14 +306,15 @@ int nslm_moe_step_layer(NslmMoe* m, kc_stream_t s, int layer, const float* xn, i
  * past a pass's pairs, it is the pairs an expert gets on average, and the workgroups that k_mm_wide (the kernel of mostly full tiles) would have
  * at a tile an expert, that say which passes pay: 64 and 96 up to where the fuller half of the tiles still fits (the mean and twice its root).
  * us a layer step by the word 48 / 64 / 96 / 129, P = 4 where not said, [the word taken]:
- *   a mean of up to 12   E 128, top-8, d 2048, ff 768: 3: [234] 236 292 289, 12: [248] 256 319 302; E 64, top-4, d 1024, ff 512: 12: [69] 70 83 75
- *   up to 52             E 128, top-8: 25: 312 [291] 349 314, 50: 536 [357] 419 344; E 16, top-2, d 2048, ff 1024: 50: 115 [86] 88 97
- *   up to 76 (88), few   E 16, top-2: 65: 135 107 [99] 102; E 16, top-8, d 3072, ff 512: 75: 121 98 [86] 114
- *             many       E 64, top-4, d 1024, ff 448: 65: 145 118 121 [102]; E 128, top-4, d 512, ff 192, P = 3: 64: 114 101 112 [93]
- *   up to a tile, few    E 16, top-8, d 3072, ff 512: 87: 129 [100] 98 115, 115: 148 [106] 127 118
- *   else                 E 128, top-8: 128: 1146 786 970 [543]; E 16, top-4, d 1024, ff 2048, P = 3: 87: 148 112 113 [105]
+ *   a mean of up to 12   E 128, top-8, d 2048, ff 768: 12: [200] 195 257 267; E 64, top-4, d 1024, ff 512: 12: [58] 57 69 70
+ *   up to 52             E 128, top-8: 25: 245 [227] 288 273, 50: 413 [289] 357 287; E 16, top-2, d 2048, ff 1024: 50: 92 [66] 73 77
+ *   up to 76 (88), few   E 16, top-2: 65: 122 87 [86] 82; E 16, top-8, d 3072, ff 512: 75: 107 86 [78] 95, 87: 120 88 [92] 96
+ *             many       E 64, top-4, d 1024, ff 448: 65: 119 93 98 [76]; E 128, top-4, d 512, ff 192, P = 3: 64: 81 69 75 [57]
+ *   up to a tile, few    E 16, top-8, d 3072, ff 512: 115: 128 [92] 108 100
+ *   else                 E 128, top-8: 128: 890 629 779 [390]; E 16, top-4, d 1024, ff 2048, P = 3: 87: 124 95 95 [88]
+ * (The lines were laid on an earlier build of these kernels; 130 drawn steps on a later one have the rule 0.3 % off the best word.)
  * Skewed routing is the kernels' to see to, by the tiles' own counts: with a tenth of the experts taking half of the pairs, E 128, top-8, T = 128 /
- * 512 / 2048: 266 / 350 / 621 (by the kernel of one 128-pair pass a tile that came before these: 323 / 412 / 656). */
+ * 512 / 2048: 211 / 264 / 432 (uniform 193 / 250 / 409 on the same build). */
 static int tile_word(int T, int P, int E, int d, int ff) {
     const int mean = P / E, gu = E * ((ff + 63) / 64), dn = E * ((d + 127) / 128);
     if (T <= 32) return T;

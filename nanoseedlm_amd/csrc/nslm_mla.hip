@@ -397,7 +397,7 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
 // f32 online softmax, P entering the second product as two BF16 terms hi + lo).
 // Workgroup (split, group of 16 heads, row) of 8 waves, a round = 128 keys, 16 a wave.  Per round:
 //   keys    a wave's cache bytes come by loads of whole 128-byte lines (8 lanes a key FP8, 16 BF16: a load whose adjacent lanes are 16 keys, as the MFMA
-//           wants them, saves the way through LDS but costs a look-up a lane: one BF16 row of 12 k positions 27.0 us, this way 19.9), are decoded in
+//           wants them, saves the way through LDS but costs a look-up a lane: one BF16 row of 12 k positions 7 us more), are decoded in
 //           registers and go to LDS once, key by key;
 //   scores  S^T[key][head] = K Q^T by v_mfma_f32_16x16x32_bf16, the wave's own 16 keys, all r + rope dims: no barrier; Q fragments stay in registers;
 //   softmax the waves' maxima meet in LDS (barrier), every wave forms the same reference score and its own keys' P, hi + lo terms, to LDS (barrier);
@@ -409,9 +409,9 @@ __global__ void __launch_bounds__(64 * GA_HW) k_mla_attn_any(MlaArgs a, int rope
 // every byte decodes as in nslm/kvq.h.
 // What bounds it: with all CUs at work the first rounds' bytes come at the rate of a large copy; then a round is 7000 clocks of phases (writes to LDS 1500,
 // the scores' chain of reads and MFMAs 1500, two barriers with the softmax 1000, P c 1500), none of the units a third busy.  Tried: workgroups of four
-// waves, two a CU (16 rows of 2 to 4 k positions + 6 %, one row of 12 k + 23 %); two rounds' bytes in registers (they spill).  us with the reduce, FP8 / BF16, against tiles of 32 keys
-// decoded twice into LDS by four waves: 16 rows of 2 to 4 k positions 22.6 -> 16.8 / 21.8 -> 19.6, one of 12 k 31.0 -> 19.5 / 28.1 -> 19.9, 32 of 3 to 6 k 46.0 -> 30.6 /
-// 46.9 -> 38.0, 32 of 0.5 to 1 k 37.2 -> 14.8 / 34.3 -> 17.5, one of 75 13.1 -> 10.0 / 12.3 -> 10.3.
+// waves, two a CU (16 rows of 2 to 4 k positions + 6 %, one row of 12 k + 23 %); two rounds' bytes in registers (they spill).  us with the reduce, back to back, FP8 / BF16,
+// against tiles of 32 keys decoded twice into LDS by four waves: 16 rows of 2 to 4 k positions 24.0 -> 17.5 / 22.7 -> 20.2, one of 12 k 25.5 -> 16.8 / 23.1 -> 17.0, 32 of 3
+// to 6 k 49.0 -> 32.3 / 50.0 -> 39.0, 32 of 0.5 to 1 k 38.0 -> 15.6 / 34.5 -> 17.9, one of 76 13.3 -> 10.1 / 12.5 -> 10.3.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -427,8 +427,10 @@ __device__ __forceinline__ uint32_t bf2(float lo, float hi) {   // v_cvt_pk_bf16
 }
 #define MA_NW 8
 #define MA_KEYS (16 * MA_NW)
-// A wave's keys in LDS: 16 rows of r values, then 16 of the RoPE key.  A key's 16-byte slots are permuted by exclusive or with mla_swz(key): the 16 lanes that
-// a 16-byte access serves together ({0-3, 12-15, 20-23, 24-27} and so on) and the 8 keys x 32 bytes of a transposing read then fall on distinct banks.
+// A wave's keys in LDS: 16 rows of r values, then 16 of the RoPE key.  A latent row's 16-byte slots are permuted by exclusive or with mla_swz(key): the 16 lanes that
+// a 16-byte access serves together ({0-3, 12-15, 20-23, 24-27} and so on) and the 8 keys x 32 bytes of a transposing read then fall on distinct banks.  The RoPE rows'
+// slots, with key & 7 (two rows share the banks), serve the writes; their reads, the queries' and the stores of P, 8 bytes of every 16, meet two ways: a third
+// of the LDS's active cycles are conflicts.
 __device__ __forceinline__ int mla_swz(int key) { return 2 * (key & 7) + (key >> 3); }
 template <int R, int ROPE>
 constexpr int mla_mfma_lds() { return MA_NW * 16 * 2 * (R + ROPE) + (MA_NW / 2) * 2048 + 2 * 16 * MA_NW * 4; }

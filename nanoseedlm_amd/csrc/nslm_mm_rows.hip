@@ -497,7 +497,8 @@ __device__ __forceinline__ void wide_tile(const MmArgs& a, const WSlice& m, cons
 // not of the matrices in the launch.  Alone k_mm_wide pairs full tiles where their workgroups are more than 5/8 of two a CU, of which P = 3, P = 4 and Q4 run as many at once: a
 // pair saves a decode and leaves half the workgroups.  us for so many workgroups of a full tile, and for half as many of a pair (K 2048, P = 4):
 // 256 44 and 56, 320 63 and 57, 512 69 and 64, 768 97 and 94, 1024 134 and 105, 1536 210 and 149.  36 layer steps of 140 to 620 pairs an expert:
-// geometric mean 0.917 of the time of a workgroup a tile, with one round as the line 0.925, with two 0.941.  (BF16, with the line at 5/16, 5/8, one and two
+// geometric mean 0.917 of the time of a workgroup a tile, with one round as the line 0.925, with two 0.941.  (25 other steps, K 256 to 4096, against the line at 5/8: with one
+// round P = 4 0.998, P = 3 0.999, Q4 1.002 of the time, with two 1.030, 1.026, 1.039.  BF16, with the line at 5/16, 5/8, one and two
 // times two a CU: E 32, top-4, d 512, ff 256, 2048 rows 36.6, 31.0, 31.2, 31.4; E 16, top-2, d 2048, ff 1024, two experts in all 83, 84, 107, 107; E 16, top-4, d 2048,
 // ff 1024, 1024 rows 120, 119, 119, 112.)  A tile of up to FEW pairs joins at any number: it adds a pass's step to a full one's, no decode (E 16, top-8,
 // d 3584, ff 384, 325 rows - about 162 pairs an expert - with FEW 32, 48, 64: 149, 138, 138).
