@@ -186,22 +186,22 @@ def test_latent_attention_of_more_rows_than_the_chip_has_workgroups(be, oracle, 
     else:
         cache, kvf = dict(k=packs.f32_to_bf16_bits(kr), v=packs.f32_to_bf16_bits(lat)), be.KV_BF16
     o = be.kt_mla_attn(H, r, rope, kvf, ql, qr, cache, pos, kv0, scale, 128, 32)
-    for t in sorted({0, 1, T // 2, T - 2, T - 1, *range(2, T, 7)}):
+    for t in sorted({0, 1, T // 2, T - 2, T - 1, *range(2, T, 23)}):
         for h in (0, H - 1):
             want = oracle.mla_attn(ql[t, h], qr[t, h], lat[kv0[t]:], kr[kv0[t]:], pos[t], scale)
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
 
 
-# first splits of every row, and the further ones of the long row, with 256 CUs: 8 and 16 (32 rows), 3 and the one that is left of four (70), one and up to 23 (300), up to 7 (520: the
-# long row past the first 512), one and 15 for either of two groups of heads (90 rows of 20), seven and as many as the keys make (33); a row without positions among them
+# first splits of every row, and the further ones of the long row, with 256 CUs: 8 and 9 (32 rows), 3 and the one that is left of four (70), one and 5 (300; 520: the long
+# row past the first 512; 90 rows of 20 heads: for either of two groups), 7 and 8 (33); a row without positions among them
 @pytest.mark.parametrize("fmt", ["fp8", "bf16"])
-@pytest.mark.parametrize("T,H,ns,short,chunk", [(32, 16, 32, 200, 128), (70, 16, 4, 300, 128), (300, 16, 32, 150, 128), (520, 16, 8, 120, 128), (90, 20, 16, 600, 128),
-                                                (33, 16, 256, 140, 300)])
-def test_latent_attention_of_a_long_row_among_short_ones(be, oracle, fmt, T, H, ns, short, chunk):
+@pytest.mark.parametrize("T,H,ns,short,keys,chunk", [(32, 16, 32, 200, 8500, 128), (70, 16, 4, 300, 3300, 128), (300, 16, 32, 150, 3000, 128), (520, 16, 8, 120, 3000, 128),
+                                                     (90, 20, 16, 600, 3000, 128), (33, 16, 256, 140, 7500, 300)])
+def test_latent_attention_of_a_long_row_among_short_ones(be, oracle, fmt, T, H, ns, short, keys, chunk):
     rng = np.random.default_rng(T + H)
-    r, rope, NP, long = 512, 64, 12100, T - 5
+    r, rope, NP, long = 512, 64, keys + 60, T - 5
     pos = [int(p) for p in rng.integers(0, short, T)]
-    pos[long], pos[3], pos[T - 1] = 11999, -1, 0
+    pos[long], pos[3], pos[T - 1] = keys - 1, -1, 0
     kv0 = [int(rng.integers(0, NP - p)) for p in pos]
     ql = packs.round_bf16((rng.standard_normal((T, H, r)) * 0.3).astype(np.float32))
     qr = packs.round_bf16(rng.standard_normal((T, H, rope)).astype(np.float32))
@@ -216,7 +216,7 @@ def test_latent_attention_of_a_long_row_among_short_ones(be, oracle, fmt, T, H, 
         cache, kvf = dict(k=packs.f32_to_bf16_bits(kr), v=packs.f32_to_bf16_bits(lat)), be.KV_BF16
     o = be.kt_mla_attn(H, r, rope, kvf, ql, qr, cache, pos, kv0, scale, chunk, ns)
     assert np.isnan(o[3]).all()
-    for t in sorted({0, 1, 2, 4, 64 % T, long - 1, long, long + 1, T - 1, *range(5, T, 11)}):
+    for t in sorted({0, 1, 2, 4, 64 % T, long - 1, long, long + 1, T - 1, *range(5, T, 29)}):
         for h in (0, H - 1):
             want = oracle.mla_attn(ql[t, h], qr[t, h], lat[kv0[t]:], kr[kv0[t]:], pos[t], scale)
             assert np.all(close_bf(o[t, h], want.astype(np.float64), 2e-6)), (t, h)
